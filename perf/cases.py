@@ -1,0 +1,584 @@
+"""The work a user of this framework has it do, as measurable cases.
+
+A case names an operation, a model of `galic_amd.model.CONFIGS` (the
+configurations of this repository's tests and benchmark) and sizes.  The
+operations are the public calls of `galic_amd.runtime`:
+
+  iterate  fp32_iterate: reps of the batched FP32 path, trials drawn on the device
+  initial  the initial response pass, FP32 or plain FP64 path
+  rep      one rep of the plain FP64 path with the caller's trial velocities
+  orbits   responses of independent orbits returned to the caller, FP64 or FP32
+  field    table lookups at points
+  forces   Barnes-Hut forces at points
+  fill     a Barnes-Hut fill of the force tables from the caller's sources
+  retab    the in-place re-tabulation from the context's sources
+  targets  sampled density and dispersion targets of one component
+
+`nref` is the particle number whose merit cuts the model has: a realisation of
+n particles with the bin limits scaled by n / nref is judged on the nodes of the
+model of nref particles.
+"""
+import math
+
+import numpy as np
+import torch
+
+from galic_amd import model
+from galic_amd.runtime import GalicGPU, tree_fill, tree_forces
+
+F_STEP = 376       # operations of one leapfrog step with its lookups and binning
+F_INTERACTION = 21  # operations of one monopole interaction
+F_QUAD = 56         # ... with the quadrupole term
+F_POINT = 200       # operations of one sampled target point
+
+
+def listed():
+    return [
+        # one small rep of the plain method's model: a user tuning a halo interactively, launch latency
+        dict(name="rep32-small", op="iterate", model="halo-1e5", level=6, fg=128, n=10000, nref=100000, trials=200,
+             rep=200, k=1),
+        # odd sizes on an intermediate grid: a last rep that is not full, K = 3
+        dict(name="iterate32-odd", op="iterate", model="halo-disk-1e6", level=7, fg=256, n=30011, nref=1000000,
+             trials=3333, rep=1250, k=3),
+        # the batching configuration: halo, disk and bulge on 64^2 grids, reps of 1e4 with 8 trials each
+        dict(name="iterate32-batch", op="iterate", model="composite-4e6", level=6, fg=256, n=60000, nref=4000000,
+             trials=30000, rep=10000, k=8),
+        # the full model's reps: 512^2 tables and grids, 8 trials per particle, the cuts of 2e7 particles
+        dict(name="iterate32-full", op="iterate", model="composite-2e7", level=9, fg=512, n=60000, nref=20000000,
+             trials=15000, rep=5000, k=8),
+        # the initial pass of the full model
+        dict(name="initial32-full", op="initial", precision=32, model="composite-2e7", level=9, fg=512, n=100003,
+             nref=20000000),
+        # the initial pass of the plain path, the precision form's model
+        dict(name="initial64", op="initial", precision=64, model="halo-disk-1e6", level=6, fg=256, n=20011,
+             nref=1000000),
+        # a rep of the plain path: one fresh trial per particle
+        dict(name="rep64", op="rep", model="halo-disk-1e6", level=6, fg=256, n=12000, nref=1000000, trials=3000),
+        # a batch of single orbits with their response grids returned, as a caller of the reference's
+        # produce_orbit_response_field_mod has
+        dict(name="orbits64", op="orbits", precision=64, model="composite-4e6", level=6, fg=256, n=20000, nref=4000000,
+             orbits=64),
+        # lookups at the positions of a small set of particles: the shortest call
+        dict(name="field-1000", op="field", model="composite-4e6", level=6, fg=256, n=20000, nref=4000000, points=1000),
+        # the reference's own table fill: FP64, monopole, spline softening, 128^2 tables
+        dict(name="fill64", op="fill", model="composite-4e6", fg=128, sources=200000, mode=0),
+        # the force-field configuration's re-tabulation, once an iteration: FP32 group walk, quadrupole moments,
+        # Plummer softening, 512^2 tables
+        dict(name="retab-full", op="retab", model="composite-2e7", level=9, fg=512, n=4000, nref=20000000,
+             sources=10000000, mode=15),
+        # dispersion and density targets of the halo on 64^2 grids
+        dict(name="targets-halo", op="targets", model="composite-4e6", level=6, fg=256, n=4000, nref=4000000, type=1,
+             points=10000000),
+    ]
+
+
+def _log(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    op = rng.choice(["iterate", "iterate", "iterate", "initial", "initial", "rep", "orbits", "field", "forces", "fill",
+                     "retab", "targets"])
+    if op in ("forces", "fill"):
+        c = dict(op=op, model=rng.choice(["composite-4e6", "halo-disk-1e6"]), fg=rng.choice([64, 100, 128]),
+                 sources=_log(rng, 1000, 200000), mode=rng.choice([0, 1, 2, 7, 15]))
+        if op == "forces":
+            c["targets"] = _log(rng, 1, 50000)
+        return c
+    name, level, fg, nref = rng.choice([("halo-1e5", 6, 128, 100000), ("halo-disk-1e6", 6, 256, 1000000),
+                                        ("halo-disk-1e6", 7, 256, 1000000), ("composite-4e6", 6, 256, 4000000),
+                                        ("composite-4e6", 8, 256, 4000000), ("composite-2e7", 9, 512, 20000000)])
+    c = dict(op=op, model=name, level=level, fg=fg, nref=nref, n=_log(rng, 2000, 60000))
+    big = 1 if level <= 7 else 3
+    if op == "iterate":
+        c["trials"] = min(c["n"], _log(rng, 50, 30000 // big))
+        c["rep"] = _log(rng, max(1, c["trials"] // 6), c["trials"])
+        c["k"] = rng.choice([1, 2, 4, 5, 8, 8, 12]) if level <= 7 else rng.choice([1, 4, 8, 8])
+    elif op == "initial":
+        c["precision"] = rng.choice([32, 32, 64])
+        if c["precision"] == 64:
+            c["n"] = min(c["n"], 20000 // big)
+    elif op == "rep":
+        c["trials"] = _log(rng, 50, min(c["n"], 3000) // big)
+    elif op == "orbits":
+        c["precision"] = rng.choice([32, 64])
+        c["orbits"] = _log(rng, 1, 100 if level <= 7 else 8)
+    elif op == "field":
+        c["points"] = min(c["n"], _log(rng, 1, 60000))
+    elif op == "retab":
+        c["n"], c["mode"] = 4000, rng.choice([7, 15, 15])
+        c["sources"] = _log(rng, 10000, 2000000 if c["mode"] == 7 else 10000000)
+    elif op == "targets":
+        c["n"] = 4000
+        c["type"] = rng.choice([1, 2, 3]) if "composite" in name else rng.choice([1, 2]) if "disk" in name else 1
+        c["points"] = _log(rng, 10000, 10000000)
+    return c
+
+
+# ------------------------------------------------------------------- inputs --
+
+def _workload(case, seed):
+    share = case["n"] / case["nref"]
+    cfg = model.config(case["model"], level=case["level"], fg_nbin=case["fg"], min_per_bin_density=50 * share,
+                       min_per_bin_disp=100 * share, halo_in_table=case["op"] == "retab")
+    return cfg, model.make_workload(cfg, n=case["n"], target_samples=1000, seed=1 + seed % 1000000007)
+
+
+def _context(case, seed, targets=True):
+    """A context with the model's particles, tables and (device-sampled) targets."""
+    cfg, w = _workload(case, seed)
+    g = GalicGPU(w)
+    if targets:
+        for t in w.types:
+            beta, tabs = model.disp_tables(w.params, cfg, t)
+            g.set_disp_tables(t, beta, **tabs)
+            eg = g.sample_targets(t, 1000000, seed=1 + seed % 1000003, stream=400 + t, density=False)[1]
+            g.set_targets(t, [w.targets[t][0]] + [eg[f] for f in range(5)])
+    return cfg, w, g
+
+
+def _params(case):
+    return model.make_params(model.config(case["model"], fg_nbin=case["fg"]))
+
+
+def _sources(p, n, seed):
+    """The model's mass as n sampled points: the halo, a fifth of the points for a disk, a twentieth for a bulge."""
+    nd = n // 5 if p.Disk_Mass > 0 else 0
+    nb = n // 20 if p.Bulge_Mass > 0 else 0
+    ids = np.arange(n, dtype=np.uint64)
+    parts = [(1, p.Halo_Mass, ids[:n - nd - nb]), (2, p.Disk_Mass, ids[n - nd - nb:n - nb]), (3, p.Bulge_Mass, ids[n - nb:])]
+    parts = [(t, m, i) for t, m, i in parts if len(i)]
+    pos = np.concatenate([model.sample_type(p, t, seed, 10 + t, i) for t, m, i in parts])
+    mass = np.concatenate([np.full(len(i), m / len(i)) for t, m, i in parts])
+    return np.ascontiguousarray(pos), mass
+
+
+def _fill_sources(case, seed):
+    p = _params(case)
+    pos, mass = _sources(p, case["sources"], 1 + seed % 1000003)
+    return p, pos, mass
+
+
+def _points(p, n, seed):
+    return _sources(p, max(n, 40), 7 + seed % 1000003)[0][-n:].copy()
+
+
+def prepare(case, seed):
+    op = case["op"]
+    if op in ("fill", "forces"):
+        p, pos, mass = _fill_sources(case, seed)
+        s = dict(op=op, p=p, pos=pos, mass=mass, mode=case["mode"])
+        if op == "forces":
+            s["tpos"] = _points(p, case["targets"], seed)
+        return s
+    if op == "field":
+        cfg, w = _workload(case, seed)
+        return dict(op=op, g=GalicGPU(w), pos=np.ascontiguousarray(w.pos[model.permutation(w, seed)[:case["points"]]]))
+    if op == "retab":
+        cfg, w = _workload(case, seed)
+        n = case["sources"]
+        nd = n // 5 if w.params.Disk_Mass > 0 else 0
+        nb = n // 20 if w.params.Bulge_Mass > 0 else 0
+        w.params.SampleForceNhalo, w.params.SampleForceNdisk, w.params.SampleForceNbulge = n - nd - nb, nd, nb
+        g = GalicGPU(w)
+        g.sample_tree_sources(3 + seed % 1000003)
+        return dict(op=op, g=g, mode=case["mode"])
+    if op == "targets":
+        cfg, w = _workload(case, seed)
+        g = GalicGPU(w)
+        beta, tabs = model.disp_tables(w.params, cfg, case["type"])
+        g.set_disp_tables(case["type"], beta, **tabs)
+        return dict(op=op, g=g, type=case["type"], points=case["points"], seed=5 + seed % 1000003)
+    if op == "orbits":
+        cfg, w = _workload(case, seed)
+        i = model.permutation(w, seed)[:case["orbits"]]
+        return dict(op=op, g=GalicGPU(w), precision=case["precision"],
+                    args=[np.ascontiguousarray(a[i]) for a in (w.pos, w.vel, w.mass, w.tint, w.ptype)])
+    cfg, w, g = _context(case, seed)
+    s = dict(op=op, g=g, types=w.types, perm=model.permutation(w, 1 + seed % 1000003), at=0, passes=0, seed=seed % 1000003)
+    if op == "initial":
+        s["precision"] = case["precision"]
+    elif op == "iterate":
+        g.fp32_calc_all_response_fields()
+        g.fp32_set_fresh_trials(1)
+        s.update(trials=case["trials"], rep=case["rep"], k=case["k"])
+    else:
+        g.calc_all_response_fields()
+        m = case["trials"]
+        starts = range(0, max(1, min(w.n // m, 4)) * m, m)
+        s["slices"] = [(s["perm"][a:a + m], model.trial_velocities(w, s["perm"][a:a + m], 5 + seed % 1000003, r))
+                       for r, a in enumerate(starts)]
+    return s
+
+
+# --------------------------------------------------------------------- run --
+
+def _state(g, types):
+    vel, orbits, v2 = g.particles()
+    return dict(vel=vel, orbits=orbits, v2=v2, fit=[g.fit(t) for t in types])
+
+
+def run(s):
+    op = s["op"]
+    if op == "fill":
+        pot, dr, dz, nint = tree_fill(s["p"], s["pos"], s["mass"], precision=s["mode"])
+        return dict(pot=pot, dpotdr=dr, dpotdz=dz, interactions=nint)
+    if op == "forces":
+        acc, pot, nint = tree_forces(s["p"], s["pos"], s["mass"], s["tpos"], precision=s["mode"])
+        return dict(acc=acc, pot=pot, interactions=nint)
+    g = s["g"]
+    if op == "field":
+        acc, pot = g.field_at(s["pos"])
+        return dict(acc=acc, pot=pot)
+    if op == "retab":
+        nint = g.retabulate(s["mode"])
+        pot, dr, dz = g.force_tables()
+        return dict(pot=pot, dpotdr=dr, dpotdz=dz, interactions=nint)
+    if op == "targets":
+        dg, eg, binned, _ = g.sample_targets(s["type"], s["points"], seed=s["seed"])
+        return dict(dg=dg, eg=eg, binned=binned)
+    if op == "orbits":
+        return g.orbit_responses(*s["args"], precision=s["precision"])
+    if op == "initial":
+        if s["precision"] == 32:
+            g.fp32_calc_all_response_fields()
+        else:
+            g.calc_all_response_fields()
+        return dict(stacks=[[g.stack(t, k) for k in (0, 6, 7, 8, 9)] for t in s["types"]], fit=[g.fit(t) for t in s["types"]])
+    if op == "iterate":
+        # the next particles of the permutation, as an iteration walks it
+        m = s["trials"]
+        if s["at"] + m > len(s["perm"]):
+            s["at"] = 0
+        idx = s["perm"][s["at"]:s["at"] + m]
+        s["at"] += m
+        s["passes"] += 1
+        accept = g.fp32_iterate(idx, k=s["k"], rep_size=s["rep"], sigma_frac=0.1, seed=1000 * s["seed"] + s["passes"])
+        return dict(accept=accept, merits=g.fp32_trial_merits(m, s["k"]), **_state(g, s["types"]))
+    idx, vtry = s["slices"][s["passes"] % len(s["slices"])]
+    s["passes"] += 1
+    accept, dF = g.rep(idx, vtry)
+    return dict(accept=accept, dF=dF, **_state(g, s["types"]))
+
+
+# -------------------------------------------------------------------- work --
+
+# leapfrog steps of an orbit on grids of a level , measured: the cell-crossing limit sets in above 128^2 cells
+STEPS = {6: 3.5e3, 7: 3.6e3, 8: 5.2e3, 9: 1.03e4}
+
+
+def work(case):
+    op = case["op"]
+    if op in ("fill", "forces"):
+        n, m = case["sources"], case.get("targets") or 8 * case["fg"] ** 2
+        out = 4 * 8 * m if op == "forces" else 3 * 8 * case["fg"] ** 2
+        each = F_QUAD if case["mode"] & 2 else F_INTERACTION
+        # about 700 interactions of a target per decade of sources above 10, at theta = 0.4
+        return dict(bytes=32 * n + (24 * m if op == "forces" else 0) + out,
+                    flops=each * m * min(n, 700 * max(1.0, math.log10(n) - 1)))
+    tables = 24 * case["fg"] ** 2
+    if op == "field":
+        return dict(bytes=tables + 56 * case["points"], flops=100 * case["points"])
+    if op == "retab":
+        n, m = case["sources"], 8 * case["fg"] ** 2
+        return dict(bytes=32 * n + tables, flops=F_QUAD * m * 700 * max(1.0, math.log10(n) - 1))
+    if op == "targets":
+        return dict(bytes=6 * 8 * 4 ** case["level"], flops=F_POINT * case["points"])
+    grid = 5 * 8 * 4 ** case["level"]
+    if op == "orbits":
+        return dict(bytes=tables + (grid + 64) * case["orbits"], flops=F_STEP * STEPS[case["level"]] * case["orbits"])
+    if op == "initial":
+        return dict(bytes=tables + 100 * case["n"] + 3 * grid, flops=F_STEP * STEPS[case["level"]] * case["n"])
+    k = case.get("k", 1)
+    reps = -(-case["trials"] // case.get("rep", case["trials"]))
+    return dict(bytes=tables + 200 * case["trials"] + 60 * case["n"] + 6 * grid * reps,
+                flops=F_STEP * STEPS[case["level"]] * case["trials"] * (k + 1))
+
+
+# ------------------------------------------------------------ 64-bit values --
+# Written from the formulas, in torch and numpy.
+
+def _dev():
+    return torch.device("cuda" if torch.cuda.is_available() else "cpu")
+
+
+def _t(a):
+    return torch.as_tensor(np.ascontiguousarray(a), device=_dev())
+
+
+class _Field:
+    """Tabulated axisymmetric field plus the analytic halo and bulge."""
+
+    def __init__(self, w):
+        p = self.p = w.params
+        self.nb, self.lf = p.FG_Nbin, math.log(p.FG_Fac)
+        self.pot, self.dr, self.dz = _t(w.pot), _t(w.dpotdr), _t(w.dpotdz)
+        self.vstream = {t: _t(w.vstream[t]) for t in (1, 2, 3)}
+        self.table = p.Disk_Mass > 0 or p.SampleForceNhalo > 0
+
+    def index(self, R, z):
+        f = lambda v: torch.log(v / self.p.FG_Rmin + 1) / self.lf  # noqa: E731
+        return f(R), f(z.abs())
+
+    def bilinear(self, T, j, i, fj, fi):
+        o = i * self.nb + j
+        return (T[o] * (1 - fi) * (1 - fj) + T[o + 1] * (1 - fi) * fj + T[o + self.nb] * fi * (1 - fj) +
+                T[o + self.nb + 1] * fi * fj)
+
+    def clamped(self, jd, idx):
+        j, i = jd.clamp(max=self.nb - 2).long(), idx.clamp(max=self.nb - 2).long()
+        return j, i, (jd - j).clamp(max=1.0), (idx - i).clamp(max=1.0)
+
+    def at(self, x, y, z, want_pot=False):
+        p, R, r = self.p, torch.sqrt(x * x + y * y), torch.sqrt(x * x + y * y + z * z)
+        jd, idx = self.index(R, z)
+        c, s = torch.where(R > 0, x / R, torch.ones_like(x)), torch.where(R > 0, y / R, torch.zeros_like(x))
+        halo = p.G * p.Halo_Mass / ((r + 1e-6 * p.Halo_A) * (r + p.Halo_A) ** 2)
+        ax, ay, az, pot = (torch.zeros_like(x) for _ in range(4))
+        if self.table:
+            on = (jd < self.nb - 1) & (idx < self.nb - 1)
+            q = self.clamped(jd, idx)
+            aR, aZ = self.bilinear(self.dr, *q), self.bilinear(self.dz, *q) * torch.where(z < 0, -1.0, 1.0)
+            off = -halo * p.M200 / p.Halo_Mass
+            ax, ay, az = torch.where(on, aR * c, off * x), torch.where(on, aR * s, off * y), torch.where(on, aZ, off * z)
+            if want_pot:
+                pot = torch.where(on, self.bilinear(self.pot, *q), -p.G * p.M200 / (r + p.Halo_A))
+        f = torch.zeros_like(x)
+        if p.SampleForceNhalo == 0:
+            f = f + halo
+            pot = pot - p.G * p.Halo_Mass / (r + p.Halo_A)
+        if p.Bulge_Mass > 0:
+            f = f + p.G * p.Bulge_Mass / ((r + 1e-6 * p.Bulge_A) * (r + p.Bulge_A) ** 2)
+            pot = pot - p.G * p.Bulge_Mass / (r + p.Bulge_A)
+        return ax - f * x, ay - f * y, az - f * z, pot, jd, idx
+
+
+def _cells(x, y, z, rmin, fac, nb):
+    def one(v):
+        b = (torch.log(v / rmin + 1) / math.log(fac) - 0.5).clamp(min=0.0)
+        i = b.long().clamp(max=nb - 2)
+        return i, (b - i).clamp(max=1.0)
+    (iR, fR), (iz, fz) = one(torch.sqrt(x * x + y * y)), one(z.abs())
+    return iR, iz, fR, fz
+
+
+def _orbits(w, pos, vel, mass, tint, ptype, shared=False):
+    """Orbit-averaged responses by the leapfrog: per orbit, or summed by type (shared), and the orbits' end values."""
+    p, F, n = w.params, _Field(w), len(mass)
+    nb = 1 << p.DG_MaxLevel
+    edge = p.DG_Rmin * (p.DG_Fac ** torch.arange(nb + 1, dtype=torch.float64, device=_dev()) - 1)
+    width = edge[1:] - edge[:-1]
+    (x, y, z), (vx, vy, vz) = _t(pos).T.contiguous(), _t(vel).T.contiguous()
+    m, T, ty = _t(mass), _t(tint), _t(ptype).long()
+    cyl = torch.tensor([p.TypeOfVelocityStructure[t] == 2 for t in range(4)], device=_dev())
+    who = torch.arange(n, device=_dev())
+    out = torch.zeros((4 if shared else n) * 5 * nb * nb, dtype=torch.float64, device=_dev())
+    ends = dict(t=torch.zeros(n, dtype=torch.float64, device=_dev()), e0=None, e1=torch.zeros(n, dtype=torch.float64, device=_dev()))
+    t = torch.zeros_like(T)
+
+    streaming = [k for k in (1, 2, 3) if p.NType[k] > 0 and np.any(w.vstream[k])]
+
+    def look(want_pot=False):
+        ax, ay, az, pot, jd, idx = F.at(x, y, z, want_pot)
+        q, vstr = F.clamped(jd, idx), torch.zeros_like(x)
+        for k in streaming:
+            vstr = torch.where(ty == k, F.bilinear(F.vstream[k], *q), vstr)
+        return ax, ay, az, pot, _cells(x, y, z, p.DG_Rmin, p.DG_Fac, nb), vstr
+
+    def moments(vstr):
+        R2, r2, vR = x * x + y * y, x * x + y * y + z * z, vx * x + vy * y
+        vq = (vy * x - vx * y) / torch.sqrt(R2)
+        c = cyl[ty]
+        vr2 = torch.where(c, vR ** 2 / R2, (vR + vz * z) ** 2 / r2)
+        vt2 = torch.where(c, vz ** 2, (R2 * vz - z * vR) ** 2 / (R2 * r2))
+        return torch.stack([torch.ones_like(vq), vr2, vt2, vq ** 2, (vq - vstr) ** 2])
+
+    def bin_(cell, mom, dt):
+        iR, iz, fR, fz = cell
+        h = 0.5 * dt * m / T
+        base = (ty if shared else who) * (5 * nb * nb) + iz * nb + iR
+        field = (torch.arange(5, device=_dev()) * nb * nb)[:, None]
+        for wt, d in (((1 - fR) * (1 - fz), 0), (fR * (1 - fz), 1), ((1 - fR) * fz, nb), (fR * fz, nb + 1)):
+            out.index_add_(0, (base + d + field).reshape(-1), (h * wt * mom).reshape(-1))
+
+    ax, ay, az, pot, cell, vstr = look(True)
+    ends["e0"] = 0.5 * (vx ** 2 + vy ** 2 + vz ** 2) + pot
+    mom = moments(vstr)
+    while len(m):
+        v, a = torch.sqrt(vx ** 2 + vy ** 2 + vz ** 2), torch.sqrt(ax ** 2 + ay ** 2 + az ** 2)
+        dt = torch.minimum(p.TimeStepFactorOrbit * (p.V200 / a),
+                           p.TimeStepFactorCellCross * (width[torch.maximum(cell[0], cell[1])] / v))
+        fin = T < dt + t
+        dt = torch.where(fin, T - t, dt)
+        bin_(cell, mom, dt)
+        vx, vy, vz = vx + 0.5 * dt * ax, vy + 0.5 * dt * ay, vz + 0.5 * dt * az
+        x, y, z = x + dt * vx, y + dt * vy, z + dt * vz
+        ax, ay, az, _, cell, vstr = look()
+        vx, vy, vz = vx + 0.5 * dt * ax, vy + 0.5 * dt * ay, vz + 0.5 * dt * az
+        mom = moments(vstr)
+        bin_(cell, mom, dt)
+        t = t + dt
+        done = torch.nonzero(fin).reshape(-1)
+        if len(done):
+            pot = F.at(x, y, z, True)[3]  # (of the finished orbits' end points)
+            ends["t"][who[done]] = t[done]
+            ends["e1"][who[done]] = (0.5 * (vx ** 2 + vy ** 2 + vz ** 2) + pot)[done]
+            k = torch.nonzero(~fin).reshape(-1)
+            x, y, z, vx, vy, vz, ax, ay, az, m, T, ty, t, who = (
+                q[k] for q in (x, y, z, vx, vy, vz, ax, ay, az, m, T, ty, t, who))
+            cell, mom = tuple(q[k] for q in cell), mom[:, k]
+    return out, ends
+
+
+def _smooth(fine):
+    """The quadtree stack of a square map, coarsest level first."""
+    levels = [fine]
+    while levels[0].shape[0] > 1:
+        f = levels[0]
+        levels.insert(0, f[0::2, 0::2] + f[1::2, 0::2] + f[0::2, 1::2] + f[1::2, 1::2])
+    return torch.cat([lv.reshape(-1) for lv in levels])
+
+
+def _direct(p, pos, mass, tpos, plummer):
+    """Softened direct summation: accelerations and potentials at tpos."""
+    h, src, ms = p.ForceSoftening, _t(pos), _t(mass)
+    acc, pot = [], []
+    for tp in torch.split(_t(tpos), max(1, 40000000 // len(mass))):
+        d = [src[None, :, k] - tp[:, None, k] for k in range(3)]
+        r2 = d[0] ** 2 + d[1] ** 2 + d[2] ** 2
+        if plummer:
+            inv = (r2 + (h / 2.8) ** 2).rsqrt()
+            fac, wp = ms * inv ** 3, -ms * inv
+        else:
+            r = torch.sqrt(r2)
+            u = (r / h).clamp(max=1.0)
+            near, uu = u < 0.5, u.clamp(min=0.5)
+            fin = torch.where(near, 10.666666666667 + u * u * (32.0 * u - 38.4),
+                              21.333333333333 - 48.0 * uu + 38.4 * uu ** 2 - 10.666666666667 * uu ** 3 -
+                              0.066666666667 / uu ** 3)
+            win = torch.where(near, -2.8 + u * u * (5.333333333333 + u * u * (6.4 * u - 9.6)),
+                              -3.2 + 0.066666666667 / uu +
+                              uu * uu * (10.666666666667 + uu * (-16.0 + uu * (9.6 - 2.133333333333 * uu))))
+            fac = torch.where(r >= h, ms / (r2 * r), ms / h ** 3 * fin)
+            wp = torch.where(r >= h, -ms / r, ms / h * win)
+        acc.append(torch.stack([(fac * q).sum(1) for q in d], 1) * p.G)
+        pot.append(wp.sum(1) * p.G)
+    return torch.cat(acc), torch.cat(pot)
+
+
+def _mul(a, c):
+    """High and low words of the products of 32-bit values held in int64."""
+    lo, hi = (a & 0xFFFF) * c, (a >> 16) * c
+    low = (lo + ((hi & 0xFFFF) << 16))
+    return ((hi >> 16) + (low >> 32)) & 0xFFFFFFFF, low & 0xFFFFFFFF
+
+
+def _philox(ids, attempt, block, k0, k1):
+    """Philox4x32-10 (Salmon et al., SC 2011) of the counters (id, attempt, block) under the key (k0, k1)."""
+    c = [ids & 0xFFFFFFFF, ids >> 32, torch.full_like(ids, attempt), torch.full_like(ids, block)]
+    for _ in range(10):
+        h0, l0 = _mul(c[0], 0xD2511F53)
+        h1, l1 = _mul(c[2], 0xCD9E8D57)
+        c = [h1 ^ c[1] ^ k0, l1, h0 ^ c[3] ^ k1, l0]
+        k0, k1 = (k0 + 0x9E3779B9) & 0xFFFFFFFF, (k1 + 0xBB67AE85) & 0xFFFFFFFF
+    return c
+
+
+def _uniform(ids, attempt, k0, k1):
+    u = []
+    for block in (0, 1):
+        c = _philox(ids, attempt, block, k0, k1)
+        for a, b in ((c[0], c[1]), (c[2], c[3])):
+            u.append(((a >> 5).double() * 67108864.0 + (b >> 6).double() + 0.5) / 9007199254740992.0)
+    return u
+
+
+def _component_points(p, kind, n, seed, stream):
+    out, todo = torch.zeros((n, 3), dtype=torch.float64, device=_dev()), torch.arange(n, device=_dev())
+    attempt = 0
+    while len(todo):
+        u = _uniform(todo, attempt, seed, stream)
+        phi = u[2 if kind == 2 else 1] * 2 * math.pi
+        if kind == 2:
+            z, R = p.Disk_Z0 / 2 * torch.log(u[0] / (1 - u[0])), torch.ones_like(phi)
+            for _ in range(60):
+                R = R + ((1 + R) * torch.exp(-R) + u[1] - 1) / (R * torch.exp(-R))
+            R = R * p.Disk_H
+        else:
+            a = p.Halo_A if kind == 1 else p.Bulge_A
+            r = a * (u[0] + torch.sqrt(u[0])) / (1 - u[0])
+            c = u[2] * 2 - 1
+            R, z = r * torch.sqrt(1 - c * c), r * c
+        ok = torch.sqrt(R * R + z * z) <= p.Rmax
+        out[todo[ok]] = torch.stack([R * torch.cos(phi), R * torch.sin(phi), z], 1)[ok]
+        todo, attempt = todo[~ok], attempt + 1
+    return out
+
+
+def _targets(case, seed):
+    cfg, w = _workload(case, seed)
+    p, kind, nb = w.params, case["type"], 1 << case["level"]
+    beta, tabs = model.disp_tables(p, cfg, kind)
+    pos = _component_points(p, kind, case["points"], 5 + seed % 1000003, 100 + kind)
+    x, y, z = pos[torch.sqrt(pos[:, 0] ** 2 + pos[:, 2] ** 2) < p.Rmax].T.contiguous()
+    F, tovs = _Field(w), p.TypeOfVelocityStructure[kind]
+    if tovs <= 1:
+        b = torch.log(torch.sqrt(x * x + y * y + z * z) / p.FG_Rmin + 1) / F.lf
+        i = b.long().clamp(max=F.nb - 2)
+        f, D = (b - i).clamp(max=1.0), _t(tabs["disp_r"])
+        d0 = D[i] * (1 - f) + D[i + 1] * f
+        d = [d0] + [d0 * (1 - beta if tovs == 1 else 1.0)] * 3
+    else:
+        q = F.clamped(*F.index(torch.sqrt(x * x + y * y), z))
+        names = ("disp_z", "disp_z") if tovs == 2 else ("tilt_r", "tilt_theta")
+        d = [F.bilinear(_t(tabs[k]), *q) for k in names + ("disp_phi",)]
+        d.append(d[2] + F.bilinear(F.vstream[kind], *q) ** 2)
+
+    def cic(rmin, fac, val):
+        iR, iz, fR, fz = _cells(x, y, z, rmin, fac, nb)
+        m = torch.zeros(nb * nb, dtype=torch.float64, device=_dev())
+        for wt, k in (((1 - fR) * (1 - fz), 0), (fR * (1 - fz), 1), ((1 - fR) * fz, nb), (fR * fz, nb + 1)):
+            m.index_add_(0, iz * nb + iR + k, wt * val)
+        return _smooth((m * (p.MType[kind] / len(x))).reshape(nb, nb))
+
+    one = torch.ones_like(x)
+    return dict(dg=cic(p.DG_Rmin, p.DG_Fac, one), eg=torch.stack([cic(p.EG_Rmin, p.EG_Fac, v) for v in [one] + d]),
+                binned=None)
+
+
+def exact(case, seed):
+    op = case["op"]
+    if op == "field":
+        cfg, w = _workload(case, seed)
+        pos = w.pos[model.permutation(w, seed)[:case["points"]]]
+        ax, ay, az, pot, _, _ = _Field(w).at(*_t(pos).T, want_pot=True)
+        return dict(acc=torch.stack([ax, ay, az], 1), pot=pot)
+    if op in ("forces", "fill"):
+        # the tree's answer is within its opening angle's error of the sum over all sources
+        p, pos, mass = _fill_sources(case, seed)
+        if op == "forces":
+            acc, pot = _direct(p, pos, mass, _points(p, case["targets"], seed), bool(case["mode"] & 4))
+            return dict(acc=acc, pot=pot, interactions=None)
+        node = p.FG_Rmin * (p.FG_Fac ** np.arange(p.FG_Nbin) - 1.0)
+        z, R = (a.ravel() for a in np.meshgrid(node, node, indexing="ij"))
+        tot = [0.0, 0.0, 0.0]
+        for s in range(8):
+            c, sn = math.cos(2 * math.pi / 8 * s), math.sin(2 * math.pi / 8 * s)
+            acc, pot = _direct(p, pos, mass, np.stack([R * c, R * sn, z], 1), bool(case["mode"] & 4))
+            tot = [tot[0] + pot / 8, tot[1] + (acc[:, 0] * c + acc[:, 1] * sn) / 8, tot[2] + acc[:, 2] / 8]
+        return dict(pot=tot[0], dpotdr=tot[1], dpotdz=tot[2], interactions=None)
+    if op == "targets":
+        return _targets(case, seed)
+    if op == "orbits" and case["level"] <= 7:
+        cfg, w = _workload(case, seed)
+        i = model.permutation(w, seed)[:case["orbits"]]
+        out, ends = _orbits(w, *(a[i] for a in (w.pos, w.vel, w.mass, w.tint, w.ptype)))
+        return dict(fields=out.reshape(len(i), 5, -1), t=ends["t"], orbits=None, steps=None, e0=ends["e0"], e1=ends["e1"])
+    if op == "initial" and case["level"] <= 6:
+        cfg, w = _workload(case, seed)
+        out, _ = _orbits(w, w.pos, w.vel, w.mass, w.tint, w.ptype, shared=True)
+        nb = 1 << case["level"]
+        grids = out.reshape(4, 5, nb, nb)
+        # the stacks in run()'s order: mass, then the r, t, q and p moments
+        return dict(stacks=[[_smooth(grids[t][f]) for f in range(5)] for t in w.types], fit=[None] * len(w.types))
+    return None  # the trials' choices branch on differences of a rounding: no value in 64 bits to hold them to
