@@ -45,7 +45,7 @@ def listed():
              trials=30000, rep=10000, k=8),
         # the full model's reps: 512^2 tables and grids, 8 trials per particle, the cuts of 2e7 particles
         dict(name="iterate32-full", op="iterate", model="composite-2e7", level=9, fg=512, n=60000, nref=20000000,
-             trials=15000, rep=5000, k=8),
+             trials=9000, rep=3000, k=8),
         # the initial pass of the full model
         dict(name="initial32-full", op="initial", precision=32, model="composite-2e7", level=9, fg=512, n=100003,
              nref=20000000),
@@ -91,7 +91,7 @@ def draw(rng):
     c = dict(op=op, model=name, level=level, fg=fg, nref=nref, n=_log(rng, 2000, 60000))
     big = 1 if level <= 7 else 3
     if op == "iterate":
-        c["trials"] = min(c["n"], _log(rng, 50, 30000 // big))
+        c["trials"] = min(c["n"], _log(rng, 50, 27000 // big))
         c["rep"] = _log(rng, max(1, c["trials"] // 6), c["trials"])
         c["k"] = rng.choice([1, 2, 4, 5, 8, 8, 12]) if level <= 7 else rng.choice([1, 4, 8, 8])
     elif op == "initial":
