@@ -236,6 +236,7 @@ galic::OrbitArgs orbit_args(galic::Ctx &c, int n) {
   A.omass = c.o_mass; A.otint = c.o_tint; A.otype = c.o_type;
   A.tall = c.o_tall; A.e0 = c.o_e0; A.e1 = c.o_e1;
   A.norbit = c.o_norbit; A.status = c.o_status; A.steps = c.o_steps; A.bbox = c.o_bbox;
+  A.vstream_nz = c.vstream_nz64;
   A.slot_stride = (size_t)galic::kFields * c.Ngrid;
   A.stats = c.orbit_stats;
   return A;
@@ -275,8 +276,24 @@ int launch_orbit64(galic::Ctx &c, galic::OrbitArgs A) {
   HIPCHK(hipMemsetAsync(c.counter, 0, sizeof(unsigned int), c.stream));
   HIPCHK(hipMemsetAsync(c.orbit_stats, 0, 4 * sizeof(unsigned long long), c.stream));
   HIPCHK(hipEventRecord(c.ev0, c.stream));
-  const int bs = 256;
-  hipLaunchKernelGGL(galic::k_orbit64, dim3(orbit_grid(A.n, bs)), dim3(bs), 0, c.stream, c.M, A);
+  // A quad of lanes per orbit, at least 4 quads a wave (waves of one or two quads ran 1.5 times
+  // slower once four of them shared a CU; alone on their CU they are the fastest), the wave
+  // filled before a SIMD takes a second wave.  Three waves per SIMD are resident.
+  int cus = 256;
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device);
+  const int simds = 4 * cus, waves = 3 * simds;
+  const int qpw = A.n <= cus ? 1 : std::max(4, std::min(16, nblocks(A.n, simds)));
+  if(A.n > 16 * waves) {
+    // more orbits than resident quads: the longest expected first
+    CHK(alloc_sort_scratch(c, A.n));
+    hipLaunchKernelGGL(galic::k_expect_steps, dim3(nblocks(A.n, 256)), dim3(256), 0, c.stream, c.M, A.n, A.ox, A.oy,
+                       A.oz, A.ovx, A.ovy, A.ovz, A.otint, c.t_key, c.t_ord);
+    HIPCHK(hipGetLastError());
+    if(galic::sort_desc(A.n, c.t_key, c.t_key2, c.t_ord, c.t_ord2, &c.sort_tmp, &c.sort_tmp_bytes, c.stream) != 0)
+      return set_err(GALIC_ERR_HIP, "sorting the orbits by expected length failed");
+    A.order = c.t_ord2;
+  }
+  hipLaunchKernelGGL(galic::k_orbit64, dim3(std::min(nblocks(A.n, qpw), waves)), dim3(64), 0, c.stream, c.M, A, qpw);
   HIPCHK(hipGetLastError());
   HIPCHK(hipEventRecord(c.ev1, c.stream));
   HIPCHK(hipEventSynchronize(c.ev1));
@@ -996,7 +1013,7 @@ int galic_create(const galic_params *p, int device, galic_ctx **out) {
   CHK(dalloc(&c.FG_Vstream, (size_t)GALIC_NTYPES * c.FG_Ngrid));
   CHK(dalloc(&c.FG_Acc_f, c.FG_Ngrid));
   CHK(dalloc(&c.FG_Vstream_f, (size_t)GALIC_NTYPES * c.FG_Ngrid));
-  c.vstream_nz = 0;
+  c.vstream_nz = c.vstream_nz64 = 0;
   CHK(dalloc(&c.DG_CellSize, c.Ngrid));
   CHK(dalloc(&c.DG_CellSize_f, c.Ngrid));
   CHK(dalloc(&c.DG_Cell1_f, (size_t)c.Nbin));
@@ -1241,13 +1258,15 @@ int galic_set_vstream(galic_ctx *ctx, int type, const double *vstream) {
   if(vstream) memcpy(v.data(), vstream, n * sizeof(double));
   HIPCHK(hipMemcpy(c.FG_Vstream + (size_t)type * n, v.data(), n * sizeof(double), hipMemcpyHostToDevice));
   std::vector<float> f(n);
-  bool nz = false;
+  bool nz = false, nz64 = false;
   for(size_t i = 0; i < n; i++) {
     f[i] = (float)v[i];
     nz = nz || f[i] != 0.f;
+    nz64 = nz64 || v[i] != 0;
   }
   HIPCHK(hipMemcpy(c.FG_Vstream_f + (size_t)type * n, f.data(), n * sizeof(float), hipMemcpyHostToDevice));
   c.vstream_nz = nz ? (c.vstream_nz | (1u << type)) : (c.vstream_nz & ~(1u << type));
+  c.vstream_nz64 = nz64 ? (c.vstream_nz64 | (1u << type)) : (c.vstream_nz64 & ~(1u << type));
   return GALIC_OK;
 }
 

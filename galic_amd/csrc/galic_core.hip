@@ -24,159 +24,328 @@ namespace galic {
 
 // ------------------------------------------------------------------ orbits --
 
-// Register-resident accumulator for consecutive binning events that hit the
-// same 2x2 block of cells: flushed to memory only when the block changes.
+// Four lanes integrate one orbit.  A launch has far fewer orbits than the GPU has lanes (a rep's
+// trials, a batch of single orbits), so its time is the longest orbit's chain of steps, and a
+// step's latency is mostly the length of its instruction stream: about 1100 FP64 instructions
+// with one lane per orbit, 600 with four.  The lanes of a quad hold the same state bit for bit
+// and share the step's independent pieces, one each: the three square roots, the four log
+// indices (R and z on the force and the density grid, with their divisions), the divisions of
+// the force and of the velocity components, the four table taps and the four cells of a binning
+// event.  Every value is formed by the operations, in the order, of the lookups in
+// galic_device.h, so the results do not depend on the split.  Measured against one lane per
+// orbit: a single orbit's step 2.5 -> 1.5 us; 6000 orbits on 64^2 grids 32 -> 16 ms; the initial
+// pass of 2e4 particles 35 -> 22 ms, of 2e5 (bound by the atomics on the Loc grids) 217 -> 138 ms.
+
+// Lane k's value in all four lanes of the quad.
+template <int K>
+__device__ __forceinline__ double quad_get(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), K * 0x55, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), K * 0x55, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+
+__device__ __forceinline__ int quad_first(int v) { return __builtin_amdgcn_mov_dpp(v, 0, 0xF, 0xF, true); }
+
+// Register-resident accumulator of the lane's cell of the 2x2 block (lane bit 0: R + 1, bit 1:
+// z + 1) for consecutive binning events that hit the same block: flushed to memory only when
+// the block changes.
 struct Run64 {
   int quad;  // iz*Nbin + iR of the lower-left cell, -1 when empty
-  double w[kFields][4];
+  double w[kFields];
 };
 
-__device__ __forceinline__ void run_reset(Run64 &r, int quad) {
-  r.quad = quad;
-#pragma unroll
-  for(int f = 0; f < kFields; f++)
-#pragma unroll
-    for(int c = 0; c < 4; c++) r.w[f][c] = 0;
-}
-
-// Write a run either into the orbit's private slot (trial evaluation) or with
-// atomics into the Loc grid of the particle's type (initial response pass).
-__device__ __forceinline__ void run_flush(const Run64 &r, int nb, int ngrid, double fac, double *slot,
+// Adds a run to the orbit's private slot (trial evaluation; cell-major: a cell's 5 fields are
+// contiguous) or to the Loc grid of the particle's type (initial response pass).  Atomics without
+// return in both: the slot belongs to one orbit, but a load, add and store would make the wave
+// wait for memory at every flush.
+__device__ __forceinline__ void run_flush(const Run64 &r, int q, int nb, int ngrid, double fac, double *slot,
                                           double *loc) {
   if(r.quad < 0) return;
-  const int c0 = r.quad, c1 = r.quad + 1, c2 = r.quad + nb, c3 = r.quad + nb + 1;
+  const int c = r.quad + (q & 1) + (q >> 1) * nb;
   if(slot) {
-    // cell-major slot: the 5 fields of a cell are contiguous, so a flush
-    // touches two short row segments instead of ten field rows
-    double *s0 = slot + (size_t)c0 * kFields, *s2 = slot + (size_t)c2 * kFields;
+    double *s = slot + (size_t)c * kFields;
 #pragma unroll
-    for(int f = 0; f < kFields; f++) {
-      s0[f] += fac * r.w[f][0];
-      s0[kFields + f] += fac * r.w[f][1];
-      s2[f] += fac * r.w[f][2];
-      s2[kFields + f] += fac * r.w[f][3];
-    }
+    for(int f = 0; f < kFields; f++) atomicAdd(&s[f], fac * r.w[f]);
   } else {
 #pragma unroll
-    for(int f = 0; f < kFields; f++) {
-      double *s = loc + (size_t)f * ngrid;
-      atomicAdd(&s[c0], fac * r.w[f][0]);
-      atomicAdd(&s[c1], fac * r.w[f][1]);
-      atomicAdd(&s[c2], fac * r.w[f][2]);
-      atomicAdd(&s[c3], fac * r.w[f][3]);
-    }
+    for(int f = 0; f < kFields; f++) atomicAdd(&loc[(size_t)f * ngrid + c], fac * r.w[f]);
   }
 }
 
-// One binning event: trapezoid half weights (orbit_response.c:277-319).
-__device__ __forceinline__ void bin_event64(Run64 &r, int nb, int ngrid, double fac, double *slot, double *loc,
-                                            int iR, int iz, double fR, double fz, double dt, double vr2,
-                                            double vt2, double vq2, double vp2, int4 &bb) {
-  double m00 = 0.5 * dt * (1 - fR) * (1 - fz);
-  double m10 = 0.5 * dt * (fR) * (1 - fz);
-  double m01 = 0.5 * dt * (1 - fR) * (fz);
-  double m11 = 0.5 * dt * (fR) * (fz);
-  int quad = iz * nb + iR;
-  if(quad != r.quad) {
-    run_flush(r, nb, ngrid, fac, slot, loc);
-    run_reset(r, quad);
-    bb.x = min(bb.x, iR);
-    bb.y = max(bb.y, iR + 1);
-    bb.z = min(bb.z, iz);
-    bb.w = max(bb.w, iz + 1);
-  }
-  r.w[F_M][0] += m00; r.w[F_M][1] += m10; r.w[F_M][2] += m01; r.w[F_M][3] += m11;
-  r.w[F_R][0] += m00 * vr2; r.w[F_R][1] += m10 * vr2; r.w[F_R][2] += m01 * vr2; r.w[F_R][3] += m11 * vr2;
-  r.w[F_T][0] += m00 * vt2; r.w[F_T][1] += m10 * vt2; r.w[F_T][2] += m01 * vt2; r.w[F_T][3] += m11 * vt2;
-  r.w[F_Q][0] += m00 * vq2; r.w[F_Q][1] += m10 * vq2; r.w[F_Q][2] += m01 * vq2; r.w[F_Q][3] += m11 * vq2;
-  r.w[F_P][0] += m00 * vp2; r.w[F_P][1] += m10 * vp2; r.w[F_P][2] += m01 * vp2; r.w[F_P][3] += m11 * vp2;
+// Starts an empty run in the block of cell (iR, iz).
+__device__ __forceinline__ void run_start(Run64 &r, int nb, int iR, int iz, int4 &bb) {
+  r.quad = iz * nb + iR;
+#pragma unroll
+  for(int f = 0; f < kFields; f++) r.w[f] = 0;
+  bb.x = min(bb.x, iR);
+  bb.y = max(bb.y, iR + 1);
+  bb.z = min(bb.z, iz);
+  bb.w = max(bb.w, iz + 1);
 }
 
-// Persistent lanes: every lane pulls the next orbit from an atomic counter when
-// its current orbit ends, so orbits of very different length keep the wave busy.
-// Every lane leaves once the counter passes the orbit count.
-__global__ void __launch_bounds__(256) k_orbit64(DevModel M, OrbitArgs A) {
-  const int nb = M.DG_Nbin, ngrid = nb * nb;
+// One binning event in the run's block: trapezoid half weights (orbit_response.c:277-319).
+__device__ __forceinline__ void bin_event64(Run64 &r, int q, double fR, double fz, double dt, double vr2, double vt2,
+                                            double vq2, double vp2) {
+  const double m = 0.5 * dt * ((q & 1) ? fR : 1 - fR) * ((q & 2) ? fz : 1 - fz);
+  r.w[F_M] += m;
+  r.w[F_R] += m * vr2;
+  r.w[F_T] += m * vt2;
+  r.w[F_Q] += m * vq2;
+  r.w[F_P] += m * vp2;
+}
+
+// Persistent quads: qpw quads of each wave take orbits from the launch's counter, the next one
+// when their orbit ends, so orbits of different length keep the wave busy.  A freshly taken orbit
+// spends one pass of the loop on the lookups at its start point.  Every quad leaves once the
+// counter passes the orbit count.
+__global__ void __launch_bounds__(64) k_orbit64(DevModel M, OrbitArgs A, int qpw) {
+  const int lane = threadIdx.x, q = lane & 3;
+  if((lane >> 2) >= qpw) return;
+  const int nb = M.DG_Nbin, ngrid = nb * nb, fb = M.FG_Nbin;
+  const bool odd = q & 1, upper = q & 2;
+  // the lane's constants: log index (lanes 0, 1 the force grid, 2, 3 the density grid), force term
+  // (lane 2 the halo, 3 the bulge) and timestep limit (odd lanes the orbital one)
+  const double l_rmin = upper ? M.DG_Rmin : M.FG_Rmin, l_lf = upper ? M.DG_logFac : M.FG_logFac;
+  const double l_off = upper ? 0.5 : 0.0, l_fac = odd ? M.fo : M.fc;
+  const double l_GM = odd ? M.G * M.Bulge_Mass : M.G * M.Halo_Mass;
+  const double l_a = odd ? M.Bulge_A : M.Halo_A, l_eps = 1.0e-6 * l_a;
+
+  int o = 0, type = 0, tovs = 0;
+  double x = 0, y = 0, z = 0, vx = 0, vy = 0, vz = 0, timespan = 0, fac = 0;
+  double ax = 0, ay = 0, az = 0, cellsize = 0, fR = 0, fz = 0, E0 = 0;
+  double vr2 = 0, vt2 = 0, vq2 = 0, vp2 = 0, tall = 0, radsign_previous = 0, dt = 0;
+  double *slot = nullptr, *loc = nullptr;
+  int iR = 0, iz = 0, norbit = 0, flag = 0, status = 0;
+  long long steps = 0;
+  Run64 run;
+  run.quad = -1;
+  int4 bb = make_int4(nb, -1, nb, -1);
+  bool take = true, fresh = false, streams = false;
   while(true) {
-    int o = (int)atomicAdd(A.counter, 1u);
-    if(o >= A.n) break;
-    const int type = A.otype[o];
-    const int tovs = M.tovs[type];
-    double x = A.ox[o], y = A.oy[o], z = A.oz[o];
-    double vx = A.ovx[o], vy = A.ovy[o], vz = A.ovz[o];
-    const double timespan = A.otint[o];
-    const double fac = A.omass[o] / timespan;  // mass/t with t == timespan at the end (see tall)
-    double *slot = A.slots ? A.slots + (size_t)(o - A.slot_base) * A.slot_stride : nullptr;
-    double *loc = A.loc ? A.loc + (size_t)type * kFields * ngrid : nullptr;
-
-    FgIndex64 g = fg_index64(M, x, y, z);
-    double ax, ay, az;
-    accel64(M, x, y, z, g, ax, ay, az);
-    int iR, iz;
-    double fR, fz;
-    cell64(x, y, z, M.DG_Rmin, M.DG_logFac, nb, iR, iz, fR, fz);
-    int icell = iz * nb + iR;
-    const double E0 = 0.5 * (vx * vx + vy * vy + vz * vz) + potential64(M, x, y, z);
-    double vr2, vt2, vq2, vp2;
-    decompose64(M, tovs, type, x, y, z, vx, vy, vz, g, vr2, vt2, vq2, vp2);
-
-    Run64 run;
-    run.quad = -1;
-    int4 bb = make_int4(nb, -1, nb, -1);
-    double tall = 0, radsign_previous = 0;
-    int norbit = 0, flag = 0, status = 0;
-    long long steps = 0;
-    if(!(timespan > 0)) status = GALIC_ERR_ARG;  // the reference would loop until its step cap
-    while(!flag && status == 0) {
+    if(take) {
+      int t = 0;
+      if(q == 0) t = (int)atomicAdd(A.counter, 1u);
+      o = quad_first(t);
+      if(o >= A.n) break;
+      if(A.order) o = A.order[o];
+      type = A.otype[o];
+      tovs = M.tovs[type];
+      streams = (A.vstream_nz >> type) & 1u;
+      x = A.ox[o]; y = A.oy[o]; z = A.oz[o];
+      vx = A.ovx[o]; vy = A.ovy[o]; vz = A.ovz[o];
+      timespan = A.otint[o];
+      fac = A.omass[o] / timespan;  // mass/t with t == timespan at the end (see tall)
+      slot = A.slots ? A.slots + (size_t)(o - A.slot_base) * A.slot_stride : nullptr;
+      loc = A.loc ? A.loc + (size_t)type * kFields * ngrid : nullptr;
+      E0 = 0.5 * (vx * vx + vy * vy + vz * vz) + potential64(M, x, y, z);
+      run.quad = -1;
+      bb = make_int4(nb, -1, nb, -1);
+      tall = radsign_previous = 0;
+      norbit = flag = status = 0;
+      steps = 0;
+      take = false;
+      fresh = true;
+    }
+    if(!fresh) {
       // get_timestep (orbit_response.c:16-26), with the cell of the previous position
-      double v = sqrt(vx * vx + vy * vy + vz * vz);
-      double aa = sqrt(ax * ax + ay * ay + az * az);
-      double torbit = M.V200 / aa;
-      double tcross = M.DG_CellSize[icell] / v;
-      double t1 = M.fo * torbit, t2 = M.fc * tcross;
-      double dt = (t1 < t2) ? t1 : t2;
+      const double v2 = vx * vx + vy * vy + vz * vz, a2 = ax * ax + ay * ay + az * az;
+      const double tl = l_fac * ((odd ? M.V200 : cellsize) / sqrt(odd ? a2 : v2));
+      const double t1 = quad_get<1>(tl), t2 = quad_get<0>(tl);
+      dt = (t1 < t2) ? t1 : t2;
       if(timespan < dt + tall) {
         dt = timespan - tall;
         flag = 1;
       }
       if(!(dt >= 0 && dt <= timespan)) {  // NaN state: stop instead of running to the step cap
         status = GALIC_ERR_ARG;
-        break;
+      } else {
+        bin_event64(run, q, fR, fz, dt, vr2, vt2, vq2, vp2);  // (in the block of the step before)
+        vx += 0.5 * dt * ax;
+        vy += 0.5 * dt * ay;
+        vz += 0.5 * dt * az;
+        x += dt * vx;
+        y += dt * vy;
+        z += dt * vz;
       }
-      bin_event64(run, nb, ngrid, fac, slot, loc, iR, iz, fR, fz, dt, vr2, vt2, vq2, vp2, bb);
-      vx += 0.5 * dt * ax;
-      vy += 0.5 * dt * ay;
-      vz += 0.5 * dt * az;
-      x += dt * vx;
-      y += dt * vy;
-      z += dt * vz;
-      g = fg_index64(M, x, y, z);
-      accel64(M, x, y, z, g, ax, ay, az);
-      vx += 0.5 * dt * ax;
-      vy += 0.5 * dt * ay;
-      vz += 0.5 * dt * az;
-      cell64(x, y, z, M.DG_Rmin, M.DG_logFac, nb, iR, iz, fR, fz);
-      icell = iz * nb + iR;
-      // the decomposition at the end of this step is also the one at the start of the next
-      decompose64(M, tovs, type, x, y, z, vx, vy, vz, g, vr2, vt2, vq2, vp2);
-      bin_event64(run, nb, ngrid, fac, slot, loc, iR, iz, fR, fz, dt, vr2, vt2, vq2, vp2, bb);
-      tall += dt;
-      double radsign = vx * x + vy * y + vz * z;
-      if(radsign > 0 && radsign_previous < 0) norbit++;
-      radsign_previous = radsign;
-      steps++;
-      if(steps > M.max_steps) status = GALIC_ERR_STEPCAP;
     }
-    run_flush(run, nb, ngrid, fac, slot, loc);
-    A.tall[o] = tall;
-    A.norbit[o] = norbit;
-    A.steps[o] = steps;
-    A.e0[o] = E0;
-    A.e1[o] = 0.5 * (vx * vx + vy * vy + vz * vz) + potential64(M, x, y, z);
-    A.bbox[o] = bb;
-    A.status[o] = status;
-    orbit_stats_add(A.stats, steps, status, o);
+    if(status == 0) {
+      const double R2 = x * x + y * y, r2 = x * x + y * y + z * z;
+      // orbit_response.c:222-273: Q and T of the velocity decomposition
+      double Q0, Q1, Q2, q2;
+      if(tovs == 2) {
+        Q0 = -y;
+        Q1 = x;
+        Q2 = 0;
+        q2 = Q0 * Q0 + Q1 * Q1;
+      } else {
+        Q0 = y * (-1.0) - z * 0.0;
+        Q1 = z * 0.0 - x * (-1.0);
+        Q2 = x * 0.0 - y * 0.0;
+        q2 = Q0 * Q0 + Q1 * Q1 + Q2 * Q2;
+      }
+      const double root = sqrt(upper ? q2 : odd ? r2 : R2);
+      const double R = quad_get<0>(root), r = quad_get<1>(root), qn = quad_get<2>(root);
+      const double bin = log((odd ? fabs(z) : R) / l_rmin + 1.0) / l_lf - l_off;
+      const double jd = quad_get<0>(bin), id = quad_get<1>(bin);
+      double br = quad_get<2>(bin), bz = quad_get<3>(bin);
+      // densitygrid_get_cell (grid.c:494-534)
+      if(br < 0) br = 0;
+      if(bz < 0) bz = 0;
+      iR = (int)br;
+      fR = br - iR;
+      iz = (int)bz;
+      fz = bz - iz;
+      if(iR >= nb - 1) {
+        iR = nb - 2;
+        fR = 1;
+      }
+      if(iz >= nb - 1) {
+        iz = nb - 2;
+        fz = 1;
+      }
+      // the lane's taps: its node of the force tables and of the streaming table, and the cell size
+      const int jbin = (int)jd, ibin = (int)id;
+      const double jfac = jd - jbin, ifac = id - ibin;
+      const bool on = M.use_table && ibin < fb - 1 && jbin < fb - 1;
+      double tR = 0, tz = 0;
+      if(on) {
+        const int k = (ibin + (q >> 1)) * fb + jbin + (q & 1);
+        tR = M.FG_DPotDR[k];
+        tz = M.FG_DPotDz[k];
+      }
+      // get_vstream (disp_fields.c:118-132) through forcegrid_get_cell (grid.c:15-55)
+      double sR = jd < 0 ? 0 : jd, sz = id < 0 ? 0 : id;
+      int jR = (int)sR, jz = (int)sz;
+      double gR = sR - jR, gz = sz - jz;
+      if(jR >= fb - 1) {
+        jR = fb - 2;
+        gR = 1;
+      }
+      if(jz >= fb - 1) {
+        jz = fb - 2;
+        gz = 1;
+      }
+      // (a table of zeros, as the isotropic components have, gives vstr = 0 without its load)
+      const double tv = streams ? M.FG_Vstream[type][(jz + (q >> 1)) * fb + jR + (q & 1)] : 0;
+      cellsize = M.DG_CellSize[iz * nb + iR];
+      // forcegrid_get_acceleration (grid.c:122-197): lanes 0, 1 the direction cosines, 2, 3 the
+      // closed forms of halo and bulge
+      const double quot = (upper ? l_GM : odd ? y : x) / (upper ? (r + l_eps) * (r + l_a) * (r + l_a) : R);
+      const double hal = quad_get<2>(quot), bul = quad_get<3>(quot);
+      ax = ay = az = 0;
+      if(on) {
+        const double wi = upper ? ifac : 1 - ifac, wj = odd ? jfac : 1 - jfac;
+        const double pR = tR * wi * wj, pz = tz * wi * wj;
+        const double accR = quad_get<0>(pR) + quad_get<1>(pR) + quad_get<2>(pR) + quad_get<3>(pR);
+        double accz = quad_get<0>(pz) + quad_get<1>(pz) + quad_get<2>(pz) + quad_get<3>(pz);
+        if(z < 0) accz = -accz;
+        const double c = quad_get<0>(quot), s = quad_get<1>(quot);
+        ax = accR * (R > 0 ? c : 1.0);
+        ay = accR * (R > 0 ? s : 0.0);
+        az = accz;
+      } else if(M.use_table) {
+        ax = -hal * x * M.halo_offgrid_fac;
+        ay = -hal * y * M.halo_offgrid_fac;
+        az = -hal * z * M.halo_offgrid_fac;
+      }
+      if(M.add_halo) {
+        ax += -hal * x;
+        ay += -hal * y;
+        az += -hal * z;
+      }
+      if(M.add_bulge) {
+        ax += -bul * x;
+        ay += -bul * y;
+        az += -bul * z;
+      }
+      if(!fresh) {
+        vx += 0.5 * dt * ax;
+        vy += 0.5 * dt * ay;
+        vz += 0.5 * dt * az;
+      }
+      // the decomposition at the end of a step is also the one at the start of the next
+      double vstr = 0;
+      if(streams) {
+        const double pv = tv * (odd ? gR : 1 - gR) * (upper ? gz : 1 - gz);
+        vstr = quad_get<0>(pv) + quad_get<2>(pv) + quad_get<1>(pv) + quad_get<3>(pv);
+      }
+      double num, den;
+      if(tovs == 2) {
+        const double v_dot_x = vx * x + vy * y, v_dot_Q = vx * Q0 + vy * Q1;
+        num = odd ? v_dot_Q : v_dot_x * v_dot_x;
+        den = odd ? qn : R2;
+      } else {
+        const double v_dot_x = vx * x + vy * y + vz * z, v_dot_Q = vx * Q0 + vy * Q1 + vz * Q2;
+        const double T0 = y * Q2 - z * Q1, T1 = z * Q0 - x * Q2, T2 = x * Q1 - y * Q0;
+        const double v_dot_T = vx * T0 + vy * T1 + vz * T2;
+        num = upper ? v_dot_T * v_dot_T : odd ? v_dot_Q : v_dot_x * v_dot_x;
+        den = upper ? T0 * T0 + T1 * T1 + T2 * T2 : odd ? qn : r2;
+      }
+      const double comp = num / den;
+      vr2 = quad_get<0>(comp);
+      vt2 = tovs == 2 ? vz * vz : quad_get<2>(comp);
+      const double vq = quad_get<1>(comp);
+      vq2 = vq * vq;
+      vp2 = (vq - vstr) * (vq - vstr);
+      if(fresh) {
+        fresh = false;
+        if(timespan > 0) {
+          run_start(run, nb, iR, iz, bb);
+          continue;
+        }
+        status = GALIC_ERR_ARG;  // the reference would loop until its step cap
+      } else {
+        if(iz * nb + iR != run.quad) {
+          run_flush(run, q, nb, ngrid, fac, slot, loc);
+          run_start(run, nb, iR, iz, bb);
+        }
+        bin_event64(run, q, fR, fz, dt, vr2, vt2, vq2, vp2);
+        tall += dt;
+        const double radsign = vx * x + vy * y + vz * z;
+        if(radsign > 0 && radsign_previous < 0) norbit++;
+        radsign_previous = radsign;
+        steps++;
+        if(steps > M.max_steps) status = GALIC_ERR_STEPCAP;
+      }
+    }
+    if(flag || status) {
+      if(steps > 0)
+        run_flush(run, q, nb, ngrid, fac, slot, loc);
+      else
+        bb = make_int4(nb, -1, nb, -1);  // nothing was binned
+      const double e1 = 0.5 * (vx * vx + vy * vy + vz * vz) + potential64(M, x, y, z);
+      if(q == 0) {
+        A.tall[o] = tall;
+        A.norbit[o] = norbit;
+        A.steps[o] = steps;
+        A.e0[o] = E0;
+        A.e1[o] = e1;
+        A.bbox[o] = bb;
+        A.status[o] = status;
+        orbit_stats_add(A.stats, steps, status, o);
+      }
+      take = true;
+    }
   }
+}
+
+// Expected steps of each orbit, its time span over the timestep at its start (orbit_response.c:16-26):
+// the key by which a launch takes its longest orbits first.
+__global__ void k_expect_steps(DevModel M, int n, const double *ox, const double *oy, const double *oz,
+                               const double *ovx, const double *ovy, const double *ovz, const double *otint,
+                               unsigned int *key, int *ord) {
+  const int o = blockIdx.x * blockDim.x + threadIdx.x;
+  if(o >= n) return;
+  const double x = ox[o], y = oy[o], z = oz[o], vx = ovx[o], vy = ovy[o], vz = ovz[o];
+  double ax, ay, az, fR, fz;
+  int iR, iz;
+  accel64(M, x, y, z, fg_index64(M, x, y, z), ax, ay, az);
+  cell64(x, y, z, M.DG_Rmin, M.DG_logFac, M.DG_Nbin, iR, iz, fR, fz);
+  const double t1 = M.fo * M.V200 / sqrt(ax * ax + ay * ay + az * az);
+  const double t2 = M.fc * M.DG_CellSize[iz * M.DG_Nbin + iR] / sqrt(vx * vx + vy * vy + vz * vz);
+  const double s = otint[o] / (t1 < t2 ? t1 : t2);
+  key[o] = s > 0 && s < 4e9 ? (unsigned int)s : 0u;
+  ord[o] = o;
 }
 
 // --------------------------------------------------- instantaneous moments --

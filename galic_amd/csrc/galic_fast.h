@@ -134,6 +134,9 @@ int sort_trials_by_steps(int ntrial, const int *tidx, const int *psteps, unsigne
                          int *ord, int *ord2, void **tmp, size_t *tmp_bytes, hipStream_t stream);
 int sort_trials_by_records(int n, int K, const int *slot_pos, const int *log_n, unsigned int *key, unsigned int *key2,
                            int *ord, int *ord2, void **tmp, size_t *tmp_bytes, hipStream_t stream);
+// (key, ord) pairs sorted by decreasing key into (key2, ord2), stable; *tmp grown as needed.
+int sort_desc(int n, unsigned int *key, unsigned int *key2, int *ord, int *ord2, void **tmp, size_t *tmp_bytes,
+              hipStream_t stream);
 __global__ void k_pack_merit(const double *stacks, const double *weights, double2 *bw, float2 *bwf, int Nstack);
 template <bool USE_O, bool GMEM, int LF>
 __global__ void k_eval_log32(DevModel M, EvalArgs32 A);

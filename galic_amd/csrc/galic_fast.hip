@@ -691,9 +691,6 @@ __global__ void k_record_keys(int n, int K, const int *slot_pos, const int *log_
   ord[b] = b;
 }
 
-int sort_desc(int n, unsigned int *key, unsigned int *key2, int *ord, int *ord2, void **tmp, size_t *tmp_bytes,
-              hipStream_t stream);
-
 __global__ void k_fill_u32(unsigned int *p, unsigned int v, size_t n) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if(i < n) p[i] = v;

@@ -24,6 +24,8 @@ struct OrbitArgs {
   const double *ovx, *ovy, *ovz;  // start velocity of each orbit
   const double *omass, *otint;    // mass and integration time of each orbit
   const int *otype;
+  const int *order;    // the orbits in the order they are taken, or null: 0 .. n-1
+  unsigned int vstream_nz;  // bit t: type t's streaming table has a nonzero node (else it is not read)
   double *slots;       // private response per orbit (trial evaluation), or null
   size_t slot_stride;  // doubles per slot (5*Ngrid)
   int slot_base;       // orbit index of slot 0
@@ -68,7 +70,10 @@ struct FitArgs {
   double lowdisp;
 };
 
-__global__ void k_orbit64(DevModel M, OrbitArgs A);
+__global__ void k_orbit64(DevModel M, OrbitArgs A, int qpw);
+__global__ void k_expect_steps(DevModel M, int n, const double *ox, const double *oy, const double *oz,
+                               const double *ovx, const double *ovy, const double *ovz, const double *otint,
+                               unsigned int *key, int *ord);
 
 // Per-lane totals of an orbit launch folded into three counters (no per-orbit download).
 __device__ __forceinline__ void orbit_stats_add(unsigned long long *stats, long long steps, int status, int o) {
