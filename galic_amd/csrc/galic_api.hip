@@ -469,12 +469,11 @@ galic::FastModel fast_model(galic::Ctx &c) {
   galic::FastModel F;
   memset(&F, 0, sizeof(F));
   const galic_params &p = c.p;
-  F.use_table = c.M.use_table;
-  F.add_halo = c.M.add_halo;
-  F.add_bulge = c.M.add_bulge;
+  F.forces = (c.M.use_table ? 1 : 0) | (c.M.add_halo ? 2 : 0) | (c.M.add_bulge ? 4 : 0);
   for(int t = 0; t < GALIC_NTYPES; t++) F.tovs[t] = p.TypeOfVelocityStructure[t];
   F.fg_nbin = p.FG_Nbin;
   F.dg_nbin = c.Nbin;
+  F.dg_L = c.L;
   F.fg_invRmin = (float)(1.0 / p.FG_Rmin);
   F.fg_invlog2Fac = (float)(1.0 / log2(p.FG_Fac));
   F.dg_invRmin = (float)(1.0 / p.DG_Rmin);
@@ -494,7 +493,6 @@ galic::FastModel fast_model(galic::Ctx &c) {
   F.vstream_nz = c.vstream_nz;
   F.cellsize = c.DG_CellSize_f;
   F.cell1 = c.cell1_ok ? c.DG_Cell1_f : nullptr;
-  for(int f = 0; f < 5; f++) F.qscale[f] = c.fp32_scale[f];
   return F;
 }
 

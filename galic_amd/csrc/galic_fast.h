@@ -9,9 +9,9 @@ namespace galic {
 
 // FP32 forms of the model constants (reciprocals and log2 are fine here).
 struct FastModel {
-  int use_table, add_halo, add_bulge;
+  int forces;  // bit 0: the tables, 1: the analytic halo, 2: the analytic bulge
   int tovs[GALIC_NTYPES];
-  int fg_nbin, dg_nbin;
+  int fg_nbin, dg_nbin, dg_L;  // dg_nbin = 2^dg_L
   float fg_invRmin, fg_invlog2Fac, dg_invRmin, dg_invlog2Fac;
   float halo_GM, halo_a, halo_eps, offgrid_fac;
   float bulge_GM, bulge_a, bulge_eps;
@@ -22,7 +22,6 @@ struct FastModel {
   unsigned int vstream_nz;  // bit t: type t's streaming table has a nonzero node (else it is not read)
   const float *cellsize;
   const float *cell1;      // or null: cellsize[iz * nb + iR] = cell1[max(iR, iz)] (staged in LDS)
-  double qscale[kFields];  // fixed-point scale per orbit-averaged field
 };
 
 constexpr int kCell1Max = 1024;  // density-grid cells per side the LDS cell-size table holds
@@ -30,12 +29,12 @@ constexpr int kCell1Max = 1024;  // density-grid cells per side the LDS cell-siz
 struct OrbitArgs32 {
   int n;
   unsigned int *counter;
+  const int *order;    // the orbits in the order they are taken, or null: 0 .. n-1
   const double *ox, *oy, *oz, *ovx, *ovy, *ovz, *omass, *otint;
   const int *otype;
   float *slots;        // private FP32 response per orbit, or null
   size_t slot_stride;  // floats per slot (5*Ngrid)
   int slot_base;
-  long long *locq;     // fixed-point Loc grids [type][5][Ngrid] for direct atomics, or null
   double *tall;
   int *norbit, *status;
   long long *steps;

@@ -24,233 +24,53 @@
 
 namespace galic {
 
-// ------------------------------------------------------------ FP32 lookups --
+// ------------------------------------------------------------- FP32 orbits --
 
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 __device__ __forceinline__ float fast_rsq(float x) { return __builtin_amdgcn_rsqf(x); }
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
-struct Fg32 {
-  float R, invR, jd, id;
-};
-
-__device__ __forceinline__ Fg32 fg_index32(const FastModel &F, float x, float y, float z) {
-  Fg32 g;
-  float R2 = x * x + y * y;
-  g.invR = fast_rsq(R2);
-  g.R = R2 * g.invR;
-  if(!(R2 > 0)) {
-    g.R = 0;
-    g.invR = 0;
-  }
-  g.jd = fast_log2(g.R * F.fg_invRmin + 1.0f) * F.fg_invlog2Fac;
-  g.id = fast_log2(fabsf(z) * F.fg_invRmin + 1.0f) * F.fg_invlog2Fac;
-  return g;
-}
-
-// Every table value one point of the orbit needs, loaded together so a step
-// waits on memory once: the four force-table nodes and the four streaming
-// velocity nodes around the point (both on the force grid, indices clamped
-// into the table; the off-grid force below does not use the force taps), and
-// the density-grid cell size that sets the next step's dt (from the LDS copy of
-// its per-index table where the grid has one: the size of cell (iR, iz) is the
-// larger of the R and z widths, the same function of either index).
-struct Taps32 {
-  float2 a00, a01, a10, a11;  // (DPotDR, DPotDz) at (z row, R column) +(0,0), (0,1), (1,0), (1,1)
-  float v00, v01, v10, v11;   // streaming velocity at the same nodes
-  float cell;                 // DG_CellSize of the point's density cell
-  int jb, ib;                 // force-grid node left of / below the point (unclamped)
-};
-
-__device__ __forceinline__ Taps32 load_taps32(const FastModel &F, const Fg32 &g, int type, int iR, int iz,
-                                              const float *s_cell) {
-  Taps32 t;
-  const int nb = F.fg_nbin;
-  t.jb = max((int)g.jd, 0);
-  t.ib = max((int)g.id, 0);
-  const int k = min(t.ib, nb - 2) * nb + min(t.jb, nb - 2);
-  const float2 *T = F.acc + k;
-  const float *V = F.vstream + (size_t)type * nb * nb + k;
-  t.a00 = T[0];
-  t.a01 = T[1];
-  t.a10 = T[nb];
-  t.a11 = T[nb + 1];
-  // (a table of zeros, as the isotropic components have, gives vstr = +0 without its loads)
-  if((F.vstream_nz >> type) & 1u) {
-    t.v00 = V[0];
-    t.v01 = V[1];
-    t.v10 = V[nb];
-    t.v11 = V[nb + 1];
-  } else {
-    t.v00 = t.v01 = t.v10 = t.v11 = 0.f;
-  }
-  t.cell = F.cell1 ? s_cell[max(iR, iz)] : F.cellsize[iz * F.dg_nbin + iR];
-  return t;
-}
-
-__device__ __forceinline__ void accel32(const FastModel &F, float x, float y, float z, const Fg32 &g,
-                                        const Taps32 &t, float &ax, float &ay, float &az) {
-  ax = ay = az = 0.f;
-  if(F.use_table) {
-    const int nb = F.fg_nbin;
-    const int jb = t.jb, ib = t.ib;
-    if(ib < nb - 1 && jb < nb - 1) {
-      float jf = g.jd - jb, fi = g.id - ib;
-      float w00 = (1 - fi) * (1 - jf), w01 = (1 - fi) * jf, w10 = fi * (1 - jf), w11 = fi * jf;
-      float accR = t.a00.x * w00 + t.a01.x * w01 + t.a10.x * w10 + t.a11.x * w11;
-      float accz = t.a00.y * w00 + t.a01.y * w01 + t.a10.y * w10 + t.a11.y * w11;
-      if(z < 0) accz = -accz;
-      float c = 1.f, s = 0.f;
-      if(g.R > 0) {
-        c = x * g.invR;
-        s = y * g.invR;
-      }
-      ax = accR * c;
-      ay = accR * s;
-      az = accz;
-    } else {
-      float r = sqrtf(x * x + y * y + z * z);
-      float f = F.halo_GM * fast_rcp((r + F.halo_eps) * (r + F.halo_a) * (r + F.halo_a)) * F.offgrid_fac;
-      ax = -f * x;
-      ay = -f * y;
-      az = -f * z;
-    }
-  }
-  if(F.add_halo || F.add_bulge) {
-    float r = sqrtf(x * x + y * y + z * z);
-    float f = 0.f;
-    if(F.add_halo) f += F.halo_GM * fast_rcp((r + F.halo_eps) * (r + F.halo_a) * (r + F.halo_a));
-    if(F.add_bulge) f += F.bulge_GM * fast_rcp((r + F.bulge_eps) * (r + F.bulge_a) * (r + F.bulge_a));
-    ax -= f * x;
-    ay -= f * y;
-    az -= f * z;
-  }
-}
-
-// Bilinear streaming velocity; beyond the last node the outermost column / row
-// is used (fraction 1 of the clamped cell).
-__device__ __forceinline__ float vstream32(const FastModel &F, const Fg32 &g, const Taps32 &t) {
-  const int nb = F.fg_nbin;
-  float fR = g.jd - t.jb, fz = g.id - t.ib;
-  if(t.jb >= nb - 1) fR = 1.f;
-  if(t.ib >= nb - 1) fz = 1.f;
-  return t.v00 * (1 - fR) * (1 - fz) + t.v10 * (1 - fR) * fz + t.v01 * fR * (1 - fz) + t.v11 * fR * fz;
-}
-
-__device__ __forceinline__ void cell32(const FastModel &F, float R, float z, int &iR, int &iz, float &fR,
-                                       float &fz) {
-  const int nb = F.dg_nbin;
-  float br = fast_log2(R * F.dg_invRmin + 1.0f) * F.dg_invlog2Fac - 0.5f;
-  float bz = fast_log2(fabsf(z) * F.dg_invRmin + 1.0f) * F.dg_invlog2Fac - 0.5f;
-  br = fmaxf(br, 0.f);
-  bz = fmaxf(bz, 0.f);
-  iR = (int)br;
-  iz = (int)bz;
-  fR = br - iR;
-  fz = bz - iz;
-  if(iR >= nb - 1) {
-    iR = nb - 2;
-    fR = 1.f;
-  }
-  if(iz >= nb - 1) {
-    iz = nb - 2;
-    fz = 1.f;
-  }
-}
-
-// vr2, vt2, vq2, vp2 of orbit_response.c:222-273 in closed form:
-// spherical basis Q = (-y, x, 0), T = (-zx, -zy, R^2), |Q| = R, |T| = R r.
-__device__ __forceinline__ void decompose32(int tovs, float vstr, float x, float y, float z, float vx, float vy,
-                                            float vz, const Fg32 &g, float &vr2, float &vt2, float &vq2, float &vp2) {
-  float R2 = x * x + y * y;
-  float vq = (vy * x - vx * y) * g.invR;
-  vq2 = vq * vq;
-  vp2 = (vq - vstr) * (vq - vstr);
-  if(tovs == 2) {
-    float vdx = vx * x + vy * y;
-    vr2 = vdx * vdx * g.invR * g.invR;
-    vt2 = vz * vz;
-  } else {
-    float r2 = R2 + z * z;
-    float ir2 = fast_rcp(r2);
-    float vdx = vx * x + vy * y + vz * z;
-    vr2 = vdx * vdx * ir2;
-    float vdt = R2 * vz - z * (vx * x + vy * y);
-    vt2 = vdt * vdt * ir2 * g.invR * g.invR;
-  }
-}
-
-// ------------------------------------------------------------- FP32 orbits --
-
-struct Run32 {
-  int quad;
-  float w[kFields][4];
-};
-
-__device__ __forceinline__ void run32_reset(Run32 &r, int quad) {
-  r.quad = quad;
-#pragma unroll
-  for(int f = 0; f < kFields; f++)
-#pragma unroll
-    for(int c = 0; c < 4; c++) r.w[f][c] = 0.f;
+// Correctly rounded square root for r^2 of a position: the hardware's root, moved by an ulp where
+// its residual says so.  (Not scaled for r^2 < 2^-96, where r no longer changes r + eps.)
+__device__ __forceinline__ float root32(float s) {
+  const float q = __builtin_amdgcn_sqrtf(s);
+  const float lo = __int_as_float(__float_as_int(q) - 1), hi = __int_as_float(__float_as_int(q) + 1);
+  float r = __builtin_fmaf(-lo, q, s) <= 0.f ? lo : q;
+  return __builtin_fmaf(-hi, q, s) > 0.f ? hi : r;
 }
 
 __device__ __forceinline__ void atomic_q(long long *p, double v) {
   atomicAdd((unsigned long long *)p, (unsigned long long)__double2ll_rn(v));
 }
 
-// Adds a run's weights to the orbit's slot (cell-major: 5 fields per cell
-// contiguous, so a 2x2 block is two short row segments) or, without a slot,
-// to the fixed-point Loc grids.
-__device__ __forceinline__ void run32_flush(const Run32 &r, int nb, int ngrid, float *slot, long long *locq,
-                                            const FastModel &F) {
-  if(r.quad < 0) return;
-  const int c[4] = {r.quad, r.quad + 1, r.quad + nb, r.quad + nb + 1};
-  if(slot) {
-    float *s0 = slot + (size_t)c[0] * kFields, *s2 = slot + (size_t)c[2] * kFields;
-#pragma unroll
-    for(int f = 0; f < kFields; f++) {
-      s0[f] += r.w[f][0];
-      s0[kFields + f] += r.w[f][1];
-      s2[f] += r.w[f][2];
-      s2[kFields + f] += r.w[f][3];
-    }
-  } else {
-#pragma unroll
-    for(int f = 0; f < kFields; f++) {
-      long long *s = locq + (size_t)f * ngrid;
-      double sc = F.qscale[f];
-#pragma unroll
-      for(int k = 0; k < 4; k++) atomic_q(&s[c[k]], sc * (double)r.w[f][k]);
-    }
-  }
-}
+// Two or four table values at an 8- or 4-byte aligned address, one load.  (Pointers held in
+// registers name their address space: generic ones would load through the flat path, which also
+// waits for LDS.)
+#define GLOBAL __attribute__((address_space(1)))
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+typedef float f32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
+
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 // Append-only response log of one orbit: the lane never reads its log back,
 // so a flush is a handful of stores and the wave does not wait on memory.
 // Arena blocks are claimed LOG_CHUNK at a time per lane and handed to the
 // lane's orbits in turn: a claim is an atomic with return on one counter that
 // every lane of the chip shares, and its round trip stalls the whole wave.
-// Records are written in pairs (indices 2m and 2m + 1, 32 contiguous bytes of
-// each field's column of the block): a finished record waits in registers for
-// the next one, so the memory system receives whole 32-byte sectors instead of
-// half sectors that it would merge with what memory holds.
 struct Log32 {
   int n;              // records written
-  int blk;            // current arena block
-  bool full;          // out of block-table entries or arena blocks
-  bool held;          // rec holds a finished record not yet written
-  bool qheld;         // q0, q1: the quads of the written pair at n - 2, not yet stored (n % 4 == 2)
-  int q0, q1;
+  int blk;            // current arena block, -1: out of block-table entries or arena blocks
   unsigned int next;  // the lane's claimed blocks [next, end)
   unsigned int end;
   float tot[kFields];  // sums of the orbit's record values per field (all values are >= 0)
-  Run32 rec;
+  GLOBAL int *q;       // the arena's quads and values
+  GLOBAL char *v;
 };
 
-// Claims the arena block that record n starts, if it starts one.
+// Claims the arena block that record n (the first of a block) starts.
 __device__ __forceinline__ void log32_claim(Log32 &lg, int o, const OrbitArgs32 &A) {
-  if(lg.full || (lg.n & (LOG_B - 1)) != 0) return;
+  if(lg.blk < 0 && lg.n > 0) return;  // the log has overflowed
   const int b = lg.n / LOG_B;
   unsigned int nb = 0xffffffffu;
   if(b < A.log_M) {
@@ -261,125 +81,73 @@ __device__ __forceinline__ void log32_claim(Log32 &lg, int o, const OrbitArgs32 
     nb = lg.next++;
   }
   if(nb >= A.log_cap) {
-    lg.full = true;
+    lg.blk = -1;
   } else {
     lg.blk = (int)nb;
     A.log_blocks[(size_t)o * A.log_M + b] = (int)nb;
   }
 }
 
-__device__ __forceinline__ void log32_flush(const Run32 &r, Log32 &lg, int o, const OrbitArgs32 &A) {
-  if(r.quad < 0) return;
+// A finished run of binning events in one 2x2 block: a record of the log, or added to the
+// orbit's slot (cell-major: 5 fields per cell contiguous).
+template <bool LOG>
+__device__ __forceinline__ void run32_flush(int quad, const float (&w)[kFields][4], int nb, Log32 &lg, int o,
+                                            float *slot, const OrbitArgs32 &A) {
+#pragma clang fp contract(off)
+  if(LOG) {
 #pragma unroll
-  for(int f = 0; f < kFields; f++) lg.tot[f] += (r.w[f][0] + r.w[f][1]) + (r.w[f][2] + r.w[f][3]);
-  if(!lg.held) {
-    lg.rec = r;
-    lg.held = true;
-    return;
-  }
-  log32_claim(lg, o, A);  // n is even: the pair shares a block
-  if(!lg.full) {
-    // (the quads of two pairs go out as one 16-byte store: a pair at j % 4 == 0 holds its own)
+    for(int f = 0; f < kFields; f++) lg.tot[f] += (w[f][0] + w[f][1]) + (w[f][2] + w[f][3]);
     const int j = lg.n & (LOG_B - 1);
-    if((j & 2) == 0) {
-      lg.q0 = lg.rec.quad;
-      lg.q1 = r.quad;
-      lg.qheld = true;
-    } else {
-      *(int4 *)(A.log_q + (size_t)lg.blk * LOG_B + j - 2) = make_int4(lg.q0, lg.q1, lg.rec.quad, r.quad);
-      lg.qheld = false;
+    if(j == 0) log32_claim(lg, o, A);
+    if(lg.blk >= 0) {
+      const unsigned int rec = (unsigned int)lg.blk * LOG_B + (unsigned int)j;  // below 2^32: 84 bytes a record
+      lg.q[rec] = quad;
+      GLOBAL f32x4 *v = (GLOBAL f32x4 *)(lg.v + (unsigned long long)rec * (kFields * sizeof(f32x4)));
+#pragma unroll
+      for(int f = 0; f < kFields; f++) v[f] = f32x4{w[f][0], w[f][1], w[f][2], w[f][3]};
     }
-    float4 *v = A.log_v + ((size_t)lg.blk * LOG_B + j) * kFields;
+    lg.n++;
+  } else {
+    float *s0 = slot + (size_t)quad * kFields, *s2 = s0 + (size_t)nb * kFields;
 #pragma unroll
     for(int f = 0; f < kFields; f++) {
-      v[f] = make_float4(lg.rec.w[f][0], lg.rec.w[f][1], lg.rec.w[f][2], lg.rec.w[f][3]);
-      v[kFields + f] = make_float4(r.w[f][0], r.w[f][1], r.w[f][2], r.w[f][3]);
+      s0[f] += w[f][0];
+      s0[kFields + f] += w[f][1];
+      s2[f] += w[f][2];
+      s2[kFields + f] += w[f][3];
     }
   }
-  lg.n += 2;
-  lg.held = false;
 }
 
-// At the orbit's end: the record still held, alone.
-__device__ __forceinline__ void log32_finish(Log32 &lg, int o, const OrbitArgs32 &A) {
-  // the quads of a pair still held (in the current block: n % 4 == 2)
-  if(lg.qheld) {
-    if(!lg.full) *(int2 *)(A.log_q + (size_t)lg.blk * LOG_B + ((lg.n - 2) & (LOG_B - 1))) = make_int2(lg.q0, lg.q1);
-    lg.qheld = false;
-  }
-  if(!lg.held) return;
-  log32_claim(lg, o, A);
-  if(!lg.full) {
-    const int j = lg.n & (LOG_B - 1);
-    A.log_q[(size_t)lg.blk * LOG_B + j] = lg.rec.quad;
-    float4 *v = A.log_v + ((size_t)lg.blk * LOG_B + j) * kFields;
-#pragma unroll
-    for(int f = 0; f < kFields; f++)
-      v[f] = make_float4(lg.rec.w[f][0], lg.rec.w[f][1], lg.rec.w[f][2], lg.rec.w[f][3]);
-  }
-  lg.n++;
-  lg.held = false;
-}
-
-// Trapezoid weight h of one point of the orbit (orbit_response.c:283-319),
-// already multiplied by mass / timespan (the final scaling of :475-486),
-// accumulated in registers while the orbit stays in one 2x2 block.
-template <typename Flush>
-__device__ __forceinline__ void bin32(Run32 &r, int nb, Flush flush, int iR, int iz, float fR, float fz, float h,
-                                      float vr2, float vt2, float vq2, float vp2, int4 &bb) {
-  float m[4] = {h * (1 - fR) * (1 - fz), h * fR * (1 - fz), h * (1 - fR) * fz, h * fR * fz};
-  int quad = iz * nb + iR;
-  if(quad != r.quad) {
-    flush(r);
-    run32_reset(r, quad);
-    bb.x = min(bb.x, iR);
-    bb.y = max(bb.y, iR + 1);
-    bb.z = min(bb.z, iz);
-    bb.w = max(bb.w, iz + 1);
-  }
+// Trapezoid weight h of one point of the orbit (orbit_response.c:283-319), already multiplied by
+// mass / timespan (the final scaling of :475-486), added to the run's four cells.
+__device__ __forceinline__ void bin32(float (&w)[kFields][4], float fR, float fz, float h, float vr2, float vt2,
+                                      float vq2, float vp2) {
+#pragma clang fp contract(off)
+  const float hr = fR * h, hl = (1.0f - fR) * h, gz = 1.0f - fz;
+  const float m[4] = {gz * hl, gz * hr, fz * hl, fz * hr};
+  w[F_M][0] = __builtin_fmaf(gz, hl, w[F_M][0]);
+  w[F_M][1] = __builtin_fmaf(gz, hr, w[F_M][1]);
+  w[F_M][2] = __builtin_fmaf(fz, hl, w[F_M][2]);
+  w[F_M][3] = __builtin_fmaf(fz, hr, w[F_M][3]);
 #pragma unroll
   for(int k = 0; k < 4; k++) {
-    r.w[F_M][k] += m[k];
-    r.w[F_R][k] += m[k] * vr2;
-    r.w[F_T][k] += m[k] * vt2;
-    r.w[F_Q][k] += m[k] * vq2;
-    r.w[F_P][k] += m[k] * vp2;
+    w[F_R][k] = __builtin_fmaf(vr2, m[k], w[F_R][k]);
+    w[F_T][k] = __builtin_fmaf(vt2, m[k], w[F_T][k]);
+    w[F_Q][k] = __builtin_fmaf(vq2, m[k], w[F_Q][k]);
+    w[F_P][k] = __builtin_fmaf(vp2, m[k], w[F_P][k]);
   }
 }
-
-// State of the orbit a lane is integrating.
-struct Lane32 {
-  int o, type, tovs;
-  double timespan, tall;
-  float fac;  // mass / timespan, folded into every trapezoid weight
-  float *slot;
-  long long *locq;
-};
 
 // Takes orbits from the launch's counter until one starts cleanly; orbits with a
 // non-positive time span are finished at once with GALIC_ERR_ARG, as the FP64
-// path does.  Returns false when the launch has no orbits left.
-__device__ __forceinline__ bool take_orbit32(const OrbitArgs32 &A, int nb, Lane32 &L, float &x, float &y, float &z,
-                                             float &vx, float &vy, float &vz) {
-  const int ngrid = nb * nb;
+// path does.  Returns the orbit, or -1 when the launch has none left.
+__device__ __forceinline__ int take_orbit32(const OrbitArgs32 &A, int nb) {
   while(true) {
-    unsigned int q = atomicAdd(A.counter, 1u);
-    if(q >= (unsigned int)A.n) return false;
-    const int o = (int)q;
-    L.o = o;
-    L.type = A.otype[o];
-    L.timespan = A.otint[o];
-    L.tall = 0;
-    x = (float)A.ox[o];
-    y = (float)A.oy[o];
-    z = (float)A.oz[o];
-    vx = (float)A.ovx[o];
-    vy = (float)A.ovy[o];
-    vz = (float)A.ovz[o];
-    L.fac = (float)(A.omass[o] / L.timespan);
-    L.slot = A.slots ? A.slots + (size_t)(o - A.slot_base) * A.slot_stride : nullptr;
-    L.locq = A.locq ? A.locq + (size_t)L.type * kFields * ngrid : nullptr;
-    if(L.timespan > 0) return true;
+    const unsigned int q = atomicAdd(A.counter, 1u);
+    if(q >= (unsigned int)A.n) return -1;
+    const int o = A.order ? A.order[q] : (int)q;
+    if(A.otint[o] > 0) return o;
     A.tall[o] = 0;
     A.norbit[o] = 0;
     A.steps[o] = 0;
@@ -393,164 +161,283 @@ __device__ __forceinline__ bool take_orbit32(const OrbitArgs32 &A, int nb, Lane3
   }
 }
 
+// Keeps a kernel argument in a scalar register: the loop has more of them than the compiler
+// likes to hold, and each reload from the argument segment stalls the wave's step.
+#define HOLD(v) asm volatile("" : "+s"(v))
+
 // Persistent orbit integration with per-lane refill: a lane whose orbit ends
 // writes it out and takes the next one at once, so the lanes of a wave stay
 // busy however uneven the orbit lengths are.  A freshly taken orbit spends one
-// pass of the loop on the lookups at its start point (the pre-loop lookups of
-// orbit_response.c:199-210); every later pass is one step of :211-458.
-template <bool LOG>
+// pass of the loop, with dt = 0, on the lookups at its start point (the pre-loop
+// lookups of orbit_response.c:199-210); every later pass is one step of :211-458.
+//
+// The step is bound by the latency of its own instruction stream (a launch lasts as long as its
+// longest orbits), so the loop is one straight line: the arguments stay in registers, the cell
+// size comes from LDS without a generic load, the flush of a run and the end of an orbit are the
+// only branches a step usually takes.  The products and sums are written out as they round
+// (contraction off), so that every kernel that integrates an orbit gives the same bits.
+// Measured with one wave per SIMD (64^2 grids): 1.4 -> 0.8 us a step; 81000 orbits on 512^2 grids
+// 74 -> 42 ms, where the longest takes 37000 steps.
+template <bool LOG, bool CELL1>
 __device__ __forceinline__ void orbit32_body(const FastModel &F, const OrbitArgs32 &A, const float *s_cell) {
-  const int nb = F.dg_nbin, ngrid = nb * nb;
-  Lane32 L;
+#pragma clang fp contract(off)
+  const int nb = F.dg_nbin, nbL = F.dg_L;
+  float fginv = F.fg_invRmin, fgil = F.fg_invlog2Fac, dginv = F.dg_invRmin, dgil = F.dg_invlog2Fac;
+  float hGM = F.halo_GM, ha = F.halo_a, heps = F.halo_eps, bGM = F.bulge_GM, ba = F.bulge_a, beps = F.bulge_eps;
+  float fo = F.fo_v200, fc = F.fc;
+  int fgn = F.fg_nbin, forces = F.forces;
+  unsigned int vnz = F.vstream_nz;
+  HOLD(fginv); HOLD(fgil); HOLD(dginv); HOLD(dgil);
+  HOLD(hGM); HOLD(ha); HOLD(heps); HOLD(bGM); HOLD(ba); HOLD(beps);
+  HOLD(fo); HOLD(fc); HOLD(fgn); HOLD(forces); HOLD(vnz);
+  const GLOBAL char *acc = (const GLOBAL char *)F.acc, *vst = (const GLOBAL char *)F.vstream;
+  unsigned int max_steps = (unsigned int)F.max_steps;
+  HOLD(acc); HOLD(vst); HOLD(max_steps);
   Log32 lg;
-  lg.n = 0;
-  lg.blk = 0;
-  lg.full = false;
-  lg.held = false;
-  lg.qheld = false;
-  lg.q0 = lg.q1 = 0;
+  if(LOG) {
+    lg.q = (GLOBAL int *)A.log_q;
+    lg.v = (GLOBAL char *)A.log_v;
+    HOLD(lg.q); HOLD(lg.v);
+  }
+
+  int o = take_orbit32(A, nb);
+  if(o < 0) return;
+  lg.blk = -1;
   lg.next = lg.end = 0;
+  float x, y, z, vx, vy, vz, ax, ay, az, cellsize, fR, fz, vr2, vt2, vq2, vp2, hprev, radsign_prev, fac;
+  float w[kFields][4];
+  double timespan, tall;
+  float *slot = nullptr;
+  int type, tovs, quad, run, norbit, steps;
+  u16x2 blo, bhi;  // touched cells (R, z): lowest and highest lower-left corner
+  auto begin = [&]() {
+    type = A.otype[o];
+    tovs = F.tovs[type];
+    timespan = A.otint[o];
+    fac = (float)(A.omass[o] / timespan);  // mass / timespan, folded into every trapezoid weight
+    if(!LOG) slot = A.slots + (size_t)(o - A.slot_base) * A.slot_stride;
+    x = (float)A.ox[o];
+    y = (float)A.oy[o];
+    z = (float)A.oz[o];
+    vx = (float)A.ovx[o];
+    vy = (float)A.ovy[o];
+    vz = (float)A.ovz[o];
+    ax = ay = az = cellsize = fR = fz = vr2 = vt2 = vq2 = vp2 = hprev = radsign_prev = 0.f;
+    tall = 0;
+    quad = run = -1;
+    norbit = 0;
+    steps = -1;  // the pass of the start point
+    blo = (unsigned short)nb;
+    bhi = (unsigned short)0;
+    lg.n = 0;
 #pragma unroll
-  for(int f = 0; f < kFields; f++) lg.tot[f] = 0.f;
-  auto flush = [&](const Run32 &r) {
-    if(LOG)
-      log32_flush(r, lg, L.o, A);
-    else
-      run32_flush(r, nb, ngrid, L.slot, L.locq, F);
+    for(int f = 0; f < kFields; f++) lg.tot[f] = 0.f;
+#pragma unroll
+    for(int f = 0; f < kFields; f++)
+#pragma unroll
+      for(int c = 0; c < 4; c++) w[f][c] = 0.f;
   };
-  float x, y, z, vx, vy, vz;
-  if(!take_orbit32(A, nb, L, x, y, z, vx, vy, vz)) return;
-  L.tovs = F.tovs[L.type];
-  bool fresh = true;
-  float ax = 0, ay = 0, az = 0;
-  int iR = 0, iz = 0;
-  float cellsize = 0.f;  // of the current point's density cell
-  float fR = 0, fz = 0, vr2 = 0, vt2 = 0, vq2 = 0, vp2 = 0;
-  Run32 run;
-  run.quad = -1;
-  int4 bb = make_int4(nb, -1, nb, -1);
-  float radsign_prev = 0.f;
-  int norbit = 0, flag = 0, status = 0;
-  long long steps = 0;
-  float dt = 0.f, hdt = 0.f;
-  // The trapezoid rule weights each point of the orbit by half of each step it
-  // ends or starts (orbit_response.c:283-319).  A point is binned once, with
-  // both halves: hprev, the half of the step that ended there, is added when
-  // the next step's dt is known.
-  float hprev = 0.f;
+  // the current point's block becomes the run's
+  auto change_block = [&]() {
+    if(run >= 0) run32_flush<LOG>(run, w, nb, lg, o, slot, A);
+    run = quad;
+    const u16x2 at = {(unsigned short)(quad & (nb - 1)), (unsigned short)(quad >> nbL)};
+    blo = __builtin_elementwise_min(blo, at);
+    bhi = __builtin_elementwise_max(bhi, at);
+#pragma unroll
+    for(int f = 0; f < kFields; f++)
+#pragma unroll
+      for(int c = 0; c < 4; c++) w[f][c] = 0.f;
+  };
+  begin();
   while(true) {
-    if(!fresh) {
-      float inv_v = fast_rsq(vx * vx + vy * vy + vz * vz);
-      float inv_a = fast_rsq(ax * ax + ay * ay + az * az);
-      dt = fminf(F.fo_v200 * inv_a, F.fc * cellsize * inv_v);
-      if(L.timespan < L.tall + (double)dt) {
-        dt = (float)(L.timespan - L.tall);
-        flag = 1;
+    const float inv_v = fast_rsq(__builtin_fmaf(vz, vz, __builtin_fmaf(vy, vy, vx * vx)));
+    const float inv_a = fast_rsq(__builtin_fmaf(az, az, __builtin_fmaf(ay, ay, ax * ax)));
+    float dt = __builtin_fminf(fo * inv_a, fc * cellsize * inv_v);
+    const bool fresh = steps < 0;
+    bool last = timespan < tall + (double)dt;
+    dt = last ? (float)(timespan - tall) : dt;
+    dt = fresh ? 0.f : dt;
+    last = last && !fresh;
+    int status = 0;
+    if(!(dt >= 0.f && dt < 3.0e38f)) {
+      status = GALIC_ERR_ARG;
+      dt = 0.f;
+    }
+    // The trapezoid rule weights each point of the orbit by half of each step it ends or starts
+    // (orbit_response.c:283-319).  A point is binned once, with both halves: hprev, the half of
+    // the step that ended there, is added when the next step's dt is known.
+    const float hdt = 0.5f * dt;
+    bin32(w, fR, fz, fac * __builtin_fmaf(0.5f, dt, hprev), vr2, vt2, vq2, vp2);
+    vx = __builtin_fmaf(hdt, ax, vx);
+    vy = __builtin_fmaf(hdt, ay, vy);
+    vz = __builtin_fmaf(hdt, az, vz);
+    x = __builtin_fmaf(dt, vx, x);
+    y = __builtin_fmaf(dt, vy, y);
+    z = __builtin_fmaf(dt, vz, z);
+
+    // the point's place on the force grid (log index of R and |z|) and its table values: every
+    // load of the step is issued here (indices clamped into the table; the off-grid force below
+    // does not use the force taps)
+    const float R2 = __builtin_fmaf(y, y, x * x);
+    float invR = fast_rsq(R2), R = R2 * invR;
+    if(!(R2 > 0)) R = invR = 0.f;
+    const float jd = fgil * fast_log2(__builtin_fmaf(fginv, R, 1.0f));
+    const float id = fgil * fast_log2(__builtin_fmaf(__builtin_fabsf(z), fginv, 1.0f));
+    const int jb = max((int)jd, 0), ib = max((int)id, 0);
+    const unsigned int k = __umul24(min(ib, fgn - 2), fgn) + min(jb, fgn - 2);
+    const f32x4_a8 t0 = *(const GLOBAL f32x4_a8 *)(acc + (k << 3));          // (DPotDR, DPotDz) at (z row, R column)
+    const f32x4_a8 t1 = *(const GLOBAL f32x4_a8 *)(acc + ((k + fgn) << 3));  // +(0,0), (0,1); (1,0), (1,1)
+    f32x2_a4 v0 = {0.f, 0.f}, v1 = {0.f, 0.f};
+    const bool streams = (vnz >> type) & 1u;
+    if(streams) {  // (a table of zeros, as the isotropic components have, gives vstr = +0 without its loads)
+      const GLOBAL char *V = vst + (((size_t)(unsigned int)(type * fgn) * fgn + k) << 2);
+      v0 = *(const GLOBAL f32x2_a4 *)V;
+      v1 = *(const GLOBAL f32x2_a4 *)(V + 4 * (size_t)fgn);
+    }
+    // the density cell (cell-centred log index) and its size, which sets the next step's dt
+    const float br = __builtin_fmaxf(__builtin_fmaf(dgil, fast_log2(__builtin_fmaf(R, dginv, 1.0f)), -0.5f), 0.f);
+    const float bz =
+        __builtin_fmaxf(__builtin_fmaf(dgil, fast_log2(__builtin_fmaf(__builtin_fabsf(z), dginv, 1.0f)), -0.5f), 0.f);
+    int iR = (int)br, iz = (int)bz;
+    fR = br - (float)iR;
+    fz = bz - (float)iz;
+    if(iR >= nb - 1) {
+      iR = nb - 2;
+      fR = 1.f;
+    }
+    if(iz >= nb - 1) {
+      iz = nb - 2;
+      fz = 1.f;
+    }
+    if(status == 0) quad = (iz << nbL) + iR;
+    cellsize = CELL1 ? s_cell[max(iR, iz)] : F.cellsize[(iz << nbL) + iR];
+
+    // forcegrid_get_acceleration (grid.c:122-197)
+    const float r2 = __builtin_fmaf(z, z, R2), ir2 = fast_rcp(r2);
+    float jf = jd - (float)jb, fi = id - (float)ib;
+    float ana = 0.f;
+    if(forces & 6) {
+      const float r = root32(r2);
+      if(forces & 2) ana = __builtin_fmaf(hGM, fast_rcp((r + heps) * (r + ha) * (r + ha)), 0.f);
+      if(forces & 4) ana = __builtin_fmaf(bGM, fast_rcp((r + beps) * (r + ba) * (r + ba)), ana);
+    }
+    ax = ay = az = 0.f;
+    if(forces & 1) {
+      const float w01 = jf * (1.0f - fi), w00 = (1.0f - jf) * (1.0f - fi), w10 = fi * (1.0f - jf), w11 = jf * fi;
+      const float aR = __builtin_fmaf(w11, t1.z, __builtin_fmaf(w10, t1.x, __builtin_fmaf(t0.x, w00, t0.z * w01)));
+      const float aZ = __builtin_fmaf(w11, t1.w, __builtin_fmaf(w10, t1.y, __builtin_fmaf(t0.y, w00, t0.w * w01)));
+      ax = aR * (R > 0 ? x * invR : 1.f);
+      ay = aR * (R > 0 ? y * invR : 0.f);
+      az = z < 0 ? -aZ : aZ;
+      if(max(ib, jb) >= fgn - 1) {  // off the grid
+        const float r = root32(r2);
+        const float g = hGM * fast_rcp((r + heps) * (r + ha) * (r + ha)) * -F.offgrid_fac;
+        ax = x * g;
+        ay = y * g;
+        az = z * g;
       }
-      if(!(dt >= 0.f && dt < 3.0e38f)) {
-        status = GALIC_ERR_ARG;
-        if(hprev > 0.f) bin32(run, nb, flush, iR, iz, fR, fz, L.fac * hprev, vr2, vt2, vq2, vp2, bb);
-      } else {
-        hdt = 0.5f * dt;
-        bin32(run, nb, flush, iR, iz, fR, fz, L.fac * (hprev + hdt), vr2, vt2, vq2, vp2, bb);
-        vx += hdt * ax;
-        vy += hdt * ay;
-        vz += hdt * az;
-        x += dt * vx;
-        y += dt * vy;
-        z += dt * vz;
-      }
     }
-    Fg32 g = fg_index32(F, x, y, z);
-    cell32(F, g.R, z, iR, iz, fR, fz);
-    const Taps32 taps = load_taps32(F, g, L.type, iR, iz, s_cell);
-    float nax, nay, naz;
-    accel32(F, x, y, z, g, taps, nax, nay, naz);
-    ax = nax;
-    ay = nay;
-    az = naz;
-    if(!fresh && status == 0) {
-      vx += hdt * ax;
-      vy += hdt * ay;
-      vz += hdt * az;
+    if(forces & 6) {
+      ax = __builtin_fmaf(-x, ana, ax);
+      ay = __builtin_fmaf(-y, ana, ay);
+      az = __builtin_fmaf(-z, ana, az);
     }
-    cellsize = taps.cell;
-    decompose32(L.tovs, vstream32(F, g, taps), x, y, z, vx, vy, vz, g, vr2, vt2, vq2, vp2);
-    if(fresh) {
-      fresh = false;
-      continue;
+    vx = __builtin_fmaf(hdt, ax, vx);
+    vy = __builtin_fmaf(hdt, ay, vy);
+    vz = __builtin_fmaf(hdt, az, vz);
+
+    // A run that ended is flushed here, as soon as the point's block is known and right after the
+    // wait for the loads: memory operations complete in order, so the next step's loads also wait
+    // for these stores, which now have the rest of the step and the start of the next to finish.
+    if(quad != run) change_block();
+
+    // vr2, vt2, vq2, vp2 of orbit_response.c:222-273 in closed form: spherical basis Q = (-y, x, 0),
+    // T = (-zx, -zy, R^2), |Q| = R, |T| = R r; velocity structure 2 the cylindrical one
+    const float vdR = __builtin_fmaf(x, vx, y * vy), radsign = __builtin_fmaf(z, vz, vdR);
+    const float vdT = __builtin_fmaf(R2, vz, -(z * vdR));
+    vr2 = ir2 * (radsign * radsign);
+    vt2 = invR * (invR * (ir2 * (vdT * vdT)));
+    if(tovs == 2) {
+      vr2 = invR * (invR * (vdR * vdR));
+      vt2 = vz * vz;
     }
+    // bilinear streaming velocity; beyond the last node the outermost column / row
+    float vstr = 0.f;
+    if(streams) {
+      if(jb >= fgn - 1) jf = 1.f;
+      if(ib >= fgn - 1) fi = 1.f;
+      const float gi = 1.0f - fi, gj = 1.0f - jf;
+      vstr = fi * (gj * v1.x);
+      vstr = __builtin_fmaf(gi, gj * v0.x, vstr);
+      vstr = __builtin_fmaf(gi, jf * v0.y, vstr);
+      vstr = __builtin_fmaf(fi, jf * v1.y, vstr);
+    }
+    const float cross = __builtin_fmaf(x, vy, -(y * vx));
+    const float vq = invR * cross, vp = __builtin_fmaf(invR, cross, -vstr);
+    vq2 = vq * vq;
+    vp2 = vp * vp;
+
     if(status == 0) {
       hprev = hdt;
-      if(flag) bin32(run, nb, flush, iR, iz, fR, fz, L.fac * hprev, vr2, vt2, vq2, vp2, bb);  // the orbit's last point
-      L.tall += (double)dt;
-      float radsign = vx * x + vy * y + vz * z;
-      if(radsign > 0 && radsign_prev < 0) norbit++;
-      radsign_prev = radsign;
+      tall += (double)dt;
+      norbit += (radsign > 0 && radsign_prev < 0) ? 1 : 0;
+      radsign_prev = fresh ? 0.f : radsign;
       steps++;
-      if(steps > F.max_steps) status = GALIC_ERR_STEPCAP;
+      if(steps > 0 && (unsigned int)steps > max_steps) status = GALIC_ERR_STEPCAP;
     }
-    if(flag || status) {
-      flush(run);
-      const int o = L.o;
+    if(last || status) {
+      if(last && status != GALIC_ERR_ARG) bin32(w, fR, fz, fac * hprev, vr2, vt2, vq2, vp2);  // the orbit's last point
+      const int n = max(steps, 0);
+      if(n > 0) run32_flush<LOG>(run, w, nb, lg, o, slot, A);
       if(LOG) {
-        log32_finish(lg, o, A);
-        A.log_n[o] = lg.full ? -1 : lg.n;
-        if(lg.full) atomicAdd(&A.stats[3], 1ull);
+        const bool full = lg.n > 0 && lg.blk < 0;
+        A.log_n[o] = full ? -1 : lg.n;
+        if(full) atomicAdd(&A.stats[3], 1ull);
 #pragma unroll
-        for(int f = 0; f < kFields; f++) {
-          A.log_tot[(size_t)o * kFields + f] = lg.tot[f];
-          lg.tot[f] = 0.f;
-        }
-        lg.n = 0;
-        lg.full = false;
+        for(int f = 0; f < kFields; f++) A.log_tot[(size_t)o * kFields + f] = lg.tot[f];
       }
-      A.tall[o] = L.tall;
+      A.tall[o] = tall;
       A.norbit[o] = norbit;
-      A.steps[o] = steps;
-      A.bbox[o] = bb;
+      A.steps[o] = n;
+      A.bbox[o] = n == 0 ? make_int4(nb, -1, nb, -1) : make_int4(blo.x, bhi.x + 1, blo.y, bhi.y + 1);
       A.status[o] = status;
       if(A.fin) {
-        float *fo = A.fin + (size_t)o * 6;
-        fo[0] = x;
-        fo[1] = y;
-        fo[2] = z;
-        fo[3] = vx;
-        fo[4] = vy;
-        fo[5] = vz;
+        float *e = A.fin + (size_t)o * 6;
+        e[0] = x;
+        e[1] = y;
+        e[2] = z;
+        e[3] = vx;
+        e[4] = vy;
+        e[5] = vz;
       }
-      orbit_stats_add(A.stats, steps, status, o);
-      if(!take_orbit32(A, nb, L, x, y, z, vx, vy, vz)) break;
-      L.tovs = F.tovs[L.type];
-      fresh = true;
-      run.quad = -1;
-      bb = make_int4(nb, -1, nb, -1);
-      radsign_prev = 0.f;
-      norbit = 0;
-      flag = 0;
-      status = 0;
-      steps = 0;
-      hprev = 0.f;
+      orbit_stats_add(A.stats, n, status, o);
+      o = take_orbit32(A, nb);
+      if(o < 0) break;
+      begin();
     }
   }
 }
 
 // (the cell-size table into LDS before any lane can leave)
-__device__ __forceinline__ void stage_cell1(const FastModel &F, float *s_cell) {
-  if(F.cell1)
+template <bool LOG>
+__device__ __forceinline__ void orbit32_run(const FastModel &F, const OrbitArgs32 &A, float *s_cell) {
+  if(F.cell1) {
     for(int i = threadIdx.x; i < F.dg_nbin; i += blockDim.x) s_cell[i] = F.cell1[i];
-  __syncthreads();
+    __syncthreads();
+    orbit32_body<LOG, true>(F, A, s_cell);
+  } else {
+    orbit32_body<LOG, false>(F, A, s_cell);
+  }
 }
 
 __global__ void __launch_bounds__(256) k_orbit32(FastModel F, OrbitArgs32 A) {
   __shared__ float s_cell[kCell1Max];
-  stage_cell1(F, s_cell);
-  orbit32_body<false>(F, A, s_cell);
+  orbit32_run<false>(F, A, s_cell);
 }
 __global__ void __launch_bounds__(256) k_orbit32_log(FastModel F, OrbitArgs32 A) {
   __shared__ float s_cell[kCell1Max];
-  stage_cell1(F, s_cell);
-  orbit32_body<true>(F, A, s_cell);
+  orbit32_run<true>(F, A, s_cell);
 }
 
 // ------------------------------------------------------------ trial draws --

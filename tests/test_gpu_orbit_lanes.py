@@ -50,3 +50,27 @@ def test_fp64_initial_pass_sorted(composite):
     assert np.array_equal(orbits, r["orbits"])
     assert g.stack(1, 0)[0] == pytest.approx(w.params.MType[1], rel=1e-12)
     g.close()
+
+
+# one lane, a full wave and one more, a full workgroup and one more, more orbits than resident lanes
+@pytest.mark.parametrize("n", [1, 64, 65, 257, 300001])
+def test_fp32_orbits_do_not_depend_on_the_launch(n):
+    """Batched FP32 orbits equal the same orbits integrated alone, bit for bit, and follow the FP64 path: the energies
+    at the start to rounding, the mass response of every orbit sums to its particle's mass (FP32 sums of some hundred
+    records: 1e-4)."""
+    cfg = model.config("composite-4e6", max_steps=2000000, torbit_fac=0.05, level=4)
+    w = model.make_workload(cfg, n=2000, target_samples=20000)
+    print(f"[gpu] fp32 orbits n={n}", flush=True)
+    i = np.arange(n) % w.n
+    g = GalicGPU(w)
+    few = n <= 257
+    r = g.orbit_responses(w.pos[i], w.vel[i], w.mass[i], w.tint[i], w.ptype[i], fields=few, precision=32)
+    for k in np.unique([0, n // 3, n // 2, n - 1]):
+        j = i[k]
+        one = g.orbit_responses(w.pos[j], w.vel[j], w.mass[j], w.tint[j], w.ptype[j], precision=32)
+        for key in ("t", "orbits", "steps", "e0", "e1") + (("fields",) if few else ()):
+            assert np.array_equal(r[key][k], one[key][0]), (n, k, key)
+        assert one["fields"][0][0].sum() == pytest.approx(w.mass[j], rel=1e-4)
+        assert one["e0"][0] == pytest.approx(g.orbit_responses(w.pos[j], w.vel[j], w.mass[j], w.tint[j], w.ptype[j],
+                                                              fields=False)["e0"][0], rel=1e-12)
+    g.close()
