@@ -100,19 +100,6 @@ void smooth_stack_host(double *data, int maxlevel) {
   }
 }
 
-// The set of nodes where calc_stack_difference's recursion stops
-// (grid.c:1090: l >= maxlevel or ref1 < thresh).  Positions never move, so
-// the reference's cuts are the same at every call.
-void mark_cut(const double *ref, double thresh, int l, int i, int j, int L, std::vector<char> &cut) {
-  int o = GALIC_STACKOFFSET(l, i, j);
-  if(l >= L || ref[o] < thresh) {
-    cut[o] = 1;
-    return;
-  }
-  for(int ii = 2 * i; ii <= 2 * i + 1; ii++)
-    for(int jj = 2 * j; jj <= 2 * j + 1; jj++) mark_cut(ref, thresh, l + 1, ii, jj, L, cut);
-}
-
 bool type_present(const galic_params &p, int t) { return p.NType[t] > 0; }
 
 int alloc_orbit_scratch(galic::Ctx &c, int n) {
@@ -323,85 +310,33 @@ galic::FitArgs fit_args(galic_ctx *ctx) {
   return F;
 }
 
-// Cut-A weights (density cut, fixed by DGs_MassTarget) and, once EGs_MassResponse
-// is known, the cut-B flags and the fine cell -> cut-B node map.
-int build_weights(galic_ctx *ctx, bool with_cutB) {
-  galic::Ctx &c = ctx->c;
-  const int Ns = c.Nstack, L = c.L, nb = c.Nbin;
-  ctx->weights.assign((size_t)GALIC_NTYPES * galic::W_COUNT * Ns, 0.0);
-  ctx->cutB_of.assign((size_t)GALIC_NTYPES * c.Ngrid, 0);
-  // per 16 x 16-cell tile (Morton index), the levels of its cut-A nodes: bit u for level L-u
-  // inside the tile (u = 0..4), bit 5 when the tile lies inside a cut-A node above its level
-  const int lt = L - 4, ntile = lt >= 0 ? 1 << (2 * lt) : 0;
-  std::vector<unsigned char> tcut((size_t)GALIC_NTYPES * ntile, 0);
-  std::vector<double> emr(Ns);
+// The cuts' weights, the fine cell -> cut-B node map and the tiles' cut levels, from the targets and
+// EGs_MassResponse (on the device, after the fit's stacks).
+int build_weights(galic::Ctx &c) {
+  const int lt = c.L - 4, ntile = lt >= 0 ? 1 << (2 * lt) : 0;
+  if(ntile > 0 && !c.tcut) CHK(dalloc(&c.tcut, (size_t)GALIC_NTYPES * ntile));
+  galic::CutArgs A;
+  memset(&A, 0, sizeof(A));
+  A.L = c.L;
   for(int t = 1; t < GALIC_NTYPES; t++) {
-    if(!type_present(c.p, t) || !c.targets_set[t]) continue;
-    double *W = &ctx->weights[(size_t)t * galic::W_COUNT * Ns];
-    const std::vector<double> &Tm = ctx->targets[t][0];
-    double thr_d = c.p.MinParticlesPerBinForDensityMeasurement * c.p.MType[t] / c.p.NType[t];
-    std::vector<char> cutA(Ns, 0);
-    mark_cut(Tm.data(), thr_d, 0, 0, 0, L, cutA);
-    for(int tz = 0; tz < (1 << std::max(lt, 0)) && lt >= 0; tz++)
-      for(int tr = 0; tr < (1 << lt); tr++) {
-        unsigned char m = 0;
-        for(int u = 0; u <= 4; u++) {
-          const int n = 16 >> u, l = L - u;
-          for(int i = 0; i < n && !(m & (1 << u)); i++)
-            for(int j = 0; j < n; j++)
-              if(cutA[GALIC_STACKOFFSET(l, tz * n + i, tr * n + j)]) {
-                m |= (unsigned char)(1 << u);
-                break;
-              }
-        }
-        for(int l = 0; l < lt; l++)
-          if(cutA[GALIC_STACKOFFSET(l, tz >> (lt - l), tr >> (lt - l))]) m |= 32;
-        int code = 0;
-        for(int b = 0; b < 6; b++) code |= (((tr >> b) & 1) << (2 * b)) | (((tz >> b) & 1) << (2 * b + 1));
-        tcut[(size_t)t * ntile + code] = m;
-      }
-    const double rlim = c.p.R200 / 20.0;
-    for(int o = 0; o < Ns; o++) {
-      if(!cutA[o]) continue;
-      double d = ctx->distance[o];
-      W[galic::W_A * Ns + o] = (d < rlim) ? d : rlim;  // min() of grid.c:1078-1084
-      // S-term weights Tm/E_x for E_x > 0 (grid.c:1128-1133), fields r, t, q, p
-      const int e_of[4] = {2, 3, 5, 4};  // targets[] order: Tm, MT, Er, Et, Ep, Eq
-      for(int k = 0; k < 4; k++) {
-        double e = ctx->targets[t][e_of[k]][o];
-        W[(galic::W_SR + k) * Ns + o] = (e > 0) ? Tm[o] / e : 0.0;
-      }
-    }
-    if(with_cutB) {
-      HIPCHK(hipMemcpy(emr.data(), c.stacks + ((size_t)t * galic::ST_COUNT + galic::ST_EMR) * Ns,
-                       sizeof(double) * Ns, hipMemcpyDeviceToHost));
-      double thr_s = c.p.MinParticlesPerBinForDispersionMeasurement * c.p.MType[t] / c.p.NType[t];
-      std::vector<char> cutB(Ns, 0);
-      mark_cut(emr.data(), thr_s, 0, 0, 0, L, cutB);
-      for(int o = 0; o < Ns; o++) W[galic::W_B * Ns + o] = cutB[o] ? 1.0 : 0.0;
-      int *cb = &ctx->cutB_of[(size_t)t * c.Ngrid];
-      for(int iz = 0; iz < nb; iz++)
-        for(int iR = 0; iR < nb; iR++) {
-          int node = -1;
-          for(int l = 0; l <= L && node < 0; l++) {
-            int o = GALIC_STACKOFFSET(l, iz >> (L - l), iR >> (L - l));
-            if(cutB[o]) node = o;
-          }
-          cb[iz * nb + iR] = node;
-        }
-    }
+    A.present[t] = (type_present(c.p, t) && c.targets_set[t]) ? 1 : 0;
+    if(!A.present[t]) continue;
+    A.thr_d[t] = c.p.MinParticlesPerBinForDensityMeasurement * c.p.MType[t] / c.p.NType[t];
+    A.thr_s[t] = c.p.MinParticlesPerBinForDispersionMeasurement * c.p.MType[t] / c.p.NType[t];
   }
-  HIPCHK(hipMemcpy(c.weights, ctx->weights.data(), sizeof(double) * ctx->weights.size(), hipMemcpyHostToDevice));
-  if(ntile > 0) {
-    if(!c.tcut) CHK(dalloc(&c.tcut, tcut.size()));
-    HIPCHK(hipMemcpy(c.tcut, tcut.data(), tcut.size(), hipMemcpyHostToDevice));
-  }
-  if(with_cutB)
-    HIPCHK(hipMemcpy(c.cutB_of, ctx->cutB_of.data(), sizeof(int) * ctx->cutB_of.size(), hipMemcpyHostToDevice));
+  A.rlim = c.p.R200 / 20.0;
+  A.stacks = c.stacks;
+  A.weights = c.weights;
+  A.cutB_of = c.cutB_of;
+  A.tcut = c.tcut;
+  hipLaunchKernelGGL(galic::k_cut_weights, dim3(nblocks(c.Nstack, 256), GALIC_NTYPES), dim3(256), 0, c.stream, A);
+  hipLaunchKernelGGL(galic::k_cut_cells, dim3(nblocks(c.Ngrid, 256), GALIC_NTYPES), dim3(256), 0, c.stream, A);
+  if(ntile > 0) hipLaunchKernelGGL(galic::k_cut_tiles, dim3(ntile, GALIC_NTYPES), dim3(64), 0, c.stream, A);
+  HIPCHK(hipGetLastError());
   return GALIC_OK;
 }
 
-// The fit's kernels on c.stream (the first call also sets the cuts, which waits for the stream).
+// The fit's kernels on c.stream (the first call also sets the cuts).
 int global_fit_launch(galic_ctx *ctx) {
   galic::Ctx &c = ctx->c;
   galic::FitArgs F = fit_args(ctx);
@@ -415,8 +350,7 @@ int global_fit_launch(galic_ctx *ctx) {
   }
   HIPCHK(hipGetLastError());
   if(!c.cuts_ready) {
-    HIPCHK(hipStreamSynchronize(c.stream));
-    CHK(build_weights(ctx, true));
+    CHK(build_weights(c));
     c.cuts_ready = true;
   }
   hipLaunchKernelGGL(galic::k_fit_partial, dim3(galic::kFitBlocks, 3), dim3(256), 0, c.stream, F, c.fit_part,
@@ -1045,8 +979,6 @@ int galic_create(const galic_params *p, int device, galic_ctx **out) {
   CHK(galic_density_geometry(p, ctx->cellsize.data(), nullptr, ctx->distance.data()));
   HIPCHK(hipMemcpy(c.DG_CellSize, ctx->cellsize.data(), sizeof(double) * c.Ngrid, hipMemcpyHostToDevice));
   CHK(upload_cell_sizes_f(c, ctx->cellsize.data()));
-  for(int t = 1; t < GALIC_NTYPES; t++)
-    for(int k = 0; k < 6; k++) ctx->targets[t][k].assign(c.Nstack, 0.0);
 
   // device model
   galic::DevModel &M = c.M;
@@ -1278,7 +1210,6 @@ int galic_set_targets(galic_ctx *ctx, int type, const double *dgs_mass_target, c
   const double *src[6] = {dgs_mass_target, egs_mass_target, egs_r, egs_t, egs_p, egs_q};
   const int dst[6] = {galic::ST_MT, galic::ST_EMT, galic::ST_ER, galic::ST_ET, galic::ST_EP, galic::ST_EQ};
   for(int k = 0; k < 6; k++) {
-    ctx->targets[type][k].assign(src[k], src[k] + c.Nstack);
     HIPCHK(hipMemcpy(c.stacks + ((size_t)type * galic::ST_COUNT + dst[k]) * c.Nstack, src[k],
                      sizeof(double) * c.Nstack, hipMemcpyHostToDevice));
   }
@@ -1542,7 +1473,6 @@ int galic_calc_all_response_fields(galic_ctx *ctx) {
   HIPCHK(hipMemsetAsync(c.locM, 0, sizeof(double) * GALIC_NTYPES * c.Ngrid, c.stream));
   HIPCHK(hipMemsetAsync(c.fit, 0, sizeof(double) * GALIC_NTYPES * 16, c.stream));
   c.cuts_ready = false;
-  CHK(build_weights(ctx, false));
   hipLaunchKernelGGL(galic::k_prepare_all, dim3(nblocks(n, 256)), dim3(256), 0, c.stream, n, 0, c.P, orbit_in(c));
   HIPCHK(hipGetLastError());
   galic::OrbitArgs A = orbit_args(c, n);
@@ -1840,7 +1770,6 @@ int galic_fp32_calc_all_response_fields(galic_ctx *ctx) {
   HIPCHK(hipMemsetAsync(c.locM_q, 0, sizeof(long long) * nm, c.stream));
   HIPCHK(hipMemsetAsync(c.fit, 0, sizeof(double) * GALIC_NTYPES * 16, c.stream));
   c.cuts_ready = false;
-  CHK(build_weights(ctx, false));
   hipLaunchKernelGGL(galic::k_prepare_all, dim3(nblocks(n, 256)), dim3(256), 0, c.stream, n, 0, c.P, orbit_in(c));
   HIPCHK(hipGetLastError());
   // the orbits into response logs, chunk by chunk as the arena holds them, each chunk's

@@ -563,6 +563,82 @@ __global__ void k_commit(double *loc, double *delta, size_t n) {
   delta[k] = 0;
 }
 
+// The cuts of calc_stack_difference (grid.c:1090: the recursion stops where l >= maxlevel or ref
+// < thresh) and what the merit needs on them.  Positions never move and the targets are fixed, so
+// the cuts are the same at every call.  A node is on a cut when it stops the recursion and none of
+// its ancestors does: every node, tile and cell looks down its own path from the root, so the
+// passes over the stacks (30 ms a type on the host at 512^2 cells) are a few microseconds here.
+__device__ __forceinline__ int cut_level(const double *ref, double thresh, int L, int l, int i, int j) {
+  for(int a = 0; a < l; a++)
+    if(ref[GALIC_STACKOFFSET(a, i >> (l - a), j >> (l - a))] < thresh) return a;
+  return (l >= L || ref[GALIC_STACKOFFSET(l, i, j)] < thresh) ? l : l + 1;  // (l + 1: the recursion goes on)
+}
+
+// Per node: min(dist, R200/20) and Tm/E_x on the cut of DGs_MassTarget (grid.c:1078-1084,
+// 1128-1133), 1 on the cut of EGs_MassResponse.
+__global__ void k_cut_weights(CutArgs A) {
+  const int o = blockIdx.x * blockDim.x + threadIdx.x, t = blockIdx.y, L = A.L, Ns = GALIC_NSTACK(L);
+  if(o >= Ns) return;
+  int l = 0;
+  while(l < L && o >= GALIC_STACKOFFSET(l + 1, 0, 0)) l++;
+  const int k = o - GALIC_STACKOFFSET(l, 0, 0), i = k >> l, j = k & ((1 << l) - 1);
+  const double *S = A.stacks + (size_t)t * ST_COUNT * Ns;
+  double *W = A.weights + (size_t)t * W_COUNT * Ns;
+  double w[W_COUNT] = {0, 0, 0, 0, 0, 0};
+  if(A.present[t]) {
+    const double *Tm = S + ST_MT * Ns;
+    if(cut_level(Tm, A.thr_d[t], L, l, i, j) == l) {
+      const double d = S[ST_DIST * Ns + o];
+      w[W_A] = (d < A.rlim) ? d : A.rlim;
+      const int st[4] = {ST_ER, ST_ET, ST_EQ, ST_EP};
+      for(int f = 0; f < 4; f++) {
+        const double e = S[st[f] * Ns + o];
+        w[W_SR + f] = (e > 0) ? Tm[o] / e : 0.0;
+      }
+    }
+    if(cut_level(S + ST_EMR * Ns, A.thr_s[t], L, l, i, j) == l) w[W_B] = 1.0;
+  }
+  for(int f = 0; f < W_COUNT; f++) W[(size_t)f * Ns + o] = w[f];
+}
+
+// Per fine cell: its node on the cut of EGs_MassResponse.
+__global__ void k_cut_cells(CutArgs A) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x, t = blockIdx.y, L = A.L, ng = 1 << (2 * L);
+  if(c >= ng) return;
+  const int i = c >> L, j = c & ((1 << L) - 1);
+  int node = 0;
+  if(A.present[t]) {
+    const int l = cut_level(A.stacks + ((size_t)t * ST_COUNT + ST_EMR) * GALIC_NSTACK(L), A.thr_s[t], L, L, i, j);
+    node = GALIC_STACKOFFSET(l, i >> (L - l), j >> (L - l));
+  }
+  A.cutB_of[(size_t)t * ng + c] = node;
+}
+
+// Per 16 x 16-cell tile (Morton index), the levels of its nodes on the cut of DGs_MassTarget: bit u
+// for level L-u inside the tile (u = 0..4), bit 5 when the tile lies inside a cut node above its
+// level.  One wave per tile.
+__global__ void __launch_bounds__(64) k_cut_tiles(CutArgs A) {
+  const int L = A.L, lt = L - 4, ntile = 1 << (2 * lt), m = blockIdx.x, t = blockIdx.y, lane = threadIdx.x;
+  int tz = 0, tr = 0;
+  for(int b = 0; b < lt; b++) {
+    tr |= ((m >> (2 * b)) & 1) << b;
+    tz |= ((m >> (2 * b + 1)) & 1) << b;
+  }
+  unsigned int bits = 0;
+  if(A.present[t]) {
+    const double *Tm = A.stacks + ((size_t)t * ST_COUNT + ST_MT) * GALIC_NSTACK(L);
+    for(int u = 0; u <= 4; u++) {
+      const int n = 16 >> u;
+      bool on = false;
+      for(int q = lane; q < n * n; q += 64)
+        on = on || cut_level(Tm, A.thr_d[t], L, L - u, tz * n + q / n, tr * n + q % n) == L - u;
+      if(__ballot(on)) bits |= 1u << u;
+    }
+    if(cut_level(Tm, A.thr_d[t], L, lt, tz, tr) < lt) bits |= 32u;
+  }
+  if(lane == 0) A.tcut[(size_t)t * ntile + m] = (unsigned char)bits;
+}
+
 // One workgroup per (type, stack): copy the fine level from a Loc grid and
 // build the coarse levels as in smooth_stack (grid.c:1247-1265).
 __global__ void k_fit_stacks(FitArgs A) {

@@ -8,12 +8,8 @@
 
 struct galic_ctx {
   galic::Ctx c;
-  // host copies of the targets (DGs_MassTarget, EGs_MassTarget, EGs_EgyTarget_r, _t, _p, _q)
-  // and of the geometry, used to build the cuts
-  std::vector<double> targets[GALIC_NTYPES][6];
+  // host copies of the geometry
   std::vector<double> distance, cellsize;
-  std::vector<double> weights;  // [type][W_COUNT][Nstack]
-  std::vector<int> cutB_of;     // [type][Ngrid]
   bool initial_done = false;
   bool fp32_initial_done = false;
 };

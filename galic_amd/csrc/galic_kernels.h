@@ -70,6 +70,20 @@ struct FitArgs {
   double lowdisp;
 };
 
+struct CutArgs {
+  int L;
+  int present[GALIC_NTYPES];
+  double thr_d[GALIC_NTYPES], thr_s[GALIC_NTYPES];  // thresholds of the density and the dispersion cut
+  double rlim;                                      // R200 / 20
+  const double *stacks;
+  double *weights;
+  int *cutB_of;
+  unsigned char *tcut;
+};
+__global__ void k_cut_weights(CutArgs A);
+__global__ void k_cut_cells(CutArgs A);
+__global__ void k_cut_tiles(CutArgs A);
+
 __global__ void k_orbit64(DevModel M, OrbitArgs A, int qpw);
 __global__ void k_expect_steps(DevModel M, int n, const double *ox, const double *oy, const double *oz,
                                const double *ovx, const double *ovy, const double *ovz, const double *otint,
