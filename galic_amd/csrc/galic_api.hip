@@ -170,14 +170,15 @@ void swap_orbit_set(galic::Ctx &c) {
 // The other set's stream, events and counters (its arrays grow on demand when it is active).
 int ensure_alt_set(galic::Ctx &c) {
   if(c.alt_ready) return GALIC_OK;
+  const int log_M = c.log_M;
   swap_orbit_set(c);
   int rc = GALIC_OK;
-  c.log_M = 64;
+  c.log_M = log_M;
   if(hipStreamCreate(&c.stream) != hipSuccess || hipEventCreate(&c.ev0) != hipSuccess ||
      hipEventCreate(&c.ev1) != hipSuccess)
     rc = set_err(GALIC_ERR_HIP, "creating the second orbit stream failed");
   if(rc == GALIC_OK) rc = dalloc(&c.counter, 1);
-  if(rc == GALIC_OK) rc = dalloc(&c.orbit_stats, 4);
+  if(rc == GALIC_OK) rc = dalloc(&c.orbit_stats, 6);
   if(rc == GALIC_OK) rc = dalloc(&c.log_next, 1);
   swap_orbit_set(c);
   if(rc == GALIC_OK) c.alt_ready = true;
@@ -242,7 +243,8 @@ int orbit_grid(int n, int bs, int per_cu = 8) {
 }
 
 // Steps and the first failure of an orbit launch (orbit_response.c:449-456 exits on the step cap).
-int finish_orbit_launch(galic::Ctx &c, int n) {
+// pidx (device, or null): the particle of each orbit, named in place of the orbit.
+int finish_orbit_launch(galic::Ctx &c, int n, const int *pidx = nullptr) {
   unsigned long long st[3];
   HIPCHK(hipMemcpyAsync(st, c.orbit_stats, sizeof(st), hipMemcpyDeviceToHost, c.stream));
   HIPCHK(hipStreamSynchronize(c.stream));
@@ -251,6 +253,7 @@ int finish_orbit_launch(galic::Ctx &c, int n) {
   if(st[1]) {
     long long status = (long long)st[2];
     int o = (int)(st[1] - 1);
+    if(pidx) HIPCHK(hipMemcpy(&o, pidx + o, sizeof(int), hipMemcpyDeviceToHost));
     if(status == GALIC_ERR_STEPCAP)
       return set_err(GALIC_ERR_STEPCAP, "orbit %d exceeded the step cap of %lld steps", o, (long long)c.M.max_steps);
     return set_err(GALIC_ERR_ARG, "orbit %d has a non-positive or non-finite timestep", o);
@@ -261,7 +264,7 @@ int finish_orbit_launch(galic::Ctx &c, int n) {
 int launch_orbit64(galic::Ctx &c, galic::OrbitArgs A) {
   if(A.n <= 0) return GALIC_OK;
   HIPCHK(hipMemsetAsync(c.counter, 0, sizeof(unsigned int), c.stream));
-  HIPCHK(hipMemsetAsync(c.orbit_stats, 0, 4 * sizeof(unsigned long long), c.stream));
+  HIPCHK(hipMemsetAsync(c.orbit_stats, 0, 6 * sizeof(unsigned long long), c.stream));
   HIPCHK(hipEventRecord(c.ev0, c.stream));
   // A quad of lanes per orbit, at least 4 quads a wave (waves of one or two quads ran 1.5 times
   // slower once four of them shared a CU; alone on their CU they are the fastest), the wave
@@ -447,7 +450,7 @@ galic::OrbitArgs32 orbit_args32(galic::Ctx &c, int n) {
 int launch_orbit32(galic::Ctx &c, galic::OrbitArgs32 A) {
   if(A.n <= 0) return GALIC_OK;
   HIPCHK(hipMemsetAsync(c.counter, 0, sizeof(unsigned int), c.stream));
-  HIPCHK(hipMemsetAsync(c.orbit_stats, 0, 4 * sizeof(unsigned long long), c.stream));
+  HIPCHK(hipMemsetAsync(c.orbit_stats, 0, 6 * sizeof(unsigned long long), c.stream));
   HIPCHK(hipEventRecord(c.ev0, c.stream));
   const int bs = 256;
   hipLaunchKernelGGL(galic::k_orbit32, dim3(orbit_grid(A.n, bs, c.fp32_bpc)), dim3(bs), 0, c.stream, fast_model(c),
@@ -483,10 +486,11 @@ void log_setup(galic::Ctx &c) {
 
 size_t log_block_bytes() { return (size_t)galic::LOG_B * (sizeof(int) + galic::kFields * sizeof(float4)); }
 
-// The log arena (the `slots` buffer): reallocated only when it is below half of
-// what a call could use, so repeated calls reuse one allocation.
+// The log arena (the `slots` buffer), kept across calls: reallocated only when it is so far below
+// what a call could use (kLogFitMargin / kLogPlanMargin of it) that the call would need another
+// launch.
 int ensure_arena(galic::Ctx &c, size_t want, size_t need) {
-  if(c.slot_bytes >= need && 2 * c.slot_bytes >= want) return GALIC_OK;
+  if(c.slot_bytes >= need && c.slot_bytes >= want / 100 * 89) return GALIC_OK;
   if(c.slots) (void)hipFree(c.slots);
   c.slots = nullptr;
   c.slot_bytes = 0;
@@ -496,11 +500,24 @@ int ensure_arena(galic::Ctx &c, size_t want, size_t need) {
   return GALIC_OK;
 }
 
-// Arena blocks planned for a launch of n orbits: the running estimate per orbit
-// with a margin, and the blocks the lanes may claim and leave unused.
+// Blocks the lanes of a launch may claim and leave unused.
+double log_blocks_slack(const galic::Ctx &c, int n) {
+  return (double)orbit_grid(n, 256, c.fp32_bpc) * 256 * galic::LOG_CHUNK + 64;
+}
+
+// Arena blocks planned for a launch of n orbits: the blocks an orbit's log took in the last launch
+// (counted exactly, also where the arena ran out) with a margin for other orbits.  The arena is
+// sized with the larger margin and a launch with the smaller, so that a call whose logs grew a
+// little since the arena was allocated still goes out as one launch: two launches last twice as
+// long as their longest orbits.
+constexpr double kLogPlanMargin = 1.2, kLogFitMargin = 1.06;
 double log_blocks_planned(const galic::Ctx &c, int n) {
-  const double lanes = (double)orbit_grid(n, 256, c.fp32_bpc) * 256;
-  return (double)n * (c.log_est_blocks + 1.0) * 1.25 + lanes * galic::LOG_CHUNK + 64;
+  return (double)n * c.log_est_blocks * kLogPlanMargin + log_blocks_slack(c, n);
+}
+// Orbits, of a call of n, that fit the arena at once.
+double log_orbits_fit(const galic::Ctx &c, int n) {
+  const double blocks = (double)(c.slot_bytes / ((size_t)galic::LOG_B * (sizeof(int) + galic::kFields * sizeof(float4))));
+  return (blocks - log_blocks_slack(c, n)) / (c.log_est_blocks * kLogFitMargin);
 }
 
 constexpr int kLogArenaFull = 1;  // launch_orbit32_log: the arena ran out, plan a smaller launch
@@ -539,7 +556,7 @@ int orbit32_log_begin(galic::Ctx &c, galic::OrbitArgs32 &A) {
   A.log_cap = (unsigned int)std::min<size_t>(cap, 0xf0000000u);  // claims past the cap stay below 2^32
   HIPCHK(hipMemsetAsync(c.log_next, 0, sizeof(unsigned int), c.stream));
   HIPCHK(hipMemsetAsync(c.counter, 0, sizeof(unsigned int), c.stream));
-  HIPCHK(hipMemsetAsync(c.orbit_stats, 0, 4 * sizeof(unsigned long long), c.stream));
+  HIPCHK(hipMemsetAsync(c.orbit_stats, 0, 6 * sizeof(unsigned long long), c.stream));
   HIPCHK(hipEventRecord(c.ev0, c.stream));
   hipLaunchKernelGGL(galic::k_orbit32_log, dim3(orbit_grid(A.n, 256, c.fp32_bpc)), dim3(256), 0, c.stream,
                      fast_model(c), A);
@@ -549,33 +566,30 @@ int orbit32_log_begin(galic::Ctx &c, galic::OrbitArgs32 &A) {
 }
 
 // Waits for the launch of orbit32_log_begin.  If an orbit needed more blocks than its table
-// holds, the table grows and kLogTableFull asks for the same launch again (the orbits and their
-// logs do not depend on the launch, so the result is the same); if the arena ran out, the block
-// estimate doubles and kLogArenaFull asks the caller for a smaller launch.
+// holds, the tables grow to the longest log and kLogTableFull asks for the same launch again (the
+// orbits and their logs do not depend on the launch, so the result is the same); if the arena ran
+// out, kLogArenaFull asks the caller for a smaller launch, planned with the blocks it needed.
 int orbit32_log_end(galic::Ctx &c, const galic::OrbitArgs32 &A) {
   const size_t cap = c.slot_bytes / log_block_bytes();
   HIPCHK(hipEventSynchronize(c.ev1));
   float ms = 0;
   HIPCHK(hipEventElapsedTime(&ms, c.ev0, c.ev1));
-  unsigned long long st[4];
+  unsigned long long st[6];
   unsigned int used = 0;
   HIPCHK(hipMemcpyAsync(st, c.orbit_stats, sizeof(st), hipMemcpyDeviceToHost, c.stream));
   HIPCHK(hipMemcpyAsync(&used, c.log_next, sizeof(used), hipMemcpyDeviceToHost, c.stream));
   HIPCHK(hipStreamSynchronize(c.stream));
+  c.log_est_blocks = std::max(1.0, (double)st[4] / A.n);
   if(st[3] == 0) {
     c.last_orbit_ms = ms;
     c.acc_orbit_ms += ms;
     c.acc_orbit_launches++;
-    c.log_est_blocks = std::max(1.0, (double)std::min<size_t>(used, cap) / A.n);
-    return finish_orbit_launch(c, A.n);
+    return finish_orbit_launch(c, A.n, A.pidx);
   }
   c.acc_log_relaunches++;
-  if((size_t)used >= cap) {
-    c.log_est_blocks *= 2;
-    return kLogArenaFull;
-  }
-  c.log_M *= 2;  // an orbit needed more blocks than its table holds
-  return kLogTableFull;
+  const size_t blocks = (size_t)(st[5] / galic::LOG_B) + 1;
+  while((size_t)c.log_M < blocks) c.log_M *= 2;
+  return (size_t)used >= cap ? kLogArenaFull : kLogTableFull;
 }
 
 // One launch of the logging orbit kernel, waited on (tables grown and the launch repeated as
@@ -612,9 +626,6 @@ size_t slot_budget(galic::Ctx &c) {
   return std::max<size_t>((size_t)1 << 30, std::min(cap, have));
 }
 
-// The orbits of the initial pass (prepared at o_* [0, n)) through the logging kernel in
-// chunks the arena holds, each chunk's logs added to the Loc grids by k_log_to_loc.  The
-// first chunk is small: it sets the estimate of log blocks per orbit for the others.
 // Adds logs to dst (fixed-point Loc grids [type][5][Ngrid]) through region buckets: the
 // entries of each (type, region) are counted on the device, their buckets laid out here, the
 // entries scattered, then summed region chunk by region chunk (galic_commit.hip).  A.n items,
@@ -759,33 +770,68 @@ int commit_logs_launch(galic::Ctx &c, galic::CommitArgs A, long long *dst, size_
   return GALIC_OK;
 }
 
+// Every particle's orbit through the logging kernel and its records into the Loc grids.  The
+// orbits are taken longest expected first, in as many launches as the arena asks for, each a
+// strided share of that order: the launches are alike, so one plan holds for all of them, and each
+// ends with its short orbits.  (Integer sums: the grids do not depend on the order.)
 int fp32_initial_logs(galic::Ctx &c, int n) {
-  const size_t bb = log_block_bytes();
+  const galic::Particles &P = c.P;
+  CHK(alloc_sort_scratch(c, n));
+  hipLaunchKernelGGL(galic::k_expect_steps, dim3(nblocks(n, 256)), dim3(256), 0, c.stream, c.M, n, (const double *)P.x,
+                     (const double *)P.y, (const double *)P.z, (const double *)P.vx, (const double *)P.vy,
+                     (const double *)P.vz, (const double *)P.tint, c.t_key, c.t_ord);
+  HIPCHK(hipGetLastError());
+  if(c.log_est_blocks <= 0) {
+    // nothing measured yet: about a record per two expected steps
+    unsigned long long sum[2];
+    HIPCHK(hipMemsetAsync(c.orbit_stats, 0, sizeof(sum), c.stream));
+    hipLaunchKernelGGL(galic::k_sum_keys, dim3(std::min(nblocks(n, 256), 1024)), dim3(256), 0, c.stream, n,
+                       (const unsigned int *)c.t_key, c.orbit_stats);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(sum, c.orbit_stats, sizeof(sum), hipMemcpyDeviceToHost, c.stream));
+    HIPCHK(hipStreamSynchronize(c.stream));
+    const double mean = std::min(1e6, (double)sum[0] / n), longest = std::min(1e6, (double)sum[1]);
+    c.log_est_blocks = 1 + 0.5 * mean / galic::LOG_B;
+    while(c.log_M < 0.5 * longest / galic::LOG_B) c.log_M *= 2;
+  }
+  if(galic::sort_desc(n, c.t_key, c.t_key2, c.t_ord, c.t_ord2, &c.sort_tmp, &c.sort_tmp_bytes, c.stream) != 0)
+    return set_err(GALIC_ERR_HIP, "sorting the particles by expected orbit length failed");
   {
+    const size_t bb = log_block_bytes();
     const size_t all = (size_t)(log_blocks_planned(c, n) * bb);
-    const size_t one = (size_t)(log_blocks_planned(c, std::min(n, 4096)) * bb);
+    const size_t one = (size_t)(log_blocks_planned(c, std::min(n, 1024)) * bb);
     CHK(ensure_arena(c, std::min(all, slot_budget(c)), one));
   }
-  int a = 0;
-  bool first = true;
-  while(a < n) {
-    const double blocks = (double)(c.slot_bytes / bb);
-    const double lanes = (double)orbit_grid(n - a, 256, c.fp32_bpc) * 256;
-    double fit = (blocks - 64 - lanes * galic::LOG_CHUNK) / ((c.log_est_blocks + 1.0) * 1.25);
-    if(first) fit = std::min(fit, 65536.0);
-    const int m = (int)std::max(1.0, std::min((double)(n - a), fit));
+  struct Share {
+    int first, stride;
+  };
+  std::vector<Share> todo;
+  {
+    const int shares = (int)std::min((double)n, std::ceil(n / std::max(1.0, log_orbits_fit(c, n))));
+    for(int k = shares - 1; k >= 0; k--) todo.push_back({k, shares});
+  }
+  while(!todo.empty()) {
+    const Share sh = todo.back();
+    todo.pop_back();
+    const int m = (n - sh.first + sh.stride - 1) / sh.stride;
+    CHK(alloc_orbit_scratch(c, m));
+    hipLaunchKernelGGL(galic::k_prepare_list, dim3(nblocks(m, 256)), dim3(256), 0, c.stream, m,
+                       (const int *)c.t_ord2, sh.first, sh.stride, P, orbit_in(c));
+    HIPCHK(hipGetLastError());
     galic::OrbitArgs32 A = orbit_args32(c, m);
-    A.ox += a; A.oy += a; A.oz += a;
-    A.ovx += a; A.ovy += a; A.ovz += a;
-    A.omass += a; A.otint += a; A.otype += a;
-    A.tall += a; A.norbit += a; A.status += a; A.steps += a; A.bbox += a;
+    A.pidx = c.o_pidx;
     const int lr = launch_orbit32_log(c, A);
     if(lr == kLogArenaFull) {
       if(m <= 1) return set_err(GALIC_ERR_NOMEM, "the response log of one orbit does not fit in device memory");
-      continue;  // the estimate has doubled: plan the chunk again
+      todo.push_back({sh.first + sh.stride, 2 * sh.stride});
+      todo.push_back({sh.first, 2 * sh.stride});
+      continue;
     }
     CHK(lr);
-    // every record of the chunk's orbits into the Loc grids, in runs of orbits whose bucket
+    hipLaunchKernelGGL(galic::k_store_list, dim3(nblocks(m, 256)), dim3(256), 0, c.stream, m, (const int *)c.o_pidx,
+                       (const int *)c.o_norbit, (const long long *)c.o_steps, P.orbits, c.psteps);
+    HIPCHK(hipGetLastError());
+    // every record of the share's orbits into the Loc grids, in runs of orbits whose bucket
     // entries (about 1.3 per record) stay within kCommitEntries
     const double per_orbit = std::max(1.0, c.log_est_blocks * galic::LOG_B * 1.3);
     const int run = (int)std::max(1.0, std::min((double)m, (double)kCommitEntries / per_orbit));
@@ -794,11 +840,9 @@ int fp32_initial_logs(galic::Ctx &c, int n) {
       memset(&C, 0, sizeof(C));
       C.n = std::min(run, m - b0);
       C.orbit_base = b0;
-      C.otype = c.o_type + a + b0;
+      C.otype = c.o_type + b0;
       CHK(commit_logs(c, C, c.locA_q));
     }
-    a += m;
-    first = false;
   }
   return GALIC_OK;
 }
@@ -970,7 +1014,7 @@ int galic_create(const galic_params *p, int device, galic_ctx **out) {
   CHK(dalloc(&c.fit, (size_t)GALIC_NTYPES * 16));
   CHK(dalloc(&c.fit_part, (size_t)3 * galic::kFitBlocks * 5));
   CHK(dalloc(&c.counter, 1));
-  CHK(dalloc(&c.orbit_stats, 4));
+  CHK(dalloc(&c.orbit_stats, 6));
   CHK(dalloc(&c.log_next, 1));
 
   // geometry
@@ -1760,7 +1804,6 @@ int galic_fp32_calc_all_response_fields(galic_ctx *ctx) {
   if(n <= 0) return set_err(GALIC_ERR_STATE, "no particles set");
   for(int t = 1; t < GALIC_NTYPES; t++)
     if(type_present(c.p, t) && !c.targets_set[t]) return set_err(GALIC_ERR_STATE, "targets of type %d not set", t);
-  CHK(alloc_orbit_scratch(c, n));
   const size_t na = (size_t)GALIC_NTYPES * galic::kFields * c.Ngrid, ni = (size_t)GALIC_NTYPES * 4 * c.Ngrid,
                nm = (size_t)GALIC_NTYPES * c.Ngrid;
   HIPCHK(hipMemsetAsync(c.locA_q, 0, sizeof(long long) * na, c.stream));
@@ -1770,17 +1813,11 @@ int galic_fp32_calc_all_response_fields(galic_ctx *ctx) {
   HIPCHK(hipMemsetAsync(c.locM_q, 0, sizeof(long long) * nm, c.stream));
   HIPCHK(hipMemsetAsync(c.fit, 0, sizeof(double) * GALIC_NTYPES * 16, c.stream));
   c.cuts_ready = false;
-  hipLaunchKernelGGL(galic::k_prepare_all, dim3(nblocks(n, 256)), dim3(256), 0, c.stream, n, 0, c.P, orbit_in(c));
-  HIPCHK(hipGetLastError());
-  // the orbits into response logs, chunk by chunk as the arena holds them, each chunk's
+  // the orbits into response logs, launch by launch as the arena holds them, each launch's
   // records then added to the fixed-point Loc grids (the logging kernel keeps its lanes
   // integrating; atomics at every flush would stall them)
   log_setup(c);
   CHK(fp32_initial_logs(c, n));
-  hipLaunchKernelGGL(galic::k_store_orbits, dim3(nblocks(n, 256)), dim3(256), 0, c.stream, n, 0, c.o_norbit,
-                     c.P.orbits);
-  hipLaunchKernelGGL(galic::k_store_steps, dim3(nblocks(n, 256)), dim3(256), 0, c.stream, n,
-                     (const long long *)c.o_steps, c.psteps);
   hipLaunchKernelGGL(galic::k_inst_init_q, dim3(nblocks(n, 256)), dim3(256), 0, c.stream, c.M, c.P, c.locI_q,
                      c.locM_q, c.Ngrid, c.fp32_iscale, c.fp32_scale[0]);
   HIPCHK(hipGetLastError());
@@ -1803,7 +1840,7 @@ int galic_fp32_autotune(galic_ctx *ctx, int nsample, int *variant, int *blocks_p
   // no more orbits than the response logs of one launch fit in half the memory the arena may
   // take (the other half covers the blocks the lanes claim and leave unused)
   const double arena_blocks = (double)slot_budget(c) / log_block_bytes();
-  const double per_orbit = (c.log_est_blocks + 1.0) * 1.25;
+  const double per_orbit = c.log_est_blocks * kLogPlanMargin;
   const int fit_n = (int)std::max(1024.0, std::min(2e9, 0.5 * arena_blocks / per_orbit));
   const int n = std::min(std::min(nsample, c.P.n), fit_n);
   CHK(alloc_orbit_scratch(c, n));
@@ -1962,10 +1999,7 @@ int fp32_run(galic_ctx *ctx, int ntrial, const int *idx, int K, int rep_size, co
   const int bpc_alone = c.fp32_bpc, bpc_beside = c.fp32_bpc_overlap > 0 ? c.fp32_bpc_overlap : c.fp32_bpc;
   // trials whose orbits' logs fit in the arena at the current estimate (and the caller's cap)
   auto group_cap = [&]() {
-    const double blocks = (double)(c.slot_bytes / log_block_bytes());
-    const double per_trial = (K + 1) * (c.log_est_blocks + 1.0) * 1.25;
-    const double lanes = (double)orbit_grid(std::max(ntrial, 1) * (K + 1), 256, c.fp32_bpc) * 256;
-    double cap = std::min((double)std::max(ntrial, 1), (blocks - 64 - lanes * galic::LOG_CHUNK) / per_trial);
+    double cap = std::min((double)std::max(ntrial, 1), log_orbits_fit(c, std::max(ntrial, 1) * (K + 1)) / (K + 1));
     if(c.max_group_trials > 0) cap = std::min(cap, (double)c.max_group_trials);
     return (int)std::max(1.0, cap);
   };
@@ -2105,7 +2139,7 @@ int fp32_run(galic_ctx *ctx, int ntrial, const int *idx, int K, int rep_size, co
       }
       if(r != kLogArenaFull) return r;
       if(s1 - s0 <= 1) return set_err(GALIC_ERR_NOMEM, "the response logs of one trial do not fit in device memory");
-      cap = group_cap();
+      cap = std::max(1, std::min(group_cap(), (s1 - s0) / 4 * 3));
       s1 = plan(s0);
       CHK(start(s0, s1, A));
     }

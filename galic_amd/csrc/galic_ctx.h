@@ -150,7 +150,8 @@ struct Ctx {
   int4 *o_bbox = nullptr;
   unsigned int *counter = nullptr;
   unsigned long long *orbit_stats = nullptr;  // [0] steps of the launch, [1] first failed orbit + 1, [2] its status,
-                                              // [3] orbits whose response log overflowed
+                                              // [3] response logs that overflowed, [4] log blocks needed,
+                                              // [5] records of the longest log
 
   // per-trial scratch
   int max_trials = 0;
@@ -193,7 +194,7 @@ struct Ctx {
   unsigned int *log_next = nullptr;
   int *log_q = nullptr;          // the last launch's arena: quads, then values
   float4 *log_v = nullptr;
-  double log_est_blocks = 12;    // running estimate of arena blocks per orbit
+  double log_est_blocks = 0;     // arena blocks an orbit's log takes, of the last launch (0: none yet)
   float log_scale[5] = {0, 0, 0, 0, 0};  // record value -> exact int64 sum units (a power of two)
   double log_unit[5] = {0, 0, 0, 0, 0};   // its inverse
   double log_to_loc[5] = {0, 0, 0, 0, 0}; // int64 sum units -> Loc fixed point
@@ -235,7 +236,7 @@ struct Ctx {
   long long acc_orbit_launches = 0;
   long long acc_orbits = 0, acc_steps = 0;
   int fp32_variant = 0;   // orbit kernel variant (one so far)
-  int fp32_bpc = 4;       // persistent workgroups per CU for k_orbit32 (autotuned)
+  int fp32_bpc = 3;       // persistent workgroups per CU for k_orbit32 (autotuned)
   int fp32_bpc_overlap = 0;  // the same for the launches beside a group's judging (0: fp32_bpc)
   int fp32_nfresh = 0;    // device trials per particle drawn fresh (optimize()'s distribution)
   bool fp32_tuned = false;

@@ -39,7 +39,9 @@ struct OrbitArgs32 {
   int *norbit, *status;
   long long *steps;
   int4 *bbox;
-  unsigned long long *stats;
+  unsigned long long *stats;  // OrbitArgs' three, [3] logs that overflowed, [4] blocks the logs need, [5] the
+                              // longest log's records (both counted for overflowed logs too)
+  const int *pidx;     // the orbits' particles, for messages (host), or null
   float *fin;  // final x, y, z, vx, vy, vz per orbit, or null
   // response logs (k_orbit32_log): every flushed 2x2 run is appended as a record
   // (quad index, 4 cells x 5 fields of fac * weight in FP32) to the orbit's blocks
@@ -125,7 +127,10 @@ __global__ void k_draw_trials(DevModel M, int ntrial, int K, int nfresh, const i
                               const int *tovs_of_type, double *vtx, double *vty, double *vtz);
 __global__ void k_prepare_ktrials(int ntrial, int K, const int *order, const int *tidx, const double *vtx,
                                   const double *vty, const double *vtz, Particles P, OrbitIn O);
-__global__ void k_store_steps(int n, const long long *osteps, int *psteps);
+__global__ void k_prepare_list(int n, const int *order, int first, int stride, Particles P, OrbitIn O);
+__global__ void k_store_list(int n, const int *pidx, const int *norbit, const long long *osteps, int *orbits,
+                             int *psteps);
+__global__ void k_sum_keys(int n, const unsigned int *key, unsigned long long *sum);
 __global__ void k_invert_order(int n, const int *ord, int *inv);
 __global__ void k_energy32(DevModel M, int n, const double *ox, const double *oy, const double *oz, const double *ovx,
                            const double *ovy, const double *ovz, const float *fin, double *e0, double *e1);

@@ -394,6 +394,8 @@ __device__ __forceinline__ void orbit32_body(const FastModel &F, const OrbitArgs
         const bool full = lg.n > 0 && lg.blk < 0;
         A.log_n[o] = full ? -1 : lg.n;
         if(full) atomicAdd(&A.stats[3], 1ull);
+        atomicAdd(&A.stats[4], (unsigned long long)((lg.n + LOG_B - 1) / LOG_B));
+        atomicMax(&A.stats[5], (unsigned long long)lg.n);
 #pragma unroll
         for(int f = 0; f < kFields; f++) A.log_tot[(size_t)o * kFields + f] = lg.tot[f];
       }
@@ -562,9 +564,47 @@ __global__ void k_step_keys(int ntrial, const int *tidx, const int *psteps, unsi
   ord[i] = i;
 }
 
-__global__ void k_store_steps(int n, const long long *osteps, int *psteps) {
-  int o = blockIdx.x * blockDim.x + threadIdx.x;
-  if(o < n) psteps[o] = (int)min(osteps[o], (long long)0x7fffffff);
+// Orbits of particles order[first + j * stride], j = 0 .. n-1, at their current velocities.
+__global__ void k_prepare_list(int n, const int *order, int first, int stride, Particles P, OrbitIn O) {
+  const int o = blockIdx.x * blockDim.x + threadIdx.x;
+  if(o >= n) return;
+  const int p = order[(size_t)first + (size_t)o * stride];
+  O.pidx[o] = p;
+  O.ox[o] = P.x[p];
+  O.oy[o] = P.y[p];
+  O.oz[o] = P.z[p];
+  O.ovx[o] = P.vx[p];
+  O.ovy[o] = P.vy[p];
+  O.ovz[o] = P.vz[p];
+  O.omass[o] = P.mass[p];
+  O.otint[o] = P.tint[p];
+  O.otype[o] = P.type[p];
+}
+
+// Pericentre passages and steps of a launch's orbits to their particles.
+__global__ void k_store_list(int n, const int *pidx, const int *norbit, const long long *osteps, int *orbits,
+                             int *psteps) {
+  const int o = blockIdx.x * blockDim.x + threadIdx.x;
+  if(o >= n) return;
+  orbits[pidx[o]] = norbit[o];
+  psteps[pidx[o]] = (int)min(osteps[o], (long long)0x7fffffff);
+}
+
+// sum[0] += the keys' sum, sum[1] = their maximum.
+__global__ void __launch_bounds__(256) k_sum_keys(int n, const unsigned int *key, unsigned long long *sum) {
+  unsigned long long s = 0, m = 0;
+  for(int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    s += key[i];
+    m = max(m, (unsigned long long)key[i]);
+  }
+  for(int d = 32; d > 0; d >>= 1) {
+    s += __shfl_xor(s, d);
+    m = max(m, (unsigned long long)__shfl_xor(m, d));
+  }
+  if((threadIdx.x & 63) == 0) {
+    atomicAdd(&sum[0], s);
+    atomicMax(&sum[1], m);
+  }
 }
 
 // Records of each trial's K+1 logs (the merit kernel's work for it).
