@@ -45,20 +45,26 @@ constexpr int kMaxDepth = 21;
 struct Tree {
   int nsrc = 0;
   int cap = 0;
-  // sorted sources
-  double *x = nullptr, *y = nullptr, *z = nullptr, *m = nullptr;
+  double corner[3] = {0, 0, 0}, dlen = 1;  // the domain cube
+  // sorted sources: position and mass
+  double4 *src = nullptr;
   unsigned long long *key = nullptr;
   int *nextp = nullptr;  // next walk entry after each particle
   // nodes
-  int *first = nullptr, *count = nullptr, *depth = nullptr;
+  int *first = nullptr, *count = nullptr;
   int *child = nullptr;  // [node][8]: -1, particle (< nsrc) or nsrc + node
-  double *mass = nullptr, *sx = nullptr, *sy = nullptr, *sz = nullptr;
+  double4 *com = nullptr;  // centre of mass and mass
+  int4 *meta = nullptr;    // side length (float bits), sibling, nextnode, 1 for a leaf bucket
   double *quad = nullptr;  // [6][node] traceless quadrupole xx, yy, zz, xy, xz, yz (with quadrupole moments)
   float4 *quadf = nullptr; // [node][2] the same in FP32 for the FP32 walk: (xx, yy, zz, xy), (xz, yz, 0, 0)
-  float *len = nullptr;
-  int *sibling = nullptr, *nextnode = nullptr, *bucket = nullptr;
   int *counter = nullptr;
   std::vector<int> level_lo;  // nodes of depth d are [level_lo[d], level_lo[d+1])
+};
+
+// Points of the host's interleaved arrays (stride 3) or of one array per coordinate (stride 1).
+struct Points {
+  const double *x, *y, *z;
+  int stride;
 };
 
 __device__ __forceinline__ unsigned long long spread3(unsigned long long v) {
@@ -76,26 +82,51 @@ __device__ __forceinline__ unsigned long long mantissa(double d) {
 }
 
 // forcetree.c:197-210 integer positions; Morton key from bits 51..31 of each
-__global__ void k_keys(int n, const double *px, const double *py, const double *pz, double cx, double cy, double cz,
-                       double inv_len, unsigned long long *key, int *idx) {
+__global__ void k_keys(int n, Points P, double cx, double cy, double cz, double inv_len, unsigned long long *key,
+                       int *idx) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if(i >= n) return;
-  unsigned long long xb = mantissa(((px[i] - cx) * inv_len) + 1.0) >> 31;
-  unsigned long long yb = mantissa(((py[i] - cy) * inv_len) + 1.0) >> 31;
-  unsigned long long zb = mantissa(((pz[i] - cz) * inv_len) + 1.0) >> 31;
+  const size_t k = (size_t)i * P.stride;
+  unsigned long long xb = mantissa(((P.x[k] - cx) * inv_len) + 1.0) >> 31;
+  unsigned long long yb = mantissa(((P.y[k] - cy) * inv_len) + 1.0) >> 31;
+  unsigned long long zb = mantissa(((P.z[k] - cz) * inv_len) + 1.0) >> 31;
   key[i] = spread3(xb) | (spread3(yb) << 1) | (spread3(zb) << 2);
   idx[i] = i;
 }
 
-__global__ void k_gather(int n, const int *idx, const double *px, const double *py, const double *pz,
-                         const double *pm, double *x, double *y, double *z, double *m) {
+__global__ void k_gather(int n, const int *idx, Points P, const double *pm, double4 *src) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if(i >= n) return;
-  int j = idx[i];
-  x[i] = px[j];
-  y[i] = py[j];
-  z[i] = pz[j];
-  m[i] = pm[j];
+  const int j = idx[i];
+  const size_t k = (size_t)j * P.stride;
+  src[i] = make_double4(P.x[k], P.y[k], P.z[k], pm[j]);
+}
+
+// Extent of the points: the smallest x, y, z then the largest, per workgroup.
+__global__ void __launch_bounds__(256) k_extent(int n, Points P, double *out) {
+  __shared__ double s[256];
+  double v[6] = {1e30, 1e30, 1e30, -1e30, -1e30, -1e30};
+  for(int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    const size_t k = (size_t)i * P.stride;
+    const double x[3] = {P.x[k], P.y[k], P.z[k]};
+    for(int j = 0; j < 3; j++) {
+      if(v[j] > x[j]) v[j] = x[j];
+      if(v[3 + j] < x[j]) v[3 + j] = x[j];
+    }
+  }
+  for(int j = 0; j < 6; j++) {
+    s[threadIdx.x] = v[j];
+    __syncthreads();
+    for(int d = 128; d > 0; d >>= 1) {
+      if((int)threadIdx.x < d) {
+        const double a = s[threadIdx.x], b = s[threadIdx.x + d];
+        s[threadIdx.x] = j < 3 ? (a > b ? b : a) : (a < b ? b : a);
+      }
+      __syncthreads();
+    }
+    if(threadIdx.x == 0) out[blockIdx.x * 6 + j] = s[0];
+    __syncthreads();
+  }
 }
 
 __device__ __forceinline__ int digit_at(unsigned long long key, int d) {  // child digit below depth d
@@ -105,17 +136,17 @@ __device__ __forceinline__ int digit_at(unsigned long long key, int d) {  // chi
 // Split every node of depth d into its 8 child ranges (binary search on the
 // sorted keys); ranges of >= 2 particles become nodes of depth d+1.
 __global__ void k_split(int lo, int hi, int d, int nsrc, int cap, const unsigned long long *key, int *first,
-                        int *count, int *depth, int *child, int *bucket, int *counter) {
+                        int *count, int *child, int4 *meta, int *counter) {
   int nd = lo + blockIdx.x * blockDim.x + threadIdx.x;
   if(nd >= hi) return;
   int f = first[nd], c = count[nd];
   int *ch = child + (size_t)nd * 8;
   for(int k = 0; k < 8; k++) ch[k] = -1;
   if(c >= 2 && d >= kMaxDepth) {  // particles closer than the key resolution: a leaf bucket
-    bucket[nd] = 1;
+    meta[nd].w = 1;
     return;
   }
-  bucket[nd] = 0;
+  meta[nd].w = 0;
   int b[9];
   b[0] = f;
   b[8] = f + c;
@@ -142,7 +173,6 @@ __global__ void k_split(int lo, int hi, int d, int nsrc, int cap, const unsigned
       }
       first[id] = b[dg];
       count[id] = cnt;
-      depth[id] = d + 1;
       ch[dg] = nsrc + id;
     }
   }
@@ -163,36 +193,32 @@ __device__ __forceinline__ void add_quad(double q[6], double m, double dx, doubl
 // Monopole moments of the nodes of one depth (forcetree.c:619-697), children in order 0..7.
 // With quad (nnodes per component), also the traceless quadrupole about the
 // centre of mass, from the children's own quadrupoles shifted to it.
-__global__ void k_moments(int lo, int hi, int nsrc, int nnodes, const int *child, const int *bucket, const int *first,
-                          const int *count, const double *x, const double *y, const double *z, const double *m,
-                          double *mass, double *sx, double *sy, double *sz, double *quad) {
+// The node's side length (NODE.len, allvars.h:1095, held in float) goes beside them.
+__global__ void k_moments(int lo, int hi, int nsrc, int nnodes, float len, const int *child, const int *first,
+                          const int *count, const double4 *src, double4 *com, int4 *meta, double *quad) {
   int nd = lo + blockIdx.x * blockDim.x + threadIdx.x;
   if(nd >= hi) return;
   double ms = 0, s0 = 0, s1 = 0, s2 = 0;
-  if(bucket[nd]) {
+  meta[nd].x = __float_as_int(len);
+  const bool bucket = meta[nd].w;
+  if(bucket) {
     for(int p = first[nd]; p < first[nd] + count[nd]; p++) {
-      ms += m[p];
-      s0 += m[p] * x[p];
-      s1 += m[p] * y[p];
-      s2 += m[p] * z[p];
+      const double4 v = src[p];
+      ms += v.w;
+      s0 += v.w * v.x;
+      s1 += v.w * v.y;
+      s2 += v.w * v.z;
     }
   } else {
     const int *ch = child + (size_t)nd * 8;
     for(int k = 0; k < 8; k++) {
       int c = ch[k];
       if(c < 0) continue;
-      if(c < nsrc) {
-        ms += m[c];
-        s0 += m[c] * x[c];
-        s1 += m[c] * y[c];
-        s2 += m[c] * z[c];
-      } else {
-        int q = c - nsrc;
-        ms += mass[q];
-        s0 += mass[q] * sx[q];
-        s1 += mass[q] * sy[q];
-        s2 += mass[q] * sz[q];
-      }
+      const double4 v = c < nsrc ? src[c] : com[c - nsrc];
+      ms += v.w;
+      s0 += v.w * v.x;
+      s1 += v.w * v.y;
+      s2 += v.w * v.z;
     }
   }
   if(ms) {
@@ -200,26 +226,23 @@ __global__ void k_moments(int lo, int hi, int nsrc, int nnodes, const int *child
     s1 /= ms;
     s2 /= ms;
   }
-  mass[nd] = ms;
-  sx[nd] = s0;
-  sy[nd] = s1;
-  sz[nd] = s2;
+  com[nd] = make_double4(s0, s1, s2, ms);
   if(!quad) return;
   double q[6] = {0, 0, 0, 0, 0, 0};
-  if(bucket[nd]) {
-    for(int p = first[nd]; p < first[nd] + count[nd]; p++) add_quad(q, m[p], x[p] - s0, y[p] - s1, z[p] - s2);
+  if(bucket) {
+    for(int p = first[nd]; p < first[nd] + count[nd]; p++) {
+      const double4 v = src[p];
+      add_quad(q, v.w, v.x - s0, v.y - s1, v.z - s2);
+    }
   } else {
     const int *ch = child + (size_t)nd * 8;
     for(int k = 0; k < 8; k++) {
       int c = ch[k];
       if(c < 0) continue;
-      if(c < nsrc) {
-        add_quad(q, m[c], x[c] - s0, y[c] - s1, z[c] - s2);
-      } else {
-        int r = c - nsrc;
-        for(int j = 0; j < 6; j++) q[j] += quad[(size_t)j * nnodes + r];
-        add_quad(q, mass[r], sx[r] - s0, sy[r] - s1, sz[r] - s2);
-      }
+      const double4 v = c < nsrc ? src[c] : com[c - nsrc];
+      if(c >= nsrc)
+        for(int j = 0; j < 6; j++) q[j] += quad[(size_t)j * nnodes + (c - nsrc)];
+      add_quad(q, v.w, v.x - s0, v.y - s1, v.z - s2);
     }
   }
   for(int j = 0; j < 6; j++) quad[(size_t)j * nnodes + nd] = q[j];
@@ -227,27 +250,27 @@ __global__ void k_moments(int lo, int hi, int nsrc, int nnodes, const int *child
 
 // nextnode = first child; the sibling of a child is the next child, the last
 // child inherits its parent's sibling (forcetree.c:624-638).
-__global__ void k_thread(int lo, int hi, int nsrc, const int *child, const int *bucket, int *sibling, int *nextnode,
-                         int *nextp) {
+__global__ void k_thread(int lo, int hi, int nsrc, const int *child, int4 *meta, int *nextp) {
   int nd = lo + blockIdx.x * blockDim.x + threadIdx.x;
   if(nd >= hi) return;
-  int sib = sibling[nd];
-  if(bucket[nd]) {
-    nextnode[nd] = sib;  // opened buckets are walked inline
+  const int sib = nd == 0 ? -1 : meta[nd].y;
+  if(nd == 0) meta[nd].y = -1;
+  if(meta[nd].w) {
+    meta[nd].z = sib;  // opened buckets are walked inline
     return;
   }
   const int *ch = child + (size_t)nd * 8;
   int list[8], n = 0;
   for(int k = 0; k < 8; k++)
     if(ch[k] >= 0) list[n++] = ch[k];
-  nextnode[nd] = n ? list[0] : sib;
+  meta[nd].z = n ? list[0] : sib;
   for(int k = 0; k < n; k++) {
     int nx = (k + 1 < n) ? list[k + 1] : sib;
     int c = list[k];
     if(c < nsrc)
       nextp[c] = nx;
     else
-      sibling[c - nsrc] = nx;
+      meta[c - nsrc].y = nx;
   }
 }
 
@@ -260,24 +283,20 @@ __global__ void k_quadf(int nnodes, const double *quad, float4 *quadf) {
   quadf[2 * nd + 1] = make_float4((float)quad[4 * nn + nd], (float)quad[5 * nn + nd], 0.f, 0.f);
 }
 
-__global__ void k_len(int lo, int hi, double dlen, float *len) {
-  int nd = lo + blockIdx.x * blockDim.x + threadIdx.x;
-  if(nd < hi) len[nd] = (float)dlen;
-}
-
 struct WalkArgs {
   int nsrc, ntarget;
-  const double *tx, *ty, *tz;
-  const double *x, *y, *z, *m;
-  const int *nextp, *first, *count, *bucket, *sibling, *nextnode;
-  const double *mass, *sx, *sy, *sz;
+  Points X;             // the targets
+  const int *order;     // per-target walks: the targets in walk order, or null
+  const double4 *src;
+  const int *nextp, *first, *count;
+  const double4 *com;
+  const int4 *meta;     // side length, sibling, nextnode, bucket (Tree)
   const double *quad;   // [6][nnodes] or null: monopole only
   const float4 *quadf;  // [nnodes][2] FP32 copy (FP32 walk)
   int nnodes;
-  const float *len;
   const int *child;     // [node][8] (the group walk)
-  int blk_nb;           // group walk: targets are the (section, z, R) table nodes of nb x nb grids,
-                        // a group an 8 x 8 block of one section; 0: 64 consecutive targets
+  int blk_nb;           // targets are the (section, z, R) table nodes of nb x nb grids, a wave's an
+                        // 8 x 8 block of one section; 0: 64 consecutive targets
   double theta, h, G;
   int plummer;          // Plummer softening of length eps instead of the spline of length h
   double eps;
@@ -361,161 +380,144 @@ __device__ __forceinline__ void quad_term(const T q[6], T dx, T dy, T dz, T s2, 
   pot += (T)-0.5 * dqd * s5;
 }
 
-// forcetree_walk.c:58-192 for one target per lane (mode 0, one task)
-__global__ void __launch_bounds__(256) k_walk64(WalkArgs A) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if(t >= A.ntarget) return;
-  const double px = A.tx[t], py = A.ty[t], pz = A.tz[t];
-  double acc_x = 0, acc_y = 0, acc_z = 0, potv = 0, fac, wp;
-  unsigned long long nint = 0;
-  int no = A.nsrc;  // root
-  while(no >= 0) {
-    double dx, dy, dz, r2, mass;
-    if(no < A.nsrc) {
-      dx = A.x[no] - px;
-      dy = A.y[no] - py;
-      dz = A.z[no] - pz;
-      r2 = dx * dx + dy * dy + dz * dz;
-      mass = A.m[no];
-      no = A.nextp[no];
-    } else {
-      int q = no - A.nsrc;
-      mass = A.mass[q];
-      dx = A.sx[q] - px;
-      dy = A.sy[q] - py;
-      dz = A.sz[q] - pz;
-      r2 = dx * dx + dy * dy + dz * dz;
-      float l = A.len[q];
-      float l2 = l * l;
-      if(l2 > r2 * A.theta * A.theta) {
-        if(A.bucket[q]) {
-          for(int p = A.first[q]; p < A.first[q] + A.count[q]; p++) {
-            double ex = A.x[p] - px, ey = A.y[p] - py, ez = A.z[p] - pz;
-            double e2 = ex * ex + ey * ey + ez * ez;
-            if(A.m[p]) {
-              if(A.plummer)
-                plummer64(A.m[p], e2, A.eps, fac, wp);
-              else
-                interact64(A.m[p], e2, A.h, fac, wp);
-              acc_x += ex * fac;
-              acc_y += ey * fac;
-              acc_z += ez * fac;
-              potv += wp;
-              nint++;
-            }
-          }
-          no = A.sibling[q];
-        } else {
-          no = A.nextnode[q];
-        }
-        continue;
-      }
-      no = A.sibling[q];
-      if(A.quad && mass) {
-        const size_t nn = A.nnodes;
-        const double qq[6] = {A.quad[q], A.quad[nn + q], A.quad[2 * nn + q],
-                              A.quad[3 * nn + q], A.quad[4 * nn + q], A.quad[5 * nn + q]};
-        const double s2 = A.plummer ? r2 + A.eps * A.eps : r2;
-        if(A.plummer || s2 >= A.h * A.h) quad_term(qq, dx, dy, dz, s2, 1.0 / sqrt(s2), acc_x, acc_y, acc_z, potv);
-      }
-    }
-    if(mass) {
-      if(A.plummer)
-        plummer64(mass, r2, A.eps, fac, wp);
-      else
-        interact64(mass, r2, A.h, fac, wp);
-      acc_x += dx * fac;
-      acc_y += dy * fac;
-      acc_z += dz * fac;
-      potv += wp;
-      nint++;
-    }
+// The target of a lane: an 8 x 8 block of a section's table nodes per wave, or 64 targets in turn.
+__device__ __forceinline__ long long wave_target(const WalkArgs &A, int g, int lane) {
+  if(A.blk_nb > 0) {
+    const int nbb = A.blk_nb / 8, s = g / (nbb * nbb), b = g % (nbb * nbb);
+    return ((long long)s * A.blk_nb + (b / nbb) * 8 + lane / 8) * A.blk_nb + (b % nbb) * 8 + lane % 8;
   }
-  A.ax[t] = acc_x * A.G;
-  A.ay[t] = acc_y * A.G;
-  A.az[t] = acc_z * A.G;
-  A.pot[t] = potv * A.G;
-  atomicAdd(A.nint, nint);
+  return (long long)g * 64 + lane;
 }
 
-// The same walk with FP32 interactions: separations are formed in FP64 (node
-// centres of mass and particles stay FP64) and rounded once, the kernel and the
-// sums run in FP32 per target, totals in FP64.
-__global__ void __launch_bounds__(256) k_walk32(WalkArgs A) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if(t >= A.ntarget) return;
-  const double px = A.tx[t], py = A.ty[t], pz = A.tz[t];
-  float acc_x = 0, acc_y = 0, acc_z = 0, potv = 0, fac, wp;
-  const float h = (float)A.h, th2 = (float)(A.theta * A.theta), eps = (float)A.eps;
+// Adds the interaction with a point of mass `mass` at offset (dx, dy, dz).
+__device__ __forceinline__ void interact(const WalkArgs &A, double mass, double dx, double dy, double dz, double r2,
+                                         double &ax, double &ay, double &az, double &pot) {
+  double fac, wp;
+  if(A.plummer)
+    plummer64(mass, r2, A.eps, fac, wp);
+  else
+    interact64(mass, r2, A.h, fac, wp);
+  ax += dx * fac;
+  ay += dy * fac;
+  az += dz * fac;
+  pot += wp;
+}
+__device__ __forceinline__ void interact(const WalkArgs &A, float mass, float dx, float dy, float dz, float r2,
+                                         float &ax, float &ay, float &az, float &pot) {
+  float fac, wp;
+  if(A.plummer)
+    plummer32(mass, r2, (float)A.eps, fac, wp);
+  else
+    interact32(mass, r2, (float)A.h, fac, wp);
+  ax += dx * fac;
+  ay += dy * fac;
+  az += dz * fac;
+  pot += wp;
+}
+
+// forcetree_walk.c:58-192 (mode 0, one task), one target per lane, the 64 targets of a wave on one
+// path.  The wave walks the nodes any of its targets opens; a lane whose target accepts a node
+// waits until the walk reaches that node's sibling.  Every target interacts with the nodes and
+// particles of its own walk in its own order, but the entry being walked is the same for the whole
+// wave, so its moments and links are scalar loads: with each lane on its own path they were
+// gathers of 64 lines, one after the other.  Neighbouring targets share most of their paths (the
+// targets come in 8 x 8 blocks of a table section or in Morton order).  2e5 sources, 8 x 128^2
+// targets, FP64: 11.7 -> 5.3 ms.
+// T = float: separations formed in FP64 (node centres of mass and particles stay FP64) and rounded
+// once, the kernel and the sums in FP32 per target.
+template <typename T>
+__device__ __forceinline__ void walk_body(const WalkArgs &A) {
+  const int lane = threadIdx.x & 63;
+  long long t = wave_target(A, blockIdx.x, lane);
+  const bool live = t < A.ntarget;
+  if(live && A.order) t = A.order[t];
+  const size_t tk = live ? (size_t)t * A.X.stride : 0;
+  const double px = live ? A.X.x[tk] : 0, py = live ? A.X.y[tk] : 0, pz = live ? A.X.z[tk] : 0;
+  T ax = 0, ay = 0, az = 0, pot = 0;
+  const T h = (T)A.h, eps = (T)A.eps, th2 = (T)(A.theta * A.theta);
   unsigned int nint = 0;
-  int no = A.nsrc;
+  constexpr int kGo = -2, kDead = -3;
+  int resume = live ? kGo : kDead;  // kGo: the lane walks; an entry: it waits for it
+  int no = A.nsrc;                  // root
   while(no >= 0) {
-    float dx, dy, dz, r2, mass;
+    no = __builtin_amdgcn_readfirstlane(no);
+    if(resume == no) resume = kGo;
+    const bool act = resume == kGo;
     if(no < A.nsrc) {
-      dx = (float)(A.x[no] - px);
-      dy = (float)(A.y[no] - py);
-      dz = (float)(A.z[no] - pz);
-      r2 = dx * dx + dy * dy + dz * dz;
-      mass = (float)A.m[no];
-      no = A.nextp[no];
-    } else {
-      int q = no - A.nsrc;
-      mass = (float)A.mass[q];
-      dx = (float)(A.sx[q] - px);
-      dy = (float)(A.sy[q] - py);
-      dz = (float)(A.sz[q] - pz);
-      r2 = dx * dx + dy * dy + dz * dz;
-      float l = A.len[q];
-      if(l * l > r2 * th2) {
-        if(A.bucket[q]) {
-          for(int p = A.first[q]; p < A.first[q] + A.count[q]; p++) {
-            float ex = (float)(A.x[p] - px), ey = (float)(A.y[p] - py), ez = (float)(A.z[p] - pz);
-            float e2 = ex * ex + ey * ey + ez * ez;
-            if(A.m[p] != 0) {
-              if(A.plummer)
-                plummer32((float)A.m[p], e2, eps, fac, wp);
-              else
-                interact32((float)A.m[p], e2, h, fac, wp);
-              acc_x += ex * fac;
-              acc_y += ey * fac;
-              acc_z += ez * fac;
-              potv += wp;
-              nint++;
-            }
-          }
-          no = A.sibling[q];
-        } else {
-          no = A.nextnode[q];
-        }
-        continue;
+      const double4 s = A.src[no];
+      const T dx = (T)(s.x - px), dy = (T)(s.y - py), dz = (T)(s.z - pz), mass = (T)s.w;
+      if(act && mass != 0) {
+        interact(A, mass, dx, dy, dz, dx * dx + dy * dy + dz * dz, ax, ay, az, pot);
+        nint++;
       }
-      no = A.sibling[q];
-      if(A.quadf && mass != 0) {
-        const float4 qa = A.quadf[2 * q], qb = A.quadf[2 * q + 1];
-        const float qq[6] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y};
-        const float s2 = A.plummer ? r2 + eps * eps : r2;
-        if(A.plummer || s2 >= h * h)
-          quad_term(qq, dx, dy, dz, s2, __builtin_amdgcn_rsqf(s2), acc_x, acc_y, acc_z, potv);
+      no = A.nextp[no];
+      continue;
+    }
+    const int q = no - A.nsrc;
+    const double4 s = A.com[q];
+    const int4 m = A.meta[q];
+    const T dx = (T)(s.x - px), dy = (T)(s.y - py), dz = (T)(s.z - pz), mass = (T)s.w;
+    const T r2 = dx * dx + dy * dy + dz * dz;
+    const float l = __int_as_float(m.x), l2 = l * l;
+    const bool wide = sizeof(T) == 8 ? l2 > r2 * A.theta * A.theta : l2 > r2 * th2;
+    const bool open = act && wide;
+    if(act && !wide) {
+      if(A.quad && mass != 0) {
+        T qq[6];
+        if(sizeof(T) == 8) {
+          const size_t nn = A.nnodes;
+          for(int k = 0; k < 6; k++) qq[k] = A.quad[k * nn + q];
+        } else {
+          const float4 qa = A.quadf[2 * q], qb = A.quadf[2 * q + 1];
+          qq[0] = qa.x;
+          qq[1] = qa.y;
+          qq[2] = qa.z;
+          qq[3] = qa.w;
+          qq[4] = qb.x;
+          qq[5] = qb.y;
+        }
+        const T s2 = A.plummer ? r2 + eps * eps : r2;
+        if(A.plummer || s2 >= h * h) {
+          const T sinv = sizeof(T) == 8 ? (T)(1.0 / sqrt((double)s2)) : (T)__builtin_amdgcn_rsqf((float)s2);
+          quad_term(qq, dx, dy, dz, s2, sinv, ax, ay, az, pot);
+        }
+      }
+      if(mass != 0) {
+        interact(A, mass, dx, dy, dz, r2, ax, ay, az, pot);
+        nint++;
       }
     }
-    if(mass != 0) {
-      if(A.plummer)
-        plummer32(mass, r2, eps, fac, wp);
-      else
-        interact32(mass, r2, h, fac, wp);
-      acc_x += dx * fac;
-      acc_y += dy * fac;
-      acc_z += dz * fac;
-      potv += wp;
-      nint++;
+    if(__ballot(open) == 0) {
+      no = m.y;
+    } else if(m.w) {
+      // a leaf bucket, its particles one by one
+      const int p0 = A.first[q], p1 = p0 + A.count[q];
+      for(int p = p0; p < p1; p++) {
+        const double4 v = A.src[p];
+        const T ex = (T)(v.x - px), ey = (T)(v.y - py), ez = (T)(v.z - pz);
+        if(open && v.w != 0) {
+          interact(A, (T)v.w, ex, ey, ez, ex * ex + ey * ey + ez * ez, ax, ay, az, pot);
+          nint++;
+        }
+      }
+      no = m.y;
+    } else {
+      if(act && !wide) resume = m.y;
+      no = m.z;
     }
   }
-  A.ax[t] = (double)acc_x * A.G;
-  A.ay[t] = (double)acc_y * A.G;
-  A.az[t] = (double)acc_z * A.G;
-  A.pot[t] = (double)potv * A.G;
-  atomicAdd(A.nint, (unsigned long long)nint);
+  if(live) {
+    A.ax[t] = (double)ax * A.G;
+    A.ay[t] = (double)ay * A.G;
+    A.az[t] = (double)az * A.G;
+    A.pot[t] = (double)pot * A.G;
+  }
+  unsigned long long n = nint;
+  for(int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
+  if(lane == 0) atomicAdd(A.nint, n);
 }
+__global__ void __launch_bounds__(64) k_walk64(WalkArgs A) { walk_body<double>(A); }
+__global__ void __launch_bounds__(64) k_walk32(WalkArgs A) { walk_body<float>(A); }
 
 // Table projection of grid.c:719-750: radial and vertical components summed
 // over the FG_SECTIONS azimuthal sections in order, then averaged.
@@ -625,13 +627,31 @@ inline int nb256(size_t n) { return (int)((n + 255) / 256); }
 // moments, threading), walk, and the interaction count.
 double g_last_build_ms = 0, g_last_walk_ms = 0, g_last_interactions = 0;
 
+// Device buffers of one call, carved from a few allocations (each twice what the call has taken so
+// far, 16 MiB at least): a call has some thirty of them, and an allocation and its release cost
+// about 0.1 ms.
 struct DevBufs {
   std::vector<void *> ptrs;
+  char *at = nullptr;
+  size_t left = 0, taken = 0;
   template <typename T>
   hipError_t alloc(T **p, size_t n) {
-    hipError_t e = hipMalloc((void **)p, std::max<size_t>(n, 1) * sizeof(T));
-    if(e == hipSuccess) ptrs.push_back((void *)*p);
-    return e;
+    const size_t bytes = (std::max<size_t>(n, 1) * sizeof(T) + 255) & ~(size_t)255;
+    if(bytes > left) {
+      size_t want = std::max(bytes, std::max<size_t>(2 * taken, (size_t)16 << 20));
+      void *q = nullptr;
+      hipError_t e = hipMalloc(&q, want);
+      if(e == hipErrorOutOfMemory && want > bytes) e = hipMalloc(&q, want = bytes);
+      if(e != hipSuccess) return e;
+      ptrs.push_back(q);
+      at = (char *)q;
+      left = want;
+      taken += want;
+    }
+    *p = (T *)at;
+    at += bytes;
+    left -= bytes;
+    return hipSuccess;
   }
   ~DevBufs() {
     for(void *p : ptrs) (void)hipFree(p);
@@ -647,21 +667,16 @@ int tree_moments_dev(hipStream_t st, Tree &T, double dlen) {
   for(int d = ndepth - 1; d >= 0; d--) {
     int lo = T.level_lo[d], hi = T.level_lo[d + 1];
     if(hi <= lo) continue;
-    hipLaunchKernelGGL(k_moments, dim3(nb256(hi - lo)), dim3(256), 0, st, lo, hi, nsrc, nnodes,
-                       (const int *)T.child, (const int *)T.bucket, (const int *)T.first, (const int *)T.count,
-                       (const double *)T.x, (const double *)T.y, (const double *)T.z, (const double *)T.m, T.mass,
-                       T.sx, T.sy, T.sz, T.quad);
-    hipLaunchKernelGGL(k_len, dim3(nb256(hi - lo)), dim3(256), 0, st, lo, hi, ldexp(dlen, -d), T.len);
+    hipLaunchKernelGGL(k_moments, dim3(nb256(hi - lo)), dim3(256), 0, st, lo, hi, nsrc, nnodes, (float)ldexp(dlen, -d),
+                       (const int *)T.child, (const int *)T.first, (const int *)T.count, (const double4 *)T.src, T.com,
+                       T.meta, T.quad);
     if(hipGetLastError() != hipSuccess) return terr(GALIC_ERR_HIP, "tree moments launch failed");
   }
-  int minus1 = -1;
-  if(hipMemcpyAsync(T.sibling, &minus1, sizeof(int), hipMemcpyHostToDevice, st) != hipSuccess)
-    return terr(GALIC_ERR_HIP, "tree threading: copy failed");
   for(int d = 0; d < ndepth; d++) {
     int lo = T.level_lo[d], hi = T.level_lo[d + 1];
     if(hi <= lo) continue;
-    hipLaunchKernelGGL(k_thread, dim3(nb256(hi - lo)), dim3(256), 0, st, lo, hi, nsrc, (const int *)T.child,
-                       (const int *)T.bucket, T.sibling, T.nextnode, T.nextp);
+    hipLaunchKernelGGL(k_thread, dim3(nb256(hi - lo)), dim3(256), 0, st, lo, hi, nsrc, (const int *)T.child, T.meta,
+                       T.nextp);
     if(hipGetLastError() != hipSuccess) return terr(GALIC_ERR_HIP, "tree threading launch failed");
   }
   if(T.quad && T.quadf) {
@@ -674,8 +689,8 @@ int tree_moments_dev(hipStream_t st, Tree &T, double dlen) {
 // Builds the tree of nsrc sources (device SoA inputs, domain cube at corner with side dlen)
 // into T, its buffers owned by B.  sorted (optional) receives the device array giving, for each
 // sorted source, its index among the inputs.
-int tree_build_dev(const galic_params *p, hipStream_t st, int nsrc, const double *dpx, const double *dpy,
-                   const double *dpz, const double *dpm, const double corner[3], double dlen, int precision,
+int tree_build_dev(const galic_params *p, hipStream_t st, int nsrc, Points S, const double *dpm,
+                   const double corner[3], double dlen, int precision,
                    DevBufs &B, Tree &T, int **sorted, float *build_ms) {
   int rc = GALIC_OK;
   unsigned long long *keys_in = nullptr;
@@ -685,6 +700,8 @@ int tree_build_dev(const galic_params *p, hipStream_t st, int nsrc, const double
   hipEvent_t eb = nullptr, ee = nullptr;
   (void)p;
   T.nsrc = nsrc;
+  for(int j = 0; j < 3; j++) T.corner[j] = corner[j];
+  T.dlen = dlen;
   TCHK(hipEventCreate(&eb));
   TCHK(hipEventCreate(&ee));
   TCHK(hipEventRecord(eb, st));
@@ -692,20 +709,16 @@ int tree_build_dev(const galic_params *p, hipStream_t st, int nsrc, const double
   TCHK(B.alloc(&T.key, nsrc));
   TCHK(B.alloc(&idx_in, nsrc));
   TCHK(B.alloc(&idx, nsrc));
-  TCHK(B.alloc(&T.x, nsrc));
-  TCHK(B.alloc(&T.y, nsrc));
-  TCHK(B.alloc(&T.z, nsrc));
-  TCHK(B.alloc(&T.m, nsrc));
+  TCHK(B.alloc(&T.src, nsrc));
   TCHK(B.alloc(&T.nextp, nsrc));
   if(nsrc > 0) {
-    hipLaunchKernelGGL(k_keys, dim3(nb256(nsrc)), dim3(256), 0, st, nsrc, dpx, dpy, dpz, corner[0], corner[1],
-                       corner[2], 1.0 / dlen, keys_in, idx_in);
+    hipLaunchKernelGGL(k_keys, dim3(nb256(nsrc)), dim3(256), 0, st, nsrc, S, corner[0], corner[1], corner[2],
+                       1.0 / dlen, keys_in, idx_in);
     TCHK(hipGetLastError());
     TCHK(rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys_in, T.key, idx_in, idx, (unsigned int)nsrc, 0, 63, st));
     TCHK(B.alloc((char **)&tmp, tmp_bytes));
     TCHK(rocprim::radix_sort_pairs(tmp, tmp_bytes, keys_in, T.key, idx_in, idx, (unsigned int)nsrc, 0, 63, st));
-    hipLaunchKernelGGL(k_gather, dim3(nb256(nsrc)), dim3(256), 0, st, nsrc, (const int *)idx, dpx, dpy, dpz, dpm, T.x,
-                       T.y, T.z, T.m);
+    hipLaunchKernelGGL(k_gather, dim3(nb256(nsrc)), dim3(256), 0, st, nsrc, (const int *)idx, S, dpm, T.src);
     TCHK(hipGetLastError());
   }
   if(sorted) *sorted = idx;
@@ -717,14 +730,12 @@ int tree_build_dev(const galic_params *p, hipStream_t st, int nsrc, const double
     for(int attempt = 0; attempt < 6; attempt++) {
       TCHK(B.alloc(&T.first, T.cap));
       TCHK(B.alloc(&T.count, T.cap));
-      TCHK(B.alloc(&T.depth, T.cap));
       TCHK(B.alloc(&T.child, (size_t)T.cap * 8));
-      TCHK(B.alloc(&T.bucket, T.cap));
+      TCHK(B.alloc(&T.meta, T.cap));
       TCHK(B.alloc(&T.counter, 1));
-      int root[3] = {0, nsrc, 0}, one = 1;
+      int root[2] = {0, nsrc}, one = 1;
       TCHK(hipMemcpyAsync(T.first, &root[0], sizeof(int), hipMemcpyHostToDevice, st));
       TCHK(hipMemcpyAsync(T.count, &root[1], sizeof(int), hipMemcpyHostToDevice, st));
-      TCHK(hipMemcpyAsync(T.depth, &root[2], sizeof(int), hipMemcpyHostToDevice, st));
       TCHK(hipMemcpyAsync(T.counter, &one, sizeof(int), hipMemcpyHostToDevice, st));
       T.level_lo.assign(1, 0);
       int lo = 0, hi = 1, d = 0;
@@ -732,7 +743,7 @@ int tree_build_dev(const galic_params *p, hipStream_t st, int nsrc, const double
       while(lo < hi) {
         T.level_lo.push_back(hi);
         hipLaunchKernelGGL(k_split, dim3(nb256(hi - lo)), dim3(256), 0, st, lo, hi, d, nsrc, T.cap,
-                           (const unsigned long long *)T.key, T.first, T.count, T.depth, T.child, T.bucket, T.counter);
+                           (const unsigned long long *)T.key, T.first, T.count, T.child, T.meta, T.counter);
         TCHK(hipGetLastError());
         int nhi = 0;
         TCHK(hipMemcpyAsync(&nhi, T.counter, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -755,17 +766,11 @@ int tree_build_dev(const galic_params *p, hipStream_t st, int nsrc, const double
   }
   {
     const int nnodes = T.level_lo.back();
-    TCHK(B.alloc(&T.mass, nnodes));
-    TCHK(B.alloc(&T.sx, nnodes));
-    TCHK(B.alloc(&T.sy, nnodes));
-    TCHK(B.alloc(&T.sz, nnodes));
-    TCHK(B.alloc(&T.len, nnodes));
+    TCHK(B.alloc(&T.com, nnodes));
     if(precision & GALIC_TREE_QUADRUPOLE) {
       TCHK(B.alloc(&T.quad, (size_t)6 * nnodes));
       if(precision & GALIC_TREE_FP32) TCHK(B.alloc(&T.quadf, (size_t)2 * nnodes));
     }
-    TCHK(B.alloc(&T.sibling, nnodes));
-    TCHK(B.alloc(&T.nextnode, nnodes));
     if((rc = tree_moments_dev(st, T, dlen)) != GALIC_OK) goto done;
   }
   TCHK(hipEventRecord(ee, st));
@@ -796,18 +801,12 @@ __device__ __forceinline__ void group_interact(const WalkArgs &A, int e, double 
   if(e >= 0) {
     float dx, dy, dz, mass;
     int q = -1;
-    if(e < A.nsrc) {
-      dx = (float)(A.x[e] - px);
-      dy = (float)(A.y[e] - py);
-      dz = (float)(A.z[e] - pz);
-      mass = (float)A.m[e];
-    } else {
-      q = e - A.nsrc;
-      dx = (float)(A.sx[q] - px);
-      dy = (float)(A.sy[q] - py);
-      dz = (float)(A.sz[q] - pz);
-      mass = (float)A.mass[q];
-    }
+    if(e >= A.nsrc) q = e - A.nsrc;
+    const double4 s = q < 0 ? A.src[e] : A.com[q];
+    dx = (float)(s.x - px);
+    dy = (float)(s.y - py);
+    dz = (float)(s.z - pz);
+    mass = (float)s.w;
     if(mass == 0) return;
     const float r2 = dx * dx + dy * dy + dz * dz;
     if(q >= 0 && A.quadf) {
@@ -829,13 +828,14 @@ __device__ __forceinline__ void group_interact(const WalkArgs &A, int e, double 
     // an opened leaf bucket: its particles one by one
     const int q = ~e, p0 = A.first[q], p1 = p0 + A.count[q];
     for(int p = p0; p < p1; p++) {
-      if(A.m[p] == 0) continue;
-      const float ex = (float)(A.x[p] - px), ey = (float)(A.y[p] - py), ez = (float)(A.z[p] - pz);
+      const double4 s = A.src[p];
+      if(s.w == 0) continue;
+      const float ex = (float)(s.x - px), ey = (float)(s.y - py), ez = (float)(s.z - pz);
       const float e2 = ex * ex + ey * ey + ez * ez;
       if(A.plummer)
-        plummer32((float)A.m[p], e2, eps, fac, wp);
+        plummer32((float)s.w, e2, eps, fac, wp);
       else
-        interact32((float)A.m[p], e2, h, fac, wp);
+        interact32((float)s.w, e2, h, fac, wp);
       ax += ex * fac;
       ay += ey * fac;
       az += ez * fac;
@@ -858,16 +858,11 @@ __global__ void __launch_bounds__(64) k_walk32g(WalkArgs A) {
   __shared__ int stk[kGStack];
   __shared__ int lst[kGList];
   const int lane = threadIdx.x, g = blockIdx.x;
-  long long t;
-  if(A.blk_nb > 0) {
-    const int nbb = A.blk_nb / 8, s = g / (nbb * nbb), b = g % (nbb * nbb);
-    t = ((long long)s * A.blk_nb + (b / nbb) * 8 + lane / 8) * A.blk_nb + (b % nbb) * 8 + lane % 8;
-  } else {
-    t = (long long)g * 64 + lane;
-  }
+  const long long t = wave_target(A, g, lane);
   const bool live = t < A.ntarget;
   const long long tl = live ? t : (long long)g * 64;  // (dead lanes: the group's first target)
-  const double px = A.tx[tl], py = A.ty[tl], pz = A.tz[tl];
+  const size_t tk = (size_t)tl * A.X.stride;
+  const double px = A.X.x[tk], py = A.X.y[tk], pz = A.X.z[tk];
   const double bx0 = wave_min(px), by0 = wave_min(py), bz0 = wave_min(pz);
   const double bx1 = wave_max(px), by1 = wave_max(py), bz1 = wave_max(pz);
   const float h = (float)A.h, th2 = (float)(A.theta * A.theta), eps = (float)A.eps;
@@ -894,13 +889,15 @@ __global__ void __launch_bounds__(64) k_walk32g(WalkArgs A) {
         item = e;
       } else {
         const int q = e - A.nsrc;
-        const double cx = A.sx[q], cy = A.sy[q], cz = A.sz[q];
+        const double4 cm = A.com[q];
+        const int4 mt = A.meta[q];
+        const double cx = cm.x, cy = cm.y, cz = cm.z;
         const float dx = (float)fmax(fmax(bx0 - cx, cx - bx1), 0.0);
         const float dy = (float)fmax(fmax(by0 - cy, cy - by1), 0.0);
         const float dz = (float)fmax(fmax(bz0 - cz, cz - bz1), 0.0);
-        const float l = A.len[q];
+        const float l = __int_as_float(mt.x);
         if(l * l > (dx * dx + dy * dy + dz * dz) * th2) {
-          if(A.bucket[q]) {
+          if(mt.w) {
             listed = true;
             item = ~q;
           } else {
@@ -938,8 +935,7 @@ __global__ void __launch_bounds__(64) k_walk32g(WalkArgs A) {
 // multiplies the walk's sums by G afterwards, gravtree.c:455-463).
 // blk_nb > 0: the targets are table nodes (section, z, R) of blk_nb x blk_nb grids, which the group
 // walk takes in 8 x 8 blocks.
-int tree_walk_dev(const galic_params *p, hipStream_t st, const Tree &T, int ntarget, const double *dtx,
-                  const double *dty, const double *dtz, double *dax, double *day, double *daz, double *dpot,
+int tree_walk_dev(const galic_params *p, hipStream_t st, const Tree &T, int ntarget, Points X, double *dax, double *day, double *daz, double *dpot,
                   int precision, double G, long long *ninteractions, float *walk_ms, int blk_nb = 0) {
   int rc = GALIC_OK;
   DevBufs B;
@@ -950,24 +946,14 @@ int tree_walk_dev(const galic_params *p, hipStream_t st, const Tree &T, int ntar
   TCHK(hipMemsetAsync(nint, 0, sizeof(unsigned long long), st));
   W.nsrc = T.nsrc;
   W.ntarget = ntarget;
-  W.tx = dtx;
-  W.ty = dty;
-  W.tz = dtz;
-  W.x = T.x;
-  W.y = T.y;
-  W.z = T.z;
-  W.m = T.m;
+  W.X = X;
+  W.order = nullptr;
+  W.src = T.src;
   W.nextp = T.nextp;
   W.first = T.first;
   W.count = T.count;
-  W.bucket = T.bucket;
-  W.sibling = T.sibling;
-  W.nextnode = T.nextnode;
-  W.mass = T.mass;
-  W.sx = T.sx;
-  W.sy = T.sy;
-  W.sz = T.sz;
-  W.len = T.len;
+  W.com = T.com;
+  W.meta = T.meta;
   W.child = T.child;
   W.blk_nb = 0;
   W.quad = (precision & GALIC_TREE_QUADRUPOLE) ? T.quad : nullptr;
@@ -996,14 +982,35 @@ int tree_walk_dev(const galic_params *p, hipStream_t st, const Tree &T, int ntar
   TCHK(hipEventCreate(&e1));
   TCHK(hipEventRecord(e0, st));
   if(ntarget > 0) {
+    // table nodes in 8 x 8 blocks; other targets as they come in the group walk, whose groups are
+    // the caller's, and in Morton order where each target walks for itself
+    const bool blk = blk_nb > 0 && blk_nb % 8 == 0 && (long long)ntarget % ((long long)blk_nb * blk_nb) == 0;
+    const dim3 grid((unsigned int)(((long long)ntarget + 63) / 64)), block(64);
+    W.blk_nb = blk ? blk_nb : 0;
     if(precision & GALIC_TREE_GROUP) {
-      const bool blk = blk_nb > 0 && blk_nb % 8 == 0 && (long long)ntarget % ((long long)blk_nb * blk_nb) == 0;
-      W.blk_nb = blk ? blk_nb : 0;
-      hipLaunchKernelGGL(k_walk32g, dim3((unsigned int)(((long long)ntarget + 63) / 64)), dim3(64), 0, st, W);
-    } else if(!(precision & GALIC_TREE_FP32)) {
-      hipLaunchKernelGGL(k_walk64, dim3(nb256(ntarget)), dim3(256), 0, st, W);
+      hipLaunchKernelGGL(k_walk32g, grid, block, 0, st, W);
     } else {
-      hipLaunchKernelGGL(k_walk32, dim3(nb256(ntarget)), dim3(256), 0, st, W);
+      if(!blk && ntarget > 64) {
+        unsigned long long *k0 = nullptr, *k1 = nullptr;
+        int *i0 = nullptr, *i1 = nullptr;
+        char *tmp = nullptr;
+        size_t tmp_bytes = 0;
+        TCHK(B.alloc(&k0, ntarget));
+        TCHK(B.alloc(&k1, ntarget));
+        TCHK(B.alloc(&i0, ntarget));
+        TCHK(B.alloc(&i1, ntarget));
+        hipLaunchKernelGGL(k_keys, dim3(nb256(ntarget)), dim3(256), 0, st, ntarget, X, T.corner[0], T.corner[1],
+                           T.corner[2], 1.0 / T.dlen, k0, i0);
+        TCHK(hipGetLastError());
+        TCHK(rocprim::radix_sort_pairs(nullptr, tmp_bytes, k0, k1, i0, i1, (unsigned int)ntarget, 0, 63, st));
+        TCHK(B.alloc(&tmp, tmp_bytes));
+        TCHK(rocprim::radix_sort_pairs(tmp, tmp_bytes, k0, k1, i0, i1, (unsigned int)ntarget, 0, 63, st));
+        W.order = i1;
+      }
+      if(!(precision & GALIC_TREE_FP32))
+        hipLaunchKernelGGL(k_walk64, grid, block, 0, st, W);
+      else
+        hipLaunchKernelGGL(k_walk32, grid, block, 0, st, W);
     }
     TCHK(hipGetLastError());
   }
@@ -1021,18 +1028,17 @@ done:
   return rc;
 }
 
-// Build the tree of nsrc sources (device SoA inputs) and walk ntarget targets.
-int tree_forces_dev(const galic_params *p, hipStream_t st, int nsrc, const double *dpx, const double *dpy,
-                    const double *dpz, const double *dpm, int ntarget, const double *dtx, const double *dty,
-                    const double *dtz, double corner[3], double dlen, double *dax, double *day, double *daz,
-                    double *dpot, int precision, long long *ninteractions, float *walk_ms, int blk_nb = 0) {
+// Build the tree of nsrc sources (device inputs) and walk ntarget targets.
+int tree_forces_dev(const galic_params *p, hipStream_t st, int nsrc, Points S, const double *dpm, int ntarget, Points X,
+                    double corner[3], double dlen, double *dax, double *day, double *daz, double *dpot, int precision,
+                    long long *ninteractions, float *walk_ms, int blk_nb = 0) {
   DevBufs B;
   Tree T;
   float build_ms = 0, wms = 0;
   long long ni = 0;
-  int rc = tree_build_dev(p, st, nsrc, dpx, dpy, dpz, dpm, corner, dlen, precision, B, T, nullptr, &build_ms);
+  int rc = tree_build_dev(p, st, nsrc, S, dpm, corner, dlen, precision, B, T, nullptr, &build_ms);
   if(rc != GALIC_OK) return rc;
-  rc = tree_walk_dev(p, st, T, ntarget, dtx, dty, dtz, dax, day, daz, dpot, precision, p->G, &ni, &wms, blk_nb);
+  rc = tree_walk_dev(p, st, T, ntarget, X, dax, day, daz, dpot, precision, p->G, &ni, &wms, blk_nb);
   if(rc != GALIC_OK) return rc;
   if(ninteractions) *ninteractions = ni;
   if(walk_ms) *walk_ms = wms;
@@ -1042,21 +1048,46 @@ int tree_forces_dev(const galic_params *p, hipStream_t st, int nsrc, const doubl
   return GALIC_OK;
 }
 
-// domain_box.c:20-65 over sources and targets
-void domain_extent(int nsrc, const double *spos, int ntarget, const double *tpos, double corner[3], double *len) {
-  double xmin[3] = {1e30, 1e30, 1e30}, xmax[3] = {-1e30, -1e30, -1e30}, l = 0;
-  for(int i = 0; i < nsrc + ntarget; i++) {
-    const double *x = i < nsrc ? &spos[3 * (size_t)i] : &tpos[3 * (size_t)(i - nsrc)];
+// The extent of points on the device, widened into lo and hi (domain_box.c:20-65).
+int extend_domain(hipStream_t st, DevBufs &B, int n, Points P, double lo[3], double hi[3]) {
+  if(n <= 0) return GALIC_OK;
+  int rc = GALIC_OK;
+  const int nblk = std::min(nb256(n), 512);
+  double *d = nullptr;
+  std::vector<double> h((size_t)nblk * 6);
+  TCHK(B.alloc(&d, h.size()));
+  hipLaunchKernelGGL(k_extent, dim3(nblk), dim3(256), 0, st, n, P, d);
+  TCHK(hipGetLastError());
+  TCHK(hipMemcpyAsync(h.data(), d, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st));
+  TCHK(hipStreamSynchronize(st));
+  for(int b = 0; b < nblk; b++)
     for(int j = 0; j < 3; j++) {
-      if(xmin[j] > x[j]) xmin[j] = x[j];
-      if(xmax[j] < x[j]) xmax[j] = x[j];
+      if(lo[j] > h[6 * b + j]) lo[j] = h[6 * b + j];
+      if(hi[j] < h[6 * b + 3 + j]) hi[j] = h[6 * b + 3 + j];
     }
-  }
+done:
+  return rc;
+}
+
+// The cube over an extent (domain_box.c:20-65).
+void domain_cube(const double lo[3], const double hi[3], double corner[3], double *len) {
+  double l = 0;
   for(int j = 0; j < 3; j++)
-    if(xmax[j] - xmin[j] > l) l = xmax[j] - xmin[j];
+    if(hi[j] - lo[j] > l) l = hi[j] - lo[j];
   l *= 1.00001;
-  for(int j = 0; j < 3; j++) corner[j] = 0.5 * (xmin[j] + xmax[j]) - 0.5 * l;
+  for(int j = 0; j < 3; j++) corner[j] = 0.5 * (lo[j] + hi[j]) - 0.5 * l;
   *len = l;
+}
+
+// The host's interleaved points onto the device.
+int upload_points(hipStream_t st, DevBufs &B, int n, const double *aos, Points *P) {
+  int rc = GALIC_OK;
+  double *d = nullptr;
+  TCHK(B.alloc(&d, 3 * (size_t)std::max(n, 1)));
+  if(n > 0) TCHK(hipMemcpyAsync(d, aos, 3 * sizeof(double) * (size_t)n, hipMemcpyHostToDevice, st));
+  *P = Points{d, d + 1, d + 2, 3};
+done:
+  return rc;
 }
 
 int upload_soa(hipStream_t st, int n, const double *aos, double *dx, double *dy, double *dz) {
@@ -1086,6 +1117,22 @@ void fill_nodes(const galic_params *p, std::vector<double> &rj, std::vector<doub
   }
 }
 
+// The extent of the table fill's targets (R_j cos phi_s, R_j sin phi_s, z_k), widened into lo, hi.
+void fill_extent(const std::vector<double> &rj, const std::vector<double> &cs, const std::vector<double> &sn,
+                 double lo[3], double hi[3]) {
+  for(size_t s = 0; s < cs.size(); s++)
+    for(double r : rj) {
+      lo[0] = std::min(lo[0], r * cs[s]);
+      hi[0] = std::max(hi[0], r * cs[s]);
+      lo[1] = std::min(lo[1], r * sn[s]);
+      hi[1] = std::max(hi[1], r * sn[s]);
+    }
+  for(double r : rj) {
+    lo[2] = std::min(lo[2], r);
+    hi[2] = std::max(hi[2], r);
+  }
+}
+
 // ------------------------------------------------ forcetree drop-ins' state --
 
 // P[] of the forcetree drop-ins (allvars.h:844-868), caller-owned as the reference's P[]:
@@ -1110,7 +1157,6 @@ struct BoundTree {
   std::vector<int> targets;      // TargetList: the Type-5 particles (gravtree.c:115-119)
   double corner[3] = {0, 0, 0}, len = 0;
   galic_params p;
-  double *tbuf = nullptr;        // device: one target's position, acceleration and potential
 } g_T;
 
 void tree_release() {
@@ -1155,19 +1201,20 @@ int tree_build_bound(int npart, int precision) {
     }
   }
   const int nsrc = (int)g_T.src_of.size();
-  double *px, *py, *pz, *pm;
-  domain_extent(nsrc, spos.data(), (int)g_T.targets.size(), tp.data(), g_T.corner, &g_T.len);
+  double *pm;
+  Points S, X;
+  double lo[3] = {1e30, 1e30, 1e30}, hi[3] = {-1e30, -1e30, -1e30};
   g_T.B = new DevBufs();
   TCHK(hipSetDevice(g_T.device));
   TCHK(hipStreamCreate(&g_T.st));
-  TCHK(g_T.B->alloc(&px, nsrc));
-  TCHK(g_T.B->alloc(&py, nsrc));
-  TCHK(g_T.B->alloc(&pz, nsrc));
   TCHK(g_T.B->alloc(&pm, nsrc));
-  TCHK(g_T.B->alloc(&g_T.tbuf, 8));
-  if((rc = upload_soa(g_T.st, nsrc, spos.data(), px, py, pz)) != GALIC_OK) goto done;
+  if((rc = upload_points(g_T.st, *g_T.B, nsrc, spos.data(), &S)) != GALIC_OK) goto done;
+  if((rc = upload_points(g_T.st, *g_T.B, (int)g_T.targets.size(), tp.data(), &X)) != GALIC_OK) goto done;
+  if((rc = extend_domain(g_T.st, *g_T.B, nsrc, S, lo, hi)) != GALIC_OK) goto done;
+  if((rc = extend_domain(g_T.st, *g_T.B, (int)g_T.targets.size(), X, lo, hi)) != GALIC_OK) goto done;
+  domain_cube(lo, hi, g_T.corner, &g_T.len);
   if(nsrc > 0) TCHK(hipMemcpy(pm, sm.data(), sizeof(double) * nsrc, hipMemcpyHostToDevice));
-  rc = tree_build_dev(&g_T.p, g_T.st, nsrc, px, py, pz, pm, g_T.corner, g_T.len, precision, *g_T.B, g_T.T,
+  rc = tree_build_dev(&g_T.p, g_T.st, nsrc, S, pm, g_T.corner, g_T.len, precision, *g_T.B, g_T.T,
                       &g_T.sorted, nullptr);
   if(rc == GALIC_OK) g_T.built = true;
 done:
@@ -1179,13 +1226,13 @@ done:
 int tree_walk_bound(int n, const double *pos, double *acc, double *pot, double G, long long *nint) {
   int rc = GALIC_OK;
   DevBufs B;
-  double *tx, *ty, *tz, *ax, *ay, *az, *pt;
+  double *ax, *ay, *az, *pt;
+  Points X;
   std::vector<double> h;
   TCHK(hipSetDevice(g_T.device));
-  TCHK(B.alloc(&tx, n)); TCHK(B.alloc(&ty, n)); TCHK(B.alloc(&tz, n));
   TCHK(B.alloc(&ax, n)); TCHK(B.alloc(&ay, n)); TCHK(B.alloc(&az, n)); TCHK(B.alloc(&pt, n));
-  if((rc = upload_soa(g_T.st, n, pos, tx, ty, tz)) != GALIC_OK) goto done;
-  if((rc = tree_walk_dev(&g_T.p, g_T.st, g_T.T, n, tx, ty, tz, ax, ay, az, pt, 0, G, nint, nullptr)) != GALIC_OK)
+  if((rc = upload_points(g_T.st, B, n, pos, &X)) != GALIC_OK) goto done;
+  if((rc = tree_walk_dev(&g_T.p, g_T.st, g_T.T, n, X, ax, ay, az, pt, 0, G, nint, nullptr)) != GALIC_OK)
     goto done;
   h.resize(std::max(n, 1));
   {
@@ -1318,28 +1365,14 @@ int galic_retabulate(galic_ctx *ctx, int precision, long long *ninteractions) {
   const size_t nn = (size_t)nb * nb, ns = GALIC_FG_SECTIONS * nn;
   std::vector<double> rj, cs, sn;
   fill_nodes(p, rj, cs, sn);
-  // the domain over sources and targets, as domain_extent() forms it for galic_tree_fill
-  double xmin[3], xmax[3], corner[3], len = 0;
+  // the domain over sources and targets, as galic_tree_fill forms it
+  double lo[3], hi[3], corner[3], len = 0;
   for(int j = 0; j < 3; j++) {
-    xmin[j] = c.tsrc_lo[j];
-    xmax[j] = c.tsrc_hi[j];
+    lo[j] = c.tsrc_lo[j];
+    hi[j] = c.tsrc_hi[j];
   }
-  for(int s = 0; s < GALIC_FG_SECTIONS; s++)
-    for(int j = 0; j < nb; j++) {
-      const double x = rj[j] * cs[s], y = rj[j] * sn[s];
-      xmin[0] = std::min(xmin[0], x);
-      xmax[0] = std::max(xmax[0], x);
-      xmin[1] = std::min(xmin[1], y);
-      xmax[1] = std::max(xmax[1], y);
-    }
-  for(int k = 0; k < nb; k++) {
-    xmin[2] = std::min(xmin[2], rj[k]);
-    xmax[2] = std::max(xmax[2], rj[k]);
-  }
-  for(int j = 0; j < 3; j++)
-    if(xmax[j] - xmin[j] > len) len = xmax[j] - xmin[j];
-  len *= 1.00001;
-  for(int j = 0; j < 3; j++) corner[j] = 0.5 * (xmin[j] + xmax[j]) - 0.5 * len;
+  fill_extent(rj, cs, sn, lo, hi);
+  domain_cube(lo, hi, corner, &len);
   int rc = GALIC_OK;
   DevBufs B;
   Tree T;
@@ -1356,11 +1389,11 @@ int galic_retabulate(galic_ctx *ctx, int precision, long long *ninteractions) {
   hipLaunchKernelGGL(k_fill_targets, dim3(nb256(ns)), dim3(256), 0, c.stream, nb, (const double *)drj,
                      (const double *)dcs, (const double *)dsn, tx, ty, tz);
   TCHK(hipGetLastError());
-  if((rc = tree_build_dev(p, c.stream, nsrc, c.tsrc, c.tsrc + nsrc, c.tsrc + 2 * (size_t)nsrc,
+  if((rc = tree_build_dev(p, c.stream, nsrc, Points{c.tsrc, c.tsrc + nsrc, c.tsrc + 2 * (size_t)nsrc, 1},
                           c.tsrc + 3 * (size_t)nsrc, corner, len, precision, B, T, nullptr, &bms)) != GALIC_OK)
     goto done;
-  if((rc = tree_walk_dev(p, c.stream, T, (int)ns, tx, ty, tz, ax, ay, az, pt, precision, p->G, &ni, &wms, nb)) !=
-     GALIC_OK)
+  if((rc = tree_walk_dev(p, c.stream, T, (int)ns, Points{tx, ty, tz, 1}, ax, ay, az, pt, precision, p->G, &ni, &wms,
+                         nb)) != GALIC_OK)
     goto done;
   // installed as the context's tables: FG_DPotDR, FG_DPotDz, FG_Pot and the FP32 copy
   hipLaunchKernelGGL(k_project, dim3(nb256(nn)), dim3(256), 0, c.stream, nb, (const double *)ax, (const double *)ay,
@@ -1387,23 +1420,23 @@ int galic_tree_forces(const galic_params *p, int device, int nsrc, const double 
     return terr(GALIC_ERR_ARG, "mode: GALIC_TREE_FP32 | GALIC_TREE_QUADRUPOLE | GALIC_TREE_PLUMMER | "
                                "GALIC_TREE_GROUP (with GALIC_TREE_FP32)");
   int rc = GALIC_OK;
-  hipStream_t st = nullptr;
+  const hipStream_t st = hipStreamPerThread;
   DevBufs B;
-  double *px, *py, *pz, *pm, *tx, *ty, *tz, *ax, *ay, *az, *pt;
-  double corner[3], len;
+  double *pm, *ax, *ay, *az, *pt;
+  Points S, X;
+  double lo[3] = {1e30, 1e30, 1e30}, hi[3] = {-1e30, -1e30, -1e30}, corner[3], len;
   float ms = 0;
   std::vector<double> h;
   TCHK(hipSetDevice(device));
-  TCHK(hipStreamCreate(&st));
-  domain_extent(nsrc, spos, ntarget, tpos, corner, &len);
-  TCHK(B.alloc(&px, nsrc)); TCHK(B.alloc(&py, nsrc)); TCHK(B.alloc(&pz, nsrc)); TCHK(B.alloc(&pm, nsrc));
-  TCHK(B.alloc(&tx, ntarget)); TCHK(B.alloc(&ty, ntarget)); TCHK(B.alloc(&tz, ntarget));
+  TCHK(B.alloc(&pm, nsrc));
   TCHK(B.alloc(&ax, ntarget)); TCHK(B.alloc(&ay, ntarget)); TCHK(B.alloc(&az, ntarget)); TCHK(B.alloc(&pt, ntarget));
-  if((rc = upload_soa(st, nsrc, spos, px, py, pz)) != GALIC_OK) goto done;
-  if((rc = upload_soa(st, ntarget, tpos, tx, ty, tz)) != GALIC_OK) goto done;
-  if(nsrc > 0) TCHK(hipMemcpy(pm, smass, sizeof(double) * nsrc, hipMemcpyHostToDevice));
-  rc = tree_forces_dev(p, st, nsrc, px, py, pz, pm, ntarget, tx, ty, tz, corner, len, ax, ay, az, pt, precision,
-                       ninteractions, &ms);
+  if((rc = upload_points(st, B, nsrc, spos, &S)) != GALIC_OK) goto done;
+  if((rc = upload_points(st, B, ntarget, tpos, &X)) != GALIC_OK) goto done;
+  if(nsrc > 0) TCHK(hipMemcpyAsync(pm, smass, sizeof(double) * nsrc, hipMemcpyHostToDevice, st));
+  if((rc = extend_domain(st, B, nsrc, S, lo, hi)) != GALIC_OK) goto done;
+  if((rc = extend_domain(st, B, ntarget, X, lo, hi)) != GALIC_OK) goto done;
+  domain_cube(lo, hi, corner, &len);
+  rc = tree_forces_dev(p, st, nsrc, S, pm, ntarget, X, corner, len, ax, ay, az, pt, precision, ninteractions, &ms);
   if(rc != GALIC_OK) goto done;
   h.resize(std::max(ntarget, 1));
   {
@@ -1415,7 +1448,7 @@ int galic_tree_forces(const galic_params *p, int device, int nsrc, const double 
     if(ntarget > 0) TCHK(hipMemcpy(pot, pt, sizeof(double) * ntarget, hipMemcpyDeviceToHost));
   }
 done:
-  if(st) (void)hipStreamDestroy(st);
+  (void)hipStreamSynchronize(st);  // (the buffers go next)
   return rc;
 }
 
@@ -1429,55 +1462,46 @@ int galic_tree_fill(const galic_params *p, int device, int nsrc, const double *s
   const int nb = p->FG_Nbin;
   const size_t ns = (size_t)GALIC_FG_SECTIONS * nb * nb;
   if(ns > 0x7fffffff) return terr(GALIC_ERR_ARG, "FG_Nbin too large");
-  // targets of grid.c:680-704: (R_j cos phi_s, R_j sin phi_s, z_k)
-  std::vector<double> tpos(3 * ns), cs(GALIC_FG_SECTIONS), sn(GALIC_FG_SECTIONS);
-  for(int s = 0; s < GALIC_FG_SECTIONS; s++) {
-    double phi = 2 * M_PI / GALIC_FG_SECTIONS * s;
-    cs[s] = cos(phi);
-    sn[s] = sin(phi);
-  }
-  size_t n = 0;
-  for(int s = 0; s < GALIC_FG_SECTIONS; s++)
-    for(int k = 0; k < nb; k++)
-      for(int j = 0; j < nb; j++, n++) {
-        double r1 = p->FG_Rmin * (pow(p->FG_Fac, j) - 1.0);
-        double z1 = p->FG_Rmin * (pow(p->FG_Fac, k) - 1.0);
-        tpos[3 * n] = r1 * cs[s];
-        tpos[3 * n + 1] = r1 * sn[s];
-        tpos[3 * n + 2] = z1;
-      }
+  // targets of grid.c:680-704: (R_j cos phi_s, R_j sin phi_s, z_k), formed on the device
+  std::vector<double> rj, cs, sn;
+  fill_nodes(p, rj, cs, sn);
   int rc = GALIC_OK;
-  hipStream_t st = nullptr;
+  const hipStream_t st = hipStreamPerThread;
   DevBufs B;
-  double *px, *py, *pz, *pm, *tx, *ty, *tz, *ax, *ay, *az, *pt, *dcs, *dsn, *r0, *r1, *r2;
-  double corner[3], len;
+  double *pm, *tx, *ty, *tz, *ax, *ay, *az, *pt, *drj, *dcs, *dsn, *r0, *r1, *r2;
+  Points S;
+  double lo[3] = {1e30, 1e30, 1e30}, hi[3] = {-1e30, -1e30, -1e30}, corner[3], len;
   float ms = 0;
   TCHK(hipSetDevice(device));
-  TCHK(hipStreamCreate(&st));
-  domain_extent(nsrc, spos, (int)ns, tpos.data(), corner, &len);
-  TCHK(B.alloc(&px, nsrc)); TCHK(B.alloc(&py, nsrc)); TCHK(B.alloc(&pz, nsrc)); TCHK(B.alloc(&pm, nsrc));
+  TCHK(B.alloc(&pm, nsrc));
   TCHK(B.alloc(&tx, ns)); TCHK(B.alloc(&ty, ns)); TCHK(B.alloc(&tz, ns));
   TCHK(B.alloc(&ax, ns)); TCHK(B.alloc(&ay, ns)); TCHK(B.alloc(&az, ns)); TCHK(B.alloc(&pt, ns));
-  TCHK(B.alloc(&dcs, GALIC_FG_SECTIONS)); TCHK(B.alloc(&dsn, GALIC_FG_SECTIONS));
+  TCHK(B.alloc(&drj, nb)); TCHK(B.alloc(&dcs, GALIC_FG_SECTIONS)); TCHK(B.alloc(&dsn, GALIC_FG_SECTIONS));
   TCHK(B.alloc(&r0, (size_t)nb * nb)); TCHK(B.alloc(&r1, (size_t)nb * nb)); TCHK(B.alloc(&r2, (size_t)nb * nb));
-  if((rc = upload_soa(st, nsrc, spos, px, py, pz)) != GALIC_OK) goto done;
-  if((rc = upload_soa(st, (int)ns, tpos.data(), tx, ty, tz)) != GALIC_OK) goto done;
-  if(nsrc > 0) TCHK(hipMemcpy(pm, smass, sizeof(double) * nsrc, hipMemcpyHostToDevice));
-  TCHK(hipMemcpy(dcs, cs.data(), sizeof(double) * GALIC_FG_SECTIONS, hipMemcpyHostToDevice));
-  TCHK(hipMemcpy(dsn, sn.data(), sizeof(double) * GALIC_FG_SECTIONS, hipMemcpyHostToDevice));
-  rc = tree_forces_dev(p, st, nsrc, px, py, pz, pm, (int)ns, tx, ty, tz, corner, len, ax, ay, az, pt, precision,
+  if((rc = upload_points(st, B, nsrc, spos, &S)) != GALIC_OK) goto done;
+  if(nsrc > 0) TCHK(hipMemcpyAsync(pm, smass, sizeof(double) * nsrc, hipMemcpyHostToDevice, st));
+  TCHK(hipMemcpyAsync(drj, rj.data(), sizeof(double) * nb, hipMemcpyHostToDevice, st));
+  TCHK(hipMemcpyAsync(dcs, cs.data(), sizeof(double) * GALIC_FG_SECTIONS, hipMemcpyHostToDevice, st));
+  TCHK(hipMemcpyAsync(dsn, sn.data(), sizeof(double) * GALIC_FG_SECTIONS, hipMemcpyHostToDevice, st));
+  hipLaunchKernelGGL(k_fill_targets, dim3(nb256(ns)), dim3(256), 0, st, nb, (const double *)drj, (const double *)dcs,
+                     (const double *)dsn, tx, ty, tz);
+  TCHK(hipGetLastError());
+  if((rc = extend_domain(st, B, nsrc, S, lo, hi)) != GALIC_OK) goto done;
+  fill_extent(rj, cs, sn, lo, hi);
+  domain_cube(lo, hi, corner, &len);
+  rc = tree_forces_dev(p, st, nsrc, S, pm, (int)ns, Points{tx, ty, tz, 1}, corner, len, ax, ay, az, pt, precision,
                        ninteractions, &ms, nb);
   if(rc != GALIC_OK) goto done;
   hipLaunchKernelGGL(k_project, dim3(nb256((size_t)nb * nb)), dim3(256), 0, st, nb, (const double *)ax,
                      (const double *)ay, (const double *)az, (const double *)pt, (const double *)dcs,
                      (const double *)dsn, r1, r2, r0);
   TCHK(hipGetLastError());
+  TCHK(hipMemcpyAsync(dpotdr, r1, sizeof(double) * nb * nb, hipMemcpyDeviceToHost, st));
+  TCHK(hipMemcpyAsync(dpotdz, r2, sizeof(double) * nb * nb, hipMemcpyDeviceToHost, st));
+  TCHK(hipMemcpyAsync(pot, r0, sizeof(double) * nb * nb, hipMemcpyDeviceToHost, st));
   TCHK(hipStreamSynchronize(st));
-  TCHK(hipMemcpy(dpotdr, r1, sizeof(double) * nb * nb, hipMemcpyDeviceToHost));
-  TCHK(hipMemcpy(dpotdz, r2, sizeof(double) * nb * nb, hipMemcpyDeviceToHost));
-  TCHK(hipMemcpy(pot, r0, sizeof(double) * nb * nb, hipMemcpyDeviceToHost));
 done:
-  if(st) (void)hipStreamDestroy(st);
+  (void)hipStreamSynchronize(st);  // (the buffers and the host arrays of the copies go next)
   return rc;
 }
 

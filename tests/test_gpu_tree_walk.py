@@ -1,0 +1,54 @@
+"""The per-target tree walk, 64 targets on one path: each target's result is that of its own walk."""
+import numpy as np
+import pytest
+
+from galic_amd import model
+from galic_amd.runtime import TREE_FP32, TREE_PLUMMER, TREE_QUADRUPOLE, direct_forces, tree_forces
+
+pytestmark = pytest.mark.gpu
+
+
+def sources(p, n):
+    pos = np.concatenate([model.sample_halo(p, 5, 1, np.arange(n, dtype=np.uint64)),
+                          model.sample_halo(p, 5, 2, np.arange(n, dtype=np.uint64), a=p.Bulge_A)])
+    mass = np.full(len(pos), 1.0 / len(pos))
+    if n > 10:
+        pos[7:10] = pos[6]   # a leaf bucket of coincident points
+        mass[11] = 0.0       # a source without mass
+    return pos, mass
+
+
+# one target, one short of a wave, a wave, one more, many waves in Morton order
+@pytest.mark.parametrize("ntarget", [1, 63, 64, 65, 1000])
+@pytest.mark.parametrize("mode", [0, TREE_FP32, TREE_QUADRUPOLE, TREE_FP32 | TREE_QUADRUPOLE | TREE_PLUMMER])
+def test_each_target_walks_for_itself(mode, ntarget):
+    p = model.make_params(model.config("composite-4e6"))
+    pos, mass = sources(p, 1500)
+    t = 0.5 * pos[np.arange(ntarget) * 3 % len(pos)]   # inside the sources' extent: the same domain cube for any subset
+    print(f"[gpu] walk mode={mode} ntarget={ntarget}", flush=True)
+    acc, pot, nint = tree_forces(p, pos, mass, t, precision=mode)
+    total = 0
+    picks = np.arange(ntarget) if ntarget <= 65 else np.array([0, 1, 500, 998, 999])
+    for k in picks:
+        a1, p1, n1 = tree_forces(p, pos, mass, t[k:k + 1], precision=mode)
+        assert np.array_equal(acc[k], a1[0]) and pot[k] == p1[0], k
+        total += n1
+    if ntarget <= 65:
+        assert total == nint
+
+
+@pytest.mark.parametrize("nsrc", [0, 1, 2, 9])
+def test_few_sources_equal_direct_summation(nsrc):
+    """Down to no source at all, theta -> 0: every source on its own, FP64 to 1e-12."""
+    p = model.make_params(model.config("composite-4e6", theta=1e-6))
+    pos, mass = sources(p, 10)
+    pos, mass = pos[:nsrc], mass[:nsrc]
+    t = model.sample_halo(p, 6, 3, np.arange(70, dtype=np.uint64))
+    acc, pot, nint = tree_forces(p, pos, mass, t)
+    assert nint == 70 * nsrc
+    if nsrc:
+        da, dp = direct_forces(p, pos, mass, t)
+        np.testing.assert_allclose(acc, da, rtol=1e-12, atol=1e-12 * np.abs(da).max())
+        np.testing.assert_allclose(pot, dp, rtol=1e-12)
+    else:
+        assert not acc.any() and not pot.any()
