@@ -794,53 +794,87 @@ done:
 // (a depth-first descent needs at most 7 entries per level).
 constexpr int kGStack = 1024, kGList = 1024, kGDeep = 7 * (kMaxDepth + 3);
 
-__device__ __forceinline__ void group_interact(const WalkArgs &A, int e, double px, double py, double pz, float h,
-                                               float eps, float &ax, float &ay, float &az, float &pot,
-                                               unsigned int &nint) {
+// One list entry's data: a node (q >= 0) with its moments, or a particle.
+struct GroupEntry {
+  int q;
+  double4 s;
+  float4 qa, qb;
+};
+
+// e uniform over the wave, not a bucket: scalar loads.
+__device__ __forceinline__ GroupEntry group_load(const WalkArgs &A, int e) {
+  GroupEntry g;
+  g.q = e - A.nsrc;
+  const double4 *s = g.q >= 0 ? A.com + g.q : A.src + e;
+  g.s = *s;
+  if(A.quadf) {
+    const float4 *m = A.quadf + 2 * (size_t)max(g.q, 0);
+    g.qa = m[0];
+    g.qb = m[1];
+  }
+  return g;
+}
+
+__device__ __forceinline__ void group_add(const WalkArgs &A, const GroupEntry &g, double px, double py, double pz,
+                                          float h, float eps, float &ax, float &ay, float &az, float &pot,
+                                          unsigned int &nint) {
   float fac, wp;
-  if(e >= 0) {
-    float dx, dy, dz, mass;
-    int q = -1;
-    if(e >= A.nsrc) q = e - A.nsrc;
-    const double4 s = q < 0 ? A.src[e] : A.com[q];
-    dx = (float)(s.x - px);
-    dy = (float)(s.y - py);
-    dz = (float)(s.z - pz);
-    mass = (float)s.w;
-    if(mass == 0) return;
-    const float r2 = dx * dx + dy * dy + dz * dz;
-    if(q >= 0 && A.quadf) {
-      const float4 qa = A.quadf[2 * q], qb = A.quadf[2 * q + 1];
-      const float qq[6] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y};
-      const float s2 = A.plummer ? r2 + eps * eps : r2;
-      if(A.plummer || s2 >= h * h) quad_term(qq, dx, dy, dz, s2, __builtin_amdgcn_rsqf(s2), ax, ay, az, pot);
-    }
-    if(A.plummer)
-      plummer32(mass, r2, eps, fac, wp);
-    else
-      interact32(mass, r2, h, fac, wp);
-    ax += dx * fac;
-    ay += dy * fac;
-    az += dz * fac;
-    pot += wp;
-    nint++;
-  } else {
-    // an opened leaf bucket: its particles one by one
-    const int q = ~e, p0 = A.first[q], p1 = p0 + A.count[q];
-    for(int p = p0; p < p1; p++) {
-      const double4 s = A.src[p];
-      if(s.w == 0) continue;
-      const float ex = (float)(s.x - px), ey = (float)(s.y - py), ez = (float)(s.z - pz);
-      const float e2 = ex * ex + ey * ey + ez * ez;
-      if(A.plummer)
-        plummer32((float)s.w, e2, eps, fac, wp);
-      else
-        interact32((float)s.w, e2, h, fac, wp);
-      ax += ex * fac;
-      ay += ey * fac;
-      az += ez * fac;
-      pot += wp;
-      nint++;
+  const float mass = (float)g.s.w;
+  if(mass == 0) return;
+  const float dx = (float)(g.s.x - px), dy = (float)(g.s.y - py), dz = (float)(g.s.z - pz);
+  const float r2 = dx * dx + dy * dy + dz * dz;
+  if(g.q >= 0 && A.quadf) {
+    const float qq[6] = {g.qa.x, g.qa.y, g.qa.z, g.qa.w, g.qb.x, g.qb.y};
+    const float s2 = A.plummer ? r2 + eps * eps : r2;
+    if(A.plummer || s2 >= h * h) quad_term(qq, dx, dy, dz, s2, __builtin_amdgcn_rsqf(s2), ax, ay, az, pot);
+  }
+  if(A.plummer)
+    plummer32(mass, r2, eps, fac, wp);
+  else
+    interact32(mass, r2, h, fac, wp);
+  ax += dx * fac;
+  ay += dy * fac;
+  az += dz * fac;
+  pot += wp;
+  nint++;
+}
+
+// An opened leaf bucket: its particles one by one.
+__device__ __forceinline__ void group_bucket(const WalkArgs &A, int q, double px, double py, double pz, float h,
+                                             float eps, float &ax, float &ay, float &az, float &pot,
+                                             unsigned int &nint) {
+  const int p0 = A.first[q], p1 = p0 + A.count[q];
+  for(int p = p0; p < p1; p++) {
+    const GroupEntry g{-1, A.src[p], {}, {}};
+    if(g.s.w != 0) group_add(A, g, px, py, pz, h, eps, ax, ay, az, pot, nint);
+  }
+}
+
+// Adds the list's entries in their order to the lane's target, kGBatch at a time: the batch's
+// loads go out together, so their latency (an LDS read, then a scalar load that depends on it) is
+// paid once a batch instead of once an entry.
+constexpr int kGBatch = 4;
+__device__ __forceinline__ void group_flush(const WalkArgs &A, const int *lst, int nl, double px, double py, double pz,
+                                            float h, float eps, float &ax, float &ay, float &az, float &pot,
+                                            unsigned int &nint) {
+  for(int i = 0; i < nl; i += kGBatch) {
+    const int4 e4 = *(const int4 *)(lst + i);  // (entries beyond nl are not used)
+    const int e[kGBatch] = {__builtin_amdgcn_readfirstlane(e4.x), __builtin_amdgcn_readfirstlane(e4.y),
+                            __builtin_amdgcn_readfirstlane(e4.z), __builtin_amdgcn_readfirstlane(e4.w)};
+    if(i + kGBatch <= nl && (e[0] | e[1] | e[2] | e[3]) >= 0) {
+      GroupEntry g[kGBatch];
+#pragma unroll
+      for(int k = 0; k < kGBatch; k++) g[k] = group_load(A, e[k]);
+#pragma unroll
+      for(int k = 0; k < kGBatch; k++) group_add(A, g[k], px, py, pz, h, eps, ax, ay, az, pot, nint);
+    } else {
+      for(int k = 0; k < kGBatch && i + k < nl; k++) {
+        const int ek = __builtin_amdgcn_readfirstlane(lst[i + k]);
+        if(ek >= 0)
+          group_add(A, group_load(A, ek), px, py, pz, h, eps, ax, ay, az, pot, nint);
+        else
+          group_bucket(A, ~ek, px, py, pz, h, eps, ax, ay, az, pot, nint);
+      }
     }
   }
 }
@@ -856,7 +890,7 @@ __device__ __forceinline__ double wave_max(double v) {
 
 __global__ void __launch_bounds__(64) k_walk32g(WalkArgs A) {
   __shared__ int stk[kGStack];
-  __shared__ int lst[kGList];
+  __shared__ __align__(16) int lst[kGList];
   const int lane = threadIdx.x, g = blockIdx.x;
   const long long t = wave_target(A, g, lane);
   const bool live = t < A.ntarget;
@@ -874,8 +908,7 @@ __global__ void __launch_bounds__(64) k_walk32g(WalkArgs A) {
   while(top > 0) {
     const int k = (kGStack - top >= 7 * 64 + kGDeep) ? min(64, top) : 1;
     if(nl + k > kGList) {
-      for(int i = 0; i < nl; i++)
-        group_interact(A, __builtin_amdgcn_readfirstlane(lst[i]), px, py, pz, h, eps, ax, ay, az, pot, nint);
+      group_flush(A, lst, nl, px, py, pz, h, eps, ax, ay, az, pot, nint);
       nl = 0;
     }
     const int e = lane < k ? stk[top - 1 - lane] : -1;
@@ -920,8 +953,7 @@ __global__ void __launch_bounds__(64) k_walk32g(WalkArgs A) {
     }
     __syncthreads();
   }
-  for(int i = 0; i < nl; i++)
-    group_interact(A, __builtin_amdgcn_readfirstlane(lst[i]), px, py, pz, h, eps, ax, ay, az, pot, nint);
+  group_flush(A, lst, nl, px, py, pz, h, eps, ax, ay, az, pot, nint);
   if(live) {
     A.ax[t] = (double)ax * A.G;
     A.ay[t] = (double)ay * A.G;
