@@ -852,7 +852,9 @@ __device__ __forceinline__ void group_bucket(const WalkArgs &A, int q, double px
 
 // Adds the list's entries in their order to the lane's target, kGBatch at a time: the batch's
 // loads go out together, so their latency (an LDS read, then a scalar load that depends on it) is
-// paid once a batch instead of once an entry.
+// paid once a batch instead of once an entry: that latency bounded the walk (512^2 x 8 targets and
+// 2e6 sources, 9.1e9 interactions: 40.7 ms one entry at a time, 32.2 ms four at a time).  A batch
+// with a bucket in it, and the list's end, go one by one.
 constexpr int kGBatch = 4;
 __device__ __forceinline__ void group_flush(const WalkArgs &A, const int *lst, int nl, double px, double py, double pz,
                                             float h, float eps, float &ax, float &ay, float &az, float &pot,

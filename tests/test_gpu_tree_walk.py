@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 from galic_amd import model
-from galic_amd.runtime import TREE_FP32, TREE_PLUMMER, TREE_QUADRUPOLE, direct_forces, tree_forces
+from galic_amd.runtime import TREE_FP32, TREE_GROUP, TREE_PLUMMER, TREE_QUADRUPOLE, direct_forces, tree_forces
 
 pytestmark = pytest.mark.gpu
 
@@ -52,3 +52,25 @@ def test_few_sources_equal_direct_summation(nsrc):
         np.testing.assert_allclose(pot, dp, rtol=1e-12)
     else:
         assert not acc.any() and not pot.any()
+
+
+# list lengths around the batch of four, a bucket (from 12 sources on), several flushes of a list
+@pytest.mark.parametrize("nsrc", [1, 3, 4, 5, 8, 12, 13, 64, 2999])
+def test_group_lists_of_any_length_equal_direct_summation(nsrc):
+    """theta -> 0: the group's list holds every source.  A term's FP32 chain (difference, r^2, two
+    reciprocal roots, products) is within 32 roundings, a sum of n terms within n more: each
+    component within (32 + n) 2^-24 of the sum of its terms' magnitudes."""
+    p = model.make_params(model.config("composite-4e6", theta=1e-6))
+    pos, mass = sources(p, 1500)
+    pos, mass = pos[:nsrc], mass[:nsrc]
+    t = model.sample_halo(p, 6, 3, np.arange(70, dtype=np.uint64))
+    print(f"[gpu] group list nsrc={nsrc}", flush=True)
+    acc, pot, nint = tree_forces(p, pos, mass, t, precision=TREE_FP32 | TREE_PLUMMER | TREE_GROUP)
+    assert nint == 70 * np.count_nonzero(mass)
+    da, dp = direct_forces(p, pos, mass, t, plummer=True)
+    d = pos[None] - t[:, None]
+    r = np.sqrt((d ** 2).sum(axis=2))
+    tol = (32 + nsrc) * 2.0 ** -24
+    scale = p.G * (mass[None, :, None] * np.abs(d) / np.maximum(r, 1e-300)[..., None] ** 3).sum(axis=1)
+    assert (np.abs(acc - da) <= tol * scale).all()
+    assert (np.abs(pot - dp) <= tol * np.abs(dp)).all()
