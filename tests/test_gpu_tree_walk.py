@@ -74,3 +74,42 @@ def test_group_lists_of_any_length_equal_direct_summation(nsrc):
     scale = p.G * (mass[None, :, None] * np.abs(d) / np.maximum(r, 1e-300)[..., None] ** 3).sum(axis=1)
     assert (np.abs(acc - da) <= tol * scale).all()
     assert (np.abs(pot - dp) <= tol * np.abs(dp)).all()
+
+
+def count_interactions(pos, mass, t, theta, depth=21):
+    """An octree of its own: the interactions of every target's walk."""
+    both = np.concatenate([pos, t])
+    lo, hi = both.min(axis=0), both.max(axis=0)
+    size = (hi - lo).max() * 1.00001
+    key = np.floor((pos - 0.5 * (lo + hi) + 0.5 * size) / size * 2 ** depth).astype(np.int64)
+
+    def node(idx, d, tt, width):
+        if len(idx) == 1:
+            return len(tt)
+        com = mass[idx] @ pos[idx] / mass[idx].sum()
+        opened = np.float32(width * width) > ((com - t[tt]) ** 2).sum(axis=1) * theta * theta
+        n, tt = np.count_nonzero(~opened), tt[opened]
+        if len(tt) == 0 or d == depth:
+            return n + len(tt) * len(idx)
+        octant = ((key[idx] >> (depth - 1 - d)) & 1) @ np.array([1, 2, 4])
+        return n + sum(node(idx[octant == k], d + 1, tt, width / 2) for k in set(octant))
+
+    return node(np.arange(len(pos)), 0, np.arange(len(t)), size)
+
+
+# a workgroup's 128 nodes of a level: fewer, as many, one more; deep chains (pairs closer than a node)
+@pytest.mark.parametrize("npair", [1, 127, 128, 129, 1025])
+def test_tree_of_close_pairs_equals_direct_summation(npair):
+    """Pairs far closer than their distance to the next pair: every pair a node of its own on many
+    levels; theta -> 0, FP64 to 1e-12 (a pair smaller than 1e-6 of its distance counts once)."""
+    p = model.make_params(model.config("composite-4e6", theta=1e-6))
+    c = model.sample_halo(p, 7, 1, np.arange(npair, dtype=np.uint64))
+    pos = np.concatenate([c, c * (1 + 1e-5)])
+    mass = np.linspace(0.5, 1.5, len(pos)) / len(pos)
+    t = model.sample_halo(p, 7, 3, np.arange(70, dtype=np.uint64))
+    print(f"[gpu] tree of {npair} pairs", flush=True)
+    acc, pot, nint = tree_forces(p, pos, mass, t)
+    assert nint == count_interactions(pos, mass, t, p.ErrTolTheta)
+    da, dp = direct_forces(p, pos, mass, t)
+    np.testing.assert_allclose(acc, da, rtol=1e-12, atol=1e-12 * np.abs(da).max())
+    np.testing.assert_allclose(pot, dp, rtol=1e-12)
