@@ -1168,7 +1168,7 @@ int galic_sample_tree_sources(galic_ctx *ctx, unsigned int seed) {
     A.pos_out = dpts;
     A.counts = cnt;
     A.count = 1;
-    if(galic::launch_sample_targets(A, orbit_grid(n, 256, 8), 0, c.stream) != 0)
+    if(galic::launch_sample_targets(A, 256, orbit_grid(n, 256, 8), 0, c.stream) != 0)
       rc = set_err(GALIC_ERR_HIP, "source sampling launch failed");
     unsigned long long hc[2] = {0, 0};
     if(rc == GALIC_OK && (hipMemcpy(pos.data() + 3 * at, dpts, sizeof(double) * 3 * n, hipMemcpyDeviceToHost) != hipSuccess ||
@@ -1298,6 +1298,8 @@ int galic_set_disp_tables(galic_ctx *ctx, int type, double beta, const double *d
   return GALIC_OK;
 }
 
+constexpr long long kTargetMany = 65536;
+
 int galic_sample_targets(galic_ctx *ctx, int type, long long nsamples, unsigned int seed, unsigned int stream,
                          double stretch, double *dgs_mass_target, double *egs_targets, double *points,
                          long long *nbinned, float *kernel_ms) {
@@ -1337,7 +1339,11 @@ int galic_sample_targets(galic_ctx *ctx, int type, long long nsamples, unsigned 
     A.tilt_r = A.disp_phi + n2;
     A.tilt_theta = A.tilt_r + n2;
   }
-  A.dg = dgs_mass_target ? maps : nullptr;
+  // where the density and the energy grid are the same, the density map is the energy grid's mass map
+  const bool same_grid = dgs_mass_target && egs_targets && c.M.DG_Nbin == c.M.EG_Nbin && c.M.DG_Rmin == c.M.EG_Rmin &&
+                         c.M.DG_logFac == c.M.EG_logFac;
+  const bool own_dg = dgs_mass_target && !same_grid;
+  A.dg = own_dg ? maps : nullptr;
   A.eg = egs_targets ? maps + ng : nullptr;
   A.qdg = ldexp(1.0, 32);
   A.qeg[0] = ldexp(1.0, 32);
@@ -1357,31 +1363,37 @@ int galic_sample_targets(galic_ctx *ctx, int type, long long nsamples, unsigned 
     CHK(dalloc(&dpts, 3 * (size_t)nsamples));
     A.pos_out = dpts;
   }
-  const int grid = orbit_grid((int)std::min<long long>(nsamples, 1 << 30), 256, 8);
-  // The maps are summed per workgroup in LDS where they fit in target_lds bytes (64^2
-  // grids: the density map, then the five energy maps two at a time), so the
-  // atomics on the small maps in memory are few; each launch draws the same points
-  // again (cheap beside the atomics), and only the first counts them and writes them out.
-  // (64 KiB keeps two workgroups per CU; less where the device gives less)
-  size_t target_lds = 65536;
+  // The maps are summed per workgroup in LDS where one fits, so the atomics on memory are few.  A
+  // launch takes as many of them as the LDS holds, in as few launches of about as many maps each as
+  // they need: each draws the same points again, and the draw is most of its work (64^2 grids, 1e7
+  // points of the halo: four launches of two maps 2.4 ms, two of three 1.4 ms, one of the five energy
+  // maps 0.6 ms; 128^2 grids: a launch a map 3.6 ms, 24.4 ms with atomics on memory).  Workgroups of 1024 threads then share a
+  // CU's maps; from kTargetMany points on they are the faster (64^2 grids, the call: 5e4 points 0.21
+  // ms with 256 threads, 0.22 with 1024; 1e5 0.25 and 0.23; 1e6 0.57 and 0.40), and so are maps over
+  // 64 KiB in LDS (128^2 grids: 5e4 points 0.39 ms with atomics on memory, 0.44 in LDS; 1e5 0.50
+  // and 0.48; 1e6 2.7 and 0.79).  Only the first launch counts the points and writes them out.
+  size_t lds = 65536;
   {
     int v = 0;
-    if(hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, c.device) == hipSuccess && v > 0)
-      target_lds = std::min(target_lds, (size_t)v);
+    if(hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, c.device) == hipSuccess && v > 0) lds = v;
   }
-  const size_t per_map = ng * sizeof(long long), fit = target_lds / per_map;
+  const bool many = nsamples >= kTargetMany;
+  const size_t per_map = ng * sizeof(long long);
+  const size_t fit = many || per_map <= 65536 ? lds / per_map : 0;
+  const int nmaps = (own_dg ? 1 : 0) + (egs_targets ? 5 : 0);
   struct Pass {
     bool dg;
     int f0, f1;
   };
   std::vector<Pass> passes;
-  if(fit == 0) {
-    passes.push_back({dgs_mass_target != nullptr, 0, egs_targets ? 5 : 0});
-  } else {
-    if(dgs_mass_target) passes.push_back({true, 0, 0});
-    if(egs_targets)
-      for(int f0 = 0; f0 < 5; f0 += (int)fit) passes.push_back({false, f0, std::min(5, f0 + (int)fit)});
+  const int npass = fit == 0 ? 1 : (int)((nmaps + fit - 1) / fit);
+  for(int i = 0; i < npass; i++) {
+    // maps m0 .. m1-1 in the order dg, eg 0 .. 4
+    const int m0 = nmaps * i / npass, m1 = nmaps * (i + 1) / npass, e = own_dg ? 1 : 0;
+    passes.push_back({e == 1 && m0 == 0, std::max(m0 - e, 0), std::max(m1 - e, 0)});
   }
+  const int threads = fit > 0 && many ? galic::kTargetThreads : 256;
+  const int grid = orbit_grid((int)std::min<long long>(nsamples, 1 << 30), threads, threads == 256 ? 8 : 1);
   HIPCHK(hipEventRecord(c.ev0, c.stream));
   for(size_t i = 0; i < passes.size(); i++) {
     galic::TargetArgs P = A;
@@ -1392,7 +1404,7 @@ int galic_sample_targets(galic_ctx *ctx, int type, long long nsamples, unsigned 
     P.count = i == 0 ? 1 : 0;
     P.pos_out = i == 0 ? A.pos_out : nullptr;
     const size_t shmem = P.lds ? per_map * ((P.dg ? 1 : 0) + (size_t)(P.f1 - P.f0)) : 0;
-    if(galic::launch_sample_targets(P, grid, shmem, c.stream) != 0) {
+    if(galic::launch_sample_targets(P, threads, grid, shmem, c.stream) != 0) {
       dfree(maps);
       dfree(counts);
       dfree(dpts);
@@ -1422,7 +1434,7 @@ int galic_sample_targets(galic_ctx *ctx, int type, long long nsamples, unsigned 
     smooth_stack_host(st.data(), c.L);
     memcpy(out, st.data(), sizeof(double) * c.Nstack);
   };
-  if(dgs_mass_target) finish(hq.data(), A.qdg, dgs_mass_target);
+  if(dgs_mass_target) finish(hq.data() + (same_grid ? ng : 0), A.qdg, dgs_mass_target);
   if(egs_targets)
     for(int f = 0; f < 5; f++) finish(hq.data() + (1 + f) * ng, A.qeg[f], egs_targets + (size_t)f * c.Nstack);
   if(nbinned) *nbinned = (long long)hc[0];

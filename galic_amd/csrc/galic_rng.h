@@ -37,15 +37,19 @@ __device__ __forceinline__ double u01(uint32_t a, uint32_t b) {
   return ((double)(a >> 5) * 67108864.0 + (double)(b >> 6) + 0.5) / 9007199254740992.0;
 }
 
+// Uniforms 2 * half and 2 * half + 1 of (id, attempt, block)
+__device__ __forceinline__ void uniform2(uint64_t id, uint32_t attempt, uint32_t block, int half, uint32_t seed,
+                                         uint32_t stream, double u[2]) {
+  uint32_t c[4] = {(uint32_t)id, (uint32_t)(id >> 32), attempt, 2 * block + half};
+  philox4x32(c, seed, stream);
+  u[0] = u01(c[0], c[1]);
+  u[1] = u01(c[2], c[3]);
+}
+
 // Four uniforms for (id, attempt, block), as rng.uniforms
 __device__ __forceinline__ void uniform4(uint64_t id, uint32_t attempt, uint32_t block, uint32_t seed, uint32_t stream,
                                          double u[4]) {
-  for(int half = 0; half < 2; half++) {
-    uint32_t c[4] = {(uint32_t)id, (uint32_t)(id >> 32), attempt, 2 * block + half};
-    philox4x32(c, seed, stream);
-    u[2 * half] = u01(c[0], c[1]);
-    u[2 * half + 1] = u01(c[2], c[3]);
-  }
+  for(int half = 0; half < 2; half++) uniform2(id, attempt, block, half, seed, stream, u + 2 * half);
 }
 
 // Four standard normals for (id, attempt, block), as rng.gaussians (Box-Muller)

@@ -41,7 +41,9 @@ struct TargetArgs {
                             // of 8 bytes per cell of each map: dg first, then eg maps f0 .. f1-1)
 };
 
-// Grid-stride launch over the sample ids on stream s.
-int launch_sample_targets(const TargetArgs &A, int grid, size_t shmem, hipStream_t s);
+constexpr int kTargetThreads = 1024;
+
+// Grid-stride launch over the sample ids on stream s, with workgroups of 256 or kTargetThreads.
+int launch_sample_targets(const TargetArgs &A, int threads, int grid, size_t shmem, hipStream_t s);
 
 }  // namespace galic

@@ -138,7 +138,7 @@ __device__ __forceinline__ int digit_at(unsigned long long key, int d) {  // chi
 // lev[k] counts the nodes of depth k: the nodes of a depth follow those of the depth above, so the
 // levels are launched one after the other without the host reading their sizes.  A workgroup takes
 // the ids of the nodes that its kSplitNodes nodes open with one atomic: atomics on one word bounded
-// the split (2e6 sources, all levels: 7.3 ms with a thread and up to 8 atomics a node, 6.3 ms with
+// the split (1e7 sources, all levels: 7.3 ms with a thread and up to 8 atomics a node, 6.3 ms with
 // an atomic a wave, 0.72 ms with an atomic a workgroup).  Ids in the order of the workgroups also
 // keep the nodes that a walk opens together near each other (k_walk32g below: 32.2 -> 29.5 ms).
 constexpr int kSplitNodes = 128;
@@ -864,7 +864,7 @@ __device__ __forceinline__ void group_bucket(const WalkArgs &A, int q, double px
 // Adds the list's entries in their order to the lane's target, kGBatch at a time: the batch's
 // loads go out together, so their latency (an LDS read, then a scalar load that depends on it) is
 // paid once a batch instead of once an entry: that latency bounded the walk (512^2 x 8 targets and
-// 2e6 sources, 9.1e9 interactions: 40.7 ms one entry at a time, 32.2 ms four at a time).  A batch
+// 1e7 sources, 9.1e9 interactions: 40.7 ms one entry at a time, 32.2 ms four at a time).  A batch
 // with a bucket in it, and the list's end, go one by one.
 constexpr int kGBatch = 4;
 __device__ __forceinline__ void group_flush(const WalkArgs &A, const int *lst, int nl, double px, double py, double pz,
