@@ -171,6 +171,30 @@ int alloc_slots(galic::Ctx &c, int norbits, size_t bytes_per_orbit) {
   return GALIC_OK;
 }
 
+// Cell-major slots of n orbits to the host as five grids per orbit, through a buffer of at most
+// 64 MB (one orbit's, where that is more); the slots are zero again.
+template <typename T>
+int fields_out(galic::Ctx &c, int n, T *slots, double *fields) {
+  const size_t per = (size_t)galic::kFields * c.Ngrid;
+  const int most = (int)std::max<size_t>(1, std::min<size_t>((size_t)n, ((size_t)64 << 20) / (sizeof(double) * per)));
+  if(c.fields_len < most * per) {
+    dfree(c.fields_buf);
+    c.fields_len = 0;
+    CHK(dalloc(&c.fields_buf, most * per));
+    c.fields_len = most * per;
+  }
+  const int nblk = nblocks(c.Ngrid, galic::kFieldCells);
+  for(int o = 0; o < n; o += most) {
+    const int m = std::min(most, n - o);
+    hipLaunchKernelGGL(galic::k_fields_out<T>, dim3((unsigned int)m * nblk), dim3(galic::kFieldCells), 0, c.stream,
+                       (int)c.Ngrid, nblk, slots + o * per, c.fields_buf);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(fields + o * per, c.fields_buf, sizeof(double) * m * per, hipMemcpyDeviceToHost, c.stream));
+  }
+  HIPCHK(hipStreamSynchronize(c.stream));
+  return GALIC_OK;
+}
+
 // Exchanges the active orbit set with the other one (see galic::OrbitSet).
 void swap_orbit_set(galic::Ctx &c) {
 #define GALIC_OS_SWAP(T, f) std::swap(c.f, c.alt.f);
@@ -1104,6 +1128,7 @@ int galic_destroy(galic_ctx *ctx) {
   dfree(c.tile_aux);
   dfree(c.tdesc);
   dfree(c.tpart);
+  dfree(c.fields_buf);
   dfree(c.cm_cnt); dfree(c.cm_start); dfree(c.cm_chunks); dfree(c.cm_buf); dfree(c.cm_aux); dfree(c.cm_bound);
   dfree(c.merit_prof);
   dfree(c.lookup_buf);
@@ -1725,18 +1750,7 @@ int galic_orbit_responses(galic_ctx *ctx, int norbit, const double *pos, const d
     CHK(launch_orbit64(c, A));
     if(!fields) HIPCHK(hipMemsetAsync(c.locA_d, 0, sizeof(double) * GALIC_NTYPES * galic::kFields * c.Ngrid, c.stream));
     HIPCHK(hipStreamSynchronize(c.stream));
-    if(fields) {
-      // slots are cell-major [cell][field]; the ABI returns 5 grids per orbit
-      std::vector<double> cm((size_t)n * galic::kFields * c.Ngrid);
-      HIPCHK(hipMemcpy(cm.data(), c.slots, per * n, hipMemcpyDeviceToHost));
-      for(int o = 0; o < n; o++) {
-        const double *src = cm.data() + (size_t)o * galic::kFields * c.Ngrid;
-        double *dst = fields + (size_t)(base + o) * galic::kFields * c.Ngrid;
-        for(int cell = 0; cell < c.Ngrid; cell++)
-          for(int f = 0; f < galic::kFields; f++) dst[(size_t)f * c.Ngrid + cell] = src[(size_t)cell * galic::kFields + f];
-      }
-    }
-    if(fields) HIPCHK(hipMemset(c.slots, 0, per * n));
+    if(fields) CHK(fields_out(c, n, (double *)c.slots, fields + (size_t)base * galic::kFields * c.Ngrid));
     if(t) HIPCHK(hipMemcpy(t + base, c.o_tall, sizeof(double) * n, hipMemcpyDeviceToHost));
     if(orbits) HIPCHK(hipMemcpy(orbits + base, c.o_norbit, sizeof(int) * n, hipMemcpyDeviceToHost));
     if(steps) HIPCHK(hipMemcpy(steps + base, c.o_steps, sizeof(long long) * n, hipMemcpyDeviceToHost));
@@ -1762,7 +1776,6 @@ int galic_fp32_orbit_responses(galic_ctx *ctx, int norbit, const double *pos, co
   float *fin = nullptr;
   HIPCHK(hipMalloc(&fin, sizeof(float) * 6 * chunk));
   std::vector<double> tmp(chunk);
-  std::vector<float> cm(fields ? (size_t)chunk * galic::kFields * c.Ngrid : 0);
   int rc = GALIC_OK;
   for(int base = 0; base < norbit && rc == GALIC_OK; base += chunk) {
     const int n = std::min(chunk, norbit - base);
@@ -1791,16 +1804,9 @@ int galic_fp32_orbit_responses(galic_ctx *ctx, int norbit, const double *pos, co
       rc = hip_ok(hipGetLastError());
     }
     if(rc == GALIC_OK) rc = hip_ok(hipStreamSynchronize(c.stream));
-    if(rc == GALIC_OK && fields) {
-      rc = hip_ok(hipMemcpy(cm.data(), c.slots, per * n, hipMemcpyDeviceToHost));
-      for(int o = 0; o < n && rc == GALIC_OK; o++) {
-        const float *src = cm.data() + (size_t)o * galic::kFields * c.Ngrid;
-        double *dst = fields + (size_t)(base + o) * galic::kFields * c.Ngrid;
-        for(int cell = 0; cell < c.Ngrid; cell++)
-          for(int f = 0; f < galic::kFields; f++) dst[(size_t)f * c.Ngrid + cell] = src[(size_t)cell * galic::kFields + f];
-      }
-    }
-    if(rc == GALIC_OK) rc = hip_ok(hipMemset(c.slots, 0, per * n));
+    if(rc == GALIC_OK && fields)
+      rc = fields_out(c, n, (float *)c.slots, fields + (size_t)base * galic::kFields * c.Ngrid);
+    if(rc == GALIC_OK && !fields) rc = hip_ok(hipMemset(c.slots, 0, per * n));
     if(rc == GALIC_OK && t) rc = hip_ok(hipMemcpy(t + base, c.o_tall, sizeof(double) * n, hipMemcpyDeviceToHost));
     if(rc == GALIC_OK && orbits) rc = hip_ok(hipMemcpy(orbits + base, c.o_norbit, sizeof(int) * n, hipMemcpyDeviceToHost));
     if(rc == GALIC_OK && steps) rc = hip_ok(hipMemcpy(steps + base, c.o_steps, sizeof(long long) * n, hipMemcpyDeviceToHost));

@@ -212,6 +212,8 @@ struct Ctx {
   size_t g32_scratch_len = 0;
   unsigned int *tile_list = nullptr;  // FP32 merit, tile form: the records' tile lists, per workgroup
   size_t tile_list_len = 0;
+  double *fields_buf = nullptr;       // response fields on their way to the host
+  size_t fields_len = 0;
   int4 *tdesc = nullptr;              // 16x16-tile form: the lists' tiles of a rep's trials
   size_t tdesc_len = 0;
   double *tpart = nullptr;            // ... and their orbit terms, [trial][5][K]

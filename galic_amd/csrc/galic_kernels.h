@@ -113,6 +113,9 @@ struct OrbitIn {
 __global__ void k_prepare_trials(int ntrial, const int *tidx, const double *tvx, const double *tvy,
                                  const double *tvz, Particles P, OrbitIn O);
 __global__ void k_prepare_all(int n, int base, Particles P, OrbitIn O);
+constexpr int kFieldCells = 256;
+template <typename T>
+__global__ void k_fields_out(int ngrid, int nblk, T *slots, double *out);
 __global__ void k_store_orbits(int n, int base, const int *norbit, int *orbits);
 
 }  // namespace galic
