@@ -71,18 +71,6 @@ void dfree(T *&ptr) {
   ptr = nullptr;
 }
 
-constexpr int kListTrials = 512;
-
-// Room for a 64-bit sum per rep of a group.
-int ensure_rep_bounds(galic::Ctx &c, int nrep) {
-  if(c.cm_bound_len >= nrep) return GALIC_OK;
-  dfree(c.cm_bound);
-  c.cm_bound_len = 0;
-  CHK(dalloc(&c.cm_bound, (size_t)nrep));
-  c.cm_bound_len = nrep;
-  return GALIC_OK;
-}
-
 inline int nblocks(size_t n, int bs) { return (int)((n + bs - 1) / bs); }
 
 // Newton solve for the spacing factor (grid.c:353-374 and the FG/EG copies).
@@ -1126,8 +1114,6 @@ int galic_destroy(galic_ctx *ctx) {
   dfree(c.g32_scratch);
   dfree(c.tile_list);
   dfree(c.tile_aux);
-  dfree(c.tdesc);
-  dfree(c.tpart);
   dfree(c.fields_buf);
   dfree(c.cm_cnt); dfree(c.cm_start); dfree(c.cm_chunks); dfree(c.cm_buf); dfree(c.cm_aux); dfree(c.cm_bound);
   dfree(c.merit_prof);
@@ -2078,10 +2064,11 @@ int fp32_run(galic_ctx *ctx, int ntrial, const int *idx, int K, int rep_size, co
   // tiles restricted to the nodes the logs touch, where their LDS fits (form 3; the dense
   // tiles measured faster so far and are the automatic choice)
   auto use_sparse = [&]() { return use_tiles() && c.merit_form == 3 && sparse_lds() <= lds_max; };
-  // 16x16 tiles in the particle's own int32 fixed point (k_t16_lists, k_t16_merit): the automatic
-  // choice where it applies (form 4 asks for it)
+  // 16x16 tiles in the particle's own int32 fixed point (k_eval_t16): the automatic choice
+  // where it applies (form 4 asks for it)
+  const size_t t16_lds = galic::t16_lds_bytes(std::max(c.L, 4), K, K <= 8 ? 8 : 16) + 1024;
   const bool t16 = (c.merit_form == 0 || c.merit_form == 4) && c.L >= 4 && c.L <= galic::T16_MAX_LEVEL &&
-                   K <= galic::T16_MAX_K;
+                   K <= galic::T16_MAX_K && t16_lds <= lds_max;
   const bool gmem = c.L > 7;
   const int kGBlocks = 512;
   auto eval_lds_gmem = [&]() {
@@ -2187,7 +2174,7 @@ int fp32_run(galic_ctx *ctx, int ntrial, const int *idx, int K, int rep_size, co
     const bool gmem_now = !t16 && !tiles && (gmem || eval_lds(1) > lds_max);
     const bool use_o = gmem_now || eval_lds(2) <= lds_max;
     const bool bwl = tiles && tile_lds_bw(true) <= lds_max;
-    const size_t shmem = (t16      ? 1024 * (size_t)(K + 2)  // the K+1 grids of a tile
+    const size_t shmem = (t16      ? t16_lds
                           : sparse ? sparse_lds()
                           : tiles  ? tile_lds_bw(bwl)
                           : gmem_now ? eval_lds_gmem()
@@ -2203,67 +2190,17 @@ int fp32_run(galic_ctx *ctx, int ntrial, const int *idx, int K, int rep_size, co
     // tile form: workgroups resident at once (each takes trials b, b + grid, ...), and list
     // room for the largest particle of the group (a record is listed in at most four tiles)
     int tile_grid = 0, tile_cap = 0;
-    // 16x16-tile form: trials whose lists are made at once (a rep's, unless memory is short) and the
-    // entries there is room for
-    int t16_chunk = 0;
-    size_t t16_room = 0;
-    if(t16) {
-      if((size_t)c.slot_bytes / log_block_bytes() * galic::LOG_B > 0xffffffffull)
-        return set_err(GALIC_ERR_ARG, "the log arena has more records than 32-bit list entries address");
-      const int nrep_t = (s1 - 1) / rep_size - r0 + 1;
-      CHK(ensure_rep_bounds(c, nrep_t));
-      if(!c.tile_aux) CHK(dalloc(&c.tile_aux, 4));
-      HIPCHK(hipMemsetAsync(c.tile_aux, 0, 2 * sizeof(unsigned int), c.stream));
-      HIPCHK(hipMemsetAsync(c.cm_bound, 0, sizeof(unsigned long long) * nrep_t, c.stream));
-      hipLaunchKernelGGL(galic::k_t16_bound, dim3(nblocks(ng, 256)), dim3(256), 0, c.stream, ng, K, s0, rep_size,
-                         (const int *)c.t_inv, (const int *)c.log_n, c.cm_bound, c.tile_aux);
-      HIPCHK(hipGetLastError());
-      std::vector<unsigned long long> bound(nrep_t);
-      unsigned int mx = 0;
-      HIPCHK(hipMemcpyAsync(bound.data(), c.cm_bound, sizeof(unsigned long long) * nrep_t, hipMemcpyDeviceToHost,
-                            c.stream));
-      HIPCHK(hipMemcpyAsync(&mx, c.tile_aux, sizeof(mx), hipMemcpyDeviceToHost, c.stream));
-      HIPCHK(hipStreamSynchronize(c.stream));
-      const size_t one = 4 * (size_t)mx + 64;
-      if(one > 0x7fffffffu) return set_err(GALIC_ERR_NOMEM, "a particle's response logs hold %u records", mx);
-      size_t want = 64;
-      for(unsigned long long v : bound) want = std::max(want, (size_t)v + 64);
-      t16_chunk = ng;
-      if(2 * want > c.tile_list_len) {
-        dfree(c.tile_list);
-        c.tile_list_len = 0;
-        // (a quarter more than now needed, so that the next calls' logs seldom need another)
-        size_t words = 2 * (want + want / 4);
-        if(dalloc(&c.tile_list, words) != GALIC_OK) {
-          // short of memory: kListTrials trials at a time, each with room for the largest
-          (void)hipGetLastError();
-          t16_chunk = std::min(ng, kListTrials);
-          words = 2 * (size_t)t16_chunk * one;
-          CHK(dalloc(&c.tile_list, words));
-        }
-        c.tile_list_len = words;
-      }
-      t16_room = c.tile_list_len / 2;
-      const int ntile = 1 << (2 * (c.L - 4)), nmax = std::min(ng, rep_size);
-      if(c.tdesc_len < (size_t)nmax * (ntile + 2)) {
-        dfree(c.tdesc);
-        c.tdesc_len = 0;
-        CHK(dalloc(&c.tdesc, (size_t)nmax * (ntile + 2)));
-        c.tdesc_len = (size_t)nmax * (ntile + 2);
-      }
-      if(c.tpart_len < (size_t)nmax * galic::kFields * K) {
-        dfree(c.tpart);
-        c.tpart_len = 0;
-        CHK(dalloc(&c.tpart, (size_t)nmax * galic::kFields * K));
-        c.tpart_len = (size_t)nmax * galic::kFields * K;
-      }
-    }
-    if(tiles) {
+    const int t16_kr = K <= 8 ? 8 : 16;
+    const void *t16_kern =
+        c.L == 9 ? (t16_kr == 8 ? (const void *)galic::k_eval_t16<9, 8> : (const void *)galic::k_eval_t16<9, 16>)
+                 : (t16_kr == 8 ? (const void *)galic::k_eval_t16<0, 8> : (const void *)galic::k_eval_t16<0, 16>);
+    if(tiles || t16) {
       int per_cu = 0, ncu = 0;
-      auto kern = sparse ? (c.L == 9 ? (const void *)galic::k_eval_sparse32<9> : (const void *)galic::k_eval_sparse32<0>)
+      auto kern = t16 ? t16_kern
+                  : sparse ? (c.L == 9 ? (const void *)galic::k_eval_sparse32<9> : (const void *)galic::k_eval_sparse32<0>)
                   : c.L == 9 ? (bwl ? (const void *)galic::k_eval_tile32<9, true> : (const void *)galic::k_eval_tile32<9, false>)
                              : (bwl ? (const void *)galic::k_eval_tile32<0, true> : (const void *)galic::k_eval_tile32<0, false>);
-      HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 1024, shmem));
+      HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, t16 ? 64 * galic::kFields : 1024, shmem));
       HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c.device));
       if(per_cu < 1) return set_err(GALIC_ERR_ARG, "the tile merit kernel does not fit on a CU (%zu bytes of LDS)", shmem);
       if(c.merit_wg_per_cu > 0) per_cu = std::min(per_cu, c.merit_wg_per_cu);
@@ -2287,8 +2224,10 @@ int fp32_run(galic_ctx *ctx, int ntrial, const int *idx, int K, int rep_size, co
       if(want > 0x7fffffffu) return set_err(GALIC_ERR_NOMEM, "a particle's response logs hold %u records", mx);
       tile_cap = (int)((want + 3) & ~(size_t)3);
       // the sparse form keeps a copy of each listed record (a word and five float4, 21 words);
-      // the dense form one word per entry
-      const size_t words = (size_t)tile_grid * tile_cap * (sparse ? 21 : 1);
+      // the dense form one word per entry, the 16x16 form two (the arena record index and the log)
+      if(t16 && (size_t)c.slot_bytes / log_block_bytes() * galic::LOG_B > 0xffffffffull)
+        return set_err(GALIC_ERR_ARG, "the log arena has more records than 32-bit list entries address");
+      const size_t words = (size_t)tile_grid * tile_cap * (t16 ? 2 : sparse ? 21 : 1);
       if(c.tile_list_len < words) {
         dfree(c.tile_list);
         c.tile_list_len = 0;
@@ -2350,46 +2289,42 @@ int fp32_run(galic_ctx *ctx, int ntrial, const int *idx, int K, int rep_size, co
     // launch order by decreasing record count made by rocPRIM's radix sort, or in one workgroup
     // (device_order, which a graph can hold: the radix sort sets memory with memset nodes)
     auto t16_rep = [&](galic::EvalArgs32 &E, int a, int b, bool device_order) -> int {
+      E.nblk = b - a;
       E.tlist2 = (uint2 *)c.tile_list;
-      E.tlist_room = t16_room;
-      E.tcursor = (unsigned long long *)(c.tile_aux + 2);
-      E.tdesc = c.tdesc;
-      E.tpart = c.tpart;
+      E.tlist_cap = tile_cap;
       E.tile_err = c.tile_aux + 1;
       E.log_tot = c.log_tot;
       E.vinst = c.t_vinst;
       E.prof = c.merit_prof;
       E.tcut = c.tcut;
-      E.choose = 1;
+      E.work_order = c.t_ord2;
+      E.work_next = (int *)c.tile_aux + 2;
       if(device_order) {
-        hipLaunchKernelGGL(galic::k_record_order, dim3(1), dim3(1024), sizeof(short) * (b - a), c.stream, b - a,
+        int m = 1;
+        while(m < b - a) m <<= 1;
+        hipLaunchKernelGGL(galic::k_record_order, dim3(1), dim3(1024), sizeof(unsigned long long) * m, c.stream, b - a,
                            K, E.slot_pos, (const int *)c.log_n, c.t_ord2);
-      } else if(galic::sort_trials_by_records(b - a, K, E.slot_pos, c.log_n, c.t_key, c.t_key2, c.t_ord, c.t_ord2,
-                                              &c.sort_tmp, &c.sort_tmp_bytes, c.stream) != 0) {
-        return set_err(GALIC_ERR_HIP, "sorting the trials by record count failed");
+        hipLaunchKernelGGL(galic::k_fill_u32, dim3(1), dim3(64), 0, c.stream, c.tile_aux + 2, 0u, (size_t)1);
+      } else {
+        if(galic::sort_trials_by_records(b - a, K, E.slot_pos, c.log_n, c.t_key, c.t_key2, c.t_ord, c.t_ord2,
+                                         &c.sort_tmp, &c.sort_tmp_bytes, c.stream) != 0)
+          return set_err(GALIC_ERR_HIP, "sorting the trials by record count failed");
+        HIPCHK(hipMemsetAsync(E.work_next, 0, sizeof(int), c.stream));
       }
-      // instantaneous terms before, the sums of the fields and the write-back of the choice after
-      E.nblk = b - a;
+      const int grid = std::min(b - a, tile_grid);
+      // instantaneous terms before, the write-back of the choice after the merit kernel
       hipLaunchKernelGGL(galic::k_trial_inst, dim3(nblocks((size_t)(b - a) * K, 256)), dim3(256), 0, c.stream, c.M, E,
                          c.t_vinst);
-      const auto lists = c.L == 9 ? galic::k_t16_lists<9> : galic::k_t16_lists<0>;
-      const auto merit = c.L == 9 ? (K <= 4   ? galic::k_t16_merit<9, 4>
-                                     : K <= 8 ? galic::k_t16_merit<9, 8>
-                                              : galic::k_t16_merit<9, 16>)
-                                  : (K <= 4   ? galic::k_t16_merit<0, 4>
-                                     : K <= 8 ? galic::k_t16_merit<0, 8>
-                                              : galic::k_t16_merit<0, 16>);
-      const size_t lists_lds = 2 * sizeof(int) << (2 * (c.L - 4));
-      for(int i = 0; i < b - a; i += t16_chunk) {
-        E.nblk = std::min(t16_chunk, b - a - i);
-        E.work_order = c.t_ord2 + i;
-        const int grid = nblocks(E.nblk, galic::kXcd) * galic::kXcd * galic::kFields;
-        hipLaunchKernelGGL(galic::k_fill_u32, dim3(1), dim3(64), 0, c.stream, c.tile_aux + 2, 0u, (size_t)2);
-        hipLaunchKernelGGL(lists, dim3(E.nblk), dim3(galic::T16_LT), lists_lds, c.stream, c.M, E);
-        hipLaunchKernelGGL(merit, dim3(grid), dim3(64), shmem, c.stream, c.M, E);
-      }
+      const dim3 tb(64 * galic::kFields);
+      if(c.L == 9 && t16_kr == 8)
+        hipLaunchKernelGGL((galic::k_eval_t16<9, 8>), dim3(grid), tb, shmem, c.stream, c.M, E);
+      else if(c.L == 9)
+        hipLaunchKernelGGL((galic::k_eval_t16<9, 16>), dim3(grid), tb, shmem, c.stream, c.M, E);
+      else if(t16_kr == 8)
+        hipLaunchKernelGGL((galic::k_eval_t16<0, 8>), dim3(grid), tb, shmem, c.stream, c.M, E);
+      else
+        hipLaunchKernelGGL((galic::k_eval_t16<0, 16>), dim3(grid), tb, shmem, c.stream, c.M, E);
       HIPCHK(hipGetLastError());
-      E.nblk = b - a;
       hipLaunchKernelGGL(galic::k_apply_best, dim3(nblocks(b - a, 256)), dim3(256), 0, c.stream, c.M, E);
       HIPCHK(hipGetLastError());
       return GALIC_OK;
@@ -2417,8 +2352,16 @@ int fp32_run(galic_ctx *ctx, int ntrial, const int *idx, int K, int rep_size, co
       nrep_g++;
       max_n = std::max(max_n, std::min({ntrial, (r + 1) * rep_size, s1}) - std::max(r * rep_size, s0));
     }
-    if(t16 && c.use_graph && c.cuts_ready && max_n <= galic::kOrderMax) {
-      CHK(ensure_rep_bounds(c, nrep_g));
+    int m_order = 1;
+    while(m_order < max_n) m_order <<= 1;
+    if(t16 && c.use_graph && c.cuts_ready && max_n <= galic::kOrderMax &&
+       sizeof(unsigned long long) * m_order <= lds_max) {
+      if(c.cm_bound_len < nrep_g) {
+        dfree(c.cm_bound);
+        c.cm_bound_len = 0;
+        CHK(dalloc(&c.cm_bound, (size_t)nrep_g));
+        c.cm_bound_len = nrep_g;
+      }
       hipLaunchKernelGGL(galic::k_fill_u32, dim3(nblocks(2 * (size_t)nrep_g, 256)), dim3(256), 0, c.stream,
                          (unsigned int *)c.cm_bound, 0u, 2 * (size_t)nrep_g);
       hipLaunchKernelGGL(galic::k_commit_bound, dim3(nblocks(ng, 256)), dim3(256), 0, c.stream, ng, K, s0, rep_size,

@@ -232,12 +232,13 @@ __global__ void __launch_bounds__(1024) k_commit_layout(const unsigned int *gcnt
 // buckets.  Trial b is trial first + b, of rep (first + b) / rep_size - first / rep_size.
 __global__ void k_commit_bound(int n, int K, int first, int rep_size, const int *slot_pos, const int *log_n,
                                unsigned long long *rep_bound) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x, b = min(g, n - 1);
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if(b >= n) return;
   const size_t o0 = (size_t)slot_pos[b] * (K + 1);
   int mx = 0;
   for(int k = 1; k <= K; k++) mx = max(mx, log_n[o0 + k]);
   const unsigned long long e = 4ull * ((unsigned long long)mx + (unsigned long long)max(log_n[o0], 0));
-  add_to_rep(rep_bound, (first + b) / rep_size - first / rep_size, g < n ? e : 0);  // (the other lanes add nothing)
+  atomicAdd(&rep_bound[(first + b) / rep_size - first / rep_size], e);
 }
 
 }  // namespace galic

@@ -214,10 +214,6 @@ struct Ctx {
   size_t tile_list_len = 0;
   double *fields_buf = nullptr;       // response fields on their way to the host
   size_t fields_len = 0;
-  int4 *tdesc = nullptr;              // 16x16-tile form: the lists' tiles of a rep's trials
-  size_t tdesc_len = 0;
-  double *tpart = nullptr;            // ... and their orbit terms, [trial][5][K]
-  size_t tpart_len = 0;
   unsigned int *tile_aux = nullptr;
   double *tsrc = nullptr;        // sources of the table fill (galic_set_tree_sources): [4][tsrc_n] x, y, z, mass
   int tsrc_n = 0;

@@ -82,17 +82,13 @@ struct EvalArgs32 {
   unsigned int *tlist;  // tile form: per workgroup, tlist_cap entries of the records' tile lists
   int tlist_cap;
   unsigned int *tile_err;  // tile form: set when a particle's lists exceed tlist_cap
-  // 16x16-tile form (k_t16_lists, k_t16_merit)
-  uint2 *tlist2;                // list entries (record index, t16_entry's word), tlist_room of them
-  unsigned long long tlist_room;
-  unsigned long long *tcursor;  // entries taken (zero at launch)
-  int4 *tdesc;                  // [trial][ntile + 2] the lists' tiles
-  double *tpart;                // [trial][5][K] orbit terms of each field
+  uint2 *tlist2;           // 16x16-tile form: per workgroup, tlist_cap entries (record index, log)
   const float *log_tot;    // [orbit][5] sums of each log's values (k_orbit32_log)
   int no_deltas;           // the taken trial's deltas are left to the region commit (k_commit_*)
   const unsigned char *tcut;  // 16x16-tile form: [type][tile] levels of the tile's cut-A nodes (bit u: L-u
                               // inside the tile, bit 5: a cut-A node above the tile)
   const int *work_order;   // 16x16-tile form: trials in the order workgroups take them
+  int *work_next;          // ... from this counter (zero at launch)
   unsigned long long *prof;  // sparse tile form, optional: time per phase and sizes, summed over particles
   int tbl_lds;               // sparse tile form: the block tables staged in LDS (else read from log_blocks)
   const double *vinst;       // sparse tile form: instantaneous merit change of each trial (k_trial_inst)
@@ -114,7 +110,6 @@ struct EvalArgs32 {
   const long long *osteps;  // steps of each orbit of the chunk
   int *psteps;              // per particle: steps of its current orbit (updated)
   long long *locA_dq, *locI_dq;
-  int choose;               // k_apply_best sums tpart and takes the best improving trial (else accept is set)
   int *accept;
   double *dF;
   double *dFk;  // merit change of trial k of trial ti at ti * K + k
@@ -187,36 +182,30 @@ __host__ __device__ inline size_t sparse_lds_bytes(int L, int K, int log_M, bool
 }
 template <int LF>
 __global__ void k_eval_sparse32(DevModel M, EvalArgs32 A);
-// 16x16-tile form of the FP32 merit (k_t16_lists, k_t16_merit): int32 tile grids in the particle's
-// own fixed point, one wave per field, all trials of a tile per lane; at most T16_MAX_K trials.
+// 16x16-tile form of the FP32 merit (k_eval_t16): int32 tile grids in the particle's own fixed
+// point, one wave per field, all trials of a tile per lane; at most T16_MAX_K trials.
 constexpr int T16 = 16;
 constexpr int T16_MAX_K = 16;
 constexpr int T16_MAX_LEVEL = 10;  // Morton codes of up to 64 x 64 tiles; open ancestors of up to 8 levels
-constexpr int T16_LT = 256;  // threads of k_t16_lists
-constexpr int kXcd = 8;      // dies that a launch's workgroups go to in turn
-template <int LF>
-__global__ void k_t16_lists(DevModel M, EvalArgs32 A);
+// int32 words at the front of its LDS: the K+1 grids (the current orbit's, then the trials')
+// of a tile's five fields (the tile counts share them while the lists are built).
+__host__ __device__ inline int t16_grid_words(int K, int L) {
+  const int a = (K + 1) * kFields * T16 * T16, b = 1 << (2 * (L - 4));
+  return a > b ? a : b;
+}
+// words of the per-tile log masks: two tiles a word for up to 15 trials (KR the trial capacity)
+__host__ __device__ inline int t16_mask_words(int ntile, int KR) { return KR <= 15 ? (ntile + 1) / 2 : ntile; }
+// LDS of k_eval_t16 beyond its static arrays: the grids, the list offsets [ntile + 1], the
+// active tiles [ntile] (16-bit) and the masks.
+__host__ __device__ inline size_t t16_lds_bytes(int L, int K, int KR) {
+  const int ntile = 1 << (2 * (L - 4));
+  return 4 * ((size_t)t16_grid_words(K, L) + ntile + 1 + (ntile + 1) / 2 + t16_mask_words(ntile, KR));
+}
 template <int LF, int KR>
-__global__ void k_t16_merit(DevModel M, EvalArgs32 A);
-__global__ void k_t16_bound(int n, int K, int first, int rep_size, const int *slot_pos, const int *log_n,
-                            unsigned long long *rep_bound, unsigned int *most);
+__global__ void k_eval_t16(DevModel M, EvalArgs32 A);
 __global__ void k_trial_inst(DevModel M, EvalArgs32 A, double *vinst);
 __global__ void k_apply_best(DevModel M, EvalArgs32 A);
 __global__ void k_log_totals(int n, int K, const int *slot_pos, const int *log_n, unsigned int *maxsum);
-
-#if defined(__HIPCC__)
-// sum[rep] += v for every lane of a wave: one atomic where the wave's lanes are of one rep (a lane
-// each, 3e4 trials' atomics on three words took 0.36 ms).
-__device__ __forceinline__ void add_to_rep(unsigned long long *sum, int rep, unsigned long long v) {
-  if(__all(rep == __builtin_amdgcn_readfirstlane(rep))) {
-    for(int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    if((threadIdx.x & 63) == 0) atomicAdd(&sum[rep], v);
-  } else {
-    atomicAdd(&sum[rep], v);
-  }
-}
-#endif
-
 
 // Logs into the fixed-point Loc grids through region buckets (galic_commit.hip).
 struct CommitArgs {

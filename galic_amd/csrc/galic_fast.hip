@@ -623,39 +623,37 @@ __global__ void k_fill_u32(unsigned int *p, unsigned int v, size_t n) {
   if(i < n) p[i] = v;
 }
 
-// Trials by decreasing record count in one workgroup, to 3%: a counting sort over 32 classes per
-// power of two (the order within a class is any; it decides when a trial is judged, not the result).
-// The bitonic sort of the exact counts it replaces took 0.28 ms for 1e4 trials, this 0.14.
-// (dynamic LDS: 2 bytes per trial)
+// The order of k_record_keys + sort_desc in one workgroup: (inverted key, index) pairs in LDS
+// (dynamic, 8 bytes per element of the power of two above n), bitonic sort ascending.
 __global__ void __launch_bounds__(1024) k_record_order(int n, int K, const int *slot_pos, const int *log_n, int *ord) {
-  extern __shared__ unsigned short cls[];
-  __shared__ unsigned int at[1024], wsum[16];
-  const int tid = threadIdx.x, lane = tid & 63;
-  at[tid] = 0;
-  __syncthreads();
-  for(int b = tid; b < n; b += 1024) {
-    const size_t o0 = (size_t)slot_pos[b] * (K + 1);
-    unsigned int s = 0;
-    for(int o = 0; o <= K; o++) s += (unsigned int)max(log_n[o0 + o], 0);
-    // exponent and five bits of the mantissa
-    const int c = 1023 - (int)(__float_as_uint((float)max(s, 1u)) >> 18) + (127 << 5);
-    cls[b] = (unsigned short)max(c, 0);
-    atomicAdd(&at[max(c, 0)], 1u);
+  extern __shared__ unsigned long long ko[];
+  int m = 1;
+  while(m < n) m <<= 1;
+  for(int b = threadIdx.x; b < m; b += blockDim.x) {
+    unsigned long long v = ~0ull;
+    if(b < n) {
+      const size_t o0 = (size_t)slot_pos[b] * (K + 1);
+      unsigned int s = 0;
+      for(int o = 0; o <= K; o++) s += (unsigned int)max(log_n[o0 + o], 0);
+      v = ((unsigned long long)(~s) << 32) | (unsigned int)b;
+    }
+    ko[b] = v;
   }
   __syncthreads();
-  // exclusive scan of the classes' counts
-  const unsigned int v = at[tid];
-  unsigned int s = v;
-  for(int d = 1; d < 64; d <<= 1) {
-    const unsigned int y = __shfl_up(s, d);
-    if(lane >= d) s += y;
-  }
-  if(lane == 63) wsum[tid >> 6] = s;
-  __syncthreads();
-  for(int w = 0; w < tid >> 6; w++) s += wsum[w];
-  at[tid] = s - v;
-  __syncthreads();
-  for(int b = tid; b < n; b += 1024) ord[atomicAdd(&at[cls[b]], 1u)] = b;
+  for(int size = 2; size <= m; size <<= 1)
+    for(int stride = size >> 1; stride > 0; stride >>= 1) {
+      for(int i = threadIdx.x; i < m / 2; i += blockDim.x) {
+        const int lo = 2 * i - (i & (stride - 1)), hi = lo + stride;
+        const bool up = (lo & size) == 0;
+        const unsigned long long a = ko[lo], c = ko[hi];
+        if((a > c) == up) {
+          ko[lo] = c;
+          ko[hi] = a;
+        }
+      }
+      __syncthreads();
+    }
+  for(int b = threadIdx.x; b < n; b += blockDim.x) ord[b] = (int)(unsigned int)ko[b];
 }
 
 // Trials in order of decreasing expected orbit length (stable, so the order is
@@ -872,7 +870,6 @@ constexpr int kDppQuadXor1 = 0xB1;  // quad_perm [1,0,3,2]
 constexpr int kDppQuadXor2 = 0x4E;  // quad_perm [2,3,0,1]
 constexpr int kDppRowRor4 = 0x124;
 constexpr int kDppRowRor8 = 0x128;
-constexpr int kDppWaveShr1 = 0x138;  // the lane below
 
 template <int CTRL>
 __device__ __forceinline__ long long dpp_i64(long long v) {
@@ -1429,22 +1426,6 @@ __global__ void k_log_totals(int n, int K, const int *slot_pos, const int *log_n
   atomicMax(maxsum, s);
 }
 
-// List entries that the trials of each rep of a group need at most (a record is listed in up to four
-// tiles), and the largest record count of one trial's K+1 logs.  Trial b is trial first + b, of rep (first + b) / rep_size - first / rep_size.
-__global__ void k_t16_bound(int n, int K, int first, int rep_size, const int *slot_pos, const int *log_n,
-                            unsigned long long *rep_bound, unsigned int *most) {
-  const int b = min((int)(blockIdx.x * blockDim.x + threadIdx.x), n - 1);
-  const bool own = blockIdx.x * blockDim.x + threadIdx.x < (unsigned int)n;  // (the other lanes add nothing)
-  const size_t o0 = (size_t)slot_pos[b] * (K + 1);
-  unsigned long long s = 0;
-  if(own)
-    for(int o = 0; o <= K; o++) s += (unsigned int)max(log_n[o0 + o], 0);
-  add_to_rep(rep_bound, (first + b) / rep_size - first / rep_size, 4 * s);
-  unsigned int mx = (unsigned int)min(s, 0xffffffffull);
-  for(int o = 32; o > 0; o >>= 1) mx = max(mx, (unsigned int)__shfl_xor((int)mx, o));
-  if((threadIdx.x & 63) == 0) atomicMax(most, mx);
-}
-
 template <int LF, bool BWL>
 __global__ void __launch_bounds__(1024) k_eval_tile32(DevModel M, EvalArgs32 A) {
   extern __shared__ double lds_d[];
@@ -1737,26 +1718,6 @@ __global__ void k_apply_best(DevModel M, EvalArgs32 A) {
   const int K = A.K, ti = A.trial_base + bid;
   const int j = A.slot_pos ? A.slot_pos[bid] : bid;
   const int p = A.tidx[ti], t = A.P.type[p];
-  if(A.choose) {
-    // the best improving trial, if any
-    int bk = -1;
-    double bv = 0;
-    const double *fit = A.fit + (size_t)t * 16;
-    for(int k = 0; k < K; k++) {
-      const size_t qk = (size_t)ti * K + k;
-      double orbit_terms = 0;
-      for(int f = 0; f < kFields; f++) orbit_terms += A.tpart[((size_t)bid * kFields + f) * K + k];
-      const double v = orbit_terms + fit[5] / fit[6] * A.vinst[qk];
-      A.dFk[qk] = v;
-      if(v < bv) {
-        bv = v;
-        bk = k;
-      }
-    }
-    A.accept[ti] = bk + 1;
-    A.dF[ti] = bk >= 0 ? bv : A.dFk[(size_t)ti * K];
-    if(A.prof && bk >= 0) atomicAdd(&A.prof[8], 1ull);
-  }
   const int best = A.accept[ti] - 1;
   const size_t o0 = (size_t)j * (K + 1), oc = (best >= 0) ? o0 + 1 + best : o0;
   A.P.orbits[p] = A.norbit[oc];
@@ -2231,12 +2192,11 @@ template __global__ void k_eval_sparse32<9>(DevModel M, EvalArgs32 A);
 //    kp[f] = 30 - e with the largest total of the particle's K+1 orbits (k_orbit32_log's
 //    log_tot) below 2^e.  Every sum of one orbit's values then stays below 2^30 (+ one unit
 //    per record of rounding), so tile grids and node sums are exact int32.
-//  * Tiles of 16 x 16 cells, taken in Morton order.  k_t16_lists lists the records of the K+1 logs
-//    by tile (arena record index, place in the tile and log; a record whose 2x2 cells straddle a
-//    tile edge is listed in each tile it reaches).
-//  * k_t16_merit evaluates one field of one particle per wave, a workgroup of its own: a tile's
-//    K+1 grids of the field in LDS, node-major: the four cells of a 2x2 node are one 16-byte
-//    word.  Lane j owns the tile's 2x2 node j (lanes in Morton order, so
+//  * Tiles of 16 x 16 cells, taken in Morton order.  The records of the K+1 logs are listed by
+//    tile (arena record index, log index; a record whose 2x2 cells straddle a tile edge is
+//    listed in each tile it reaches).  A tile's K+1 grids of all five fields sit in LDS at once,
+//    node-major: the four cells of a 2x2 node are one 16-byte word.
+//  * Wave f evaluates field f.  Lane j owns the tile's 2x2 node j (lanes in Morton order, so
 //    groups of 4 and 16 lanes are the 4x4 and 8x8 nodes and the wave is the tile); its
 //    (residual, weight) pairs stay in registers for all trials, and for each trial the lane forms
 //    D on its four cells, the node sum, the quad and row sums (DPP) and the tile sum, and adds
@@ -2244,16 +2204,9 @@ template __global__ void k_eval_sparse32<9>(DevModel M, EvalArgs32 A);
 //  * Levels above the tiles: a tile's ancestor at level l is complete once the walk reaches a
 //    tile with another ancestor at l.  Lane k keeps trial k's partial sums of the open
 //    ancestors (a stack of one sum per level) and closes them level by level.
-// Then k_apply_best sums the fields, adds the instantaneous terms (k_trial_inst) and makes the
-// choice; the deltas of the taken trial are the region commit's (k_commit_*).
-//
-// Why one wave a workgroup: five waves (a particle's fields) in one workgroup always put two on the
-// same SIMD, so at 128 registers a CU held two such workgroups, ten waves, where sixteen of these
-// fit; and between barriers each tile cost the wait of its gathers (65% of the waves' time).  3000
-// particles with 8 trials on 512^2 grids: 8.5 ms in workgroups of five that list and evaluate, 1.2
-// (lists) + 6.4 apart; there the gathers bound it: 21 GB at 3.4 TB/s, each record's line fetched
-// about twice for its five fields.  10000 on 64^2 grids: 2.4 ms, 0.44 + 1.9: waits for the lists of
-// its few long tiles.
+// Then the choice (the instantaneous terms come from k_trial_inst; the write-back follows in
+// k_apply_best) and the deltas of the taken trial: exact int64 sums at the log scale on
+// blocks of 32 x 32 cells (four consecutive tiles), the same values as k_eval_tile32.
 
 __device__ __forceinline__ int spread6(int x) {
   x &= 63;
@@ -2273,24 +2226,21 @@ __device__ __forceinline__ int compact6(int x) {
 __device__ __forceinline__ int t16_code(int tz, int tr) { return spread6(tr) | (spread6(tz) << 1); }
 __device__ __forceinline__ int t16_z(int m) { return compact6(m >> 1); }
 __device__ __forceinline__ int t16_r(int m) { return compact6(m); }
-// A list entry's word for log o: the 2x2 cells from tile-local (lz, lr), each -1 .. 15 (-1 and 16
-// outside the tile).  A cell's word in the node-major 16 x 16 grid is the Morton code of (lz, lr):
-// bits 0-7 hold the first cell's, 8-15 the last cell's (the even bits are lr's, the odd ones lz's,
-// so the other two cells' mix them), 16-19 which of the four cells the tile holds, 20 on the log.
-__device__ __forceinline__ unsigned int t16_entry(int lz, int lr, unsigned int o) {
-  const unsigned int w0 = t16_code(lz & 15, lr & 15), w1 = t16_code((lz + 1) & 15, (lr + 1) & 15);
-  const unsigned int z0 = lz >= 0 ? 3u : 0u, z1 = lz < 15 ? 12u : 0u, r0 = lr >= 0 ? 5u : 0u, r1 = lr < 15 ? 10u : 0u;
-  return w0 | w1 << 8 | ((z0 | z1) & (r0 | r1)) << 16 | o << 20;
+// Word of tile-local cell (cz, cr) in a node-major 16 x 16 grid.
+__device__ __forceinline__ int t16_cell(int cz, int cr) {
+  return ((spread6(cr >> 1) | (spread6(cz >> 1) << 1)) << 2) | ((cz & 1) << 1) | (cr & 1);
 }
 
-// Calls visit(tile, lz, lr) for the tiles beyond its first that the 2x2 cells from (iz, iR) reach.
+// Tiles (Morton codes) reached by the 2x2 cells of quad.
 template <typename Visit>
-__device__ __forceinline__ void t16_straddle(int iz, int iR, Visit visit) {
-  const int z0 = iz >> 4, r0 = iR >> 4, lz = iz & 15, lr = iR & 15;
-  if(lr == 15) visit(t16_code(z0, r0 + 1), lz, -1);
-  if(lz == 15) {
-    visit(t16_code(z0 + 1, r0), -1, lr);
-    if(lr == 15) visit(t16_code(z0 + 1, r0 + 1), -1, -1);
+__device__ __forceinline__ void t16_visit(int quad, int L, Visit visit) {
+  const int iz = quad >> L, iR = quad & ((1 << L) - 1);
+  const int z0 = iz >> 4, z1 = (iz + 1) >> 4, r0 = iR >> 4, r1 = (iR + 1) >> 4;
+  visit(t16_code(z0, r0));
+  if(r1 != r0) visit(t16_code(z0, r1));
+  if(z1 != z0) {
+    visit(t16_code(z1, r0));
+    if(r1 != r0) visit(t16_code(z1, r1));
   }
 }
 
@@ -2304,354 +2254,342 @@ __device__ __forceinline__ int dpp_i32(int v) {
   return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
 }
 
-static_assert(LOG_B == 64, "a log block is a wave's records");
-constexpr int T16_LB = 8;  // log blocks a wave takes at once in the list passes
-constexpr int T16_U = 2;   // list entries of a tile that a lane fetches ahead
-constexpr int T16_UR = 4;  // ... and takes at once of a longer list
-
-// The tile lists of each trial of the launch: tdesc[trial] = {tiles with entries, -, first entry's
-// index in tlist2 (two words)}, then per tile in Morton order {tile, logs reaching it (bit 0 the
-// current orbit's, bit k + 1 trial k's), its first entry, its cut byte} and an end.  One workgroup
-// per trial, the longest first.
-template <int LF>
-__global__ void __launch_bounds__(T16_LT) k_t16_lists(DevModel M, EvalArgs32 A) {
-  extern __shared__ int lds_l[];
-  const int tid = threadIdx.x, lane = tid & 63, K = A.K;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int L = LF ? LF : M.DG_L, nb = 1 << L, ntile = 1 << (2 * (L - 4));
-  int *tcnt = lds_l;                                   // [ntile] counts, then each list's next place
-  unsigned int *tmask = (unsigned int *)(tcnt + ntile);  // [ntile]
-  __shared__ int s_off[T16_MAX_K + 2], s_cnt[T16_MAX_K + 1];
-  __shared__ unsigned long long s_base;
-  const int bid = A.work_order[blockIdx.x], ti = A.trial_base + bid;
-  const int t = A.P.type[A.tidx[ti]];
-  const size_t o0 = (size_t)(A.slot_pos ? A.slot_pos[bid] : bid) * (K + 1);
-  const unsigned long long tp0 = A.prof ? wall_clock64() : 0;
-  if(tid == 0) {
-    // the logs' 64-record blocks in turn: s_off their prefix counts, s_cnt the records
-    int s = 0;
-    for(int o = 0; o <= K; o++) {
-      s_off[o] = s;
-      s_cnt[o] = max(A.log_n[o0 + o], 0);
-      s += (s_cnt[o] + LOG_B - 1) / LOG_B;
-    }
-    s_off[K + 1] = s;
-  }
-  for(int q = tid; q < 2 * ntile; q += T16_LT) tcnt[q] = 0;
-  __syncthreads();
-  // A wave takes T16_LB blocks of 64 records at once, a record a lane, their loads issued together.
-  // Consecutive records are consecutive cells of an orbit, mostly of one tile: a run of lanes in a
-  // tile takes its list places with one LDS atomic (a lane each: up to 64 on one word).
-  const int boff = lane <= K + 1 ? s_off[lane] : 0, bcnt = lane <= K ? s_cnt[lane] : 0;
-  const int nblk = __builtin_amdgcn_readlane(boff, K + 1);
-  auto records = [&](auto visit_run, auto visit_one) {
-    for(int b0 = wave; b0 < nblk; b0 += T16_LT / 64 * T16_LB) {
-      unsigned int rec[T16_LB], ob[T16_LB];
-      int quad[T16_LB];
-#pragma unroll
-      for(int u = 0; u < T16_LB; u++) {
-        const int b = b0 + u * (T16_LT / 64);
-        const unsigned int o = __popcll(__ballot(lane >= 1 && lane <= K && b >= boff));
-        const int q = b - __builtin_amdgcn_readlane(boff, o);
-        quad[u] = -1;
-        rec[u] = 0;
-        ob[u] = o;
-        if(b < nblk) {
-          rec[u] = (unsigned int)A.log_blocks[(o0 + o) * A.log_M + q] * LOG_B + lane;
-          if(q * LOG_B + lane < __builtin_amdgcn_readlane(bcnt, o)) quad[u] = A.log_q[rec[u]];
-        }
-      }
-#pragma unroll
-      for(int u = 0; u < T16_LB; u++) {
-        if(b0 + u * (T16_LT / 64) >= nblk) break;
-        const int iz = quad[u] >> L, iR = quad[u] & (nb - 1);
-        const int m = quad[u] >= 0 ? t16_code(iz >> 4, iR >> 4) : -1;
-        const int mp = __builtin_amdgcn_update_dpp(-2, m, kDppWaveShr1, 0xF, 0xF, false);
-        const unsigned long long heads = __ballot(m != mp);
-        visit_run(rec[u], ob[u], m, iz & 15, iR & 15, heads);
-        if(m >= 0) t16_straddle(iz, iR, [&](int m2, int lz, int lr) { visit_one(rec[u], ob[u], m2, lz, lr); });
-      }
-    }
-  };
-  auto mark = [&](int m, unsigned int o) {
-    if(!(tmask[m] & (1u << o))) atomicOr(&tmask[m], 1u << o);
-  };
-  // lanes from a head on, up to the next (lane: a head)
-  auto run_length = [&](unsigned long long heads) {
-    const unsigned long long after = lane < 63 ? heads >> (lane + 1) : 0ull;
-    return after ? __ffsll((long long)after) : 64 - lane;
-  };
-  records(
-      [&](unsigned int, unsigned int o, int m, int, int, unsigned long long heads) {
-        if(m >= 0 && (heads >> lane & 1)) {
-          atomicAdd(&tcnt[m], run_length(heads));
-          mark(m, o);
-        }
-      },
-      [&](unsigned int, unsigned int o, int m, int, int) {
-        atomicAdd(&tcnt[m], 1);
-        mark(m, o);
-      });
-  __syncthreads();
-  if(wave == 0) {
-    int4 *desc = A.tdesc + (size_t)bid * (ntile + 2);
-    const unsigned char *cut = A.tcut + (size_t)t * ntile;
-    int total = 0, nact = 0;
-    for(int q = 0; q < ntile; q += 64) {
-      const int m = q + lane, n = m < ntile ? tcnt[m] : 0;
-      const unsigned long long act = __ballot(n > 0);
-      if(act == 0) continue;
-      int s = n;
-#pragma unroll
-      for(int d = 1; d < 64; d <<= 1) {
-        const int y = __shfl_up(s, d);
-        if(lane >= d) s += y;
-      }
-      if(n > 0) {
-        tcnt[m] = total + s - n;
-        desc[1 + nact + __popcll(act & ((1ull << lane) - 1))] = make_int4(m, (int)tmask[m], total + s - n, cut[m]);
-      }
-      total += __shfl(s, 63);
-      nact += __popcll(act);
-    }
-    if(lane == 0) {
-      unsigned long long base = atomicAdd(A.tcursor, (unsigned long long)total);
-      if(base + total > A.tlist_room) {
-        // cannot happen with the room of the launch's records; reported, not evaluated
-        atomicOr(A.tile_err, 1u);
-        base = ~0ull;
-        nact = total = 0;
-      }
-      s_base = base;
-      desc[0] = make_int4(nact, 0, (int)(unsigned int)base, (int)(unsigned int)(base >> 32));
-      desc[1 + nact] = make_int4(0, 0, total, 0);
-      if(A.prof) {
-        atomicAdd(&A.prof[5], (unsigned long long)nact);
-        atomicAdd(&A.prof[6], (unsigned long long)total);
-        atomicAdd(&A.prof[7], 1ull);
-        atomicMax(&A.prof[12], (unsigned long long)total);
-      }
-    }
-  }
-  __syncthreads();
-  if(s_base == ~0ull) return;
-  uint2 *list = A.tlist2 + s_base;
-  records(
-      [&](unsigned int rec, unsigned int o, int m, int lz, int lr, unsigned long long heads) {
-        int base = 0;
-        if(m >= 0 && (heads >> lane & 1)) base = atomicAdd(&tcnt[m], run_length(heads));
-        const int hl = 63 - __clzll((long long)(heads & (~0ull >> (63 - lane))));
-        base = __shfl(base, hl);
-        if(m >= 0) list[base + lane - hl] = make_uint2(rec, t16_entry(lz, lr, o));
-      },
-      [&](unsigned int rec, unsigned int o, int m, int lz, int lr) {
-        list[atomicAdd(&tcnt[m], 1)] = make_uint2(rec, t16_entry(lz, lr, o));
-      });
-  if(A.prof && tid == 0) atomicAdd(&A.prof[0], wall_clock64() - tp0);
+// The logs reaching each tile: one bit per log (bit 0 the current orbit, bit k+1 trial k), 16
+// bits per tile for up to 15 trials, 32 above.
+template <int KR>
+__device__ __forceinline__ unsigned int t16_mask_get(const unsigned int *w, int m) {
+  if(KR <= 15) return (w[m >> 1] >> ((m & 1) * 16)) & 0xffffu;
+  return w[m];
+}
+template <int KR>
+__device__ __forceinline__ void t16_mask_or(unsigned int *w, int m, unsigned int bits) {
+  if(KR <= 15)
+    atomicOr(&w[m >> 1], bits << ((m & 1) * 16));
+  else
+    atomicOr(&w[m], bits);
 }
 
-template __global__ void k_t16_lists<0>(DevModel M, EvalArgs32 A);
-template __global__ void k_t16_lists<9>(DevModel M, EvalArgs32 A);
-
-// The orbit terms of one trial particle's trials for one field: a workgroup of one wave, the
-// longest particles first, a particle's fields on one XCD (they read the same records).
-template <int LF, int KR>
-__global__ void __launch_bounds__(64, 4) k_t16_merit(DevModel M, EvalArgs32 A) {
-  // 16-byte aligned: the grids are read and cleared four cells a lane (8 bytes off, as an array of
-  // int after static arrays, the LDS stalled on each such access for 39% of the kernel's time)
-  extern __shared__ __align__(16) int grids[];  // [K+1][256] int32: O, then G_k
-  constexpr int NSTK = (LF ? LF : T16_MAX_LEVEL) - 4;
-  // trial k's sums of the open ancestors of the walk at level l < lt: stk[l * KR + k], lane k's
-  __shared__ int stk[(NSTK > 0 ? NSTK : 1) * KR];
-  const int lane = threadIdx.x, K = A.K;
-  const int L = LF ? LF : M.DG_L, Nstack = GALIC_NSTACK(L), lt = L - 4, ntile = 1 << (2 * lt);
-  const int item = blockIdx.x / kXcd, rank = item / kFields * kXcd + blockIdx.x % kXcd, f = item % kFields;
-  if(rank >= A.nblk) return;
-  const int bid = A.work_order[rank], ti = A.trial_base + bid, t = A.P.type[A.tidx[ti]];
-  const size_t o0 = (size_t)(A.slot_pos ? A.slot_pos[bid] : bid) * (K + 1);
-  const unsigned long long tp0 = A.prof ? wall_clock64() : 0;
-  const int jx = morton_x(lane), jy = morton_y(lane);
-  for(int q = lane; q < (K + 1) * 64; q += 64) ((int4 *)grids)[q] = make_int4(0, 0, 0, 0);
-  for(int q = lane; q < (NSTK > 0 ? NSTK : 1) * KR; q += 64) stk[q] = 0;
-  int kp;
-  {
-    float mx = lane <= K ? A.log_tot[(o0 + lane) * kFields + f] : 0.f;
-    for(int o = 16; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    int e = 0;
-    (void)frexpf(mx, &e);  // mx < 2^e
-    kp = __builtin_amdgcn_readfirstlane(min(126, 30 - e));
+// Offsets of the tiles' lists (exclusive scan of the counts, off[ntile] = total) and the tiles
+// with entries in increasing order (16-bit indices); one wave.
+__device__ __forceinline__ void t16_scan(const int *cnt, int *off, unsigned short *act, int *nact, int ntile, int lane) {
+  const int per = (ntile + 63) / 64, a = min(lane * per, ntile), e = min(a + per, ntile);
+  int s = 0, na = 0;
+  for(int i = a; i < e; i++) {
+    s += cnt[i];
+    na += cnt[i] > 0;
   }
-  const float sc = ldexpf(1.0f, kp);
-  // (written by an earlier kernel: scalar loads)
-  typedef int tile_desc __attribute__((ext_vector_type(4)));
-  const auto desc = (const __attribute__((address_space(4))) tile_desc *)(uintptr_t)(A.tdesc + (size_t)bid * (ntile + 2));
-  const tile_desc head = desc[0];
-  const int nact = head.x;
-  const uint2 *list = A.tlist2 + (((unsigned long long)(unsigned int)head.w << 32) | (unsigned int)head.z);
-  auto tile = [&](int i) { return desc[min(i, nact + 1)]; };
-  unsigned long long tpa = 0, tpb = 0;
-  // (the pairs in FP32: the residual's rounding moves a term |b + D| - |b| only where b + D
-  // changes sign, by at most 2^-23 of |D|)
-  const float2 *bwf = A.merit_bwf + ((size_t)t * kFields + f) * Nstack;
-  double acc[KR];
+  int si = s, ni = na;
 #pragma unroll
-  for(int k = 0; k < KR; k++) acc[k] = 0.0;
-  double accs = 0.0;  // lane k: trial k's terms of the tile nodes and above
-  // lane 4q + j: the 4x4-node terms of trials j, j + 4, ...; lane 16r + k: trial k's 8x8 terms
-  double acc2[(KR + 3) / 4], acc3 = 0.0;
+  for(int d = 1; d < 64; d <<= 1) {
+    const int y = __shfl_up(si, d), z = __shfl_up(ni, d);
+    if(lane >= d) {
+      si += y;
+      ni += z;
+    }
+  }
+  int base = si - s, abase = ni - na;
+  for(int i = a; i < e; i++) {
+    off[i] = base;
+    base += cnt[i];
+    if(cnt[i] > 0) act[abase++] = (unsigned short)i;
+  }
+  if(lane == 63) {
+    off[ntile] = si;
+    *nact = ni;
+  }
+}
+
+constexpr int T16_LU = 8;  // records a thread takes at once in the list passes
+
+// Record index of the q-th record of the particle's logs (orbits' records in turn; s_off
+// the exclusive prefix of the K+1 counts) and its log.
+__device__ __forceinline__ unsigned int t16_record(const EvalArgs32 &A, const int *s_off, int K, size_t o0, int q,
+                                                   int &o) {
+  o = 0;
+  while(o < K && q >= s_off[o + 1]) o++;
+  const int r = q - s_off[o];
+  const int blk = A.log_blocks[(o0 + o) * A.log_M + r / LOG_B];
+  return (unsigned int)blk * LOG_B + (unsigned int)(r & (LOG_B - 1));
+}
+
+template <int LF, int KR>
+__global__ void __launch_bounds__(64 * kFields, 4) k_eval_t16(DevModel M, EvalArgs32 A) {
+  // 16-byte aligned: the grids are read and cleared four cells a lane.  As an array of int it began
+  // 8 bytes off, after the static arrays, and the LDS stalled on each such access for 39% of the
+  // kernel's time (3000 particles, 9 logs each, 512^2 grids: 11.3 ms, aligned 8.5).
+  extern __shared__ __align__(16) int lds_i[];
+  const int tid = threadIdx.x, nt = blockDim.x, K = A.K, wave = tid >> 6, lane = tid & 63;
+  const int L = LF ? LF : M.DG_L, nb = 1 << L, Nstack = GALIC_NSTACK(L);
+  const int lt = L - 4, ntile = 1 << (2 * lt);
+  const int gwords = t16_grid_words(K, L);
+  int *grids = lds_i;                                  // [K+1][5][256] int32: O, then G_k; counts while listing
+  int *tcnt = grids;                                   // [ntile] (list building only)
+  int *toff = grids + gwords;                          // [ntile + 1]
+  unsigned short *tact = (unsigned short *)(toff + ntile + 1);  // [ntile] tiles with entries, Morton order
+  unsigned int *tmask = (unsigned int *)(toff + ntile + 1 + (ntile + 1) / 2);  // logs reaching each tile
+  const int nmask = t16_mask_words(ntile, KR);
+  __shared__ double s_part[kFields][KR];
+  __shared__ double s_dF[KR];
+  __shared__ int s_off[KR + 2], s_kp[kFields], s_nact, s_best, s_item;
+  constexpr int NSTK = (LF ? LF : T16_MAX_LEVEL) - 4;
+  // trial k's sums of the open ancestors of field f's walk at level l < lt: s_stk[f][l][k]
+  __shared__ int s_stk[kFields][NSTK > 0 ? NSTK : 1][KR];
+  __shared__ float s_sc[kFields];
+  uint2 *list = A.tlist2 + (size_t)blockIdx.x * A.tlist_cap;
+  const int jx = morton_x(lane), jy = morton_y(lane);
+
+  for(int q = tid; q < gwords; q += nt) grids[q] = 0;
+  const unsigned long long t_wg0 = A.prof ? wall_clock64() : 0;
+  while(true) {
+    // the next trial from the launch's counter, longest first
+    __syncthreads();  // the previous particle's use of the shared arrays is over
+    if(tid == 0) s_item = atomicAdd(A.work_next, 1);
+    __syncthreads();
+    if(s_item >= A.nblk) {
+      if(A.prof && tid == 0) {
+        const unsigned long long tw = wall_clock64() - t_wg0;
+        atomicAdd(&A.prof[13], tw);
+        atomicMax(&A.prof[14], tw);
+        atomicAdd(&A.prof[15], 1ull);
+      }
+      break;
+    }
+    const int bid = A.work_order[s_item];
+    const int ti = A.trial_base + bid;
+    const int j = A.slot_pos ? A.slot_pos[bid] : bid;
+    const int p = A.tidx[ti];
+    const int t = A.P.type[p];
+    const size_t o0 = (size_t)j * (K + 1);
+    unsigned long long tp0 = 0, tp1 = 0, tpa = 0, tpb = 0;
+    if(A.prof && tid == 0) tp0 = wall_clock64();
+    if(tid == 0) {
+      int s = 0;
+      for(int o = 0; o <= K; o++) {
+        s_off[o] = s;
+        s += max(A.log_n[o0 + o], 0);
+      }
+      s_off[K + 1] = s;
+    }
+    if(tid < kFields) {
+      float mx = 0.f;
+      for(int o = 0; o <= K; o++) mx = fmaxf(mx, A.log_tot[(o0 + o) * kFields + tid]);
+      int e = 0;
+      (void)frexpf(mx, &e);  // mx < 2^e
+      const int kp = min(126, 30 - e);
+      s_kp[tid] = kp;
+      s_sc[tid] = ldexpf(1.0f, kp);
+    }
+    for(int q = tid; q < ntile; q += nt) tcnt[q] = 0;
+    for(int q = tid; q < nmask; q += nt) tmask[q] = 0;
+    __syncthreads();
+    const int R = s_off[K + 1];
+    // 1. the tile lists: counts, offsets, entries.  A thread takes T16_LU records at a time,
+    // their block-table and quad loads issued together.
+    auto records = [&](auto visit_record) {
+      for(int q0 = tid; q0 < R; q0 += nt * T16_LU) {
+        unsigned int rec[T16_LU];
+        int ob[T16_LU], quad[T16_LU];
 #pragma unroll
-  for(int u = 0; u < (KR + 3) / 4; u++) acc2[u] = 0.0;
-  float2 pcf[4] = {}, p1f = make_float2(0.f, 0.f), up = make_float2(0.f, 0.f);
-  float2 p2f = p1f, p3f = p1f, p4f = p1f;  // the 4x4, 8x8 and tile nodes' pairs
-  // (only the levels with cut-A nodes in the tile: the others' terms are not formed, and their
-  // loads take the field's first pair: with every load made, the compiler can count those in
-  // flight and a wait is for the needed ones only)
-  auto load_pairs = [&](tile_desc d) {
-    const int m = d.x;
-    const int gz = t16_z(m) * T16 + 2 * jy, gr = t16_r(m) * T16 + 2 * jx;
-    const unsigned int cmn = (unsigned int)d.w;
-    auto at = [&](unsigned int bit, int i) { return bwf[cmn & bit ? i : 0]; };
-    pcf[0] = at(1u, GALIC_STACKOFFSET(L, gz, gr));
-    pcf[1] = at(1u, GALIC_STACKOFFSET(L, gz, gr + 1));
-    pcf[2] = at(1u, GALIC_STACKOFFSET(L, gz + 1, gr));
-    pcf[3] = at(1u, GALIC_STACKOFFSET(L, gz + 1, gr + 1));
-    p1f = at(2u, GALIC_STACKOFFSET(L - 1, gz >> 1, gr >> 1));
-    p2f = at(4u, GALIC_STACKOFFSET(L - 2, gz >> 2, gr >> 2));
-    p3f = at(8u, GALIC_STACKOFFSET(L - 3, gz >> 3, gr >> 3));
-    p4f = at(16u, GALIC_STACKOFFSET(L - 4, t16_z(m), t16_r(m)));
-  };
-  // closes trial k's open ancestors of the tile prev (all of them, or those m does not
-  // share) from level lt - 1 upwards; up holds their pairs (lane l: level l)
-  auto close_levels = [&](int prev, int m, bool all) {
-    bool open = true;
+        for(int u = 0; u < T16_LU; u++) {
+          const int q = q0 + u * nt;
+          ob[u] = -1;
+          rec[u] = 0;
+          if(q < R) rec[u] = t16_record(A, s_off, K, o0, q, ob[u]);
+        }
 #pragma unroll
-    for(int l = NSTK - 1; l >= 0; l--) {
-      if(l < lt && open) {
-        const int sh = 2 * (lt - l);
-        if(!all && (prev >> sh) == (m >> sh)) {
-          open = false;
-        } else {
-          const double b = ldexp((double)__shfl(up.x, l), kp), w = (double)__shfl(up.y, l);
-          const int sl = lane < KR ? stk[l * KR + lane] : 0;
-          accs = t16_term(b, w, (double)sl, accs);
-          if(lane < KR) {
-            if(l > 0) stk[(l - 1) * KR + lane] += sl;
-            stk[l * KR + lane] = 0;
+        for(int u = 0; u < T16_LU; u++) quad[u] = ob[u] >= 0 ? A.log_q[rec[u]] : 0;
+#pragma unroll
+        for(int u = 0; u < T16_LU; u++)
+          if(ob[u] >= 0) visit_record(rec[u], ob[u], quad[u]);
+      }
+    };
+    records([&](unsigned int rec, int o, int quad) {
+      t16_visit(quad, L, [&](int m) {
+        atomicAdd(&tcnt[m], 1);
+        if(!(t16_mask_get<KR>(tmask, m) & (1u << o))) t16_mask_or<KR>(tmask, m, 1u << o);
+      });
+    });
+    __syncthreads();
+    if(wave == 0) t16_scan(tcnt, toff, tact, &s_nact, ntile, lane);
+    __syncthreads();
+    if(toff[ntile] > A.tlist_cap) {
+      // cannot happen when the caller sizes tlist_cap from k_log_totals; reported, not evaluated
+      for(int q = tid; q < ntile; q += nt) tcnt[q] = 0;
+      if(tid == 0) {
+        atomicOr(A.tile_err, 1u);
+        A.accept[ti] = 0;
+        A.dF[ti] = 0;
+      }
+      continue;
+    }
+    for(int q = tid; q < ntile; q += nt) tcnt[q] = 0;
+    __syncthreads();
+    records([&](unsigned int rec, int o, int quad) {
+      t16_visit(quad, L, [&](int m) { list[toff[m] + atomicAdd(&tcnt[m], 1)] = make_uint2(rec, (unsigned int)o); });
+    });
+    __syncthreads();
+    // the counts shared the grids' words: zero again for the tiles
+    for(int q = tid; q < ntile; q += nt) tcnt[q] = 0;
+    const int nact = s_nact;
+    if(A.prof && tid == 0) {
+      tp1 = wall_clock64();
+      atomicAdd(&A.prof[0], tp1 - tp0);
+      atomicAdd(&A.prof[5], (unsigned long long)nact);
+      atomicAdd(&A.prof[6], (unsigned long long)toff[ntile]);
+      atomicAdd(&A.prof[7], 1ull);
+    }
+
+    // 2. the tiles in Morton order
+    const int f = wave;
+    // (the pairs in FP32: the residual's rounding moves a term |b + D| - |b| only where b + D
+    // changes sign, by at most 2^-23 of |D|)
+    const float2 *bwf = A.merit_bwf + ((size_t)t * kFields + f) * Nstack;
+    const int kp = s_kp[f];
+    double acc[KR];
+#pragma unroll
+    for(int k = 0; k < KR; k++) acc[k] = 0.0;
+    double accs = 0.0;  // lane k: trial k's terms of the tile nodes and above
+    // lane 4q + j: the 4x4-node terms of trials j, j + 4, ...; lane 16r + k: trial k's 8x8 terms
+    double acc2[(KR + 3) / 4], acc3 = 0.0;
+#pragma unroll
+    for(int u = 0; u < (KR + 3) / 4; u++) acc2[u] = 0.0;
+    int *stk = &s_stk[f][0][0];  // [l][k], read and written by lane k of wave f only
+    if(lane < KR)
+      for(int l = 0; l < NSTK; l++) stk[l * KR + lane] = 0;
+    float2 pcf[4] = {}, p1f = make_float2(0.f, 0.f), up = make_float2(0.f, 0.f);
+    float2 p2f = p1f, p3f = p1f, p4f = p1f;  // the 4x4, 8x8 and tile nodes' pairs
+    // (only the levels with cut-A nodes in the tile: the others' terms are not formed)
+    auto load_pairs = [&](int m) {
+      const int gz = t16_z(m) * T16 + 2 * jy, gr = t16_r(m) * T16 + 2 * jx;
+      const unsigned int cmn = A.tcut[(size_t)t * ntile + m];
+      if(cmn & 1u) {
+        pcf[0] = bwf[GALIC_STACKOFFSET(L, gz, gr)];
+        pcf[1] = bwf[GALIC_STACKOFFSET(L, gz, gr + 1)];
+        pcf[2] = bwf[GALIC_STACKOFFSET(L, gz + 1, gr)];
+        pcf[3] = bwf[GALIC_STACKOFFSET(L, gz + 1, gr + 1)];
+      }
+      if(cmn & 2u) p1f = bwf[GALIC_STACKOFFSET(L - 1, gz >> 1, gr >> 1)];
+      if(cmn & 4u) p2f = bwf[GALIC_STACKOFFSET(L - 2, gz >> 2, gr >> 2)];
+      if(cmn & 8u) p3f = bwf[GALIC_STACKOFFSET(L - 3, gz >> 3, gr >> 3)];
+      if(cmn & 16u) p4f = bwf[GALIC_STACKOFFSET(L - 4, t16_z(m), t16_r(m))];
+    };
+    // closes trial k's open ancestors of the tile prev (all of them, or those m does not
+    // share) from level lt - 1 upwards; up holds their pairs (lane l: level l)
+    auto close_levels = [&](int prev, int m, bool all) {
+      bool open = true;
+#pragma unroll
+      for(int l = NSTK - 1; l >= 0; l--) {
+        if(l < lt && open) {
+          const int sh = 2 * (lt - l);
+          if(!all && (prev >> sh) == (m >> sh)) {
+            open = false;
+          } else {
+            const double b = ldexp((double)__shfl(up.x, l), kp), w = (double)__shfl(up.y, l);
+            const int sl = lane < KR ? stk[l * KR + lane] : 0;
+            accs = t16_term(b, w, (double)sl, accs);
+            if(lane < KR) {
+              if(l > 0) stk[(l - 1) * KR + lane] += sl;
+              stk[l * KR + lane] = 0;
+            }
           }
         }
       }
-    }
-  };
-  // A lane's first T16_U entries of a tile's list are fetched two tiles ahead, their values one
-  // tile ahead, so a tile's adds start with both in registers; the rest of a long list is taken
-  // T16_UR at a time.  (Every load is made, without an entry the list's or the field's first: see
-  // load_pairs.)
-  auto fetch_entries = [&](int e0, int e1, auto &en) {
-#pragma unroll
-    for(int u = 0; u < (int)(sizeof(en) / sizeof(en[0])); u++) {
-      const int e = e0 + u * 64 + lane;
-      en[u] = list[e < e1 ? e : 0];
-      if(e >= e1) en[u] = make_uint2(0u, 0u);
-    }
-  };
-  auto fetch_values = [&](const auto &en, auto &x, auto &y) {
-#pragma unroll
-    for(int u = 0; u < (int)(sizeof(en) / sizeof(en[0])); u++) {
-      y[u] = en[u].y;
-      x[u] = A.log_v[(size_t)en[u].x * kFields + f];
-    }
-  };
-  // the cells of the lane's entries into their logs' grids (cells outside the tile and lanes
-  // without an entry add 0)
-  auto add_values = [&](const auto &x, const auto &y, int left) {
-#pragma unroll
-    for(int u = 0; u < (int)(sizeof(y) / sizeof(y[0])); u++)
-      if(u * 64 < left) {
-        const unsigned int w0 = y[u] & 0xffu, w3 = (y[u] >> 8) & 0xffu;
-        int *g = grids + (y[u] >> 20) * 256;
-        const unsigned int w[4] = {w0, (w3 & 0x55u) | (w0 & 0xAAu), (w0 & 0x55u) | (w3 & 0xAAu), w3};
-        const float v[4] = {x[u].x, x[u].y, x[u].z, x[u].w};
-#pragma unroll
-        for(int c = 0; c < 4; c++)
-          atomicAdd(&g[w[c]], __float2int_rn(v[c] * sc) & -(int)((y[u] >> (16 + c)) & 1u));
+    };
+    // Phase A's list entries are fetched ahead: during tile ai's pyramid each thread loads its
+    // first entry of tile ai+2, so a tile's adds start with the entry in registers.
+    auto fetch_entry = [&](int ai2) {
+      uint2 en = make_uint2(0u, 0xffffffffu);
+      if(ai2 < nact) {
+        const int m2 = tact[ai2], e = toff[m2] + tid;
+        if(e < toff[m2 + 1]) en = list[e];
       }
-  };
-  if(nact > 0) {
-    tile_desc d0 = tile(1), d1 = tile(2), d2 = tile(3), d3 = tile(4);
+      return en;
+    };
+    // the cells of one entry inside tile (tz, tr) into its log's grids
+    auto add_values = [&](int o, int quad, const float4 (&x)[kFields], int tz, int tr) {
+      const int lz = (quad >> L) - tz * T16, lr = (quad & (nb - 1)) - tr * T16;
+#pragma unroll
+      for(int c = 0; c < 4; c++) {
+        const int cz = lz + (c >> 1), cr = lr + (c & 1);
+        if((unsigned)cz < (unsigned)T16 && (unsigned)cr < (unsigned)T16) {
+          const int w = t16_cell(cz, cr);
+#pragma unroll
+          for(int f2 = 0; f2 < kFields; f2++) {
+            const float v = c == 0 ? x[f2].x : c == 1 ? x[f2].y : c == 2 ? x[f2].z : x[f2].w;
+            if(v != 0.f) atomicAdd(&grids[(o * kFields + f2) * 256 + w], __float2int_rn(v * s_sc[f2]));
+          }
+        }
+      }
+    };
+    auto add_entry = [&](uint2 en, int tz, int tr) {
+      const unsigned int rec = en.x;
+      const int blk = (int)(rec / LOG_B), jj = (int)(rec % LOG_B);
+      float4 x[kFields];
+#pragma unroll
+      for(int f2 = 0; f2 < kFields; f2++) x[f2] = A.log_v[((size_t)blk * LOG_B + jj) * kFields + f2];
+      add_values((int)en.y, A.log_q[rec], x, tz, tr);
+    };
+    uint2 pe_cur = fetch_entry(0);
+    uint2 pe = fetch_entry(1);
+    if(nact > 0) load_pairs(tact[0]);
     int prev = -1;
-    uint2 pe[T16_U];
-    float4 x[T16_U];
-    unsigned int y[T16_U];
-    fetch_entries(d0.z, d1.z, pe);
-    fetch_values(pe, x, y);
-    fetch_entries(d1.z, d2.z, pe);
-    load_pairs(d0);
-    for(int i = 1; i <= nact; i++) {
-      const int m = d0.x;
-      if(A.prof && lane == 0) tpa = wall_clock64();
-      // phase A: the tile's entries into the logs' grids
-      add_values(x, y, d1.z - d0.z);
-      for(int e = d0.z + 64 * T16_U; e < d1.z; e += 64 * T16_UR) {
-        uint2 er[T16_UR];
-        float4 xr[T16_UR];
-        unsigned int yr[T16_UR];
-        fetch_entries(e, d1.z, er);
-        fetch_values(er, xr, yr);
-        add_values(xr, yr, d1.z - e);
-      }
-      // the grids are this wave's: its LDS operations are done in their order
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if(A.prof && f == 0 && lane == 0) {
+    for(int ai = 0; ai < nact; ai++) {
+      const int m = tact[ai], tz = t16_z(m), tr = t16_r(m);
+      if(A.prof && tid == 0) tpa = wall_clock64();
+      // phase A: the tile's entries into the logs' grids (the first one's list entry fetched
+      // ahead)
+      if(pe_cur.y != 0xffffffffu) add_entry(pe_cur, tz, tr);
+      for(int e = toff[m] + tid + nt; e < toff[m + 1]; e += nt) add_entry(list[e], tz, tr);
+      __syncthreads();
+      if(A.prof && tid == 0) {
         tpb = wall_clock64();
         atomicAdd(&A.prof[9], tpb - tpa);
       }
-      // phase B: the terms (the next tiles' values and entries on their way)
-      fetch_values(pe, x, y);
-      fetch_entries(d2.z, d3.z, pe);
+      // phase B: wave f, field f (the next tiles' entries on their way)
+      pe_cur = pe;
+      pe = fetch_entry(ai + 2);
       if(prev >= 0) close_levels(prev, m, false);
+      if(lane < lt) {
+        const int a = m >> (2 * (lt - lane));
+        up = bwf[GALIC_STACKOFFSET(lane, t16_z(a), t16_r(a))];
+      }
       {
         // the levels that hold cut-A nodes in this tile: only their terms can be nonzero (the
         // weights vanish off the cut), and the node sums are formed only if a level above the
         // cells needs them
-        const unsigned int tm = (unsigned int)d0.y, cm = (unsigned int)d0.w;
+        const unsigned int cm = A.tcut[(size_t)t * ntile + m];
         const bool cells = cm & 1u, node1 = cm & 2u, sums = cm & 0x3eu;
-        // the 4x4, 8x8 and tile nodes' pairs, used after the trials
+        // the 4x4, 8x8 and tile nodes' pairs of the levels on the cut (loaded a tile ahead with
+        // the cells' and 2x2 nodes'), used after the trials
         const float2 p2 = p2f, p3 = p3f, p4 = p4f;
         // residuals in the particle's units
         double2 pc[4];
-  #pragma unroll
+#pragma unroll
         for(int c = 0; c < 4; c++) pc[c] = make_double2(ldexp((double)pcf[c].x, kp), (double)pcf[c].y);
         const double2 p1 = make_double2(ldexp((double)p1f.x, kp), (double)p1f.y);
-        // the next tile's pairs and this tile's ancestors' (for when they close) on their way
-        {
-          const int l = min(lane, max(lt - 1, 0)), a = m >> (2 * (lt - l));
-          up = bwf[GALIC_STACKOFFSET(l, t16_z(a), t16_r(a))];
-          load_pairs(d1);
-        }
+        const unsigned int tm = t16_mask_get<KR>(tmask, m);
         // The coarser nodes' sums of trial k are handed to one lane each and their terms formed
         // after the loop: the 4x4 node's (in all four lanes of its quad after the quad sum) to
         // lane 4q + k % 4, register k / 4; the 8x8 node's (in all 16 lanes of its row) to lane
         // 16r + k; the tile's to lane k.
         int s2x[(KR + 3) / 4], s3x = 0, tsk = 0;
-  #pragma unroll
+#pragma unroll
         for(int u = 0; u < (KR + 3) / 4; u++) s2x[u] = 0;
-        int4 *og = (int4 *)grids + lane;  // O's word; trial k's: og + (k + 1) * 64
+        int4 *og = (int4 *)(grids + f * 256) + lane;  // O's word; trial k's: og + (k + 1) * kFields * 64
         const int4 o4 = *og;
         *og = make_int4(0, 0, 0, 0);
-        int4 *g0 = og + 64;
+        int4 *g0 = og + kFields * 64;
         int4 gn = *g0;
-  #pragma unroll
+#pragma unroll
         for(int k = 0; k < KR; k++) {
           if(k < K) {
             const int4 g4 = gn;
-            if(k + 1 < K) gn = g0[(k + 1) * 64];
+            if(k + 1 < K) gn = g0[(k + 1) * kFields * 64];
             // (a compiler barrier: trial k+1's word is read here, one trial ahead, not all
             // trials' words at once, which would hold 4 registers per trial)
             asm volatile("" ::: "memory");
             if(tm & (1u | (2u << k))) {
-              g0[k * 64] = make_int4(0, 0, 0, 0);
+              g0[k * kFields * 64] = make_int4(0, 0, 0, 0);
               const int4 d = make_int4(g4.x - o4.x, g4.y - o4.y, g4.z - o4.z, g4.w - o4.w);
               double a = acc[k];
               if(cells) {
@@ -2679,7 +2617,7 @@ __global__ void __launch_bounds__(64, 4) k_t16_merit(DevModel M, EvalArgs32 A) {
         }
         // the coarser nodes' terms of the lane's trials (0 for trials beyond K or not evaluated)
         if(cm & 4u)
-  #pragma unroll
+#pragma unroll
           for(int u = 0; u < (KR + 3) / 4; u++)
             acc2[u] = t16_term(ldexp((double)p2.x, kp), (double)p2.y, (double)s2x[u], acc2[u]);
         if(cm & 8u) acc3 = t16_term(ldexp((double)p3.x, kp), (double)p3.y, (double)s3x, acc3);
@@ -2687,50 +2625,68 @@ __global__ void __launch_bounds__(64, 4) k_t16_merit(DevModel M, EvalArgs32 A) {
         if((cm & 32u) && lt > 0 && lane < KR) stk[(lt - 1) * KR + lane] += tsk;
       }
       prev = m;
-      d0 = d1;
-      d1 = d2;
-      d2 = d3;
-      d3 = tile(i + 4);
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if(A.prof && f == 0 && lane == 0) atomicAdd(&A.prof[10], wall_clock64() - tpb);
+      if(ai + 1 < nact) load_pairs(tact[ai + 1]);
+      __syncthreads();
+      if(A.prof && tid == 0) atomicAdd(&A.prof[10], wall_clock64() - tpb);
     }
-    close_levels(prev, prev, true);
-  }
-  // the trials' totals (their sum over the fields and the choice are k_apply_best's)
-  const double MT = A.MType[t];
-  const double coef = f == 0 ? 1.0 / MT : (f == 1 ? A.fac[t][0] : f == 2 ? A.fac[t][1] : f == 3 ? A.fac[t][2]
-                                                                                              : A.fac[t][3]) /
-                                              MT / 4;
-  const double unit = ldexp(coef, -kp);
+    if(prev >= 0) close_levels(prev, prev, true);
+    // per-trial totals of field f
+    {
+      const double MT = A.MType[t];
+      const double coef = f == 0 ? 1.0 / MT : (f == 1 ? A.fac[t][0] : f == 2 ? A.fac[t][1] : f == 3 ? A.fac[t][2]
+                                                                                                  : A.fac[t][3]) /
+                                                  MT / 4;
+      const double unit = ldexp(coef, -kp);
 #pragma unroll
-  for(int k = 0; k < KR; k++)
-    if(k < K) {
-      double v = acc[k];
-      if((lane & 3) == (k & 3)) v += acc2[k >> 2];
-      if((lane & 15) == k) v += acc3;
-      if(lane == k) v += accs;
-      v = wave_sum(v);
-      if(lane == 0) A.tpart[((size_t)bid * kFields + f) * K + k] = v * unit;
+      for(int k = 0; k < KR; k++)
+        if(k < K) {
+          double v = acc[k];
+          if((lane & 3) == (k & 3)) v += acc2[k >> 2];
+          if((lane & 15) == k) v += acc3;
+          if(lane == k) v += accs;
+          v = wave_sum(v);
+          if(lane == 0) s_part[f][k] = v * unit;
+        }
     }
-  if(A.prof && lane == 0) {
-    const unsigned long long te = wall_clock64() - tp0;
-    atomicAdd(&A.prof[1], te);
-    atomicMax(&A.prof[4], te);
-    atomicAdd(&A.prof[11], te * te / 100);
-    atomicAdd(&A.prof[13], te);
-    atomicMax(&A.prof[14], te);
-    atomicAdd(&A.prof[15], 1ull);
+    __syncthreads();
+    // 3. the choice (the taken trial's deltas are the region commit's, k_commit_*)
+    for(int k = tid; k < K; k += nt) {
+      const size_t q = (size_t)ti * K + k;
+      const double *fit = A.fit + (size_t)t * 16;
+      double orbit_terms = 0;
+#pragma unroll
+      for(int f2 = 0; f2 < kFields; f2++) orbit_terms += s_part[f2][k];
+      s_dF[k] = orbit_terms + fit[5] / fit[6] * A.vinst[q];
+      A.dFk[q] = s_dF[k];
+    }
+    __syncthreads();
+    if(tid == 0) {
+      int bk = -1;
+      double bv = 0;
+      for(int k = 0; k < K; k++)
+        if(s_dF[k] < bv) {
+          bv = s_dF[k];
+          bk = k;
+        }
+      s_best = bk;
+      A.accept[ti] = bk + 1;
+      A.dF[ti] = (bk >= 0) ? bv : (K > 0 ? s_dF[0] : 0.0);
+      if(A.prof) {
+        const unsigned long long te = wall_clock64();
+        atomicAdd(&A.prof[1], te - tp1);
+        if(bk >= 0) atomicAdd(&A.prof[8], 1ull);
+        atomicMax(&A.prof[4], te - tp0);
+        atomicAdd(&A.prof[11], (te - tp0) * (te - tp0) / 100);
+        atomicMax(&A.prof[12], (unsigned long long)toff[ntile]);
+      }
+    }
   }
 }
 
-template __global__ void k_t16_merit<0, 4>(DevModel M, EvalArgs32 A);
-template __global__ void k_t16_merit<0, 8>(DevModel M, EvalArgs32 A);
-template __global__ void k_t16_merit<0, 16>(DevModel M, EvalArgs32 A);
-template __global__ void k_t16_merit<9, 4>(DevModel M, EvalArgs32 A);
-template __global__ void k_t16_merit<9, 8>(DevModel M, EvalArgs32 A);
-template __global__ void k_t16_merit<9, 16>(DevModel M, EvalArgs32 A);
+template __global__ void k_eval_t16<0, 8>(DevModel M, EvalArgs32 A);
+template __global__ void k_eval_t16<9, 8>(DevModel M, EvalArgs32 A);
+template __global__ void k_eval_t16<0, 16>(DevModel M, EvalArgs32 A);
+template __global__ void k_eval_t16<9, 16>(DevModel M, EvalArgs32 A);
 
 // ---------------------------------------------------- fixed point commit --
 

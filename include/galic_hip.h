@@ -249,7 +249,7 @@ int galic_fp32_set_merit_launch(galic_ctx *ctx, int wg_per_cu);
  * results are the same bits whatever the schedule. */
 int galic_fp32_set_schedule(galic_ctx *ctx, int max_group_trials, int overlap, int graph);
 
-/* Timing aid of the sparse and the 16 x 16 tile merit: on != 0 starts (or restarts) summing, per phase of
+/* Timing aid of the sparse tile merit: on != 0 starts (or restarts) summing, per phase of
  * each particle, the wall-clock ticks (100 MHz) of the kernel's thread 0; out16 (optional)
  * first receives the sums so far: [0] tile lists, [1] fields and tiles, [2] choice, [3]
  * deltas of the taken trial, [5] tiles visited, [6] list entries, [7] particles, [8] taken. */

@@ -1,5 +1,4 @@
-"""The 16 x 16-tile merit in two kernels, lists and one wave per field: trial counts on both sides of the
-kernel variants' limits, particle counts around the eight that its launch pads to."""
+"""The 16 x 16-tile merit: trial counts on both sides of the kernel variants' limits, from one particle to many."""
 import numpy as np
 import pytest
 
