@@ -838,6 +838,15 @@ int fp32_initial_logs(galic::Ctx &c, int n) {
     const Share sh = todo.back();
     todo.pop_back();
     const int m = (n - sh.first + sh.stride - 1) / sh.stride;
+    // A share planned on an estimate that a launch has since corrected is divided before it is
+    // launched, not after it ran out of the arena too (2e7 orbits, the first estimate too low: every
+    // one of 36 shares failed once, 4.9 s of 11.5 s of orbit launches).
+    const double fit = std::max(1.0, log_orbits_fit(c, n));
+    if(m > fit) {
+      const int f = (int)std::min((double)m, std::ceil(m / fit));
+      for(int k = f - 1; k >= 0; k--) todo.push_back({sh.first + k * sh.stride, f * sh.stride});
+      continue;
+    }
     CHK(alloc_orbit_scratch(c, m));
     hipLaunchKernelGGL(galic::k_prepare_list, dim3(nblocks(m, 256)), dim3(256), 0, c.stream, m,
                        (const int *)c.t_ord2, sh.first, sh.stride, P, orbit_in(c));
