@@ -152,10 +152,10 @@ int alloc_slots(galic::Ctx &c, int norbits, size_t bytes_per_orbit) {
   if(need <= c.slot_bytes) return GALIC_OK;
   if(c.slots) (void)hipFree(c.slots);
   c.slots = nullptr;
-  c.slot_bytes = 0;
+  c.slot_bytes = c.slots_zero = 0;
   HIPCHK(hipMalloc(&c.slots, need));
   HIPCHK(hipMemset(c.slots, 0, need));
-  c.slot_bytes = need;
+  c.slot_bytes = c.slots_zero = need;
   return GALIC_OK;
 }
 
@@ -517,7 +517,7 @@ int ensure_arena(galic::Ctx &c, size_t want, size_t need) {
   if(c.slot_bytes >= need && c.slot_bytes >= want / 100 * 89) return GALIC_OK;
   if(c.slots) (void)hipFree(c.slots);
   c.slots = nullptr;
-  c.slot_bytes = 0;
+  c.slot_bytes = c.slots_zero = 0;
   const size_t bytes = std::max(want, need);
   HIPCHK(hipMalloc(&c.slots, bytes));
   c.slot_bytes = bytes;
@@ -578,6 +578,7 @@ int orbit32_log_begin(galic::Ctx &c, galic::OrbitArgs32 &A) {
   A.log_v = c.log_v = (float4 *)((int *)c.slots + cap * galic::LOG_B);
   A.log_next = c.log_next;
   A.log_cap = (unsigned int)std::min<size_t>(cap, 0xf0000000u);  // claims past the cap stay below 2^32
+  c.slots_zero = 0;
   HIPCHK(hipMemsetAsync(c.log_next, 0, sizeof(unsigned int), c.stream));
   HIPCHK(hipMemsetAsync(c.counter, 0, sizeof(unsigned int), c.stream));
   HIPCHK(hipMemsetAsync(c.orbit_stats, 0, 6 * sizeof(unsigned long long), c.stream));
@@ -1592,6 +1593,13 @@ int galic_rep(galic_ctx *ctx, int ntrial, const int *idx, const double *vtry, in
   CHK(alloc_trial_scratch(c, std::max(ntrial, 1)));
   CHK(alloc_orbit_scratch(c, 2 * chunk));
   CHK(alloc_slots(c, 2 * chunk, slot_bytes_per_orbit));
+  // the slots are zero, as every rep leaves them, unless response logs or a call that failed used them since
+  size_t zero = 2 * (size_t)chunk * slot_bytes_per_orbit;
+  if(c.slots_zero < zero)
+    HIPCHK(hipMemsetAsync(c.slots, 0, zero, c.stream));
+  else
+    zero = c.slots_zero;
+  c.slots_zero = 0;
   if(ntrial > 0) {
     std::vector<double> tv(3 * (size_t)ntrial);
     for(int i = 0; i < ntrial; i++)
@@ -1675,6 +1683,7 @@ int galic_rep(galic_ctx *ctx, int ntrial, const int *idx, const double *vtry, in
     eval_ms += ms;
   }
   c.last_eval_ms = eval_ms;
+  c.slots_zero = zero;
   CHK(commit(ctx));
   if(ntrial > 0) {
     if(accept) HIPCHK(hipMemcpy(accept, c.t_accept, sizeof(int) * ntrial, hipMemcpyDeviceToHost));
@@ -1720,6 +1729,8 @@ int galic_orbit_responses(galic_ctx *ctx, int norbit, const double *pos, const d
   int chunk = (int)std::max<size_t>(1, std::min<size_t>((size_t)std::max(norbit, 1), (1ull << 30) / per));
   CHK(alloc_orbit_scratch(c, chunk));
   if(fields) CHK(alloc_slots(c, chunk, per));
+  const size_t zero = c.slots_zero;
+  if(fields) c.slots_zero = 0;
   std::vector<double> tmp(chunk);
   for(int base = 0; base < norbit; base += chunk) {
     int n = std::min(chunk, norbit - base);
@@ -1752,6 +1763,7 @@ int galic_orbit_responses(galic_ctx *ctx, int norbit, const double *pos, const d
     if(e0) HIPCHK(hipMemcpy(e0 + base, c.o_e0, sizeof(double) * n, hipMemcpyDeviceToHost));
     if(e1) HIPCHK(hipMemcpy(e1 + base, c.o_e1, sizeof(double) * n, hipMemcpyDeviceToHost));
   }
+  c.slots_zero = zero;
   return GALIC_OK;
 }
 
@@ -1768,6 +1780,8 @@ int galic_fp32_orbit_responses(galic_ctx *ctx, int norbit, const double *pos, co
   int chunk = (int)std::max<size_t>(1, std::min<size_t>((size_t)std::max(norbit, 1), (1ull << 30) / per));
   CHK(alloc_orbit_scratch(c, chunk));
   CHK(alloc_slots(c, chunk, per));
+  const size_t zero = c.slots_zero;
+  c.slots_zero = 0;
   float *fin = nullptr;
   HIPCHK(hipMalloc(&fin, sizeof(float) * 6 * chunk));
   std::vector<double> tmp(chunk);
@@ -1809,6 +1823,7 @@ int galic_fp32_orbit_responses(galic_ctx *ctx, int norbit, const double *pos, co
     if(rc == GALIC_OK && e1) rc = hip_ok(hipMemcpy(e1 + base, c.o_e1, sizeof(double) * n, hipMemcpyDeviceToHost));
   }
   (void)hipFree(fin);
+  if(rc == GALIC_OK) c.slots_zero = zero;
   return rc;
 }
 

@@ -72,7 +72,7 @@ struct Particles {
 // own fields and the other in Ctx::alt: one group's orbits integrate on one set's stream while
 // the previous group's reps are judged with the other's (swap_orbit_set in galic_api.hip).
 #define GALIC_ORBIT_SET_FIELDS(X) \
-  X(hipStream_t, stream) X(hipEvent_t, ev0) X(hipEvent_t, ev1) X(void *, slots) X(size_t, slot_bytes) \
+  X(hipStream_t, stream) X(hipEvent_t, ev0) X(hipEvent_t, ev1) X(void *, slots) X(size_t, slot_bytes) X(size_t, slots_zero) \
   X(int, max_slot_orbits) X(int, max_orbits) X(int *, o_pidx) X(int *, o_type) X(double *, o_x) X(double *, o_y) \
   X(double *, o_z) X(double *, o_vx) X(double *, o_vy) X(double *, o_vz) X(double *, o_mass) X(double *, o_tint) \
   X(double *, o_tall) X(double *, o_e0) X(double *, o_e1) X(int *, o_norbit) X(int *, o_status) \
@@ -136,6 +136,7 @@ struct Ctx {
   // orbit slots (FP64 path: double; FP32 path: float)
   void *slots = nullptr;
   size_t slot_bytes = 0;
+  size_t slots_zero = 0;         // bytes at the start of slots known to be zero (response logs leave them in any state)
   int max_slot_orbits = 0;
 
   // per-orbit scratch
