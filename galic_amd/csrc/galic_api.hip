@@ -1753,8 +1753,10 @@ int galic_orbit_responses(galic_ctx *ctx, int norbit, const double *pos, const d
       // integrate without binning into memory the caller wants: bin into a scratch Loc
       A.loc = c.locA_d;
     }
-    CHK(launch_orbit64(c, A));
+    const int rc = launch_orbit64(c, A);
+    // (the deltas of the Loc grids are zero between calls, also after one that failed)
     if(!fields) HIPCHK(hipMemsetAsync(c.locA_d, 0, sizeof(double) * GALIC_NTYPES * galic::kFields * c.Ngrid, c.stream));
+    CHK(rc);
     HIPCHK(hipStreamSynchronize(c.stream));
     if(fields) CHK(fields_out(c, n, (double *)c.slots, fields + (size_t)base * galic::kFields * c.Ngrid));
     if(t) HIPCHK(hipMemcpy(t + base, c.o_tall, sizeof(double) * n, hipMemcpyDeviceToHost));

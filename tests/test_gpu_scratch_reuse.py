@@ -51,3 +51,20 @@ def test_fp64_rep_after_orbit_fields(small, precision):
     g.calc_all_response_fields()
     same_rep(g, idx, v, ref)
     g.close()
+
+
+def test_fp64_rep_after_orbits_that_failed(small):
+    """Orbits integrated without fields bin into the rep's delta grids; one beyond the step cap ends the call early."""
+    w, idx, v, ref = small
+    cap = w.params.MaxStepsPerOrbit
+    w.params.MaxStepsPerOrbit = 20000
+    g = GalicGPU(w)
+    w.params.MaxStepsPerOrbit = cap
+    g.calc_all_response_fields()
+    with pytest.raises(RuntimeError, match="step cap"):
+        g.orbit_responses(w.pos[:50], w.vel[:50], w.mass[:50], 1000 * w.tint[:50], w.ptype[:50], fields=False)
+    same_rep(g, idx, v, ref)
+    # an accepted orbit takes the place of one of the same mass: sums of 3000 orbits, 1e-10
+    for t in w.types:
+        assert g.stack(t, 0)[0] == pytest.approx(w.params.MType[t], rel=1e-10)
+    g.close()
