@@ -34,6 +34,7 @@
 #include "../../include/galic_hip.h"
 #include "galic_ctx.h"
 #include "galic_kernels.h"
+#include "galic_pool.h"
 
 namespace galic {
 galic_ctx *bound_ctx();
@@ -643,36 +644,16 @@ inline int nb256(size_t n) { return (int)((n + 255) / 256); }
 // moments, threading), walk, and the interaction count.
 double g_last_build_ms = 0, g_last_walk_ms = 0, g_last_interactions = 0;
 
-// Device buffers of one call, carved from a few allocations (each twice what the call has taken so
-// far, 16 MiB at least): a call has some thirty of them, and an allocation and its release cost
-// about 0.1 ms.
-struct DevBufs {
-  std::vector<void *> ptrs;
-  char *at = nullptr;
-  size_t left = 0, taken = 0;
-  template <typename T>
-  hipError_t alloc(T **p, size_t n) {
-    const size_t bytes = (std::max<size_t>(n, 1) * sizeof(T) + 255) & ~(size_t)255;
-    if(bytes > left) {
-      size_t want = std::max(bytes, std::max<size_t>(2 * taken, (size_t)16 << 20));
-      void *q = nullptr;
-      hipError_t e = hipMalloc(&q, want);
-      if(e == hipErrorOutOfMemory && want > bytes) e = hipMalloc(&q, want = bytes);
-      if(e != hipSuccess) return e;
-      ptrs.push_back(q);
-      at = (char *)q;
-      left = want;
-      taken += want;
-    }
-    *p = (T *)at;
-    at += bytes;
-    left -= bytes;
-    return hipSuccess;
-  }
-  ~DevBufs() {
-    for(void *p : ptrs) (void)hipFree(p);
-  }
+// Device buffers of one call.
+struct HipMem {
+  typedef hipError_t Error;
+  static Error get(void **p, size_t n) { return hipMalloc(p, n); }
+  static void put(void *p) { (void)hipFree(p); }
+  static Error good() { return hipSuccess; }
+  static bool is_short(Error e) { return e == hipErrorOutOfMemory; }
+  static void forget() { (void)hipGetLastError(); }
 };
+typedef galic::DevPool<HipMem> DevBufs;
 
 // Moments bottom-up (monopole, and the quadrupole where T.quad is allocated), node side
 // lengths DomainLen / 2^depth (NODE.len, allvars.h:1095, held in float), then the
@@ -978,12 +959,12 @@ __global__ void __launch_bounds__(64) k_walk32g(WalkArgs A) {
 
 // Walk of ntarget targets (device SoA) through T; the results are scaled by G (gravity_tree
 // multiplies the walk's sums by G afterwards, gravtree.c:455-463).
-// blk_nb > 0: the targets are table nodes (section, z, R) of blk_nb x blk_nb grids, which the group
-// walk takes in 8 x 8 blocks.
-int tree_walk_dev(const galic_params *p, hipStream_t st, const Tree &T, int ntarget, Points X, double *dax, double *day, double *daz, double *dpot,
-                  int precision, double G, long long *ninteractions, float *walk_ms, int blk_nb = 0) {
+// blk_nb > 0: the targets are table nodes (section, z, R) of blk_nb x blk_nb grids, which a wave
+// takes in 8 x 8 blocks.
+int tree_walk_dev(const galic_params *p, hipStream_t st, DevBufs &B, const Tree &T, int ntarget, Points X, double *dax,
+                  double *day, double *daz, double *dpot, int precision, double G, long long *ninteractions,
+                  float *walk_ms, int blk_nb = 0) {
   int rc = GALIC_OK;
-  DevBufs B;
   unsigned long long *nint = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   WalkArgs W;
@@ -1074,16 +1055,15 @@ done:
 }
 
 // Build the tree of nsrc sources (device inputs) and walk ntarget targets.
-int tree_forces_dev(const galic_params *p, hipStream_t st, int nsrc, Points S, const double *dpm, int ntarget, Points X,
-                    double corner[3], double dlen, double *dax, double *day, double *daz, double *dpot, int precision,
-                    long long *ninteractions, float *walk_ms, int blk_nb = 0) {
-  DevBufs B;
+int tree_forces_dev(const galic_params *p, hipStream_t st, DevBufs &B, int nsrc, Points S, const double *dpm,
+                    int ntarget, Points X, double corner[3], double dlen, double *dax, double *day, double *daz,
+                    double *dpot, int precision, long long *ninteractions, float *walk_ms, int blk_nb = 0) {
   Tree T;
   float build_ms = 0, wms = 0;
   long long ni = 0;
   int rc = tree_build_dev(p, st, nsrc, S, dpm, corner, dlen, precision, B, T, nullptr, &build_ms);
   if(rc != GALIC_OK) return rc;
-  rc = tree_walk_dev(p, st, T, ntarget, X, dax, day, daz, dpot, precision, p->G, &ni, &wms, blk_nb);
+  rc = tree_walk_dev(p, st, B, T, ntarget, X, dax, day, daz, dpot, precision, p->G, &ni, &wms, blk_nb);
   if(rc != GALIC_OK) return rc;
   if(ninteractions) *ninteractions = ni;
   if(walk_ms) *walk_ms = wms;
@@ -1221,7 +1201,7 @@ void tree_dropin_fail(const char *what) {
 
 // Builds the bound tree over P[0..npart) without the Type-5 particles (forcetree.c:331);
 // the domain cube covers every one of them (domain_box.c:20-65).  Returns the node count.
-int tree_build_bound(int npart, int precision) {
+int tree_build_bound(int npart, int precision, bool exact = false) {
   galic_ctx *ctx = galic::bound_ctx();
   if(!ctx) return terr(GALIC_ERR_STATE, "no context bound (galic_bind): the tree takes its parameters from it");
   if(!g_P.pos || npart < 0 || npart > g_P.n)
@@ -1249,7 +1229,7 @@ int tree_build_bound(int npart, int precision) {
   double *pm;
   Points S, X;
   double lo[3] = {1e30, 1e30, 1e30}, hi[3] = {-1e30, -1e30, -1e30};
-  g_T.B = new DevBufs();
+  g_T.B = new DevBufs(exact);
   TCHK(hipSetDevice(g_T.device));
   TCHK(hipStreamCreate(&g_T.st));
   TCHK(g_T.B->alloc(&pm, nsrc));
@@ -1264,20 +1244,20 @@ int tree_build_bound(int npart, int precision) {
   if(rc == GALIC_OK) g_T.built = true;
 done:
   if(rc != GALIC_OK) tree_release();
+  if(rc == GALIC_ERR_NOMEM && !exact) return tree_build_bound(npart, precision, true);
   return rc == GALIC_OK ? g_T.T.level_lo.back() : rc;
 }
 
 // Walks n targets (positions pos, 3 each) of the bound tree; G scales the results.
-int tree_walk_bound(int n, const double *pos, double *acc, double *pot, double G, long long *nint) {
+int tree_walk_bound_with(DevBufs &B, int n, const double *pos, double *acc, double *pot, double G, long long *nint) {
   int rc = GALIC_OK;
-  DevBufs B;
   double *ax, *ay, *az, *pt;
   Points X;
   std::vector<double> h;
   TCHK(hipSetDevice(g_T.device));
   TCHK(B.alloc(&ax, n)); TCHK(B.alloc(&ay, n)); TCHK(B.alloc(&az, n)); TCHK(B.alloc(&pt, n));
   if((rc = upload_points(g_T.st, B, n, pos, &X)) != GALIC_OK) goto done;
-  if((rc = tree_walk_dev(&g_T.p, g_T.st, g_T.T, n, X, ax, ay, az, pt, 0, G, nint, nullptr)) != GALIC_OK)
+  if((rc = tree_walk_dev(&g_T.p, g_T.st, B, g_T.T, n, X, ax, ay, az, pt, 0, G, nint, nullptr)) != GALIC_OK)
     goto done;
   h.resize(std::max(n, 1));
   {
@@ -1289,6 +1269,198 @@ int tree_walk_bound(int n, const double *pos, double *acc, double *pot, double G
     if(n > 0) TCHK(hipMemcpy(pot, pt, sizeof(double) * n, hipMemcpyDeviceToHost));
   }
 done:
+  return rc;
+}
+int tree_walk_bound(int n, const double *pos, double *acc, double *pot, double G, long long *nint) {
+  return galic::with_pool<DevBufs>(GALIC_ERR_NOMEM,
+                                   [&](DevBufs &B) { return tree_walk_bound_with(B, n, pos, acc, pot, G, nint); });
+}
+
+// ---------------------------------------------------------- the tree calls --
+
+int retabulate_with(DevBufs &B, galic_ctx *ctx, int precision, long long *ninteractions) {
+  if(!ctx) return terr(GALIC_ERR_ARG, "null context");
+  if((precision & ~15) || ((precision & GALIC_TREE_GROUP) && !(precision & GALIC_TREE_FP32)))
+    return terr(GALIC_ERR_ARG, "mode: GALIC_TREE_FP32 | GALIC_TREE_QUADRUPOLE | GALIC_TREE_PLUMMER | "
+                               "GALIC_TREE_GROUP (with GALIC_TREE_FP32)");
+  galic::Ctx &c = galic::ctx_state(ctx);
+  if(!c.tsrc || c.tsrc_n < 1) return terr(GALIC_ERR_STATE, "no tree sources (galic_set_tree_sources)");
+  const galic_params *p = &c.p;
+  const int nb = p->FG_Nbin, nsrc = c.tsrc_n;
+  const size_t nn = (size_t)nb * nb, ns = GALIC_FG_SECTIONS * nn;
+  std::vector<double> rj, cs, sn;
+  fill_nodes(p, rj, cs, sn);
+  // the domain over sources and targets, as galic_tree_fill forms it
+  double lo[3], hi[3], corner[3], len = 0;
+  for(int j = 0; j < 3; j++) {
+    lo[j] = c.tsrc_lo[j];
+    hi[j] = c.tsrc_hi[j];
+  }
+  fill_extent(rj, cs, sn, lo, hi);
+  domain_cube(lo, hi, corner, &len);
+  int rc = GALIC_OK;
+  Tree T;
+  double *drj, *dcs, *dsn, *tx, *ty, *tz, *ax, *ay, *az, *pt;
+  long long ni = 0;
+  float bms = 0, wms = 0;
+  TCHK(hipSetDevice(c.device));
+  TCHK(B.alloc(&drj, nb)); TCHK(B.alloc(&dcs, GALIC_FG_SECTIONS)); TCHK(B.alloc(&dsn, GALIC_FG_SECTIONS));
+  TCHK(B.alloc(&tx, ns)); TCHK(B.alloc(&ty, ns)); TCHK(B.alloc(&tz, ns));
+  TCHK(B.alloc(&ax, ns)); TCHK(B.alloc(&ay, ns)); TCHK(B.alloc(&az, ns)); TCHK(B.alloc(&pt, ns));
+  TCHK(hipMemcpyAsync(drj, rj.data(), sizeof(double) * nb, hipMemcpyHostToDevice, c.stream));
+  TCHK(hipMemcpyAsync(dcs, cs.data(), sizeof(double) * GALIC_FG_SECTIONS, hipMemcpyHostToDevice, c.stream));
+  TCHK(hipMemcpyAsync(dsn, sn.data(), sizeof(double) * GALIC_FG_SECTIONS, hipMemcpyHostToDevice, c.stream));
+  hipLaunchKernelGGL(k_fill_targets, dim3(nb256(ns)), dim3(256), 0, c.stream, nb, (const double *)drj,
+                     (const double *)dcs, (const double *)dsn, tx, ty, tz);
+  TCHK(hipGetLastError());
+  if((rc = tree_build_dev(p, c.stream, nsrc, Points{c.tsrc, c.tsrc + nsrc, c.tsrc + 2 * (size_t)nsrc, 1},
+                          c.tsrc + 3 * (size_t)nsrc, corner, len, precision, B, T, nullptr, &bms)) != GALIC_OK)
+    goto done;
+  if((rc = tree_walk_dev(p, c.stream, B, T, (int)ns, Points{tx, ty, tz, 1}, ax, ay, az, pt, precision, p->G, &ni, &wms,
+                         nb)) != GALIC_OK)
+    goto done;
+  // installed as the context's tables: FG_DPotDR, FG_DPotDz, FG_Pot and the FP32 copy
+  hipLaunchKernelGGL(k_project, dim3(nb256(nn)), dim3(256), 0, c.stream, nb, (const double *)ax, (const double *)ay,
+                     (const double *)az, (const double *)pt, (const double *)dcs, (const double *)dsn, c.FG_DPotDR,
+                     c.FG_DPotDz, c.FG_Pot);
+  hipLaunchKernelGGL(k_acc_f, dim3(nb256(nn)), dim3(256), 0, c.stream, (int)nn, (const double *)c.FG_DPotDR,
+                     (const double *)c.FG_DPotDz, c.FG_Acc_f);
+  TCHK(hipGetLastError());
+  TCHK(hipStreamSynchronize(c.stream));
+  if(ninteractions) *ninteractions = ni;
+  g_last_build_ms = bms;
+  g_last_walk_ms = wms;
+  g_last_interactions = (double)ni;
+done:
+  return rc;
+}
+
+int tree_forces_with(DevBufs &B, const galic_params *p, int device, int nsrc, const double *spos, const double *smass,
+                      int ntarget, const double *tpos, double *acc, double *pot, int precision,
+                      long long *ninteractions) {
+  if(!p || nsrc < 0 || ntarget < 0 || (nsrc > 0 && (!spos || !smass)) || (ntarget > 0 && (!tpos || !acc || !pot)))
+    return terr(GALIC_ERR_ARG, "bad tree arguments");
+  if((precision & ~15) || ((precision & GALIC_TREE_GROUP) && !(precision & GALIC_TREE_FP32)))
+    return terr(GALIC_ERR_ARG, "mode: GALIC_TREE_FP32 | GALIC_TREE_QUADRUPOLE | GALIC_TREE_PLUMMER | "
+                               "GALIC_TREE_GROUP (with GALIC_TREE_FP32)");
+  int rc = GALIC_OK;
+  const hipStream_t st = hipStreamPerThread;
+  double *pm, *ax, *ay, *az, *pt;
+  Points S, X;
+  double lo[3] = {1e30, 1e30, 1e30}, hi[3] = {-1e30, -1e30, -1e30}, corner[3], len;
+  float ms = 0;
+  std::vector<double> h;
+  TCHK(hipSetDevice(device));
+  TCHK(B.alloc(&pm, nsrc));
+  TCHK(B.alloc(&ax, ntarget)); TCHK(B.alloc(&ay, ntarget)); TCHK(B.alloc(&az, ntarget)); TCHK(B.alloc(&pt, ntarget));
+  if((rc = upload_points(st, B, nsrc, spos, &S)) != GALIC_OK) goto done;
+  if((rc = upload_points(st, B, ntarget, tpos, &X)) != GALIC_OK) goto done;
+  if(nsrc > 0) TCHK(hipMemcpyAsync(pm, smass, sizeof(double) * nsrc, hipMemcpyHostToDevice, st));
+  if((rc = extend_domain(st, B, nsrc, S, lo, hi)) != GALIC_OK) goto done;
+  if((rc = extend_domain(st, B, ntarget, X, lo, hi)) != GALIC_OK) goto done;
+  domain_cube(lo, hi, corner, &len);
+  rc = tree_forces_dev(p, st, B, nsrc, S, pm, ntarget, X, corner, len, ax, ay, az, pt, precision, ninteractions, &ms);
+  if(rc != GALIC_OK) goto done;
+  h.resize(std::max(ntarget, 1));
+  {
+    double *src[3] = {ax, ay, az};
+    for(int k = 0; k < 3; k++) {
+      if(ntarget > 0) TCHK(hipMemcpy(h.data(), src[k], sizeof(double) * ntarget, hipMemcpyDeviceToHost));
+      for(int i = 0; i < ntarget; i++) acc[3 * (size_t)i + k] = h[i];
+    }
+    if(ntarget > 0) TCHK(hipMemcpy(pot, pt, sizeof(double) * ntarget, hipMemcpyDeviceToHost));
+  }
+done:
+  (void)hipStreamSynchronize(st);  // (the buffers go next)
+  return rc;
+}
+
+int tree_fill_with(DevBufs &B, const galic_params *p, int device, int nsrc, const double *spos, const double *smass,
+                    double *pot, double *dpotdr, double *dpotdz, int precision, long long *ninteractions) {
+  if(!p || nsrc < 0 || (nsrc > 0 && (!spos || !smass)) || !pot || !dpotdr || !dpotdz || p->FG_Nbin < 2)
+    return terr(GALIC_ERR_ARG, "bad table-fill arguments");
+  if((precision & ~15) || ((precision & GALIC_TREE_GROUP) && !(precision & GALIC_TREE_FP32)))
+    return terr(GALIC_ERR_ARG, "mode: GALIC_TREE_FP32 | GALIC_TREE_QUADRUPOLE | GALIC_TREE_PLUMMER | "
+                               "GALIC_TREE_GROUP (with GALIC_TREE_FP32)");
+  const int nb = p->FG_Nbin;
+  const size_t ns = (size_t)GALIC_FG_SECTIONS * nb * nb;
+  if(ns > 0x7fffffff) return terr(GALIC_ERR_ARG, "FG_Nbin too large");
+  // targets of grid.c:680-704: (R_j cos phi_s, R_j sin phi_s, z_k), formed on the device
+  std::vector<double> rj, cs, sn;
+  fill_nodes(p, rj, cs, sn);
+  int rc = GALIC_OK;
+  const hipStream_t st = hipStreamPerThread;
+  double *pm, *tx, *ty, *tz, *ax, *ay, *az, *pt, *drj, *dcs, *dsn, *r0, *r1, *r2;
+  Points S;
+  double lo[3] = {1e30, 1e30, 1e30}, hi[3] = {-1e30, -1e30, -1e30}, corner[3], len;
+  float ms = 0;
+  TCHK(hipSetDevice(device));
+  TCHK(B.alloc(&pm, nsrc));
+  TCHK(B.alloc(&tx, ns)); TCHK(B.alloc(&ty, ns)); TCHK(B.alloc(&tz, ns));
+  TCHK(B.alloc(&ax, ns)); TCHK(B.alloc(&ay, ns)); TCHK(B.alloc(&az, ns)); TCHK(B.alloc(&pt, ns));
+  TCHK(B.alloc(&drj, nb)); TCHK(B.alloc(&dcs, GALIC_FG_SECTIONS)); TCHK(B.alloc(&dsn, GALIC_FG_SECTIONS));
+  TCHK(B.alloc(&r0, (size_t)nb * nb)); TCHK(B.alloc(&r1, (size_t)nb * nb)); TCHK(B.alloc(&r2, (size_t)nb * nb));
+  if((rc = upload_points(st, B, nsrc, spos, &S)) != GALIC_OK) goto done;
+  if(nsrc > 0) TCHK(hipMemcpyAsync(pm, smass, sizeof(double) * nsrc, hipMemcpyHostToDevice, st));
+  TCHK(hipMemcpyAsync(drj, rj.data(), sizeof(double) * nb, hipMemcpyHostToDevice, st));
+  TCHK(hipMemcpyAsync(dcs, cs.data(), sizeof(double) * GALIC_FG_SECTIONS, hipMemcpyHostToDevice, st));
+  TCHK(hipMemcpyAsync(dsn, sn.data(), sizeof(double) * GALIC_FG_SECTIONS, hipMemcpyHostToDevice, st));
+  hipLaunchKernelGGL(k_fill_targets, dim3(nb256(ns)), dim3(256), 0, st, nb, (const double *)drj, (const double *)dcs,
+                     (const double *)dsn, tx, ty, tz);
+  TCHK(hipGetLastError());
+  if((rc = extend_domain(st, B, nsrc, S, lo, hi)) != GALIC_OK) goto done;
+  fill_extent(rj, cs, sn, lo, hi);
+  domain_cube(lo, hi, corner, &len);
+  rc = tree_forces_dev(p, st, B, nsrc, S, pm, (int)ns, Points{tx, ty, tz, 1}, corner, len, ax, ay, az, pt, precision,
+                       ninteractions, &ms, nb);
+  if(rc != GALIC_OK) goto done;
+  hipLaunchKernelGGL(k_project, dim3(nb256((size_t)nb * nb)), dim3(256), 0, st, nb, (const double *)ax,
+                     (const double *)ay, (const double *)az, (const double *)pt, (const double *)dcs,
+                     (const double *)dsn, r1, r2, r0);
+  TCHK(hipGetLastError());
+  TCHK(hipMemcpyAsync(dpotdr, r1, sizeof(double) * nb * nb, hipMemcpyDeviceToHost, st));
+  TCHK(hipMemcpyAsync(dpotdz, r2, sizeof(double) * nb * nb, hipMemcpyDeviceToHost, st));
+  TCHK(hipMemcpyAsync(pot, r0, sizeof(double) * nb * nb, hipMemcpyDeviceToHost, st));
+  TCHK(hipStreamSynchronize(st));
+done:
+  (void)hipStreamSynchronize(st);  // (the buffers and the host arrays of the copies go next)
+  return rc;
+}
+
+int direct_forces_with(DevBufs &B, const galic_params *p, int device, int nsrc, const double *spos, const double *smass,
+                             int ntarget, const double *tpos, double *acc, double *pot, int mode) {
+  if(!p || nsrc < 0 || ntarget < 0 || (nsrc > 0 && (!spos || !smass)) || (ntarget > 0 && (!tpos || !acc || !pot)))
+    return terr(GALIC_ERR_ARG, "bad direct-summation arguments");
+  if(mode != 0 && mode != GALIC_TREE_PLUMMER) return terr(GALIC_ERR_ARG, "mode: 0 or GALIC_TREE_PLUMMER");
+  int rc = GALIC_OK;
+  hipStream_t st = nullptr;
+  double *px, *py, *pz, *pm, *tx, *ty, *tz, *ax, *ay, *az, *pt;
+  std::vector<double> h;
+  TCHK(hipSetDevice(device));
+  TCHK(hipStreamCreate(&st));
+  TCHK(B.alloc(&px, nsrc)); TCHK(B.alloc(&py, nsrc)); TCHK(B.alloc(&pz, nsrc)); TCHK(B.alloc(&pm, nsrc));
+  TCHK(B.alloc(&tx, ntarget)); TCHK(B.alloc(&ty, ntarget)); TCHK(B.alloc(&tz, ntarget));
+  TCHK(B.alloc(&ax, ntarget)); TCHK(B.alloc(&ay, ntarget)); TCHK(B.alloc(&az, ntarget)); TCHK(B.alloc(&pt, ntarget));
+  if((rc = upload_soa(st, nsrc, spos, px, py, pz)) != GALIC_OK) goto done;
+  if((rc = upload_soa(st, ntarget, tpos, tx, ty, tz)) != GALIC_OK) goto done;
+  if(nsrc > 0) TCHK(hipMemcpy(pm, smass, sizeof(double) * nsrc, hipMemcpyHostToDevice));
+  if(ntarget > 0) {
+    hipLaunchKernelGGL(galic::tree::k_direct64, dim3(nb256(ntarget)), dim3(256), 0, st, nsrc, (const double *)px,
+                       (const double *)py, (const double *)pz, (const double *)pm, ntarget, (const double *)tx,
+                       (const double *)ty, (const double *)tz, p->ForceSoftening, mode == GALIC_TREE_PLUMMER ? 1 : 0,
+                       p->ForceSoftening / 2.8, p->G, ax, ay, az, pt);
+    TCHK(hipGetLastError());
+    TCHK(hipStreamSynchronize(st));
+    h.resize(ntarget);
+    double *src[3] = {ax, ay, az};
+    for(int k = 0; k < 3; k++) {
+      TCHK(hipMemcpy(h.data(), src[k], sizeof(double) * ntarget, hipMemcpyDeviceToHost));
+      for(int i = 0; i < ntarget; i++) acc[3 * (size_t)i + k] = h[i];
+    }
+    TCHK(hipMemcpy(pot, pt, sizeof(double) * ntarget, hipMemcpyDeviceToHost));
+  }
+done:
+  if(st) (void)hipStreamDestroy(st);
   return rc;
 }
 
@@ -1399,155 +1571,24 @@ done:
 }
 
 int galic_retabulate(galic_ctx *ctx, int precision, long long *ninteractions) {
-  if(!ctx) return terr(GALIC_ERR_ARG, "null context");
-  if((precision & ~15) || ((precision & GALIC_TREE_GROUP) && !(precision & GALIC_TREE_FP32)))
-    return terr(GALIC_ERR_ARG, "mode: GALIC_TREE_FP32 | GALIC_TREE_QUADRUPOLE | GALIC_TREE_PLUMMER | "
-                               "GALIC_TREE_GROUP (with GALIC_TREE_FP32)");
-  galic::Ctx &c = galic::ctx_state(ctx);
-  if(!c.tsrc || c.tsrc_n < 1) return terr(GALIC_ERR_STATE, "no tree sources (galic_set_tree_sources)");
-  const galic_params *p = &c.p;
-  const int nb = p->FG_Nbin, nsrc = c.tsrc_n;
-  const size_t nn = (size_t)nb * nb, ns = GALIC_FG_SECTIONS * nn;
-  std::vector<double> rj, cs, sn;
-  fill_nodes(p, rj, cs, sn);
-  // the domain over sources and targets, as galic_tree_fill forms it
-  double lo[3], hi[3], corner[3], len = 0;
-  for(int j = 0; j < 3; j++) {
-    lo[j] = c.tsrc_lo[j];
-    hi[j] = c.tsrc_hi[j];
-  }
-  fill_extent(rj, cs, sn, lo, hi);
-  domain_cube(lo, hi, corner, &len);
-  int rc = GALIC_OK;
-  DevBufs B;
-  Tree T;
-  double *drj, *dcs, *dsn, *tx, *ty, *tz, *ax, *ay, *az, *pt;
-  long long ni = 0;
-  float bms = 0, wms = 0;
-  TCHK(hipSetDevice(c.device));
-  TCHK(B.alloc(&drj, nb)); TCHK(B.alloc(&dcs, GALIC_FG_SECTIONS)); TCHK(B.alloc(&dsn, GALIC_FG_SECTIONS));
-  TCHK(B.alloc(&tx, ns)); TCHK(B.alloc(&ty, ns)); TCHK(B.alloc(&tz, ns));
-  TCHK(B.alloc(&ax, ns)); TCHK(B.alloc(&ay, ns)); TCHK(B.alloc(&az, ns)); TCHK(B.alloc(&pt, ns));
-  TCHK(hipMemcpyAsync(drj, rj.data(), sizeof(double) * nb, hipMemcpyHostToDevice, c.stream));
-  TCHK(hipMemcpyAsync(dcs, cs.data(), sizeof(double) * GALIC_FG_SECTIONS, hipMemcpyHostToDevice, c.stream));
-  TCHK(hipMemcpyAsync(dsn, sn.data(), sizeof(double) * GALIC_FG_SECTIONS, hipMemcpyHostToDevice, c.stream));
-  hipLaunchKernelGGL(k_fill_targets, dim3(nb256(ns)), dim3(256), 0, c.stream, nb, (const double *)drj,
-                     (const double *)dcs, (const double *)dsn, tx, ty, tz);
-  TCHK(hipGetLastError());
-  if((rc = tree_build_dev(p, c.stream, nsrc, Points{c.tsrc, c.tsrc + nsrc, c.tsrc + 2 * (size_t)nsrc, 1},
-                          c.tsrc + 3 * (size_t)nsrc, corner, len, precision, B, T, nullptr, &bms)) != GALIC_OK)
-    goto done;
-  if((rc = tree_walk_dev(p, c.stream, T, (int)ns, Points{tx, ty, tz, 1}, ax, ay, az, pt, precision, p->G, &ni, &wms,
-                         nb)) != GALIC_OK)
-    goto done;
-  // installed as the context's tables: FG_DPotDR, FG_DPotDz, FG_Pot and the FP32 copy
-  hipLaunchKernelGGL(k_project, dim3(nb256(nn)), dim3(256), 0, c.stream, nb, (const double *)ax, (const double *)ay,
-                     (const double *)az, (const double *)pt, (const double *)dcs, (const double *)dsn, c.FG_DPotDR,
-                     c.FG_DPotDz, c.FG_Pot);
-  hipLaunchKernelGGL(k_acc_f, dim3(nb256(nn)), dim3(256), 0, c.stream, (int)nn, (const double *)c.FG_DPotDR,
-                     (const double *)c.FG_DPotDz, c.FG_Acc_f);
-  TCHK(hipGetLastError());
-  TCHK(hipStreamSynchronize(c.stream));
-  if(ninteractions) *ninteractions = ni;
-  g_last_build_ms = bms;
-  g_last_walk_ms = wms;
-  g_last_interactions = (double)ni;
-done:
-  return rc;
+  return galic::with_pool<DevBufs>(GALIC_ERR_NOMEM, [&](DevBufs &B) {
+    return retabulate_with(B, ctx, precision, ninteractions);
+  });
 }
 
 int galic_tree_forces(const galic_params *p, int device, int nsrc, const double *spos, const double *smass,
                       int ntarget, const double *tpos, double *acc, double *pot, int precision,
                       long long *ninteractions) {
-  if(!p || nsrc < 0 || ntarget < 0 || (nsrc > 0 && (!spos || !smass)) || (ntarget > 0 && (!tpos || !acc || !pot)))
-    return terr(GALIC_ERR_ARG, "bad tree arguments");
-  if((precision & ~15) || ((precision & GALIC_TREE_GROUP) && !(precision & GALIC_TREE_FP32)))
-    return terr(GALIC_ERR_ARG, "mode: GALIC_TREE_FP32 | GALIC_TREE_QUADRUPOLE | GALIC_TREE_PLUMMER | "
-                               "GALIC_TREE_GROUP (with GALIC_TREE_FP32)");
-  int rc = GALIC_OK;
-  const hipStream_t st = hipStreamPerThread;
-  DevBufs B;
-  double *pm, *ax, *ay, *az, *pt;
-  Points S, X;
-  double lo[3] = {1e30, 1e30, 1e30}, hi[3] = {-1e30, -1e30, -1e30}, corner[3], len;
-  float ms = 0;
-  std::vector<double> h;
-  TCHK(hipSetDevice(device));
-  TCHK(B.alloc(&pm, nsrc));
-  TCHK(B.alloc(&ax, ntarget)); TCHK(B.alloc(&ay, ntarget)); TCHK(B.alloc(&az, ntarget)); TCHK(B.alloc(&pt, ntarget));
-  if((rc = upload_points(st, B, nsrc, spos, &S)) != GALIC_OK) goto done;
-  if((rc = upload_points(st, B, ntarget, tpos, &X)) != GALIC_OK) goto done;
-  if(nsrc > 0) TCHK(hipMemcpyAsync(pm, smass, sizeof(double) * nsrc, hipMemcpyHostToDevice, st));
-  if((rc = extend_domain(st, B, nsrc, S, lo, hi)) != GALIC_OK) goto done;
-  if((rc = extend_domain(st, B, ntarget, X, lo, hi)) != GALIC_OK) goto done;
-  domain_cube(lo, hi, corner, &len);
-  rc = tree_forces_dev(p, st, nsrc, S, pm, ntarget, X, corner, len, ax, ay, az, pt, precision, ninteractions, &ms);
-  if(rc != GALIC_OK) goto done;
-  h.resize(std::max(ntarget, 1));
-  {
-    double *src[3] = {ax, ay, az};
-    for(int k = 0; k < 3; k++) {
-      if(ntarget > 0) TCHK(hipMemcpy(h.data(), src[k], sizeof(double) * ntarget, hipMemcpyDeviceToHost));
-      for(int i = 0; i < ntarget; i++) acc[3 * (size_t)i + k] = h[i];
-    }
-    if(ntarget > 0) TCHK(hipMemcpy(pot, pt, sizeof(double) * ntarget, hipMemcpyDeviceToHost));
-  }
-done:
-  (void)hipStreamSynchronize(st);  // (the buffers go next)
-  return rc;
+  return galic::with_pool<DevBufs>(GALIC_ERR_NOMEM, [&](DevBufs &B) {
+    return tree_forces_with(B, p, device, nsrc, spos, smass, ntarget, tpos, acc, pot, precision, ninteractions);
+  });
 }
 
 int galic_tree_fill(const galic_params *p, int device, int nsrc, const double *spos, const double *smass,
                     double *pot, double *dpotdr, double *dpotdz, int precision, long long *ninteractions) {
-  if(!p || nsrc < 0 || (nsrc > 0 && (!spos || !smass)) || !pot || !dpotdr || !dpotdz || p->FG_Nbin < 2)
-    return terr(GALIC_ERR_ARG, "bad table-fill arguments");
-  if((precision & ~15) || ((precision & GALIC_TREE_GROUP) && !(precision & GALIC_TREE_FP32)))
-    return terr(GALIC_ERR_ARG, "mode: GALIC_TREE_FP32 | GALIC_TREE_QUADRUPOLE | GALIC_TREE_PLUMMER | "
-                               "GALIC_TREE_GROUP (with GALIC_TREE_FP32)");
-  const int nb = p->FG_Nbin;
-  const size_t ns = (size_t)GALIC_FG_SECTIONS * nb * nb;
-  if(ns > 0x7fffffff) return terr(GALIC_ERR_ARG, "FG_Nbin too large");
-  // targets of grid.c:680-704: (R_j cos phi_s, R_j sin phi_s, z_k), formed on the device
-  std::vector<double> rj, cs, sn;
-  fill_nodes(p, rj, cs, sn);
-  int rc = GALIC_OK;
-  const hipStream_t st = hipStreamPerThread;
-  DevBufs B;
-  double *pm, *tx, *ty, *tz, *ax, *ay, *az, *pt, *drj, *dcs, *dsn, *r0, *r1, *r2;
-  Points S;
-  double lo[3] = {1e30, 1e30, 1e30}, hi[3] = {-1e30, -1e30, -1e30}, corner[3], len;
-  float ms = 0;
-  TCHK(hipSetDevice(device));
-  TCHK(B.alloc(&pm, nsrc));
-  TCHK(B.alloc(&tx, ns)); TCHK(B.alloc(&ty, ns)); TCHK(B.alloc(&tz, ns));
-  TCHK(B.alloc(&ax, ns)); TCHK(B.alloc(&ay, ns)); TCHK(B.alloc(&az, ns)); TCHK(B.alloc(&pt, ns));
-  TCHK(B.alloc(&drj, nb)); TCHK(B.alloc(&dcs, GALIC_FG_SECTIONS)); TCHK(B.alloc(&dsn, GALIC_FG_SECTIONS));
-  TCHK(B.alloc(&r0, (size_t)nb * nb)); TCHK(B.alloc(&r1, (size_t)nb * nb)); TCHK(B.alloc(&r2, (size_t)nb * nb));
-  if((rc = upload_points(st, B, nsrc, spos, &S)) != GALIC_OK) goto done;
-  if(nsrc > 0) TCHK(hipMemcpyAsync(pm, smass, sizeof(double) * nsrc, hipMemcpyHostToDevice, st));
-  TCHK(hipMemcpyAsync(drj, rj.data(), sizeof(double) * nb, hipMemcpyHostToDevice, st));
-  TCHK(hipMemcpyAsync(dcs, cs.data(), sizeof(double) * GALIC_FG_SECTIONS, hipMemcpyHostToDevice, st));
-  TCHK(hipMemcpyAsync(dsn, sn.data(), sizeof(double) * GALIC_FG_SECTIONS, hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_fill_targets, dim3(nb256(ns)), dim3(256), 0, st, nb, (const double *)drj, (const double *)dcs,
-                     (const double *)dsn, tx, ty, tz);
-  TCHK(hipGetLastError());
-  if((rc = extend_domain(st, B, nsrc, S, lo, hi)) != GALIC_OK) goto done;
-  fill_extent(rj, cs, sn, lo, hi);
-  domain_cube(lo, hi, corner, &len);
-  rc = tree_forces_dev(p, st, nsrc, S, pm, (int)ns, Points{tx, ty, tz, 1}, corner, len, ax, ay, az, pt, precision,
-                       ninteractions, &ms, nb);
-  if(rc != GALIC_OK) goto done;
-  hipLaunchKernelGGL(k_project, dim3(nb256((size_t)nb * nb)), dim3(256), 0, st, nb, (const double *)ax,
-                     (const double *)ay, (const double *)az, (const double *)pt, (const double *)dcs,
-                     (const double *)dsn, r1, r2, r0);
-  TCHK(hipGetLastError());
-  TCHK(hipMemcpyAsync(dpotdr, r1, sizeof(double) * nb * nb, hipMemcpyDeviceToHost, st));
-  TCHK(hipMemcpyAsync(dpotdz, r2, sizeof(double) * nb * nb, hipMemcpyDeviceToHost, st));
-  TCHK(hipMemcpyAsync(pot, r0, sizeof(double) * nb * nb, hipMemcpyDeviceToHost, st));
-  TCHK(hipStreamSynchronize(st));
-done:
-  (void)hipStreamSynchronize(st);  // (the buffers and the host arrays of the copies go next)
-  return rc;
+  return galic::with_pool<DevBufs>(GALIC_ERR_NOMEM, [&](DevBufs &B) {
+    return tree_fill_with(B, p, device, nsrc, spos, smass, pot, dpotdr, dpotdz, precision, ninteractions);
+  });
 }
 
 int galic_direct_forces(const galic_params *p, int device, int nsrc, const double *spos, const double *smass,
@@ -1557,40 +1598,9 @@ int galic_direct_forces(const galic_params *p, int device, int nsrc, const doubl
 
 int galic_direct_forces_mode(const galic_params *p, int device, int nsrc, const double *spos, const double *smass,
                              int ntarget, const double *tpos, double *acc, double *pot, int mode) {
-  if(!p || nsrc < 0 || ntarget < 0 || (nsrc > 0 && (!spos || !smass)) || (ntarget > 0 && (!tpos || !acc || !pot)))
-    return terr(GALIC_ERR_ARG, "bad direct-summation arguments");
-  if(mode != 0 && mode != GALIC_TREE_PLUMMER) return terr(GALIC_ERR_ARG, "mode: 0 or GALIC_TREE_PLUMMER");
-  int rc = GALIC_OK;
-  hipStream_t st = nullptr;
-  DevBufs B;
-  double *px, *py, *pz, *pm, *tx, *ty, *tz, *ax, *ay, *az, *pt;
-  std::vector<double> h;
-  TCHK(hipSetDevice(device));
-  TCHK(hipStreamCreate(&st));
-  TCHK(B.alloc(&px, nsrc)); TCHK(B.alloc(&py, nsrc)); TCHK(B.alloc(&pz, nsrc)); TCHK(B.alloc(&pm, nsrc));
-  TCHK(B.alloc(&tx, ntarget)); TCHK(B.alloc(&ty, ntarget)); TCHK(B.alloc(&tz, ntarget));
-  TCHK(B.alloc(&ax, ntarget)); TCHK(B.alloc(&ay, ntarget)); TCHK(B.alloc(&az, ntarget)); TCHK(B.alloc(&pt, ntarget));
-  if((rc = upload_soa(st, nsrc, spos, px, py, pz)) != GALIC_OK) goto done;
-  if((rc = upload_soa(st, ntarget, tpos, tx, ty, tz)) != GALIC_OK) goto done;
-  if(nsrc > 0) TCHK(hipMemcpy(pm, smass, sizeof(double) * nsrc, hipMemcpyHostToDevice));
-  if(ntarget > 0) {
-    hipLaunchKernelGGL(galic::tree::k_direct64, dim3(nb256(ntarget)), dim3(256), 0, st, nsrc, (const double *)px,
-                       (const double *)py, (const double *)pz, (const double *)pm, ntarget, (const double *)tx,
-                       (const double *)ty, (const double *)tz, p->ForceSoftening, mode == GALIC_TREE_PLUMMER ? 1 : 0,
-                       p->ForceSoftening / 2.8, p->G, ax, ay, az, pt);
-    TCHK(hipGetLastError());
-    TCHK(hipStreamSynchronize(st));
-    h.resize(ntarget);
-    double *src[3] = {ax, ay, az};
-    for(int k = 0; k < 3; k++) {
-      TCHK(hipMemcpy(h.data(), src[k], sizeof(double) * ntarget, hipMemcpyDeviceToHost));
-      for(int i = 0; i < ntarget; i++) acc[3 * (size_t)i + k] = h[i];
-    }
-    TCHK(hipMemcpy(pot, pt, sizeof(double) * ntarget, hipMemcpyDeviceToHost));
-  }
-done:
-  if(st) (void)hipStreamDestroy(st);
-  return rc;
+  return galic::with_pool<DevBufs>(GALIC_ERR_NOMEM, [&](DevBufs &B) {
+    return direct_forces_with(B, p, device, nsrc, spos, smass, ntarget, tpos, acc, pot, mode);
+  });
 }
 
 int galic_tree_last_timings(double *out3) {
