@@ -35,17 +35,22 @@ int set_err(int code, const char *fmt, ...) {
   return code;
 }
 
+// An error that is reported is also dropped from the runtime's record: HIP keeps it until it is
+// read, and the next call's check of a launch would report it again.
 #define HIPCHK(expr)                                                                                \
   do {                                                                                              \
     hipError_t e_ = (expr);                                                                         \
-    if(e_ != hipSuccess)                                                                            \
+    if(e_ != hipSuccess) {                                                                          \
+      (void)hipGetLastError();                                                                      \
       return set_err(e_ == hipErrorOutOfMemory ? GALIC_ERR_NOMEM : GALIC_ERR_HIP, "%s: %s (%s:%d)", \
                      #expr, hipGetErrorString(e_), __FILE__, __LINE__);                             \
+    }                                                                                               \
   } while(0)
 
 // HIP status as a library status (for paths that must release memory before returning)
 int hip_ok(hipError_t e) {
   if(e == hipSuccess) return GALIC_OK;
+  (void)hipGetLastError();
   return set_err(e == hipErrorOutOfMemory ? GALIC_ERR_NOMEM : GALIC_ERR_HIP, "%s", hipGetErrorString(e));
 }
 

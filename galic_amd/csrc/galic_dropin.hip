@@ -94,7 +94,10 @@ int galic_field_at(galic_ctx *ctx, int n, const double *pos, double *acc, double
     c.lookup_buf = nullptr;
     c.lookup_len = 0;
     const size_t len = std::max<size_t>((size_t)n, 1024);
-    if(hipMalloc(&c.lookup_buf, sizeof(double) * 7 * len) != hipSuccess) return GALIC_ERR_NOMEM;
+    if(hipMalloc(&c.lookup_buf, sizeof(double) * 7 * len) != hipSuccess) {
+      (void)hipGetLastError();  // (else the next check of a launch would report it again)
+      return GALIC_ERR_NOMEM;
+    }
     c.lookup_len = len;
   }
   double *dpos = c.lookup_buf, *dacc = dpos + 3 * c.lookup_len, *dpot = dacc + 3 * c.lookup_len;

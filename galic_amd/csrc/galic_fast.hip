@@ -688,7 +688,10 @@ int sort_desc(int ntrial, unsigned int *key, unsigned int *key2, int *ord, int *
     if(*tmp) (void)hipFree(*tmp);
     *tmp = nullptr;
     *tmp_bytes = 0;
-    if(hipMalloc(tmp, need) != hipSuccess) return -1;
+    if(hipMalloc(tmp, need) != hipSuccess) {
+      (void)hipGetLastError();
+      return -1;
+    }
     *tmp_bytes = need;
   }
   if(rocprim::radix_sort_pairs_desc(*tmp, need, key, key2, ord, ord2, (unsigned int)ntrial, 0, 32, stream) !=

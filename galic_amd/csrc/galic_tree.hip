@@ -628,11 +628,13 @@ int terr(int code, const char *fmt, ...) {
   return galic::set_error(code, buf);
 }
 
+// (An error that is reported is also dropped from the runtime's record, as in galic_api.hip.)
 #define TCHK(expr)                                                                                 \
   do {                                                                                             \
     hipError_t e_ = (expr);                                                                        \
     if(e_ != hipSuccess) {                                                                         \
-      rc = terr(e_ == hipErrorOutOfMemory ? GALIC_ERR_NOMEM : GALIC_ERR_HIP, "%s: %s", #expr,     \
+      (void)hipGetLastError();                                                                     \
+      rc = terr(e_ == hipErrorOutOfMemory ? GALIC_ERR_NOMEM : GALIC_ERR_HIP, "%s: %s", #expr,      \
                 hipGetErrorString(e_));                                                            \
       goto done;                                                                                   \
     }                                                                                              \
