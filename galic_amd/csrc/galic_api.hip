@@ -109,6 +109,7 @@ bool type_present(const galic_params &p, int t) { return p.NType[t] > 0; }
 
 int alloc_orbit_scratch(galic::Ctx &c, int n) {
   if(n <= c.max_orbits) return GALIC_OK;
+  c.max_orbits = 0;  // (nothing is held if an allocation below fails)
   dfree(c.o_pidx); dfree(c.o_type); dfree(c.o_x); dfree(c.o_y); dfree(c.o_z);
   dfree(c.o_vx); dfree(c.o_vy); dfree(c.o_vz); dfree(c.o_mass); dfree(c.o_tint);
   dfree(c.o_tall); dfree(c.o_e0); dfree(c.o_e1); dfree(c.o_norbit); dfree(c.o_status);
@@ -141,6 +142,7 @@ int alloc_sort_scratch(galic::Ctx &c, int n) {
 int alloc_trial_scratch(galic::Ctx &c, int n) {
   CHK(alloc_sort_scratch(c, n));
   if(n <= c.max_trials) return GALIC_OK;
+  c.max_trials = 0;
   dfree(c.t_idx); dfree(c.t_v); dfree(c.t_accept); dfree(c.t_dF); dfree(c.t_best);
   CHK(dalloc(&c.t_idx, n));
   CHK(dalloc(&c.t_v, 3 * (size_t)n));
@@ -1120,6 +1122,10 @@ int galic_destroy(galic_ctx *ctx) {
   dfree(c.locA_q); dfree(c.locA_dq); dfree(c.locI_q); dfree(c.locI_dq);
   dfree(c.fit); dfree(c.locM_q); dfree(c.qinv); dfree(c.tovs_dev); dfree(c.t_vk); dfree(c.t_dFk); dfree(c.t_vinst);
   galic::Particles &P = c.P;
+  // (no particles are set if an allocation or a copy below fails)
+  ctx->initial_done = false;
+  ctx->fp32_initial_done = false;
+  P.n = 0;
   dfree(P.x); dfree(P.y); dfree(P.z); dfree(P.vx); dfree(P.vy); dfree(P.vz);
   dfree(P.mass); dfree(P.tint); dfree(P.vesc); dfree(P.vr2); dfree(P.vt2); dfree(P.vp2); dfree(P.vq2);
   dfree(P.type); dfree(P.orbits); dfree(P.disp);
@@ -1493,10 +1499,13 @@ int galic_set_particles(galic_ctx *ctx, int n, const double *pos, const double *
       return set_err(GALIC_ERR_ARG, "particle %d has type %d but NType[%d] is 0", i, type[i], type[i]);
   }
   galic::Particles &P = c.P;
+  // (no particles are set if an allocation or a copy below fails)
+  ctx->initial_done = false;
+  ctx->fp32_initial_done = false;
+  P.n = 0;
   dfree(P.x); dfree(P.y); dfree(P.z); dfree(P.vx); dfree(P.vy); dfree(P.vz);
   dfree(P.mass); dfree(P.tint); dfree(P.vesc); dfree(P.vr2); dfree(P.vt2); dfree(P.vp2); dfree(P.vq2);
   dfree(P.type); dfree(P.orbits); dfree(P.disp); dfree(c.psteps);
-  P.n = n;
   CHK(dalloc(&c.psteps, n));
   CHK(dalloc(&P.x, n)); CHK(dalloc(&P.y, n)); CHK(dalloc(&P.z, n));
   CHK(dalloc(&P.vx, n)); CHK(dalloc(&P.vy, n)); CHK(dalloc(&P.vz, n));
@@ -1524,8 +1533,7 @@ int galic_set_particles(galic_ctx *ctx, int n, const double *pos, const double *
   HIPCHK(hipMemcpy(P.tint, tint, sizeof(double) * n, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(P.type, type, sizeof(int) * n, hipMemcpyHostToDevice));
   if(vesc) HIPCHK(hipMemcpy(P.vesc, vesc, sizeof(double) * n, hipMemcpyHostToDevice));
-  ctx->initial_done = false;
-  ctx->fp32_initial_done = false;
+  P.n = n;
   return GALIC_OK;
 }
 
@@ -1987,6 +1995,8 @@ int fp32_run(galic_ctx *ctx, int ntrial, const int *idx, int K, int rep_size, co
   CHK(alloc_trial_scratch(c, std::max(ntrial, 1)));
   size_t nk = (size_t)std::max(ntrial, 1) * K;
   if(nk > c.max_ktrials) {
+    c.max_ktrials = 0;
+    c.last_ntrial = 0;
     dfree(c.t_vk);
     dfree(c.t_dFk);
     dfree(c.t_vinst);

@@ -31,3 +31,21 @@ def test_refusal_does_not_reach_another_context(small):
     b.fp32_rep(idx, k=2, sigma_frac=0.1, seed=5)
     a.close()
     b.close()
+
+
+def test_context_goes_on_after_a_refusal(small):
+    """The scratch that the refused call wanted to grow is grown again by the next call."""
+    w, idx = small
+    acc = []
+    for refused in (False, True):
+        g = GalicGPU(w)
+        g.fp32_calc_all_response_fields()
+        first = g.fp32_rep(idx, k=2, sigma_frac=0.1, seed=5)
+        if refused:
+            too_much(g)
+            with pytest.raises(RuntimeError):
+                g.fp32_trial_merits(len(idx), 2)
+        acc.append((first, g.fp32_rep(idx, k=2, sigma_frac=0.1, seed=6), g.fp32_trial_merits(len(idx), 2)))
+        g.close()
+    for a, b in zip(*acc):
+        assert np.array_equal(a, b)
