@@ -19,6 +19,7 @@
 #include "galic_targets.h"
 #include "galic_kernels.h"
 #include "galic_handle.h"
+#include "galic_plan.h"
 
 namespace {
 
@@ -517,20 +518,6 @@ void log_setup(galic::Ctx &c) {
 
 size_t log_block_bytes() { return (size_t)galic::LOG_B * (sizeof(int) + galic::kFields * sizeof(float4)); }
 
-// The log arena (the `slots` buffer), kept across calls: reallocated only when it is so far below
-// what a call could use (kLogFitMargin / kLogPlanMargin of it) that the call would need another
-// launch.
-int ensure_arena(galic::Ctx &c, size_t want, size_t need) {
-  if(c.slot_bytes >= need && c.slot_bytes >= want / 100 * 89) return GALIC_OK;
-  if(c.slots) (void)hipFree(c.slots);
-  c.slots = nullptr;
-  c.slot_bytes = c.slots_zero = 0;
-  const size_t bytes = std::max(want, need);
-  HIPCHK(hipMalloc(&c.slots, bytes));
-  c.slot_bytes = bytes;
-  return GALIC_OK;
-}
-
 // Blocks the lanes of a launch may claim and leave unused.
 double log_blocks_slack(const galic::Ctx &c, int n) {
   return (double)orbit_grid(n, 256, c.fp32_bpc) * 256 * galic::LOG_CHUNK + 64;
@@ -540,20 +527,47 @@ double log_blocks_slack(const galic::Ctx &c, int n) {
 // (counted exactly, also where the arena ran out) with a margin for other orbits.  The arena is
 // sized with the larger margin and a launch with the smaller, so that a call whose logs grew a
 // little since the arena was allocated still goes out as one launch: two launches last twice as
-// long as their longest orbits.
-constexpr double kLogPlanMargin = 1.2, kLogFitMargin = 1.06;
-double log_blocks_planned(const galic::Ctx &c, int n) {
-  return (double)n * c.log_est_blocks * kLogPlanMargin + log_blocks_slack(c, n);
+// long as their longest orbits.  The first estimate, from the orbits' steps at their start points, is
+// good to a factor of two (512^2 grids: 53 blocks an orbit, 71 counted), and the first arena is sized
+// for it.
+constexpr double kLogPlanMargin = 1.2, kLogFitMargin = 1.06, kLogFirstMargin = 2;
+double log_blocks_planned(const galic::Ctx &c, int n, double margin = kLogPlanMargin) {
+  return (double)n * c.log_est_blocks * margin + log_blocks_slack(c, n);
 }
 // Orbits, of a call of n, that fit the arena at once.
 double log_orbits_fit(const galic::Ctx &c, int n) {
-  const double blocks = (double)(c.slot_bytes / ((size_t)galic::LOG_B * (sizeof(int) + galic::kFields * sizeof(float4))));
+  const double blocks = (double)(c.slot_bytes / log_block_bytes());
   return (blocks - log_blocks_slack(c, n)) / (c.log_est_blocks * kLogFitMargin);
+}
+
+size_t slot_budget(galic::Ctx &c);
+
+// The log arena (the `slots` buffer), kept across calls.
+int new_arena(galic::Ctx &c, size_t bytes) {
+  if(c.slots) (void)hipFree(c.slots);
+  c.slots = nullptr;
+  c.slot_bytes = c.slots_zero = 0;
+  HIPCHK(hipMalloc(&c.slots, bytes));
+  c.slot_bytes = bytes;
+  return GALIC_OK;
+}
+
+// An arena for a call of n orbits, `least` of them in one launch; first: nothing measured yet.
+int ensure_arena(galic::Ctx &c, int n, int least, bool first = false) {
+  const size_t bb = log_block_bytes();
+  auto bytes = [&](int m, double margin) { return (size_t)(log_blocks_planned(c, m, margin) * bb); };
+  const size_t all = bytes(n, kLogPlanMargin), need = bytes(std::min(n, least), kLogPlanMargin);
+  const size_t budget = slot_budget(c);
+  const size_t want = std::min(first ? bytes(n, kLogPlanMargin * kLogFirstMargin) : all, budget);
+  const bool bounded = all > budget || c.alt.slot_bytes > 0;
+  const size_t fit = bytes(n, kLogFitMargin) + bb;  // (log_orbits_fit counts whole blocks)
+  if(galic::arena_kept(c.slot_bytes, need, want, fit, bounded)) return GALIC_OK;
+  return new_arena(c, std::max(want, need));
 }
 
 constexpr int kLogArenaFull = 1;  // launch_orbit32_log: the arena ran out, plan a smaller launch
 
-constexpr int kLogTableFull = 2;  // orbit32_log_end: an orbit outgrew its block table (log_M doubled)
+constexpr int kLogTableFull = 2;  // orbit32_log_end: an orbit outgrew its block table (log_M grown to the longest log)
 
 // One launch of the logging orbit kernel over A.n orbits into the active orbit set's arena, on
 // that set's stream, not waited on: the tables sized, the counters cleared, the launch bracketed
@@ -813,7 +827,8 @@ int fp32_initial_logs(galic::Ctx &c, int n) {
                      (const double *)P.y, (const double *)P.z, (const double *)P.vx, (const double *)P.vy,
                      (const double *)P.vz, (const double *)P.tint, c.t_key, c.t_ord);
   HIPCHK(hipGetLastError());
-  if(c.log_est_blocks <= 0) {
+  const bool first = c.log_est_blocks <= 0;
+  if(first) {
     // nothing measured yet: about a record per two expected steps
     unsigned long long sum[2];
     HIPCHK(hipMemsetAsync(c.orbit_stats, 0, sizeof(sum), c.stream));
@@ -828,12 +843,7 @@ int fp32_initial_logs(galic::Ctx &c, int n) {
   }
   if(galic::sort_desc(n, c.t_key, c.t_key2, c.t_ord, c.t_ord2, &c.sort_tmp, &c.sort_tmp_bytes, c.stream) != 0)
     return set_err(GALIC_ERR_HIP, "sorting the particles by expected orbit length failed");
-  {
-    const size_t bb = log_block_bytes();
-    const size_t all = (size_t)(log_blocks_planned(c, n) * bb);
-    const size_t one = (size_t)(log_blocks_planned(c, std::min(n, 1024)) * bb);
-    CHK(ensure_arena(c, std::min(all, slot_budget(c)), one));
-  }
+  CHK(ensure_arena(c, n, 1024, first));
   struct Share {
     int first, stride;
   };
@@ -1924,6 +1934,14 @@ int galic_fp32_autotune(galic_ctx *ctx, int nsample, int *variant, int *blocks_p
   std::vector<int> bpcs;
   for(int b = 1; b <= occ; b++) bpcs.push_back(b);
   bpcs.push_back(2 * occ);
+  // the arena for the largest grid, whose lanes may leave the most blocks unused: one for all of them
+  auto room = [&]() {
+    const int b = c.fp32_bpc;
+    c.fp32_bpc = bpcs.back();
+    const size_t bytes = (size_t)(log_blocks_planned(c, n) * log_block_bytes());
+    c.fp32_bpc = b;
+    return bytes;
+  };
   double best = 1e300;
   int bv = 0, bb = 4;
   const long long steps0 = c.acc_steps, orbits0 = c.acc_orbits;
@@ -1936,8 +1954,7 @@ int galic_fp32_autotune(galic_ctx *ctx, int nsample, int *variant, int *blocks_p
       long long s_before = c.acc_steps;
       int lr = kLogArenaFull;
       for(int attempt = 0; attempt < 6 && lr == kLogArenaFull; attempt++) {
-        const size_t bb = log_block_bytes();
-        CHK(ensure_arena(c, (size_t)(log_blocks_planned(c, n) * bb), (size_t)(log_blocks_planned(c, n) * bb)));
+        if(c.slot_bytes < room()) CHK(new_arena(c, room()));
         lr = launch_orbit32_log(c, orbit_args32(c, n));
       }
       if(lr == kLogArenaFull) return set_err(GALIC_ERR_NOMEM, "no room for the tuning sample's response logs");
@@ -2034,10 +2051,7 @@ int fp32_run(galic_ctx *ctx, int ntrial, const int *idx, int K, int rep_size, co
       const size_t half = std::max(one, (budget + c.alt.slot_bytes) / 2);
       auto fit_half = [&]() -> int {
         if(c.slot_bytes >= one && c.slot_bytes <= half + half / 8 && 2 * c.slot_bytes >= half) return GALIC_OK;
-        if(c.slots) (void)hipFree(c.slots);
-        c.slots = nullptr;
-        c.slot_bytes = 0;
-        return ensure_arena(c, half, one);
+        return new_arena(c, half);
       };
       CHK(fit_half());
       swap_orbit_set(c);
@@ -2045,7 +2059,7 @@ int fp32_run(galic_ctx *ctx, int ntrial, const int *idx, int K, int rep_size, co
       swap_orbit_set(c);
       CHK(rc);
     } else {
-      CHK(ensure_arena(c, std::min(all, budget), one));
+      CHK(ensure_arena(c, std::max(ntrial, 1) * (K + 1), std::min(std::max(ntrial, 1), 1024) * (K + 1)));
     }
   }
   // the orbit launches beside a group's judging share the CUs with the merit kernel: their own

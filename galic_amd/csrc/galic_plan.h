@@ -1,0 +1,20 @@
+// galic_plan.h -- rules by which the FP32 path plans its response logs' memory and launches.  Host
+// code without HIP (tests/test_log_plan.py runs it on the CPU).
+#pragma once
+
+#include <stddef.h>
+
+namespace galic {
+
+// Whether a call keeps the log arena of `have` bytes that it finds.  It must hold `need`; then it
+// is kept if it holds the call's orbits in one launch (`fit`), since a free and a new allocation of
+// tens of GB cost more than most calls (0.4 s for 20 GB, 8 s for 130 GB), and a call that goes out
+// in two launches lasts twice as long as its longest orbits.  A call that is `bounded`, because
+// `want` is all that the memory allows or because a second arena takes its part, goes out in several
+// launches whatever it does: it keeps an arena of half of what it wants, so that calls of different
+// kinds in turn do not each take their own.
+inline bool arena_kept(size_t have, size_t need, size_t want, size_t fit, bool bounded) {
+  return have >= need && (have >= fit || (bounded && have >= want / 2));
+}
+
+}  // namespace galic

@@ -1,0 +1,50 @@
+"""The rules that plan the response logs' memory and launches (galic_plan.h), on the CPU."""
+import pathlib
+import subprocess
+
+import pytest
+
+CSRC = pathlib.Path(__file__).resolve().parents[1] / "galic_amd" / "csrc"
+
+HARNESS = r"""
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+#include "galic_plan.h"
+
+int main(int argc, char **argv) {
+  auto arg = [&](int i) { return strtoull(argv[i], nullptr, 10); };
+  if(!strcmp(argv[1], "arena")) printf("%d\n", galic::arena_kept(arg(2), arg(3), arg(4), arg(5), arg(6)));
+  return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def plan(tmp_path_factory):
+    d = tmp_path_factory.mktemp("plan")
+    (d / "plan.cpp").write_text(HARNESS)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-I", str(CSRC), str(d / "plan.cpp"), "-o", str(d / "plan")],
+                   check=True)
+
+    def run(*args):
+        out = subprocess.run([str(d / "plan")] + [str(a) for a in args], check=True, capture_output=True, text=True)
+        return [int(x) for x in out.stdout.split()]
+    return run
+
+
+# GB: the arena there is, what one launch needs, what the call wants, what holds it in one launch, bounded, kept
+@pytest.mark.parametrize("have,need,want,fit,bounded,kept", [
+    (0, 1, 10, 9, 0, 0),          # none yet
+    (43, 1, 25, 22, 0, 1),        # a second pass after a first one sized with room
+    (21, 1, 25, 22, 0, 0),        # one that would need a second launch
+    (900, 1, 1000, 897, 0, 1),    # a tenth below what is wanted, and it fits
+    (895, 1, 1000, 897, 0, 0),    # 89.5% of what is wanted, and it does not fit: two launches in every call
+    (137, 1, 192, 180, 1, 1),     # all the memory wanted, most of it there
+    (96, 1, 160, 400, 1, 1),      # a second arena holds the other half
+    (75, 1, 160, 400, 1, 0),      # less than half
+    (96, 100, 160, 90, 1, 0),     # not one launch's orbits
+])
+def test_arena_is_kept_unless_a_launch_more_is_saved(plan, have, need, want, fit, bounded, kept):
+    gb = 1 << 30
+    assert plan("arena", have * gb, need * gb, want * gb, fit * gb, bounded) == [kept]
