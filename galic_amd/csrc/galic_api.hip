@@ -884,12 +884,18 @@ int fp32_initial_logs(galic::Ctx &c, int n) {
     HIPCHK(hipGetLastError());
     // every record of the share's orbits into the Loc grids, in runs of orbits whose bucket
     // entries (about 1.3 per record) stay within kCommitEntries
-    const double per_orbit = std::max(1.0, c.log_est_blocks * galic::LOG_B * 1.3);
-    const int run = (int)std::max(1.0, std::min((double)m, (double)kCommitEntries / per_orbit));
-    for(int b0 = 0; b0 < m; b0 += run) {
+    const double most = kCommitEntries / 1.3;
+    std::vector<int> len;
+    if(c.log_est_blocks * galic::LOG_B * m > most) {
+      len.resize(m);
+      HIPCHK(hipMemcpyAsync(len.data(), c.log_n, sizeof(int) * m, hipMemcpyDeviceToHost, c.stream));
+      HIPCHK(hipStreamSynchronize(c.stream));
+    }
+    for(int b0 = 0, run = m; b0 < m; b0 += run) {
+      if(!len.empty()) run = galic::commit_run(len.data(), b0, m, most);
       galic::CommitArgs C;
       memset(&C, 0, sizeof(C));
-      C.n = std::min(run, m - b0);
+      C.n = run;
       C.orbit_base = b0;
       C.otype = c.o_type + b0;
       CHK(commit_logs(c, C, c.locA_q));

@@ -17,4 +17,17 @@ inline bool arena_kept(size_t have, size_t need, size_t want, size_t fit, bool b
   return have >= need && (have >= fit || (bounded && have >= want / 2));
 }
 
+// Orbits, from b0 on of m, whose logs (n[b] records each) make one commit of at most `most` records:
+// one orbit at least.  Counted from the logs themselves: they are in the order of their expected
+// length, so the first of m logs hold about twice the mean.
+inline int commit_run(const int *n, int b0, int m, double most) {
+  double records = 0;
+  int b = b0;
+  for(; b < m; b++) {
+    records += n[b];
+    if(b > b0 && records > most) break;
+  }
+  return b - b0;
+}
+
 }  // namespace galic

@@ -10,11 +10,19 @@ HARNESS = r"""
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <vector>
 #include "galic_plan.h"
 
 int main(int argc, char **argv) {
   auto arg = [&](int i) { return strtoull(argv[i], nullptr, 10); };
   if(!strcmp(argv[1], "arena")) printf("%d\n", galic::arena_kept(arg(2), arg(3), arg(4), arg(5), arg(6)));
+  if(!strcmp(argv[1], "commit")) {
+    // the most records of a commit, then the logs' lengths: the runs
+    std::vector<int> n;
+    for(int i = 3; i < argc; i++) n.push_back(atoi(argv[i]));
+    const int m = (int)n.size();
+    for(int b0 = 0, run; b0 < m; b0 += run) printf("%d\n", run = galic::commit_run(n.data(), b0, m, atof(argv[2])));
+  }
   return 0;
 }
 """
@@ -48,3 +56,17 @@ def plan(tmp_path_factory):
 def test_arena_is_kept_unless_a_launch_more_is_saved(plan, have, need, want, fit, bounded, kept):
     gb = 1 << 30
     assert plan("arena", have * gb, need * gb, want * gb, fit * gb, bounded) == [kept]
+
+
+@pytest.mark.parametrize("lengths", [[5], list(range(400, 0, -1)), [900, 3, 3, 3, 800, 1], [0] * 7, [1] * 50 + [700] * 3])
+@pytest.mark.parametrize("most", [1, 700, 10000, 1e9])
+def test_commit_runs_hold_their_records(plan, lengths, most):
+    """Every log once, no commit above its size but for a log alone, none that the next log would still fit in."""
+    runs = plan("commit", most, *lengths)
+    assert sum(runs) == len(lengths) and min(runs) >= 1
+    at = 0
+    for r in runs:
+        held = sum(lengths[at:at + r])
+        assert held <= most or r == 1
+        at += r
+        assert at == len(lengths) or held + lengths[at] > most
