@@ -537,7 +537,8 @@ double log_blocks_planned(const galic::Ctx &c, int n, double margin = kLogPlanMa
 // Orbits, of a call of n, that fit the arena at once.
 double log_orbits_fit(const galic::Ctx &c, int n) {
   const double blocks = (double)(c.slot_bytes / log_block_bytes());
-  return (blocks - log_blocks_slack(c, n)) / (c.log_est_blocks * kLogFitMargin);
+  return galic::orbits_fit(blocks - 64, log_blocks_slack(c, n) - 64, galic::LOG_CHUNK, 256,
+                           c.log_est_blocks * kLogFitMargin);
 }
 
 size_t slot_budget(galic::Ctx &c);

@@ -4,6 +4,8 @@
 
 #include <stddef.h>
 
+#include <algorithm>
+
 namespace galic {
 
 // Whether a call keeps the log arena of `have` bytes that it finds.  It must hold `need`; then it
@@ -15,6 +17,14 @@ namespace galic {
 // kinds in turn do not each take their own.
 inline bool arena_kept(size_t have, size_t need, size_t want, size_t fit, bool bounded) {
   return have >= need && (have >= fit || (bounded && have >= want / 2));
+}
+
+// Orbits whose logs of `per_orbit` blocks fit `blocks`.  The lanes of a launch leave up to `chunk`
+// blocks each unused: `slack` in all for a launch that fills the grid, and chunk an orbit and `group`
+// lanes more for one that does not.  (Counted for the full grid alone, an arena below its slack,
+// 8.4 GB, took its orbits one by one.)
+inline double orbits_fit(double blocks, double slack, double chunk, double group, double per_orbit) {
+  return std::max((blocks - slack) / per_orbit, (blocks - group * chunk) / (per_orbit + chunk));
 }
 
 // Orbits, from b0 on of m, whose logs (n[b] records each) make one commit of at most `most` records:

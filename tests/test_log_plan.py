@@ -16,6 +16,8 @@ HARNESS = r"""
 int main(int argc, char **argv) {
   auto arg = [&](int i) { return strtoull(argv[i], nullptr, 10); };
   if(!strcmp(argv[1], "arena")) printf("%d\n", galic::arena_kept(arg(2), arg(3), arg(4), arg(5), arg(6)));
+  if(!strcmp(argv[1], "fit"))
+    printf("%lld\n", (long long)galic::orbits_fit(atof(argv[2]), atof(argv[3]), atof(argv[4]), atof(argv[5]), atof(argv[6])));
   if(!strcmp(argv[1], "commit")) {
     // the most records of a commit, then the logs' lengths: the runs
     std::vector<int> n;
@@ -56,6 +58,19 @@ def plan(tmp_path_factory):
 def test_arena_is_kept_unless_a_launch_more_is_saved(plan, have, need, want, fit, bounded, kept):
     gb = 1 << 30
     assert plan("arena", have * gb, need * gb, want * gb, fit * gb, bounded) == [kept]
+
+
+# arenas of a few blocks to ones far above the full grid's slack (768 workgroups of 256 lanes, 8 blocks each)
+@pytest.mark.parametrize("blocks", [3000, 30000, 300000, 1500000, 1600000, 5000000, 40000000])
+@pytest.mark.parametrize("per_orbit", [1.06, 10, 75, 300])
+def test_orbits_that_fit_leave_room_for_the_slack(plan, blocks, per_orbit):
+    """What a launch of that many orbits may need is there, and nearly all of the arena is used: a launch of one
+    workgroup more, or of 1% more orbits, would not fit."""
+    def needs(m):
+        return m * per_orbit + min(-(-m // 256), 768) * 256 * 8
+    fit, = plan("fit", blocks, 768 * 256 * 8, 8, 256, per_orbit)
+    assert fit >= 1 and needs(fit) <= blocks
+    assert needs(fit + max(512, fit // 100)) > blocks
 
 
 @pytest.mark.parametrize("lengths", [[5], list(range(400, 0, -1)), [900, 3, 3, 3, 800, 1], [0] * 7, [1] * 50 + [700] * 3])
