@@ -543,6 +543,12 @@ double log_orbits_fit(const galic::Ctx &c, int n) {
 
 size_t slot_budget(galic::Ctx &c);
 
+// Bytes the logs of both orbit sets may take together.
+size_t log_budget(galic::Ctx &c) {
+  const size_t all = slot_budget(c) + c.alt.slot_bytes;
+  return c.arena_limit > 0 ? std::min(all, c.arena_limit) : all;
+}
+
 // The log arena (the `slots` buffer), kept across calls.
 int new_arena(galic::Ctx &c, size_t bytes) {
   if(c.slots) (void)hipFree(c.slots);
@@ -553,16 +559,30 @@ int new_arena(galic::Ctx &c, size_t bytes) {
   return GALIC_OK;
 }
 
+// Bytes the active set's arena may take.  (Under a limit set by the caller, the other set's arena
+// gives way when it holds more than half.)
+size_t arena_budget(galic::Ctx &c) {
+  const size_t total = log_budget(c);
+  if(c.arena_limit > 0 && c.alt.slot_bytes > total / 2) {
+    (void)hipFree(c.alt.slots);
+    c.alt.slots = nullptr;
+    c.alt.slot_bytes = c.alt.slots_zero = 0;
+  }
+  return total - c.alt.slot_bytes;
+}
+
 // An arena for a call of n orbits, `least` of them in one launch; first: nothing measured yet.
 int ensure_arena(galic::Ctx &c, int n, int least, bool first = false) {
   const size_t bb = log_block_bytes();
   auto bytes = [&](int m, double margin) { return (size_t)(log_blocks_planned(c, m, margin) * bb); };
-  const size_t all = bytes(n, kLogPlanMargin), need = bytes(std::min(n, least), kLogPlanMargin);
-  const size_t budget = slot_budget(c);
+  const size_t all = bytes(n, kLogPlanMargin), budget = arena_budget(c);
+  size_t need = bytes(std::min(n, least), kLogPlanMargin);
+  if(c.arena_limit > 0) need = std::min(need, budget);
   const size_t want = std::min(first ? bytes(n, kLogPlanMargin * kLogFirstMargin) : all, budget);
   const bool bounded = all > budget || c.alt.slot_bytes > 0;
   const size_t fit = bytes(n, kLogFitMargin) + bb;  // (log_orbits_fit counts whole blocks)
-  if(galic::arena_kept(c.slot_bytes, need, want, fit, bounded)) return GALIC_OK;
+  const bool above = c.arena_limit > 0 && c.slot_bytes > budget;
+  if(!above && galic::arena_kept(c.slot_bytes, need, want, fit, bounded)) return GALIC_OK;
   return new_arena(c, std::max(want, need));
 }
 
@@ -885,7 +905,7 @@ int fp32_initial_logs(galic::Ctx &c, int n) {
     HIPCHK(hipGetLastError());
     // every record of the share's orbits into the Loc grids, in runs of orbits whose bucket
     // entries (about 1.3 per record) stay within kCommitEntries
-    const double most = kCommitEntries / 1.3;
+    const double most = (c.commit_limit > 0 ? (double)c.commit_limit / sizeof(uint2) : kCommitEntries) / 1.3;
     std::vector<int> len;
     if(c.log_est_blocks * galic::LOG_B * m > most) {
       len.resize(m);
@@ -1911,12 +1931,31 @@ int galic_fp32_autotune(galic_ctx *ctx, int nsample, int *variant, int *blocks_p
   galic::Ctx &c = ctx->c;
   if(!ctx->fp32_initial_done) return set_err(GALIC_ERR_STATE, "galic_fp32_calc_all_response_fields must run first");
   HIPCHK(hipSetDevice(c.device));
+  // grid sizes in workgroups per CU (the results are bit-identical; only the schedule differs)
+  int occ = 4;
+  HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void *>(galic::k_orbit32_log), 256, 0));
+  occ = std::max(1, std::min(occ, 16));
+  // every count from 1 to the resident limit, and twice that (a persistent grid larger than
+  // the CUs hold only queues)
+  const int variants[1] = {0};
+  std::vector<int> bpcs;
+  for(int b = 1; b <= occ; b++) bpcs.push_back(b);
+  bpcs.push_back(2 * occ);
   // no more orbits than the response logs of one launch fit in half the memory the arena may
   // take (the other half covers the blocks the lanes claim and leave unused)
-  const double arena_blocks = (double)slot_budget(c) / log_block_bytes();
+  const size_t budget = arena_budget(c);
   const double per_orbit = c.log_est_blocks * kLogPlanMargin;
-  const int fit_n = (int)std::max(1024.0, std::min(2e9, 0.5 * arena_blocks / per_orbit));
-  const int n = std::min(std::min(nsample, c.P.n), fit_n);
+  const int fit_n = (int)std::max(1024.0, std::min(2e9, 0.5 * ((double)budget / log_block_bytes()) / per_orbit));
+  int n = std::min(std::min(nsample, c.P.n), fit_n);
+  // the arena for the largest grid, whose lanes may leave the most blocks unused: one for all of them
+  auto room = [&]() {
+    const int b = c.fp32_bpc;
+    c.fp32_bpc = bpcs.back();
+    const size_t bytes = (size_t)(log_blocks_planned(c, n) * log_block_bytes());
+    c.fp32_bpc = b;
+    return bytes;
+  };
+  while(c.arena_limit > 0 && n > 1 && room() > budget) n /= 2;
   CHK(alloc_orbit_scratch(c, n));
   // a strided sample of the model's own orbits at their current velocities,
   // longest expected first as in a rep
@@ -1931,24 +1970,6 @@ int galic_fp32_autotune(galic_ctx *ctx, int nsample, int *variant, int *blocks_p
                      (const int *)c.t_ord2, c.t_idx, (const double *)nullptr, (const double *)nullptr,
                      (const double *)nullptr, c.P, orbit_in(c));
   HIPCHK(hipGetLastError());
-  // grid sizes in workgroups per CU (the results are bit-identical; only the schedule differs)
-  int occ = 4;
-  HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void *>(galic::k_orbit32_log), 256, 0));
-  occ = std::max(1, std::min(occ, 16));
-  // every count from 1 to the resident limit, and twice that (a persistent grid larger than
-  // the CUs hold only queues)
-  const int variants[1] = {0};
-  std::vector<int> bpcs;
-  for(int b = 1; b <= occ; b++) bpcs.push_back(b);
-  bpcs.push_back(2 * occ);
-  // the arena for the largest grid, whose lanes may leave the most blocks unused: one for all of them
-  auto room = [&]() {
-    const int b = c.fp32_bpc;
-    c.fp32_bpc = bpcs.back();
-    const size_t bytes = (size_t)(log_blocks_planned(c, n) * log_block_bytes());
-    c.fp32_bpc = b;
-    return bytes;
-  };
   double best = 1e300;
   int bv = 0, bb = 4;
   const long long steps0 = c.acc_steps, orbits0 = c.acc_orbits;
@@ -2048,16 +2069,18 @@ int fp32_run(galic_ctx *ctx, int ntrial, const int *idx, int K, int rep_size, co
   {
     const size_t bb = log_block_bytes();
     const size_t all = (size_t)(log_blocks_planned(c, std::max(ntrial, 1) * (K + 1)) * bb);
-    const size_t one = (size_t)(log_blocks_planned(c, std::min(std::max(ntrial, 1), 1024) * (K + 1)) * bb);
-    const size_t budget = slot_budget(c);
+    size_t one = (size_t)(log_blocks_planned(c, std::min(std::max(ntrial, 1), 1024) * (K + 1)) * bb);
+    const size_t both = log_budget(c), budget = both - std::min(both, c.alt.slot_bytes);
     overlap = c.overlap == 1 || (c.overlap < 0 && all > budget / 2);
     if(overlap) {
       CHK(ensure_alt_set(c));
       // each set's arena about half of what one arena could take (the one left by earlier calls
       // shrinks first, so that the other has room)
-      const size_t half = std::max(one, (budget + c.alt.slot_bytes) / 2);
+      if(c.arena_limit > 0) one = std::min(one, both / 2);
+      const size_t half = std::max(one, both / 2);
       auto fit_half = [&]() -> int {
-        if(c.slot_bytes >= one && c.slot_bytes <= half + half / 8 && 2 * c.slot_bytes >= half) return GALIC_OK;
+        const size_t most = c.arena_limit > 0 ? half : half + half / 8;
+        if(c.slot_bytes >= one && c.slot_bytes <= most && 2 * c.slot_bytes >= half) return GALIC_OK;
         return new_arena(c, half);
       };
       CHK(fit_half());
@@ -2675,6 +2698,15 @@ int galic_fp32_set_schedule(galic_ctx *ctx, int max_group_trials, int overlap, i
   ctx->c.max_group_trials = max_group_trials;
   ctx->c.overlap = overlap;
   ctx->c.use_graph = graph;
+  return GALIC_OK;
+}
+
+int galic_fp32_set_memory(galic_ctx *ctx, unsigned long long log_bytes, unsigned long long commit_bytes) {
+  if(!ctx) return set_err(GALIC_ERR_ARG, "null context");
+  if(log_bytes > 0 && log_bytes < 128 * log_block_bytes())
+    return set_err(GALIC_ERR_ARG, "log_bytes must be 0 or at least %zu", 128 * log_block_bytes());
+  ctx->c.arena_limit = (size_t)log_bytes;
+  ctx->c.commit_limit = (size_t)commit_bytes;
   return GALIC_OK;
 }
 

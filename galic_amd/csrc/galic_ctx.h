@@ -229,6 +229,7 @@ struct Ctx {
   int overlap = -1;                   // FP32 reps: integrate the next group's orbits while judging a group
                                       // (-1 when a call needs more than one launch, 0 never, 1 always)
   int merit_wg_per_cu = 0;            // FP32 merit kernel: workgroups per CU at most (0: as many as fit)
+  size_t arena_limit = 0, commit_limit = 0;  // bytes the logs, and a commit's entries, may take (0: by the memory)
   int max_group_trials = 0;           // FP32 reps: at most this many trials per orbit launch (0: the arena's)
 
   // timing of the last launches (ms), measured with HIP events on ctx stream

@@ -173,6 +173,11 @@ class GalicGPU:
         (16x16-tile merit), 0 launches them rep by rep.  The results do not depend on the schedule."""
         check(self.lib.galic_fp32_set_schedule(self.h, int(max_group_trials), int(overlap), int(graph)))
 
+    def fp32_set_memory(self, log_bytes=0, commit_bytes=0):
+        """At most log_bytes of device memory for the response logs and commit_bytes for the entries of one commit of
+        the initial pass (0: by the free memory, 2 GiB).  The results do not depend on it."""
+        check(self.lib.galic_fp32_set_memory(self.h, int(log_bytes), int(commit_bytes)))
+
     def fp32_set_fresh_trials(self, nfresh):
         """The first nfresh device trials per particle are fresh draws (main.c:383-435)."""
         check(self.lib.galic_fp32_set_fresh_trials(self.h, int(nfresh)))

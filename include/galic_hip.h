@@ -249,6 +249,13 @@ int galic_fp32_set_merit_launch(galic_ctx *ctx, int wg_per_cu);
  * results are the same bits whatever the schedule. */
 int galic_fp32_set_schedule(galic_ctx *ctx, int max_group_trials, int overlap, int graph);
 
+/* Device memory of the FP32 path's response logs: at most log_bytes for the arena (or the two
+ * arenas of an overlapped schedule), and at most about commit_bytes for the entries of one commit of
+ * the initial pass.  0 (default): logs by the free memory, 2 GiB of entries.  Calls whose logs need
+ * more go out in more launches; the results are the same bits.  A call fails with GALIC_ERR_NOMEM
+ * where the logs of one orbit (one particle's trials) do not fit.  No counterpart in the reference. */
+int galic_fp32_set_memory(galic_ctx *ctx, unsigned long long log_bytes, unsigned long long commit_bytes);
+
 /* Timing aid of the sparse tile merit: on != 0 starts (or restarts) summing, per phase of
  * each particle, the wall-clock ticks (100 MHz) of the kernel's thread 0; out16 (optional)
  * first receives the sums so far: [0] tile lists, [1] fields and tiles, [2] choice, [3]
