@@ -240,7 +240,9 @@ struct Ctx {
   long long acc_orbit_launches = 0;
   long long acc_orbits = 0, acc_steps = 0;
   int fp32_variant = 0;   // orbit kernel variant (one so far)
-  int fp32_bpc = 3;       // persistent workgroups per CU for k_orbit32 (autotuned)
+  // persistent workgroups per CU for k_orbit32 (autotuned); a call of 270000 orbits on 64^2 grids with one
+  // 26.3 ms, two 23.8, three 26.7, four 30; an initial pass of 4e5 on 512^2 grids 214, 186, 196, 191 ms
+  int fp32_bpc = 2;
   int fp32_bpc_overlap = 0;  // the same for the launches beside a group's judging (0: fp32_bpc)
   int fp32_nfresh = 0;    // device trials per particle drawn fresh (optimize()'s distribution)
   bool fp32_tuned = false;
