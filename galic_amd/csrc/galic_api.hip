@@ -456,7 +456,7 @@ galic::FastModel fast_model(galic::Ctx &c) {
   F.bulge_eps = (float)(1.0e-6 * p.Bulge_A);
   F.fo_v200 = (float)(p.TimeStepFactorOrbit * p.V200);
   F.fc = (float)p.TimeStepFactorCellCross;
-  F.max_steps = c.M.max_steps;
+  F.max_steps = galic::fp32_step_cap(c.M.max_steps);
   F.acc = c.FG_Acc_f;
   F.vstream = c.FG_Vstream_f;
   F.vstream_nz = c.vstream_nz;

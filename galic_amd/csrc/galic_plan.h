@@ -40,4 +40,9 @@ inline int commit_run(const int *n, int b0, int m, double most) {
   return b - b0;
 }
 
+// The step cap of the FP32 orbit kernel, whose counter is an int that is -1 at an orbit's start: one
+// step more than the cap must be above it and not wrap to a negative count, which would start the
+// orbit over for good.
+inline long long fp32_step_cap(long long cap) { return std::min(cap, 0x7ffffffeLL); }
+
 }  // namespace galic

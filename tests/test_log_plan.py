@@ -18,6 +18,12 @@ int main(int argc, char **argv) {
   if(!strcmp(argv[1], "arena")) printf("%d\n", galic::arena_kept(arg(2), arg(3), arg(4), arg(5), arg(6)));
   if(!strcmp(argv[1], "fit"))
     printf("%lld\n", (long long)galic::orbits_fit(atof(argv[2]), atof(argv[3]), atof(argv[4]), atof(argv[5]), atof(argv[6])));
+  if(!strcmp(argv[1], "cap")) {
+    // the counter of an orbit at the cap after one more step, and whether the kernel's test ends it there
+    const long long cap = galic::fp32_step_cap(strtoll(argv[2], nullptr, 10));
+    const int steps = (int)(unsigned int)((unsigned long long)cap + 1);
+    printf("%lld\n%d\n", cap, steps > 0 && (unsigned int)steps > (unsigned int)cap);
+  }
   if(!strcmp(argv[1], "commit")) {
     // the most records of a commit, then the logs' lengths: the runs
     std::vector<int> n;
@@ -85,3 +91,9 @@ def test_commit_runs_hold_their_records(plan, lengths, most):
         assert held <= most or r == 1
         at += r
         assert at == len(lengths) or held + lengths[at] > most
+
+
+@pytest.mark.parametrize("cap", [1, 100000000, 2**31 - 2, 2**31 - 1])
+def test_every_step_cap_ends_an_orbit(plan, cap):
+    used, ends = plan("cap", cap)
+    assert ends and cap - 1 <= used <= cap
