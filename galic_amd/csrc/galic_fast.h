@@ -29,7 +29,6 @@ constexpr int kCell1Max = 1024;  // density-grid cells per side the LDS cell-siz
 struct OrbitArgs32 {
   int n;
   unsigned int *counter;
-  const int *order;    // the orbits in the order they are taken, or null: 0 .. n-1
   const double *ox, *oy, *oz, *ovx, *ovy, *ovz, *omass, *otint;
   const int *otype;
   float *slots;        // private FP32 response per orbit, or null

@@ -31,7 +31,8 @@ __device__ __forceinline__ float fast_rsq(float x) { return __builtin_amdgcn_rsq
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
 // Correctly rounded square root for r^2 of a position: the hardware's root, moved by an ulp where
-// its residual says so.  (Not scaled for r^2 < 2^-96, where r no longer changes r + eps.)
+// its residual says so, as LLVM's AMDGPU backend expands sqrtf, whose bits it has to give.  Its
+// scaling of small arguments is left out: for r^2 < 2^-96 r no longer changes r + eps.
 __device__ __forceinline__ float root32(float s) {
   const float q = __builtin_amdgcn_sqrtf(s);
   const float lo = __int_as_float(__float_as_int(q) - 1), hi = __int_as_float(__float_as_int(q) + 1);
@@ -146,7 +147,7 @@ __device__ __forceinline__ int take_orbit32(const OrbitArgs32 &A, int nb) {
   while(true) {
     const unsigned int q = atomicAdd(A.counter, 1u);
     if(q >= (unsigned int)A.n) return -1;
-    const int o = A.order ? A.order[q] : (int)q;
+    const int o = (int)q;
     if(A.otint[o] > 0) return o;
     A.tall[o] = 0;
     A.norbit[o] = 0;

@@ -16,7 +16,8 @@
 //   4. moments bottom-up in FP64, in child order 0..7 as the reference;
 //   5. nextnode/sibling threading top-down, giving the reference's depth-first
 //      walk order;
-//   6. one target per lane walks the tree without a stack.
+//   6. the tree is walked without a stack, one target per lane, the 64 targets of a wave on one path;
+//      or by groups of targets with a list of interactions each (k_walk32g).
 // Particles that share all 21 key levels (closer than len/2^21) stay together
 // in a leaf bucket; opening it interacts with them one by one.  The reference
 // would keep splitting; this changes results only for targets within that
