@@ -315,6 +315,7 @@ struct WalkArgs {
   const int *child;     // [node][8] (the group walk)
   int blk_nb;           // targets are the (section, z, R) table nodes of nb x nb grids, a wave's an
                         // 8 x 8 block of one section; 0: 64 consecutive targets
+  int tpw;              // per-target walks: targets of a wave, a power of two up to 64
   double theta, h, G;
   int plummer;          // Plummer softening of length eps instead of the spline of length h
   double eps;
@@ -441,13 +442,16 @@ __device__ __forceinline__ void interact(const WalkArgs &A, float mass, float dx
 // gathers of 64 lines, one after the other.  Neighbouring targets share most of their paths (the
 // targets come in 8 x 8 blocks of a table section or in Morton order).  2e5 sources, 8 x 128^2
 // targets, FP64: 11.7 -> 5.3 ms.
+// A wave's time is the length of its path, and targets far from each other share little of it: where
+// the launch leaves the chip idle, waves take fewer targets (kWalkWaves below), down to one.
 // T = float: separations formed in FP64 (node centres of mass and particles stay FP64) and rounded
 // once, the kernel and the sums in FP32 per target.
 template <typename T>
 __device__ __forceinline__ void walk_body(const WalkArgs &A) {
   const int lane = threadIdx.x & 63;
-  long long t = wave_target(A, blockIdx.x, lane);
-  const bool live = t < A.ntarget;
+  const long long i = (long long)blockIdx.x * A.tpw + lane;
+  long long t = wave_target(A, (int)(i >> 6), (int)(i & 63));
+  const bool live = lane < A.tpw && t < A.ntarget;
   if(live && A.order) t = A.order[t];
   const size_t tk = live ? (size_t)t * A.X.stride : 0;
   const double px = live ? A.X.x[tk] : 0, py = live ? A.X.y[tk] : 0, pz = live ? A.X.z[tk] : 0;
@@ -960,6 +964,12 @@ __global__ void __launch_bounds__(64) k_walk32g(WalkArgs A) {
   }
 }
 
+// Waves of a per-target walk below which a wave takes fewer than 64 targets: one a SIMD.  Scattered
+// targets, 2e5 sources, FP64, the walk: 64 targets in one wave 23.8 ms, one a wave 2.7 (a lane each on
+// its own path: 6.3); 16000 in 250 waves 5.9, 1000 waves 4.0, 2000 4.8, 4000 6.7; 65000 in 1016
+// waves 5.1, 2032 4.8, 4064 5.6.
+constexpr int kWalkWaves = 1024;
+
 // Walk of ntarget targets (device SoA) through T; the results are scaled by G (gravity_tree
 // multiplies the walk's sums by G afterwards, gravtree.c:455-463).
 // blk_nb > 0: the targets are table nodes (section, z, R) of blk_nb x blk_nb grids, which a wave
@@ -1014,12 +1024,15 @@ int tree_walk_dev(const galic_params *p, hipStream_t st, DevBufs &B, const Tree 
     // table nodes in 8 x 8 blocks; other targets as they come in the group walk, whose groups are
     // the caller's, and in Morton order where each target walks for itself
     const bool blk = blk_nb > 0 && blk_nb % 8 == 0 && (long long)ntarget % ((long long)blk_nb * blk_nb) == 0;
-    const dim3 grid((unsigned int)(((long long)ntarget + 63) / 64)), block(64);
     W.blk_nb = blk ? blk_nb : 0;
+    W.tpw = 64;
+    if(!(precision & GALIC_TREE_GROUP))
+      while(W.tpw > 1 && ntarget / W.tpw < kWalkWaves) W.tpw /= 2;
+    const dim3 grid((unsigned int)(((long long)ntarget + W.tpw - 1) / W.tpw)), block(64);
     if(precision & GALIC_TREE_GROUP) {
       hipLaunchKernelGGL(k_walk32g, grid, block, 0, st, W);
     } else {
-      if(!blk && ntarget > 64) {
+      if(!blk && W.tpw > 1) {
         unsigned long long *k0 = nullptr, *k1 = nullptr;
         int *i0 = nullptr, *i1 = nullptr;
         char *tmp = nullptr;

@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 from galic_amd import model
-from galic_amd.runtime import TREE_FP32, TREE_GROUP, TREE_PLUMMER, TREE_QUADRUPOLE, direct_forces, tree_forces
+from galic_amd.runtime import TREE_FP32, TREE_GROUP, TREE_PLUMMER, TREE_QUADRUPOLE, direct_forces, tree_fill, tree_forces
 
 pytestmark = pytest.mark.gpu
 
@@ -113,3 +113,39 @@ def test_tree_of_close_pairs_equals_direct_summation(npair):
     da, dp = direct_forces(p, pos, mass, t)
     np.testing.assert_allclose(acc, da, rtol=1e-12, atol=1e-12 * np.abs(da).max())
     np.testing.assert_allclose(pot, dp, rtol=1e-12)
+
+
+# one target a wave up to 2047; two, four, 32, 64 from there on (the first and last count of each)
+@pytest.mark.parametrize("ntarget", [2047, 2048, 4097, 65535, 65537])
+@pytest.mark.parametrize("mode", [0, TREE_FP32 | TREE_QUADRUPOLE | TREE_PLUMMER])
+def test_targets_do_not_depend_on_their_wave(mode, ntarget):
+    p = model.make_params(model.config("composite-4e6"))
+    pos, mass = sources(p, 1500)
+    rng = np.random.default_rng(ntarget)
+    t = pos[rng.integers(0, len(pos), ntarget)] * rng.uniform(0.1, 0.9, (ntarget, 1))   # the domain cube is the sources'
+    print(f"[gpu] targets a wave mode={mode} ntarget={ntarget}", flush=True)
+    acc, pot, _ = tree_forces(p, pos, mass, t, precision=mode)
+    pick = np.unique(np.concatenate([np.arange(70), ntarget - 1 - np.arange(70), rng.integers(0, ntarget, 300)]))
+    a1, p1, _ = tree_forces(p, pos, mass, t[pick], precision=mode)
+    assert np.array_equal(acc[pick], a1) and np.array_equal(pot[pick], p1)
+
+
+# waves of 1, 2, 4, 8 and 32 table nodes of an 8 x 8 block
+@pytest.mark.parametrize("nb", [8, 16, 24, 32, 64])
+def test_small_fill_equals_forces_at_its_nodes(nb):
+    """The nodes' places differ by the rounding of cos and sin, the sums over sections by theirs: 1e-12."""
+    p = model.make_params(model.config("composite-4e6", fg_nbin=nb))
+    pos, mass = sources(p, 1500)
+    pot, dr, dz, n = tree_fill(p, pos, mass)
+    phi = 2 * np.pi / 8 * np.arange(8)
+    r = p.FG_Rmin * (p.FG_Fac ** np.arange(nb) - 1.0)
+    s, k, j = np.meshgrid(np.arange(8), np.arange(nb), np.arange(nb), indexing="ij")
+    t = np.stack([r[j] * np.cos(phi[s]), r[j] * np.sin(phi[s]), r[k]], axis=-1).reshape(-1, 3)
+    acc, pt, nf = tree_forces(p, pos, mass, t)
+    assert nf == n
+    acc, pt = acc.reshape(8, nb * nb, 3), pt.reshape(8, nb * nb)
+    np.testing.assert_allclose(pot, pt.mean(axis=0), rtol=1e-12)
+    rad = acc[:, :, 0] * np.cos(phi)[:, None] + acc[:, :, 1] * np.sin(phi)[:, None]
+    scale = np.abs(acc).max(axis=(0, 2))
+    assert (np.abs(dr - rad.mean(axis=0)) <= 1e-12 * scale).all()
+    assert (np.abs(dz - acc[:, :, 2].mean(axis=0)) <= 1e-12 * scale).all()
