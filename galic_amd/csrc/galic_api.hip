@@ -529,9 +529,9 @@ double log_blocks_slack(const galic::Ctx &c, int n) {
 // little since the arena was allocated still goes out as one launch: two launches last twice as
 // long as their longest orbits.  The first estimate, from the orbits' steps at their start points, is
 // up to a third too low (512^2 grids: 53 blocks an orbit, 71 counted), and the first arena is sized
-// for it, so that the second pass keeps it.  No larger: device memory
-// that was freed before costs 25 ms a GB and more when it is taken again (5e4 particles on 512^2
-// grids, 27 GB: a first pass 95 ms in fresh memory, 700 in recycled).
+// for it, so that the second pass keeps it.  No larger: device memory that was freed before costs 25
+// ms a GB and more when it is taken again (5e4 particles on 512^2 grids, 27 GB: a first pass 95 ms
+// in fresh memory, 700 in recycled).
 constexpr double kLogPlanMargin = 1.2, kLogFitMargin = 1.06, kLogFirstMargin = 1.25;
 double log_blocks_planned(const galic::Ctx &c, int n, double margin = kLogPlanMargin) {
   return (double)n * c.log_est_blocks * margin + log_blocks_slack(c, n);
